@@ -93,66 +93,7 @@ __device__ __forceinline__ float closure_feature(const DevCtx *__restrict__ x, c
   return A3(h == 0 ? fd : fn, ii, kk, jj);
 }
 
-// ---------------------------------------------------------------------------
-// network forward over 16 rows: A rows (bf16, k-contiguous, stride kLd) in
-// LDS -> z per row into zout[16] (LDS).  H (bf16 [16][72]) is LDS scratch;
-// W1, W2 rows (one per output unit) have stride ldw (64 in global memory,
-// kLd in LDS).
-// ---------------------------------------------------------------------------
 constexpr int kLd = 72;  // LDS row stride of bf16 tiles (64 + 8: no bank conflicts on the 16-byte reads)
-
-__device__ __forceinline__ void mlp_rows16(const __bf16 *Xs, const __bf16 *w1, const __bf16 *w2, int ldw, const float *theta,
-                                           __bf16 *Hs, float *P1, float *P2, float *zout) {
-  const int l = threadIdx.x & 63;
-  const int col = l & 15, rb = (l >> 4) * 4;
-  // layer 1
-#pragma unroll
-  for (int t = 0; t < 4; t++) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mma16(Xs, kLd, w1 + (t * 16) * ldw, ldw, acc);
-    acc = mma16(Xs + 32, kLd, w1 + (t * 16) * ldw + 32, ldw, acc);
-    const int o = t * 16 + col;
-    const float b = theta[kOffB1 + o];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const float pre = acc[r] + b;
-      if (P1) P1[(rb + r) * 64 + o] = pre;
-      Hs[(rb + r) * kLd + o] = (__bf16)silu_f(pre);
-    }
-  }
-  __syncthreads();
-  // layer 2 and the output layer
-  float zpart[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int t = 0; t < 4; t++) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mma16(Hs, kLd, w2 + (t * 16) * ldw, ldw, acc);
-    acc = mma16(Hs + 32, kLd, w2 + (t * 16) * ldw + 32, ldw, acc);
-    const int o = t * 16 + col;
-    const float b = theta[kOffB2 + o], w3 = theta[kOffW3 + o];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const float pre = acc[r] + b;
-      if (P2) P2[(rb + r) * 64 + o] = pre;
-      zpart[r] += silu_f(pre) * w3;
-    }
-  }
-  // sum over the 16 lanes that hold the same rows (lane bits 0..3)
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    float v = zpart[r];
-    v += __shfl_xor(v, 1);
-    v += __shfl_xor(v, 2);
-    v += __shfl_xor(v, 4);
-    v += __shfl_xor(v, 8);
-    zpart[r] = v;
-  }
-  if (col == 0) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) zout[rb + r] = zpart[r] + theta[kOffB3];
-  }
-  __syncthreads();
-}
 
 // ---------------------------------------------------------------------------
 // smag2d_km with the learned km: one wave per 64 points (64 i of one level
@@ -401,160 +342,254 @@ __global__ void __launch_bounds__(256) k_coarse_grain(CoarseList L) {
 }
 
 // ---------------------------------------------------------------------------
-// training: forward, loss and backward over rows, one wave per block; each
-// wave loops over chunks of 32 rows and accumulates its gradient, written as
-// one partial (kMlpParams + 1 floats: gradient, then the loss sum) per block.
-// Loss of a row: ((t1 + K s1)^2 + (t2 + K s2)^2) * lossnorm with
-// K = kref * softplus(z) / divisor.  BACKWARD false: forward only, z -> out.
+// training: forward, loss and backward over rows.  A block of four waves
+// works on chunks of 32 rows together: the 2 x 4 output tiles of a layer are
+// two per wave, the 4 x 4 tiles of each weight gradient four per wave (kept
+// in accumulators over the block's chunks), the sums over rows eight rows
+// per wave.  The gradient of a block is one partial (kMlpParams + 1 floats:
+// gradient, then the loss sum).  Loss of a row: ((t1 + K s1)^2 +
+// (t2 + K s2)^2) * lossnorm with K = kref * softplus(z) / divisor.
+// BACKWARD false: forward only, z -> out.
+//
+// A chunk is a chain of small matrix products with a barrier between them,
+// so a minibatch is bound by latency: how many chunks run after one another
+// and how long each takes.  The chunks go one to a block until the chip's
+// resident blocks are used (mlp_blocks).  4096 rows, forward, backward and
+// reduction: 116 us a step with one wave per block and 8 chunks after one another
+// (16 waves in flight on 1024 SIMDs), 14 us this way (10.8 + 4.1 in the kernels).
 // ---------------------------------------------------------------------------
 constexpr int kChunk = 32;
 constexpr int kLdT = 40;  // LDS stride of transposed [64][32] tiles
+constexpr int kLdP = 68;  // LDS stride of the FP32 pre-activations (the four row groups of a C tile on different banks)
+// blocks of the training kernel: two of 77 KB of LDS fit a CU, so more than
+// 512 would only queue, and each adds a partial for the reduction to read
+constexpr int kMlpMaxBlocks = 512;
+constexpr int kMlpForwardBlocks = 2048;  // forward only: 29 KB of LDS, five blocks to a CU
+__host__ inline long long mlp_blocks(long long nrows) {
+  const long long chunks = (nrows + kChunk - 1) / kChunk;
+  return chunks < kMlpMaxBlocks ? chunks : kMlpMaxBlocks;
+}
+
+// rows of one layer's tiles of this wave: C[32 x 64] = A[32 x 64] B^T, the
+// row tile wv & 1 and the column tiles 2 (wv >> 1) + {0, 1}
+__device__ __forceinline__ f32x4 mlp_tile(const __bf16 *A, const __bf16 *Bt, int rt, int ct) {
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  acc = mma16(A + rt * 16 * kLd, kLd, Bt + ct * 16 * kLd, kLd, acc);
+  return mma16(A + rt * 16 * kLd + 32, kLd, Bt + ct * 16 * kLd + 32, kLd, acc);
+}
 
 template <bool BACKWARD>
-__global__ void __launch_bounds__(64) k_mlp_train(const float *__restrict__ theta, const __bf16 *__restrict__ wbf, const __bf16 *__restrict__ X,
-                                                  const float *__restrict__ T, long long n, float lossnorm, float kref, int chunks_per_block,
-                                                  float *__restrict__ out) {
-  __shared__ __align__(16) __bf16 s_w[3][64 * kLd];  // W1, W2, W2^T
+__global__ void __launch_bounds__(256) k_mlp_train(const float *__restrict__ theta, const __bf16 *__restrict__ wbf, const __bf16 *__restrict__ X,
+                                                   const float *__restrict__ T, long long n, float lossnorm, float kref,
+                                                   float *__restrict__ out) {
+  __shared__ __align__(16) __bf16 s_w[BACKWARD ? 3 : 2][64 * kLd];  // W1, W2, W2^T
   __shared__ __align__(16) __bf16 s_x[kChunk * kLd];
-  __shared__ __align__(16) __bf16 s_xt[64 * kLdT];
   __shared__ __align__(16) __bf16 s_h1[kChunk * kLd];
-  __shared__ __align__(16) __bf16 s_h1t[64 * kLdT];
-  __shared__ __align__(16) __bf16 s_d2[kChunk * kLd];
-  __shared__ __align__(16) __bf16 s_d2t[64 * kLdT];
-  __shared__ __align__(16) __bf16 s_d1t[64 * kLdT];
-  __shared__ float s_p1[kChunk * 64];
-  __shared__ float s_p2[kChunk * 64];
-  __shared__ float s_z[kChunk];
+  __shared__ __align__(16) __bf16 s_xt[BACKWARD ? 64 * kLdT : 8];
+  __shared__ __align__(16) __bf16 s_h1t[BACKWARD ? 64 * kLdT : 8];
+  __shared__ __align__(16) __bf16 s_d2[BACKWARD ? kChunk * kLd : 8];
+  __shared__ __align__(16) __bf16 s_d2t[BACKWARD ? 64 * kLdT : 8];
+  __shared__ __align__(16) __bf16 s_d1t[BACKWARD ? 64 * kLdT : 8];
+  __shared__ float s_p1[BACKWARD ? kChunk * kLdP : 1];
+  __shared__ float s_p2[BACKWARD ? kChunk * kLdP : 1];
+  __shared__ float s_z[2][kChunk];  // the two column halves' share of z
   __shared__ float s_dz[kChunk];
-  const int l = threadIdx.x;
-  for (int m = 0; m < 3; m++)
-    for (int e = l; e < 64 * 64; e += 64) s_w[m][(e / 64) * kLd + e % 64] = wbf[m * 4096 + e];
-  __syncthreads();
+  __shared__ float s_red[BACKWARD ? 3 : 1][4][64];
+  const int t = threadIdx.x, l = t & 63, wv = t >> 6;
   const int col = l & 15, rb = (l >> 4) * 4;
-  f32x4 gw1[4][4], gw2[4][4];
+  const int rt = wv & 1, ch = wv >> 1;  // this wave's row tile and column half of a layer
+  // 16-byte pieces where the caller's pointers allow it (rows are 128 bytes)
+  const bool wide_w = ((uintptr_t)wbf & 15) == 0, wide_x = ((uintptr_t)X & 15) == 0;
+  for (int e = t; e < (BACKWARD ? 3 : 2) * 512; e += 256) {
+    const int m = e >> 9, row = (e >> 3) & 63, c = e & 7;
+    bf16x8 v;
+    if (wide_w) v = *reinterpret_cast<const bf16x8 *>(wbf + m * 4096 + row * 64 + c * 8);
+    else
+      for (int q = 0; q < 8; q++) v[q] = wbf[m * 4096 + row * 64 + c * 8 + q];
+    *reinterpret_cast<bf16x8 *>(&s_w[m][row * kLd + c * 8]) = v;
+  }
+  float b1[2], b2[2], w3c[2];
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+  for (int q = 0; q < 2; q++) {
+    const int o = (2 * ch + q) * 16 + col;
+    b1[q] = theta[kOffB1 + o];
+    b2[q] = theta[kOffB2 + o];
+    w3c[q] = theta[kOffW3 + o];
+  }
+  const float b3 = theta[kOffB3], w3 = theta[kOffW3 + l];
+  f32x4 gw1[4], gw2[4];  // rows 16 wv .. + 15 of dW1 and dW2
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-      gw1[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-      gw2[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-  float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, loss = 0.f;  // lane l: hidden unit l
-  for (int c = 0; c < chunks_per_block; c++) {
-    const long long r0 = ((long long)blockIdx.x * chunks_per_block + c) * kChunk;
-    if (r0 >= n) break;
-    // rows of the chunk (rows past n are zero and carry no loss)
-    for (int e = l; e < kChunk * kMlpIn; e += 64) {
-      const int p = e / kMlpIn, f = e % kMlpIn;
-      const __bf16 v = (r0 + p < n) ? X[(r0 + p) * kMlpIn + f] : (__bf16)0.f;
-      s_x[p * kLd + f] = v;
-      s_xt[f * kLdT + p] = v;
+  for (int b = 0; b < 4; b++) gw1[b] = gw2[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, loss = 0.f;  // hidden unit l, rows 8 wv .. + 7 of every chunk
+  const long long chunks = (n + kChunk - 1) / kChunk;
+  for (long long c = blockIdx.x; c < chunks; c += gridDim.x) {
+    const long long r0 = c * kChunk;
+    {  // rows of the chunk (rows past n are zero and carry no loss)
+      const int p = t >> 3, f = (t & 7) * 8;
+      bf16x8 v;
+#pragma unroll
+      for (int q = 0; q < 8; q++) v[q] = (__bf16)0.f;
+      if (r0 + p < n) {
+        const __bf16 *src = X + (r0 + p) * kMlpIn + f;
+        if (wide_x) v = *reinterpret_cast<const bf16x8 *>(src);
+        else
+          for (int q = 0; q < 8; q++) v[q] = src[q];
+      }
+      *reinterpret_cast<bf16x8 *>(&s_x[p * kLd + f]) = v;
+      if (BACKWARD) {
+#pragma unroll
+        for (int q = 0; q < 8; q++) s_xt[(f + q) * kLdT + p] = v[q];
+      }
     }
     __syncthreads();
-    mlp_rows16(s_x, s_w[0], s_w[1], kLd, theta, s_h1, s_p1, s_p2, s_z);
-    mlp_rows16(s_x + 16 * kLd, s_w[0], s_w[1], kLd, theta, s_h1 + 16 * kLd, s_p1 + 16 * 64, s_p2 + 16 * 64, s_z + 16);
+    // layer 1
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      const int ct = 2 * ch + q, o = ct * 16 + col;
+      const f32x4 acc = mlp_tile(s_x, s_w[0], rt, ct);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int p = rt * 16 + rb + r;
+        const float pre = acc[r] + b1[q];
+        if (BACKWARD) s_p1[p * kLdP + o] = pre;
+        s_h1[p * kLd + o] = (__bf16)silu_f(pre);
+      }
+    }
+    __syncthreads();
+    // layer 2 and the output layer's share of these columns
+    float zp[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      const int ct = 2 * ch + q, o = ct * 16 + col;
+      const f32x4 acc = mlp_tile(s_h1, s_w[1], rt, ct);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float pre = acc[r] + b2[q];
+        if (BACKWARD) s_p2[(rt * 16 + rb + r) * kLdP + o] = pre;
+        zp[r] += silu_f(pre) * w3c[q];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {  // over the 16 lanes that hold the same row
+      float v = zp[r];
+      v += __shfl_xor(v, 1);
+      v += __shfl_xor(v, 2);
+      v += __shfl_xor(v, 4);
+      v += __shfl_xor(v, 8);
+      if (col == 0) s_z[ch][rt * 16 + rb + r] = v;
+    }
+    __syncthreads();
+    if (t < kChunk) {
+      const float z = (s_z[0][t] + s_z[1][t]) + b3;
+      if (!BACKWARD) {
+        if (r0 + t < n) out[r0 + t] = z;
+      } else {  // loss and dL/dz of each row
+        float dz = 0.f;
+        if (r0 + t < n) {
+          const float *tg = T + (r0 + t) * kTargetCols;
+          const float div = tg[4];
+          const float K = kref * softplus_f(z) / div;
+          const float r1 = tg[0] + K * tg[2], r2 = tg[1] + K * tg[3];
+          loss += (r1 * r1 + r2 * r2) * lossnorm;
+          const float dK = 2.f * (r1 * tg[2] + r2 * tg[3]) * lossnorm;
+          dz = dK * kref * sigmoid_f(z) / div;
+        }
+        s_dz[t] = dz;
+      }
+    }
     if (!BACKWARD) {
-      if (l < kChunk && r0 + l < n) out[r0 + l] = s_z[l];
-      __syncthreads();
+      __syncthreads();  // the next chunk overwrites s_x, s_h1 and s_z
       continue;
     }
-    // loss and dL/dz of each row
-    if (l < kChunk) {
-      float dz = 0.f;
-      if (r0 + l < n) {
-        const float *t = T + (r0 + l) * kTargetCols;
-        const float z = s_z[l], div = t[4];
-        const float K = kref * softplus_f(z) / div;
-        const float r1 = t[0] + K * t[2], r2 = t[1] + K * t[3];
-        loss += (r1 * r1 + r2 * r2) * lossnorm;
-        const float dK = 2.f * (r1 * t[2] + r2 * t[3]) * lossnorm;
-        dz = dK * kref * sigmoid_f(z) / div;
-      }
-      s_dz[l] = dz;
-    }
     __syncthreads();
-    // output layer and dL/dpre2 (lane l: hidden unit l, all rows)
-    {
-      const float w3 = theta[kOffW3 + l];
-      for (int p = 0; p < kChunk; p++) {
-        const float pre = s_p2[p * 64 + l], s = sigmoid_f(pre), h = pre * s;
-        const float dz = s_dz[p];
-        gw3 += dz * h;
-        const float d2 = dz * w3 * (s + pre * s * (1.f - s));
-        gb2 += d2;
-        const __bf16 d2b = (__bf16)d2;
-        s_d2[p * kLd + l] = d2b;
-        s_d2t[l * kLdT + p] = d2b;
-        s_h1t[l * kLdT + p] = s_h1[p * kLd + l];
-      }
-      if (l == 0)
-        for (int p = 0; p < kChunk; p++) gb3 += s_dz[p];
+    // output layer and dL/dpre2 (hidden unit l, rows 8 wv .. + 7)
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int p = 8 * wv + q;
+      const float pre = s_p2[p * kLdP + l], s = sigmoid_f(pre), h = pre * s;
+      const float dz = s_dz[p];
+      gw3 += dz * h;
+      const float d2 = dz * w3 * (s + pre * s * (1.f - s));
+      gb2 += d2;
+      const __bf16 d2b = (__bf16)d2;
+      s_d2[p * kLd + l] = d2b;
+      s_d2t[l * kLdT + p] = d2b;
+      s_h1t[l * kLdT + p] = s_h1[p * kLd + l];
+      if (l == 0) gb3 += dz;
     }
     __syncthreads();
     // dW2[o][i] += sum_p d2[p][o] h1[p][i]
 #pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-      for (int b = 0; b < 4; b++) gw2[a][b] = mma16(s_d2t + a * 16 * kLdT, kLdT, s_h1t + b * 16 * kLdT, kLdT, gw2[a][b]);
+    for (int b = 0; b < 4; b++) gw2[b] = mma16(s_d2t + wv * 16 * kLdT, kLdT, s_h1t + b * 16 * kLdT, kLdT, gw2[b]);
     // dh1[p][i] = sum_o d2[p][o] W2[o][i], then dL/dpre1
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
+    for (int q = 0; q < 2; q++) {
+      const int ct = 2 * ch + q, ihid = ct * 16 + col;
+      const f32x4 acc = mlp_tile(s_d2, s_w[BACKWARD ? 2 : 0], rt, ct);
 #pragma unroll
-      for (int b = 0; b < 4; b++) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mma16(s_d2 + h * 16 * kLd, kLd, s_w[2] + b * 16 * kLd, kLd, acc);
-        acc = mma16(s_d2 + h * 16 * kLd + 32, kLd, s_w[2] + b * 16 * kLd + 32, kLd, acc);
-        const int ihid = b * 16 + col;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int p = h * 16 + rb + r;
-          const float pre = s_p1[p * 64 + ihid], s = sigmoid_f(pre);
-          s_d1t[ihid * kLdT + p] = (__bf16)(acc[r] * (s + pre * s * (1.f - s)));
-        }
+      for (int r = 0; r < 4; r++) {
+        const int p = rt * 16 + rb + r;
+        const float pre = s_p1[p * kLdP + ihid], s = sigmoid_f(pre);
+        s_d1t[ihid * kLdT + p] = (__bf16)(acc[r] * (s + pre * s * (1.f - s)));
       }
     }
     __syncthreads();
-    for (int p = 0; p < kChunk; p++) gb1 += (float)s_d1t[l * kLdT + p];
-    // dW1[i][f] += sum_p d1[p][i] x[p][f]
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+    for (int q = 0; q < 8; q++) gb1 += (float)s_d1t[l * kLdT + 8 * wv + q];
+    // dW1[o][f] += sum_p d1[p][o] x[p][f]
 #pragma unroll
-      for (int b = 0; b < 4; b++) gw1[a][b] = mma16(s_d1t + a * 16 * kLdT, kLdT, s_xt + b * 16 * kLdT, kLdT, gw1[a][b]);
+    for (int b = 0; b < 4; b++) gw1[b] = mma16(s_d1t + wv * 16 * kLdT, kLdT, s_xt + b * 16 * kLdT, kLdT, gw1[b]);
     __syncthreads();
   }
   if (!BACKWARD) return;
   float *g = out + (size_t)blockIdx.x * (kMlpParams + 1);
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+  for (int b = 0; b < 4; b++)
 #pragma unroll
-    for (int b = 0; b < 4; b++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = a * 16 + rb + r, cc = b * 16 + col;
-        g[kOffW1 + row * 64 + cc] = gw1[a][b][r];
-        g[kOffW2 + row * 64 + cc] = gw2[a][b][r];
-      }
-  g[kOffB1 + l] = gb1;
-  g[kOffB2 + l] = gb2;
-  g[kOffW3 + l] = gw3;
-  // the loss of the rows is spread over lanes 0..31: sum it
-  float ls = loss;
-  for (int off = 32; off > 0; off >>= 1) ls += __shfl_xor(ls, off);
-  if (l == 0) {
-    g[kOffB3] = gb3;
-    g[kMlpParams] = ls;
+    for (int r = 0; r < 4; r++) {
+      const int row = wv * 16 + rb + r, cc = b * 16 + col;
+      g[kOffW1 + row * 64 + cc] = gw1[b][r];
+      g[kOffW2 + row * 64 + cc] = gw2[b][r];
+    }
+  s_red[0][wv][l] = gb1;
+  s_red[1][wv][l] = gb2;
+  s_red[2][wv][l] = gw3;
+  if (l == 0) s_z[0][wv] = gb3;
+  __syncthreads();
+  if (wv < 3) {
+    const float sum = ((s_red[wv][0][l] + s_red[wv][1][l]) + s_red[wv][2][l]) + s_red[wv][3][l];
+    g[(wv == 0 ? kOffB1 : wv == 1 ? kOffB2 : kOffW3) + l] = sum;
+  }
+  // the loss of the rows is spread over lanes 0..31 of wave 0: sum it
+  if (wv == 0) {
+    float ls = loss;
+    for (int off = 32; off > 0; off >>= 1) ls += __shfl_xor(ls, off);
+    if (l == 0) {
+      g[kOffB3] = ((s_z[0][0] + s_z[0][1]) + s_z[0][2]) + s_z[0][3];
+      g[kMlpParams] = ls;
+    }
   }
 }
 
 // Sum of the per-block partials (fixed order), then the gradient out and,
 // with adam != 0, one Adam step on theta and fresh bf16 weight copies.
-// One thread per parameter (and one for the loss).
-__global__ void __launch_bounds__(256) k_mlp_reduce(const float *__restrict__ part, int nblocks, float *grad, float *loss, float *theta,
-                                                    float *m, float *v, __bf16 *wbf, int adam, int step, float lr) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > kMlpParams) return;
+// Block (64, 16): 64 parameters (the last one the loss), the partials dealt
+// over the 16 waves, so a thread has 1/16 of them to wait for.
+constexpr int kReduceWaves = 16;
+__global__ void __launch_bounds__(64 * kReduceWaves) k_mlp_reduce(const float *__restrict__ part, int nblocks, float *grad, float *loss,
+                                                                  float *theta, float *m, float *v, __bf16 *wbf, int adam, int step, float lr) {
+  __shared__ float s_s[kReduceWaves][64];
+  const int l = threadIdx.x, wv = threadIdx.y;
+  const int p = (int)blockIdx.x * 64 + l;
   float s = 0.f;
-  for (int b = 0; b < nblocks; b++) s += part[(size_t)b * (kMlpParams + 1) + p];
+  if (p <= kMlpParams) {
+#pragma unroll 8
+    for (int b = wv; b < nblocks; b += kReduceWaves) s += part[(size_t)b * (kMlpParams + 1) + p];
+  }
+  s_s[wv][l] = s;
+  __syncthreads();
+  if (wv != 0 || p > kMlpParams) return;
+  for (int w = 1; w < kReduceWaves; w++) s += s_s[w][l];
   if (p == kMlpParams) {
     if (loss) *loss = s;
     return;

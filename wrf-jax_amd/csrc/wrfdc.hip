@@ -1912,12 +1912,10 @@ static int mlp_err(hipError_t e, const char *what) {
   if (e == hipSuccess) return WRFDC_OK;
   return set_err(nullptr, WRFDC_EHIP, std::string(what) + ": " + hipGetErrorString(e));
 }
-constexpr int kMlpChunksPerBlock = 8;  // 256 rows per block of the training kernel
 
 long long wrfdc_mlp_work_floats(long long nrows) {
   if (nrows < 0) return -1;
-  const long long rows_per_block = (long long)kMlpChunksPerBlock * kChunk;
-  return ((nrows + rows_per_block - 1) / rows_per_block) * (long long)(kMlpParams + 1);
+  return mlp_blocks(nrows) * (long long)(kMlpParams + 1);
 }
 
 int wrfdc_mlp_pack(const float *theta, void *wbf, void *stream) {
@@ -1932,15 +1930,14 @@ static int mlp_pass(const float *theta, const void *wbf, const void *rows_x, con
     return set_err(nullptr, WRFDC_EINVAL, "theta, wbf, rows and work must not be null and nrows > 0");
   if (!(kref > 0.f)) return set_err(nullptr, WRFDC_EINVAL, "kref must be > 0");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const long long rows_per_block = (long long)kMlpChunksPerBlock * kChunk;
-  const long long nb = (nrows + rows_per_block - 1) / rows_per_block;
-  if (nb > (1LL << 30)) return set_err(nullptr, WRFDC_EINVAL, "too many rows");
-  k_mlp_train<true><<<(unsigned)nb, 64, 0, s>>>(theta, static_cast<const __bf16 *>(wbf), static_cast<const __bf16 *>(rows_x), rows_t, nrows, lossnorm,
-                                                 kref, kMlpChunksPerBlock, work);
+  if (nrows > (1LL << 38)) return set_err(nullptr, WRFDC_EINVAL, "too many rows");
+  const long long nb = mlp_blocks(nrows);
+  k_mlp_train<true><<<(unsigned)nb, 256, 0, s>>>(theta, static_cast<const __bf16 *>(wbf), static_cast<const __bf16 *>(rows_x), rows_t, nrows, lossnorm,
+                                                 kref, work);
   int rc = mlp_err(hipGetLastError(), "k_mlp_train");
   if (rc != WRFDC_OK) return rc;
   const int adam = m != nullptr;
-  k_mlp_reduce<<<(kMlpParams + 1 + 255) / 256, 256, 0, s>>>(work, (int)nb, grad, loss, const_cast<float *>(theta), m, v,
+  k_mlp_reduce<<<(kMlpParams + 1 + 63) / 64, dim3(64, kReduceWaves), 0, s>>>(work, (int)nb, grad, loss, const_cast<float *>(theta), m, v,
                                                              const_cast<__bf16 *>(static_cast<const __bf16 *>(wbf)), adam, step, lr);
   return mlp_err(hipGetLastError(), "k_mlp_reduce");
 }
@@ -1959,11 +1956,9 @@ int wrfdc_mlp_train_step(float *theta, void *wbf, const void *rows_x, const floa
 
 int wrfdc_mlp_forward(const float *theta, const void *wbf, const void *rows_x, long long nrows, float *z, void *stream) {
   if (!theta || !wbf || !rows_x || !z || nrows <= 0) return set_err(nullptr, WRFDC_EINVAL, "theta, wbf, rows_x and z must not be null");
-  const long long rows_per_block = (long long)kMlpChunksPerBlock * kChunk;
-  const long long nb = (nrows + rows_per_block - 1) / rows_per_block;
-  k_mlp_train<false><<<(unsigned)nb, 64, 0, static_cast<hipStream_t>(stream)>>>(theta, static_cast<const __bf16 *>(wbf),
-                                                                              static_cast<const __bf16 *>(rows_x), nullptr, nrows, 0.f, 1.f,
-                                                                              kMlpChunksPerBlock, z);
+  const long long nb = std::min<long long>((nrows + kChunk - 1) / kChunk, kMlpForwardBlocks);
+  k_mlp_train<false><<<(unsigned)nb, 256, 0, static_cast<hipStream_t>(stream)>>>(theta, static_cast<const __bf16 *>(wbf),
+                                                                               static_cast<const __bf16 *>(rows_x), nullptr, nrows, 0.f, 1.f, z);
   return mlp_err(hipGetLastError(), "k_mlp_train<forward>");
 }
 
