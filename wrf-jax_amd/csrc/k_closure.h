@@ -394,7 +394,7 @@ __global__ void __launch_bounds__(256) k_mlp_train(const float *__restrict__ the
   __shared__ float s_p2[BACKWARD ? kChunk * kLdP : 1];
   __shared__ float s_z[2][kChunk];  // the two column halves' share of z
   __shared__ float s_dz[kChunk];
-  __shared__ float s_red[BACKWARD ? 3 : 1][4][64];
+  float(*s_red)[4][64] = reinterpret_cast<float(*)[4][64]>(s_p1);  // [3][4][64], after the last chunk
   const int t = threadIdx.x, l = t & 63, wv = t >> 6;
   const int col = l & 15, rb = (l >> 4) * 4;
   const int rt = wv & 1, ch = wv >> 1;  // this wave's row tile and column half of a layer
