@@ -81,18 +81,6 @@ __global__ void k_closure_feat(const DevCtx xv, R3 r, ClosureNorm nm, const floa
   A3(fn, i, k, j) = (A3(FL(bn2), i, k, j) - nm.n_shift) / nm.n_scale;
 }
 
-// input slot f of the point (i, k, j) (the slot order above); stencil
-// neighbours outside the range take the nearest point of it
-__device__ __forceinline__ float closure_feature(const DevCtx *__restrict__ x, const float *fd, const float *fn, const ClosureNorm &nm,
-                                                 int i, int k, int j, int f) {
-  const int h = f >> 5, g = f & 31;
-  if (g == 27) return h == 0 ? nm.dx_feature : 0.f;
-  if (g > 27) return 0.f;
-  const int di = g % 3 - 1, dk = (g / 3) % 3 - 1, dj = g / 9 - 1;
-  const int ii = clampi(i + di, 2, x->ide - 2), kk = clampi(k + dk, 1, x->kde - 1), jj = clampi(j + dj, 2, x->jde - 2);
-  return A3(h == 0 ? fd : fn, ii, kk, jj);
-}
-
 constexpr int kLd = 72;  // LDS row stride of bf16 tiles (64 + 8: no bank conflicts on the 16-byte reads)
 
 // ---------------------------------------------------------------------------
@@ -237,21 +225,65 @@ __global__ void __launch_bounds__(256) k_closure_km(const DevCtx xv, R3 r, const
 // target columns s1, s2, divisor, Smagorinsky km of every point of the
 // smag range, row = ((j-2)*nk + (k-1))*ni + (i-2).  t1, t2 come from
 // k_subgrid_stress.
+//
+// The rows of a wave's 64 points are 8 KB of consecutive memory, written a
+// kilobyte at a time: lane l forms the 16-byte piece l%8 (input slots 8*(l%8)
+// .. + 7, so 8 stencil points of one of the two inputs) of point 8*q + l/8.
+// With a row per lane, in 64 two-byte stores 128 bytes apart, the kernel took
+// 254 us for 96x96x40 (353440 rows, 54 MB), 30 us this way.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_closure_rows(const DevCtx xv, R3 r, ClosureNorm nm, const float *__restrict__ fd,
                                                       const float *__restrict__ fn, const float *__restrict__ divisor, __bf16 *X, float *T) {
   const DevCtx *__restrict__ x = &xv;
-  GET_IKJ_P(r);
+  // the tiles of GET_IKJ_P, with the wave's lanes shared out over its points
+  const int ib = 1 + ((r.i0 - 1) & ~63);
+  const unsigned gx_ = (unsigned)(r.i1 - ib + 64) / 64u;
+  const unsigned gy_ = (unsigned)(r.k1 - r.k0 + 4) / 4u;
+  const int i0 = ib + (int)((blockIdx.x % gx_) * 64u), l = (int)threadIdx.x;
+  const int k = r.k0 + (int)(((blockIdx.x / gx_) % gy_) * 4u + wave_y());
+  const int j = r.j0 + (int)(blockIdx.x / (gx_ * gy_));
+  if (k > r.k1 || j > r.j1) return;
   const int ni = r.i1 - r.i0 + 1, nk = r.k1 - r.k0 + 1;
-  const size_t row = ((size_t)(j - r.j0) * nk + (size_t)(k - r.k0)) * ni + (size_t)(i - r.i0);
-  for (int f = 0; f < kMlpIn; f++) X[row * kMlpIn + f] = (__bf16)closure_feature(x, fd, fn, nm, i, k, j, f);
+  const size_t line = ((size_t)(j - r.j0) * nk + (size_t)(k - r.k0)) * ni;  // the row of point r.i0
+  const bool wide = ((uintptr_t)X & 15) == 0;
+  const int c = l & 7;
+  const float *f = c < 4 ? fd : fn;
+  unsigned koff[8];
+  int dis[8];
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int sp = 8 * (c & 3) + q, g = sp < 27 ? sp : 13;
+    const int di = g % 3 - 1, dk = (g / 3) % 3 - 1, dj = g / 9 - 1;
+    koff[q] = XI3(1, clampi(k + dk, 1, x->kde - 1), clampi(j + dj, 2, x->jde - 2));
+    dis[q] = di;
+  }
+  for (int g = 0; g < 8; g++) {
+    const int i = i0 + 8 * g + (l >> 3);
+    if (i < r.i0 || i > r.i1) continue;
+    float v[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = f[koff[q] + (unsigned)(clampi(i + dis[q], 2, x->ide - 2) - 1)];
+    if ((c & 3) == 3) {  // slots 27 .. 31 of either input: the spacing, then zeros
+      v[3] = c == 3 ? nm.dx_feature : 0.f;
+#pragma unroll
+      for (int q = 4; q < 8; q++) v[q] = 0.f;
+    }
+    const bf16x8 b = pack8(v);
+    __bf16 *dst = X + (line + (size_t)(i - r.i0)) * kMlpIn + c * 8;
+    if (wide) *reinterpret_cast<bf16x8 *>(dst) = b;
+    else
+      for (int q = 0; q < 8; q++) dst[q] = b[q];
+  }
+  const int i = i0 + l;
+  if (i < r.i0 || i > r.i1) return;
   const float d11 = A3(FL(defor11), i, k, j), d22 = A3(FL(defor22), i, k, j);
   const float *d12 = FL(defor12);
   const float s2 = 0.25f * (A3(d12, i, k, j) + A3(d12, i, k, j + 1) + A3(d12, i + 1, k, j) + A3(d12, i + 1, k, j + 1));
-  T[row * kTargetCols + 2] = 0.5f * (d11 - d22);
-  T[row * kTargetCols + 3] = s2;
-  T[row * kTargetCols + 4] = A3(divisor, i, k, j);
-  T[row * kTargetCols + 5] = A3(FL(xkmh), i, k, j);
+  float *t = T + (line + (size_t)(i - r.i0)) * kTargetCols;
+  t[2] = 0.5f * (d11 - d22);
+  t[3] = s2;
+  t[4] = A3(divisor, i, k, j);
+  t[5] = A3(FL(xkmh), i, k, j);
 }
 
 // Sub-grid stresses of a fine domain on the mass points of a grid coarser by
