@@ -164,6 +164,10 @@ int wrfdc_recorded_stages(wrfdc_ctx *ctx);
 int wrfdc_transport_stage(wrfdc_ctx *ctx, int rk_step, const float *const *stage, const float *q_in, const float *q_old, float *q_out);
 int wrfdc_transport_stage_adjoint(wrfdc_ctx *ctx, int rk_step, const float *const *stage, const float *qbar_out, float *qbar_old,
                                   float *qbar_in);
+/* The adjoint stages of nsteps whole steps, last to first: stages holds 5
+ * pointers for each of the 3*nsteps recorded stages in forward order,
+ * qbar_begin = M^T qbar_end on the mass points (other points untouched). */
+int wrfdc_transport_window_adjoint(wrfdc_ctx *ctx, const float *const *stages, int nsteps, const float *qbar_end, float *qbar_begin);
 
 /* ---- learned eddy viscosity (north-star extension of smag_km, the km of
  * calculate_km_kh, src/wrf_jax/dyn_em/module_diffusion_em_fast.py:773-1083;

@@ -210,11 +210,22 @@ __device__ __forceinline__ float rvw_sel(const DevCtx *__restrict__ x, float r0,
 // ---------------- scalar (theta, moist, scalars) ----------------------------
 // advect_scalar (module_advect_em.py:90-369): tend -= div(flux), mass points
 // (face-sharing blocks; r = mass points; y faces j in [2, jde-1]).
-// TEND: the theta tendency of the RK step, from zero (the cleared array) plus
-// rk_addtend_dry, written once.
-template <bool TEND>
+// MODE kAdvAdd: the tendency is added to tend; kAdvTend: the theta tendency
+// of the RK step, from zero (the cleared array) plus rk_addtend_dry, written
+// once; kAdvTransport: a stage of scalar transport with recorded dynamics,
+// the tendency from zero and then the stage's update (rk_update_scalar)
+//   tend = (m_old q_old + dt msfty [inner] t) / m_new,
+// so the tendency is not stored, cleared and read back (at 200x200x45 a stage
+// took 20 us here, 7 us for the clear and 10.5 us for the update; 22 us
+// in one pass).
+enum { kAdvAdd = 0, kAdvTend = 1, kAdvTransport = 2 };
+struct TransportUpd {
+  const float *q_old, *mu_1, *mu_2;  // stage start value and column masses (perturbation; + mub)
+  float dt;
+};
+template <int MODE>
 __global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx xv, const float *q, float *tend, const float *ru, const float *rv,
-                                                       const float *rom, R3 r, int rk) {
+                                                       const float *rom, R3 r, int rk, TransportUpd tu) {
   const DevCtx *__restrict__ x = &xv;
   __shared__ float ys[kFaceRows][64];
   GET_FACE_BLOCK(r);
@@ -250,7 +261,8 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx x
   const int k1 = imin_(k + 1, kde);
   const float fm0 = A1(FL(fnm), k), fp0 = A1(FL(fnp), k), fm1 = A1(FL(fnm), k1), fp1 = A1(FL(fnp), k1);
   const float msf = A2(FL(msftx), ic, j), rdz = A1(FL(rdnw), k);
-  const float t0 = TEND ? 0.f : elem(tend, o);
+  const float t0 = MODE == kAdvAdd ? elem(tend, o) : 0.f;
+  const float q_old = MODE == kAdvTransport ? elem(tu.q_old, o) : 0.f;
   pin6(wx);
   pin5(wz);
   if (wv == kFaceRows - 1) pin6(wn);
@@ -265,7 +277,14 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx x
   if (j >= 2 && j <= jde - 2) t -= msf * x->rdy * (fn - fs);
   if (ic >= 2 && ic <= ide - 2) t -= msf * x->rdx * (fe - fw);
   t -= rdz * (zflux_br(wz[1], wz[2], wz[3], wz[4], wt, k + 1, kde, fm1, fp1) - zflux_br(wz[0], wz[1], wz[2], wz[3], wb, k, kde, fm0, fp0));
-  if (TEND) t = addtend_t(x, ic, k, j, rk, t, rk > 1);
+  if (MODE == kAdvTend) t = addtend_t(x, ic, k, j, rk, t, rk > 1);
+  if (MODE == kAdvTransport) {
+    const int sz = x->spec_zone;
+    const bool inner = i >= 1 + sz && i <= ide - sz - 1 && j >= 1 + sz && j <= jde - sz - 1;
+    const float mub = A2(FL(mub), i, j), c1 = A1(FL(c1h), k), c2 = A1(FL(c2h), k);
+    const float oldm = c1 * (A2(tu.mu_1, i, j) + mub) + c2, newm = c1 * (A2(tu.mu_2, i, j) + mub) + c2;
+    t = (oldm * q_old + tu.dt * (inner ? t * A2(FL(msfty), i, j) : 0.f)) / newm;
+  }
   elem(tend, o) = t;
 }
 

@@ -618,7 +618,7 @@ struct Run {
   }
   void advect_scalar(const float *q, float *tend, const float *ru, const float *rv, const float *rom) const {
     R3 m = mass3();
-    k_advect_scalar<false><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(d, q, tend, ru, rv, rom, m, 0);
+    k_advect_scalar<kAdvAdd><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(d, q, tend, ru, rv, rom, m, 0, TransportUpd{});
   }
   void advect_scalar_pd(const float *q, const float *q_old, float *tend, double dt) const {
     R3 r = full3();
@@ -694,7 +694,7 @@ struct Run {
     const R3 rq{1, ide - 1, kde - 1, kde - 1, 1, jde - 1};  // levels [2, kde-2]: k_advect_w<true>
     k_cqw_inv<<<g3p(rq), b3(), 0, s>>>(d, rq);
     const R3 m = mass3();
-    k_advect_scalar<true><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(d, F(F_t_2), F(F_t_tend), F(F_ru), F(F_rv), F(F_ww), m, rk);
+    k_advect_scalar<kAdvTend><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(d, F(F_t_2), F(F_t_tend), F(F_ru), F(F_rv), F(F_ww), m, rk, TransportUpd{});
     k_tend_ph<<<g3(rw), b3(), 0, s>>>(d, rw, rk);
     spec_overlays();
   }
@@ -976,17 +976,39 @@ struct Run {
   // one stage of scalar transport with recorded dynamics (tangent-linear =
   // forward) and its adjoint; rk sets dt_rk (set_rk before)
   void transport_stage(const float *const *st, const float *q_in, const float *q_old, float *q_out) const {
-    float *tend = Scr(S_T1);
     R3 m = mass3();
-    fill(tend, X->n3);
-    advect_scalar(q_in, tend, st[0], st[1], st[2]);
-    k_tl_update<<<g3p(m), b3(), 0, s>>>(d, m, StageMass{st[3], st[4]}, q_old, tend, q_out, (float)X->dt_rk);
+    k_advect_scalar<kAdvTransport><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(d, q_in, q_out, st[0], st[1], st[2], m, 0,
+                                                                                            TransportUpd{q_old, st[3], st[4], (float)X->dt_rk});
   }
   void transport_stage_adjoint(const float *const *st, const float *qbar_out, float *qbar_old, float *qbar_in) const {
     float *tbar = Scr(S_T1);
     R3 m = mass3();
-    k_ad_update<<<g3p(m), b3(), 0, s>>>(d, m, StageMass{st[3], st[4]}, qbar_out, qbar_old, tbar, (float)X->dt_rk);
-    k_ad_advect<<<g3p(m), b3(), 0, s>>>(d, m, tbar, st[0], st[1], st[2], qbar_in);
+    k_ad_update<<<g3p(m), b3(), 0, s>>>(d, m, StageMass{st[3], st[4]}, qbar_out, qbar_old, tbar, (float)X->dt_rk, 0);
+    k_ad_advect<kAdAdd><<<g3(m), b3(), 0, s>>>(d, m, tbar, st[0], st[1], st[2], qbar_in, AdNext{});
+  }
+  // the adjoint of nsteps whole steps (stages: 5 pointers for each of their
+  // 3 * nsteps stages, in forward order): qbar_begin = M^T qbar_end on the
+  // mass points, the stages last to first.  tend_bar alternates between two
+  // scratch arrays; qbar_begin holds the accumulated q_old_bar meanwhile.
+  void transport_window_adjoint(const float *const *stages, int nsteps, const float *qbar_end, float *qbar_begin) const {
+    R3 m = mass3();
+    auto st = [&](int n) { return stages + (size_t)5 * n; };
+    auto dt = [&](int n) {
+      set_rk(n % 3 + 1);
+      return (float)X->dt_rk;
+    };
+    float *tbar = Scr(S_T1), *other = Scr(S_T2);
+    const int last = 3 * nsteps - 1;
+    k_ad_update<<<g3p(m), b3(), 0, s>>>(d, m, StageMass{st(last)[3], st(last)[4]}, qbar_end, qbar_begin, tbar, dt(last), 1);
+    for (int n = last; n >= 0; n--) {
+      const float *const *f = st(n);
+      AdNext nx{};
+      if (n > 0) nx = AdNext{StageMass{st(n - 1)[3], st(n - 1)[4]}, other, dt(n - 1)};
+      if (n == 0) k_ad_advect<kAdAdd><<<g3(m), b3(), 0, s>>>(d, m, tbar, f[0], f[1], f[2], qbar_begin, nx);
+      else if (n % 3 == 0) k_ad_advect<kAdStep><<<g3(m), b3(), 0, s>>>(d, m, tbar, f[0], f[1], f[2], qbar_begin, nx);
+      else k_ad_advect<kAdNext><<<g3(m), b3(), 0, s>>>(d, m, tbar, f[0], f[1], f[2], qbar_begin, nx);
+      std::swap(tbar, other);
+    }
   }
 
   // the mass fluxes and column masses of this stage's species update
@@ -1848,6 +1870,20 @@ int wrfdc_transport_stage_adjoint(wrfdc_ctx *x, int rk, const float *const *stag
     Run run(x);
     run.set_rk(rk);
     run.transport_stage_adjoint(stage, qbar_out, qbar_old, qbar_in);
+    return WRFDC_OK;
+  });
+}
+
+int wrfdc_transport_window_adjoint(wrfdc_ctx *x, const float *const *stages, int nsteps, const float *qbar_end, float *qbar_begin) {
+  if (!x) return set_err(nullptr, WRFDC_EINVAL, "null context");
+  if (nsteps < 1 || nsteps > (1 << 24) || !stages) return set_err(x, WRFDC_EINVAL, "a window needs at least one step and its checkpoints");
+  for (int q = 0; q < 15 * nsteps; q++)
+    if (!stages[q]) return set_err(x, WRFDC_EINVAL, "stage checkpoint pointer is null");
+  if (!qbar_end || !qbar_begin) return set_err(x, WRFDC_EINVAL, "adjoint arrays must not be null");
+  if (qbar_end == qbar_begin) return set_err(x, WRFDC_EINVAL, "qbar_begin must not alias qbar_end");
+  return guarded(x, [&]() {
+    Run run(x);
+    run.transport_window_adjoint(stages, nsteps, qbar_end, qbar_begin);
     return WRFDC_OK;
   });
 }

@@ -50,6 +50,8 @@ SIGNATURES = {
                                              ctypes.c_void_p]),
     "wrfdc_transport_stage_adjoint": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
                                                      ctypes.c_void_p, ctypes.c_void_p]),
+    "wrfdc_transport_window_adjoint": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p,
+                                                      ctypes.c_void_p]),
     "wrfdc_set_closure": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     "wrfdc_closure_row_count": (ctypes.c_longlong, [ctypes.c_void_p]),
     "wrfdc_closure_rows": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),

@@ -58,6 +58,7 @@ class Trajectory:
             lib.wrfdc_record_stages(domain.ctx, None, 0)
         if got != nst:
             raise RuntimeError(f"recorded {got} of {nst} stages")
+        self.window_ptrs = ptrs
         self._ptrs = [(ctypes.c_void_p * 5)(*[t.data_ptr() for t in st]) for st in self.stages]
 
     def stage_ptrs(self, n: int, rk: int):
@@ -81,9 +82,10 @@ class Transport:
     def forward(self, q0):
         torch = _torch()
         q_old = q0.contiguous()
-        a, b = torch.zeros_like(q_old), torch.zeros_like(q_old)
+        # the stages write and read mass points only, so only the result needs its other points cleared
+        a, b = torch.empty_like(q_old), torch.empty_like(q_old)
         for n in range(self.traj.nsteps):
-            out = torch.zeros_like(q_old)
+            out = torch.zeros_like(q_old) if n == self.traj.nsteps - 1 else torch.empty_like(q_old)
             self._check(self.lib.wrfdc_transport_stage(self.dom.ctx, 1, self.traj.stage_ptrs(n, 1), self._p(q_old), self._p(q_old),
                                                        self._p(a)), "wrfdc_transport_stage")
             self._check(self.lib.wrfdc_transport_stage(self.dom.ctx, 2, self.traj.stage_ptrs(n, 2), self._p(a), self._p(q_old),
@@ -99,18 +101,12 @@ class Transport:
     def adjoint(self, qbar_end):
         torch = _torch()
         qbar = qbar_end.contiguous()
-        for n in reversed(range(self.traj.nsteps)):
-            acc = torch.zeros_like(qbar)
-            b2 = torch.zeros_like(qbar)
-            b1 = torch.zeros_like(qbar)
-            self._check(self.lib.wrfdc_transport_stage_adjoint(self.dom.ctx, 3, self.traj.stage_ptrs(n, 3), self._p(qbar),
-                                                               self._p(acc), self._p(b2)), "wrfdc_transport_stage_adjoint")
-            self._check(self.lib.wrfdc_transport_stage_adjoint(self.dom.ctx, 2, self.traj.stage_ptrs(n, 2), self._p(b2),
-                                                               self._p(acc), self._p(b1)), "wrfdc_transport_stage_adjoint")
-            self._check(self.lib.wrfdc_transport_stage_adjoint(self.dom.ctx, 1, self.traj.stage_ptrs(n, 1), self._p(b1),
-                                                               self._p(acc), self._p(acc)), "wrfdc_transport_stage_adjoint")
-            qbar = acc
-        return qbar
+        if self.traj.nsteps < 1:
+            return qbar
+        out = torch.zeros_like(qbar)
+        self._check(self.lib.wrfdc_transport_window_adjoint(self.dom.ctx, self.traj.window_ptrs, self.traj.nsteps, self._p(qbar),
+                                                            self._p(out)), "wrfdc_transport_window_adjoint")
+        return out
 
 
 def _autograd_function():
