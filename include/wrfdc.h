@@ -76,6 +76,14 @@ int wrfdc_create(const wrfdc_config *cfg, wrfdc_ctx **out);
 void wrfdc_destroy(wrfdc_ctx *ctx);
 int wrfdc_bind(wrfdc_ctx *ctx, const char *name, void *device_ptr);
 int wrfdc_set_stream(wrfdc_ctx *ctx, void *hip_stream);
+/* Host arrays in the reference's layout, float32 and contiguous, into or out
+ * of n bound fields (indexes of wrfdc_field_name): 3-D (ide,kde,jde), 2-D
+ * (ide,jde), 1-D (kde), species (ide,kde,jde,n+1) with slot 0 unused (read
+ * back as 0), x-edge (jde,kde,bw), y-edge (ide,kde,bw), 2-D edges
+ * (jde|ide,1,bw).  Ordered on the context's stream; the host arrays are
+ * read, or written, when the call returns. */
+int wrfdc_put_reference(wrfdc_ctx *ctx, int n, const int *fields, const void *const *host);
+int wrfdc_get_reference(wrfdc_ctx *ctx, int n, const int *fields, void *const *host);
 int wrfdc_step(wrfdc_ctx *ctx, int nsteps, double dtbc0);
 /* One stage of the step on the bound state.  name is a stage name of the
  * reference's solve_em driver (rk_step_prep, rk_phys_bc_dry_1,

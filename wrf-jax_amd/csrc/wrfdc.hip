@@ -12,11 +12,14 @@
 #include <cstdio>
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cstring>
 #include <initializer_list>
 #include <mutex>
 #include <utility>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "wrfdc_common.h"
@@ -30,6 +33,7 @@
 #include "k_closure.h"
 #include "k_adjoint.h"
 #include "k_colsolve.h"
+#include "k_layout.h"
 
 // ---------------------------------------------------------------------------
 // small helper kernels local to the orchestration
@@ -217,6 +221,18 @@ static const int kCkBlocks = 512;
 // device with that device current (noalloc_scratch below).
 static __device__ __align__(256) double scratch[kCkBlocks * CK_N];
 
+// Pinned and device chunks of the reference-layout transfers: one of each and
+// an event per worker thread, allocated at the first transfer of a context
+// and kept with it (4 x 8 MB each side, or the largest i row of an array if
+// that is more).
+constexpr int kXferWorkers = 4;
+constexpr size_t kXferFloats = (size_t)2 << 20;
+struct Xfer {
+  size_t cap = 0;  // floats per chunk
+  float *pin[kXferWorkers] = {}, *dev[kXferWorkers] = {};
+  hipEvent_t ev[kXferWorkers] = {};
+};
+
 struct wrfdc_ctx {
   wrfdc_config c;
   int ide, jde, kde, ip, ns;
@@ -240,6 +256,7 @@ struct wrfdc_ctx {
   int rec_n = 0, rec_i = 0;
   int rk = 1, nsmall = 1, iteration = 1;
   double dt_rk = 0.0, dts_rk = 0.0, dtbc = 0.0;
+  Xfer xfer;
   float *dtbc_dev = nullptr;  // dtbc as the boundary kernels read it (one float)
   bool capturing = false;     // a step being captured into a graph leaves dtbc_dev to the replayer
   std::string err;
@@ -1309,6 +1326,15 @@ int wrfdc_field_count(void) { return NFIELDS; }
 const char *wrfdc_field_name(int index) { return (index >= 0 && index < NFIELDS) ? kNames[index] : nullptr; }
 int wrfdc_field_kind(int index) { return (index >= 0 && index < NFIELDS) ? (int)kKinds[index] : 0; }
 
+static void xfer_free(wrfdc_ctx *x) {
+  for (int w = 0; w < kXferWorkers; w++) {
+    if (x->xfer.pin[w]) (void)hipHostFree(x->xfer.pin[w]);
+    if (x->xfer.dev[w]) (void)hipFree(x->xfer.dev[w]);
+    if (x->xfer.ev[w]) (void)hipEventDestroy(x->xfer.ev[w]);
+  }
+  x->xfer = Xfer{};
+}
+
 int wrfdc_create(const wrfdc_config *cfg, wrfdc_ctx **out) {
   if (!cfg || !out) return set_err(nullptr, WRFDC_EINVAL, "cfg and out must not be null");
   *out = nullptr;
@@ -1366,8 +1392,184 @@ void wrfdc_destroy(wrfdc_ctx *x) {
   if (x->spec_alt) (void)hipFree(x->spec_alt);
   if (x->spec_scale) (void)hipFree(x->spec_scale);
   if (x->hds) (void)hipFree(x->hds);
+  xfer_free(x);
   delete x;
 }
+
+// ---- host arrays in the reference's layout ---------------------------------
+// extents and strides of a field (the whole of it: i0 = 0, ni as stored)
+static LayoutSeg layout_of(const wrfdc_ctx *x, int f) {
+  LayoutSeg g;
+  memset(&g, 0, sizeof(g));
+  const int ide = x->ide, jde = x->jde, kde = x->kde, ip = x->ip, bw = x->c.spec_bdy_width;
+  const char kind = kKinds[f];
+  g.reg = x->h.F[f];
+  g.np = g.nslot = 1;
+  g.nj = bw;
+  g.sj = 1;
+  g.ni = g.nipad = ide;
+  switch (kind) {
+    case '1': g.ni = g.nipad = kde; g.nj = 1; g.si = 1; break;
+    case '2': g.nj = jde; g.si = (unsigned)jde; g.rj = (size_t)ip; g.nipad = ip; break;
+    case 'X': g.ni = g.nipad = jde; g.np = kde; g.si = (unsigned)(kde * bw); g.sp = (unsigned)bw; g.rj = (size_t)kde * jde; g.rp = (size_t)jde; break;
+    case 'Y': g.np = kde; g.si = (unsigned)(kde * bw); g.sp = (unsigned)bw; g.rj = (size_t)kde * ip; g.rp = (size_t)ip; g.nipad = ip; break;
+    case 'x': g.ni = g.nipad = jde; g.si = (unsigned)bw; g.rj = (size_t)jde; break;
+    case 'y': g.si = (unsigned)bw; g.rj = (size_t)ip; g.nipad = ip; break;
+    default: {  // '3', and the species stacks with the reference's unused slot 0
+      const int n = kind == 'M' ? x->c.nmoist : kind == 'S' ? x->c.nscalar : 0;
+      g.species = kind != '3';
+      g.nslot = n + 1;
+      g.nj = jde;
+      g.np = kde;
+      g.sj = (unsigned)g.nslot;
+      g.sp = (unsigned)(jde * g.nslot);
+      g.si = (unsigned)(kde * jde * g.nslot);
+      g.rj = (size_t)kde * ip;
+      g.rp = (size_t)ip;
+      g.rs = x->n3;
+      g.nipad = ip;
+    }
+  }
+  return g;
+}
+
+// Every worker takes the next chunk's worth of segments, and copies, sends
+// and turns them (up), or turns, fetches and copies (down), all on the
+// context's stream: the host copies of one worker overlap the transfers of
+// the others.
+extern "C++" {
+template <bool UP>
+static int xfer_reference(wrfdc_ctx *x, int n, const int *fields, void *const *host) {
+  if (n < 0 || (n > 0 && (!fields || !host))) return set_err(x, WRFDC_EINVAL, "fields and host arrays must not be null");
+  struct Piece {
+    LayoutSeg g;
+    char *host;
+  };
+  struct Chunk {
+    size_t p0, p1, floats;
+  };
+  return guarded(x, [&]() {
+    try {
+      size_t cap = kXferFloats;
+      for (int q = 0; q < n; q++) {
+        if (fields[q] < 0 || fields[q] >= NFIELDS) return set_err(x, WRFDC_EINVAL, "unknown field index");
+        if (!host[q]) return set_err(x, WRFDC_EINVAL, std::string("null host array: ") + kNames[fields[q]]);
+        cap = std::max<size_t>(cap, layout_of(x, fields[q]).si);
+      }
+      Xfer &X = x->xfer;
+      if (X.cap < cap) {
+        if (X.cap) {
+          hchk(x->s ? hipStreamSynchronize(x->s) : hipDeviceSynchronize(), "transfer buffers");
+          xfer_free(x);
+        }
+        try {
+          for (int w = 0; w < kXferWorkers; w++) {
+            hchk(hipHostMalloc((void **)&X.pin[w], cap * sizeof(float), hipHostMallocDefault), "hipHostMalloc transfer");
+            hchk(hipMalloc((void **)&X.dev[w], cap * sizeof(float)), "hipMalloc transfer");
+            hchk(hipEventCreateWithFlags(&X.ev[w], hipEventDisableTiming), "transfer event");
+          }
+        } catch (const HipError &) {
+          xfer_free(x);
+          throw;
+        }
+        X.cap = cap;
+      }
+      std::vector<Piece> pieces;
+      std::vector<Chunk> chunks;
+      for (int q = 0; q < n; q++) {
+        const LayoutSeg whole = layout_of(x, fields[q]);
+        for (int i0 = 0; i0 < whole.ni;) {
+          if (chunks.empty() || chunks.back().floats + whole.si > X.cap) chunks.push_back(Chunk{pieces.size(), pieces.size(), 0});
+          Chunk &c = chunks.back();
+          Piece p{whole, (char *)host[q] + (size_t)i0 * whole.si * sizeof(float)};
+          p.g.ni = (int)std::min<size_t>((X.cap - c.floats) / whole.si, (size_t)(whole.ni - i0));
+          p.g.nipad = i0 + p.g.ni == whole.ni ? whole.nipad - i0 : p.g.ni;
+          p.g.i0 = i0;
+          p.g.ref = (unsigned)c.floats;
+          c.floats += (size_t)p.g.ni * whole.si;
+          pieces.push_back(p);
+          c.p1 = pieces.size();
+          i0 += p.g.ni;
+        }
+      }
+      int dev = 0;
+      hchk(hipGetDevice(&dev), "current device");
+      std::atomic<size_t> next{0};
+      std::atomic<int> failed{(int)hipSuccess};
+      auto turn = [&](const Chunk &c, float *buf) {
+        LayoutList L;
+        L.n = 0;
+        unsigned tiles = 0;
+        for (size_t q = c.p0; q < c.p1; q++) {
+          LayoutSeg &g = L.s[L.n++] = pieces[q].g;
+          g.tile0 = tiles;
+          tiles += layout_tiles(g);
+          if (L.n == kLayoutSegs || q + 1 == c.p1) {
+            k_layout<UP><<<tiles, dim3(kLayoutTile, 8), 0, x->s>>>(L, buf);
+            L.n = 0;
+            tiles = 0;
+          }
+        }
+        return hipGetLastError();
+      };
+      auto copy = [&](const Chunk &c, float *pin) {
+        for (size_t q = c.p0; q < c.p1; q++) {
+          const Piece &p = pieces[q];
+          const size_t bytes = (size_t)p.g.ni * p.g.si * sizeof(float);
+          if (UP) memcpy(pin + p.g.ref, p.host, bytes);
+          else memcpy(p.host, pin + p.g.ref, bytes);
+        }
+      };
+      auto work = [&](int w) {
+        hipError_t e = hipSetDevice(dev);
+        bool used = false;
+        for (size_t q; e == hipSuccess && failed.load() == (int)hipSuccess && (q = next.fetch_add(1)) < chunks.size();) {
+          const Chunk &c = chunks[q];
+          const size_t bytes = c.floats * sizeof(float);
+          if (UP) {
+            if (used) e = hipEventSynchronize(X.ev[w]);  // this worker's last chunk has left its buffers
+            if (e != hipSuccess) break;
+            copy(c, X.pin[w]);
+            e = hipMemcpyAsync(X.dev[w], X.pin[w], bytes, hipMemcpyHostToDevice, x->s);
+            if (e == hipSuccess) e = turn(c, X.dev[w]);
+            if (e == hipSuccess) e = hipEventRecord(X.ev[w], x->s);
+            used = true;
+          } else {
+            e = turn(c, X.dev[w]);
+            if (e == hipSuccess) e = hipMemcpyAsync(X.pin[w], X.dev[w], bytes, hipMemcpyDeviceToHost, x->s);
+            if (e == hipSuccess) e = hipEventRecord(X.ev[w], x->s);
+            if (e == hipSuccess) e = hipEventSynchronize(X.ev[w]);
+            if (e == hipSuccess) copy(c, X.pin[w]);
+          }
+        }
+        // the buffers are free when the call returns
+        if (UP && e == hipSuccess && used) e = hipEventSynchronize(X.ev[w]);
+        if (e != hipSuccess) failed.store((int)e);
+      };
+      const int helpers = (int)std::min<size_t>(kXferWorkers, chunks.size()) - 1;
+      std::thread pool[kXferWorkers];
+      for (int w = 1; w <= helpers; w++) {
+        try {
+          pool[w] = std::thread(work, w);
+        } catch (const std::system_error &) {
+          break;  // no more threads to be had: the ones that run do it all
+        }
+      }
+      work(0);
+      for (auto &t : pool)
+        if (t.joinable()) t.join();
+      hchk((hipError_t)failed.load(), UP ? "upload" : "download");
+      return WRFDC_OK;
+    } catch (const std::bad_alloc &) {
+      return set_err(x, WRFDC_EHIP, "out of host memory");
+    }
+  });
+}
+}  // extern "C++"
+int wrfdc_put_reference(wrfdc_ctx *x, int n, const int *fields, const void *const *host) {
+  return xfer_reference<true>(x, n, fields, const_cast<void *const *>(host));
+}
+int wrfdc_get_reference(wrfdc_ctx *x, int n, const int *fields, void *const *host) { return xfer_reference<false>(x, n, fields, host); }
 
 int wrfdc_bind(wrfdc_ctx *x, const char *name, void *device_ptr) {
   if (!x || !name) return WRFDC_EINVAL;

@@ -161,6 +161,50 @@ def from_registry(name: str, reg: np.ndarray, dims: Dims) -> np.ndarray:
     raise ValueError(kind)
 
 
+_FIELD_INDEX = {n: q for q, (n, _) in enumerate(FIELD_SPECS)}
+
+
+def reference_shape(name: str, dims: Dims) -> tuple:
+    """Shape of registry field ``name`` in the reference's layout."""
+    ide, jde, kde, bw = dims.ide, dims.jde, dims.kde, dims.spec_bdy_width
+    return {"3": (ide, kde, jde), "2": (ide, jde), "1": (kde,), "M": (ide, kde, jde, dims.nmoist + 1),
+            "S": (ide, kde, jde, dims.nscalar + 1), "X": (jde, kde, bw), "Y": (ide, kde, bw), "x": (jde, 1, bw),
+            "y": (ide, 1, bw)}[FIELD_KIND[name]]
+
+
+def _pointers(arrays):
+    return np.array([a.__array_interface__["data"][0] for a in arrays], dtype=np.uintp)
+
+
+def put_reference(dom, dims: Dims, refs: Mapping) -> None:
+    """Reference-layout host arrays (registry names) into the domain's
+    buffers.  Arrays of the expected shape go as they are and are turned on
+    the device; any other shape takes to_registry's rules on the host."""
+    fields, arrays, rest = [], [], {}
+    for name, ref in refs.items():
+        a = np.asarray(ref)
+        if a.shape != reference_shape(name, dims):
+            rest[name] = to_registry(name, ref, dims)
+            continue
+        fields.append(_FIELD_INDEX[name])
+        arrays.append(np.ascontiguousarray(a, dtype=np.float32))
+    if fields:
+        index, ptrs = np.array(fields, dtype=np.int32), _pointers(arrays)
+        dom._check(dom.lib.wrfdc_put_reference(dom.ctx, len(fields), index.ctypes.data, ptrs.ctypes.data), "wrfdc_put_reference")
+    if rest:
+        dom.upload(rest)
+
+
+def get_reference(dom, dims: Dims, names) -> dict:
+    """The domain's fields as new host arrays in the reference's layout."""
+    names = list(names)
+    out = {n: np.empty(reference_shape(n, dims), dtype=np.float32) for n in names}
+    if names:
+        index, ptrs = np.array([_FIELD_INDEX[n] for n in names], dtype=np.int32), _pointers(out.values())
+        dom._check(dom.lib.wrfdc_get_reference(dom.ctx, len(names), index.ctypes.data, ptrs.ctypes.data), "wrfdc_get_reference")
+    return out
+
+
 # the prognostic arrays a ModelState carries between steps (reference names)
 DYNAMIC_ARRAY_NAMES = tuple(sorted(reference_name(n) for n, _ in FIELD_SPECS))
 
@@ -214,8 +258,8 @@ def build_step_em_core_context(*, grid: DycoreConfig, config_flags: Mapping | No
     for name, _ in FIELD_SPECS:
         ref = reference_name(name)
         if ref in template:
-            upload[name] = to_registry(name, template[ref], dims)
-    dom.upload(upload)
+            upload[name] = template[ref]
+    put_reference(dom, dims, upload)
     return StepEmCoreContext(domain=dom, grid=cfg, config_flags=opts, fields_template=template, dynamic_only=bool(dynamic_only),
                              boundary_interval_seconds=int(boundary_interval_seconds), check_finite=bool(check_finite), dims=dims)
 
@@ -235,14 +279,14 @@ def step_em_core_once(state: ModelState, context: StepEmCoreContext) -> StepEmCo
     for ref, arr in state.as_dict().items():
         name = registry_name(ref)
         if name in FIELD_KIND:
-            upload[name] = to_registry(name, arr, dims)
-    dom.upload(upload)
+            upload[name] = arr
+    put_reference(dom, dims, upload)
     dom.step(1, float(state.time.dtbc))
     ck = dom.checksums() if context.check_finite else None
-    got = dom.download([registry_name(r) for r in state.array_names if registry_name(r) in FIELD_KIND])
+    got = get_reference(dom, dims, [registry_name(r) for r in state.array_names if registry_name(r) in FIELD_KIND])
     new_arrays = dict(state.as_dict())
     for name, a in got.items():
-        new_arrays[reference_name(name)] = from_registry(name, a, dims)
+        new_arrays[reference_name(name)] = a
     time = state.time.advance(context.grid.dt, context.boundary_interval_seconds)
     next_state = ModelState(state.array_names, tuple(new_arrays[n] for n in state.array_names), time)
     fields = dict(context.fields_template)
@@ -252,6 +296,6 @@ def step_em_core_once(state: ModelState, context: StepEmCoreContext) -> StepEmCo
 
 __all__ = [
     "DYNAMIC_ARRAY_NAMES", "ModelState", "SolveResult", "StepEmCoreContext", "StepEmCoreResult", "TimeState",
-    "build_step_em_core_context", "from_registry", "initial_step_em_state", "reference_name", "registry_name",
-    "step_em_core_once", "to_registry",
+    "build_step_em_core_context", "from_registry", "get_reference", "initial_step_em_state", "put_reference", "reference_name",
+    "reference_shape", "registry_name", "step_em_core_once", "to_registry",
 ]
