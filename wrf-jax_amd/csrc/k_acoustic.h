@@ -28,7 +28,7 @@
 // without branches around its loads: p is read at levels k-1 .. k+2 (clamped
 // into the column) and the surface / interior / top expressions of uv_iface
 // are selected on the level
-__device__ __forceinline__ float uv_vert(const DevCtx *__restrict__ x, const float *p, int i, int j, int di, int dj, int k) {
+__device__ __forceinline__ float uv_vert(CtxPtr x, const float *p, int i, int j, int di, int dj, int k) {
   const int kde = x->kde;
   const int km = imax_(k - 1, 1), kp = imin_(k + 1, kde), kq = imin_(k + 2, kde);
   const float ppm = A3(p, i, km, j) + A3(p, i - di, km, j - dj);
@@ -47,7 +47,7 @@ __device__ __forceinline__ float uv_vert(const DevCtx *__restrict__ x, const flo
 // advance_uv at an interior u point (axis 0: i [2, ide-1], j [2, jde-2]) or v
 // point (axis 1: i [2, ide-2], j [2, jde-1]); adv = u + dts * ru_tend (v +
 // dts * rv_tend) of that point, formed by the caller
-__device__ __forceinline__ float uv_interior(const DevCtx *__restrict__ x, int axis, int i, int k, int j, float dts, float adv) {
+__device__ __forceinline__ float uv_interior(CtxPtr x, int axis, int i, int k, int j, float dts, float adv) {
   const int di = axis == 0 ? 1 : 0, dj = axis == 0 ? 0 : 1;
   const unsigned o = XI3(i, k, j);
   const float *p = FL(p), *pb = FL(pb), *ph = FL(ph_2), *alt = FL(alt), *al = FL(al), *php = FL(php);
@@ -73,8 +73,8 @@ __device__ __forceinline__ float uv_interior(const DevCtx *__restrict__ x, int a
 // (its own where they apply) and the zone formula, with no branch around the
 // loads, so all of them are in flight together; the results are selected
 // and stored at the end.
-__global__ void __launch_bounds__(256) k_uv_substep(const DevCtx xv, float dts, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(256) k_uv_substep(const DevCtx *xv, float dts, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int ide = x->ide, jde = x->jde;
   const unsigned o = XI3(i, k, j);
@@ -94,8 +94,8 @@ __global__ void __launch_bounds__(256) k_uv_substep(const DevCtx xv, float dts, 
 
 // zero_grad_bdy of w: every destination (the zone ring of the mass grid)
 // copies an interior point, so rows and columns go in one race-free pass.
-__global__ void k_zero_grad_w(const DevCtx xv) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_zero_grad_w(const DevCtx *xv) {
+  const CtxPtr x = ctx_ptr(xv);
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   const int ibe = x->ide - 1, jbe = x->jde - 1;
@@ -138,8 +138,8 @@ inline int acoustic_col_npw(int kde) {
 }
 
 template <int NPW>
-__global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx xv, float dts, int first, int fin, float ns, int store_tav) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *xv, float dts, int first, int fin, float ns, int store_tav) {
+  const CtxPtr x = ctx_ptr(xv);
   constexpr int NW = kColWaves;
   constexpr int G1 = kColG1, G3 = kColG3, G4 = kColG4, G5 = kColG5, G6 = kColG6, G9 = kColG9, G10 = kColG10;
   extern __shared__ float sm[];
@@ -686,15 +686,15 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx xv
 // host launcher: instantiation by levels per wave
 // store_tav: write the acoustic theta average to t_2ave (only its last
 // substep's value is read outside the kernel)
-inline void launch_acoustic_col(const DevCtx &d, hipStream_t s, float dts, int first, int fin, float ns, int store_tav) {
+inline void launch_acoustic_col(const DevCtx &d, const DevCtx *dev, hipStream_t s, float dts, int first, int fin, float ns, int store_tav) {
   const dim3 grid((unsigned)((d.ide + 63) / 64) * (unsigned)d.jde), block(64, kColWaves);
   const size_t lds = acoustic_col_lds(d.kde);
   switch (acoustic_col_npw(d.kde)) {
-    case 4: k_acoustic_col<4><<<grid, block, lds, s>>>(d, dts, first, fin, ns, store_tav); break;
-    case 8: k_acoustic_col<8><<<grid, block, lds, s>>>(d, dts, first, fin, ns, store_tav); break;
-    case 12: k_acoustic_col<12><<<grid, block, lds, s>>>(d, dts, first, fin, ns, store_tav); break;
-    case 16: k_acoustic_col<16><<<grid, block, lds, s>>>(d, dts, first, fin, ns, store_tav); break;
-    default: k_acoustic_col<20><<<grid, block, lds, s>>>(d, dts, first, fin, ns, store_tav); break;
+    case 4: k_acoustic_col<4><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
+    case 8: k_acoustic_col<8><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
+    case 12: k_acoustic_col<12><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
+    case 16: k_acoustic_col<16><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
+    default: k_acoustic_col<20><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
   }
 }
 // raise the dynamic-LDS limit of the instantiation kde needs (beyond 64 KB)

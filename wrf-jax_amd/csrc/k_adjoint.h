@@ -25,7 +25,7 @@ struct StageCoef {
   float oldm, newm, msfty;
   bool inner;
 };
-__device__ __forceinline__ StageCoef stage_coef(const DevCtx *__restrict__ x, const StageMass &sm, int i, int k, int j) {
+__device__ __forceinline__ StageCoef stage_coef(CtxPtr x, const StageMass &sm, int i, int k, int j) {
   StageCoef c;
   const int sz = x->spec_zone;
   c.inner = i >= 1 + sz && i <= x->ide - sz - 1 && j >= 1 + sz && j <= x->jde - sz - 1;
@@ -38,9 +38,9 @@ __device__ __forceinline__ StageCoef stage_coef(const DevCtx *__restrict__ x, co
 
 // transpose of the update: q_old_bar += (m_old / m_new) q_out_bar,
 // tend_bar = dt msfty [inner] / m_new q_out_bar; first: qbar_old starts from 0
-__global__ void k_ad_update(const DevCtx xv, R3 r, StageMass sm, const float *__restrict__ qbar_out, float *__restrict__ qbar_old,
+__global__ void k_ad_update(const DevCtx *xv, R3 r, StageMass sm, const float *__restrict__ qbar_out, float *__restrict__ qbar_old,
                             float *__restrict__ tbar, float dt, int first) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const StageCoef c = stage_coef(x, sm, i, k, j);
   const float qb = A3(qbar_out, i, k, j);
@@ -122,10 +122,10 @@ struct AdNext {
 // and a division per coefficient the stage took 76 us at 200x200x45 and its
 // update 12 us in a pass of its own, 28 us together this way.
 template <int MODE>
-__global__ void __launch_bounds__(256) k_ad_advect(const DevCtx xv, R3 r, const float *__restrict__ tbar, const float *__restrict__ ru,
+__global__ void __launch_bounds__(256) k_ad_advect(const DevCtx *xv, R3 r, const float *__restrict__ tbar, const float *__restrict__ ru,
                                                    const float *__restrict__ rv, const float *__restrict__ rom, float *__restrict__ qbar,
                                                    AdNext nx) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int ide = x->ide, jde = x->jde, ktf = x->kde - 1;
   const float rdx = x->rdx, rdy = x->rdy;

@@ -200,7 +200,7 @@ __device__ __forceinline__ float zflux_w_sel(float qm2, float qm1, float q0, flo
 }
 // mass flux at a w level from the values at levels k, k-1, k-2 of the column
 // (extrapolated at the top level kde)
-__device__ __forceinline__ float rvw_sel(const DevCtx *__restrict__ x, float r0, float rm1, float rm2, int k) {
+__device__ __forceinline__ float rvw_sel(CtxPtr x, float r0, float rm1, float rm2, int k) {
   const int kde = x->kde, kc = imin_(k, kde - 1);
   const float top = (2.f - A1(FL(fnm), kde - 1)) * rm1 - A1(FL(fnp), kde - 1) * rm2;
   const float mid = A1(FL(fnm), kc) * r0 + A1(FL(fnp), kc) * rm1;
@@ -224,9 +224,9 @@ struct TransportUpd {
   float dt;
 };
 template <int MODE>
-__global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx xv, const float *q, float *tend, const float *ru, const float *rv,
+__global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx *xv, const float *q, float *tend, const float *ru, const float *rv,
                                                        const float *rom, R3 r, int rk, TransportUpd tu) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   __shared__ float ys[kFaceRows][64];
   GET_FACE_BLOCK(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
@@ -298,9 +298,9 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx x
 // a column clamped into [2, ide-1], so their loads stay in the field) and
 // used where they apply.
 template <bool TEND>
-__global__ void __launch_bounds__(64 * kFaceRows) k_advect_u(const DevCtx xv, const float *u, float *tend, const float *ru, const float *rv,
+__global__ void __launch_bounds__(64 * kFaceRows) k_advect_u(const DevCtx *xv, const float *u, float *tend, const float *ru, const float *rv,
                                                   const float *rom, R3 r, int rk) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   __shared__ float ys[kFaceRows][64];
   GET_FACE_BLOCK(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
@@ -373,9 +373,9 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_u(const DevCtx xv, co
 // gradient, Coriolis/curvature at j [2, jde-1], then rk_addtend_dry); the
 // pressure-gradient and Coriolis terms at a row clamped into [2, jde-1].
 template <bool TEND>
-__global__ void __launch_bounds__(64 * kFaceRows) k_advect_v(const DevCtx xv, const float *v, float *tend, const float *ru, const float *rv,
+__global__ void __launch_bounds__(64 * kFaceRows) k_advect_v(const DevCtx *xv, const float *v, float *tend, const float *ru, const float *rv,
                                                   const float *rom, R3 r, int rk) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   __shared__ float ys[kFaceRows][64];
   GET_FACE_BLOCK(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
@@ -450,9 +450,9 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_v(const DevCtx xv, co
 // the top, Coriolis/curvature at k [2, kde]; then rk_addtend_dry.  Buoyancy
 // and Coriolis terms at a level clamped into the range they apply to.
 template <bool TEND>
-__global__ void __launch_bounds__(64 * kFaceRows) k_advect_w(const DevCtx xv, const float *w, float *tend, const float *ru, const float *rv,
+__global__ void __launch_bounds__(64 * kFaceRows) k_advect_w(const DevCtx *xv, const float *w, float *tend, const float *ru, const float *rv,
                                                   const float *rom, R3 r, int rk) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   __shared__ float ys[kFaceRows][64];
   GET_FACE_BLOCK_LG(r, (unsigned)x->face_lg[1]);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
@@ -525,8 +525,8 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_w(const DevCtx xv, co
 // the phi tendency of the RK step over k [1, kde]: rhs_ph at k [2, kde] from
 // zero (the cleared array), then rk_addtend_dry; r = i [1, ide-1], k [1, kde],
 // j [1, jde-1]
-__global__ void __launch_bounds__(256) k_tend_ph(const DevCtx xv, R3 r, int rk) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(256) k_tend_ph(const DevCtx *xv, R3 r, int rk) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const unsigned o = XI3(i, k, j);
   // rk_addtend_dry's loads go out first (addtend_ph in two parts)
@@ -540,9 +540,9 @@ __global__ void __launch_bounds__(256) k_tend_ph(const DevCtx xv, R3 r, int rk) 
 // ---------------- positive-definite scalar advection ------------------------
 // pass 1: high-order minus upwind (antidiffusive) and upwind fluxes
 // (module_advect_em.py:537-660) on all faces the limiter and tendency read.
-__global__ void k_pd_fluxes(const DevCtx xv, const float *q, const float *q_old, const float *ru, const float *rv,
+__global__ void k_pd_fluxes(const DevCtx *xv, const float *q, const float *q_old, const float *ru, const float *rv,
                             const float *rom, const float *mut, float dt, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *c1 = FL(c1h), *c2 = FL(c2h), *msftx = FL(msftx), *msfty = FL(msfty), *rdzw = FL(rdnw);
   const float *fzm = FL(fnm), *fzp = FL(fnp);
@@ -608,8 +608,8 @@ __global__ void k_pd_fluxes(const DevCtx xv, const float *q, const float *q_old,
 }
 // pass 2: renormalisation factor of each limited cell (1 = not limited)
 // (module_advect_em.py:662-720); cells i in [2, ide-2], j in [2, jde-2].
-__global__ void k_pd_scale(const DevCtx xv, const float *q_old, const float *mub, const float *mu_old, float dt, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_pd_scale(const DevCtx *xv, const float *q_old, const float *mub, const float *mu_old, float dt, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *c1 = FL(c1h), *c2 = FL(c2h), *msftx = FL(msftx), *msfty = FL(msfty), *rdzw = FL(rdnw);
   const float *fqx = SCR(S_FQX), *fqy = SCR(S_FQY), *fqz = SCR(S_FQZ), *fqxl = SCR(S_FQXL), *fqyl = SCR(S_FQYL), *fqzl = SCR(S_FQZL);
@@ -630,8 +630,8 @@ __global__ void k_pd_scale(const DevCtx xv, const float *q_old, const float *mub
 }
 // pass 3: tendency from the renormalised faces; a face is scaled by the
 // cell its antidiffusive flux leaves (the only cell that may limit it).
-__global__ void k_pd_tend(const DevCtx xv, float *tend, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_pd_tend(const DevCtx *xv, float *tend, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *msftx = FL(msftx), *rdzw = FL(rdnw);
   const float *fqx = SCR(S_FQX), *fqy = SCR(S_FQY), *fqz = SCR(S_FQZ), *fqxl = SCR(S_FQXL), *fqyl = SCR(S_FQYL), *fqzl = SCR(S_FQZL);

@@ -7,8 +7,8 @@
 
 // ---- physical BC copy (set_physical_bc3d, no-halo specified) -------------
 // plane i = ide-1 -> ide for every j (skipped for x-staggered variables)
-__global__ void k_bc_x(const DevCtx xv, float *fl, int kend, int is2d) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_bc_x(const DevCtx *xv, float *fl, int kend, int is2d) {
+  const CtxPtr x = ctx_ptr(xv);
   const int j = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   if (j > x->jde || k > kend) return;
@@ -16,8 +16,8 @@ __global__ void k_bc_x(const DevCtx xv, float *fl, int kend, int is2d) {
   else A3(fl, x->ide, k, j) = A3(fl, x->ide - 1, k, j);
 }
 // row j = jde-1 -> jde for every i (skipped for y-staggered variables)
-__global__ void k_bc_y(const DevCtx xv, float *fl, int kend, int is2d) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_bc_y(const DevCtx *xv, float *fl, int kend, int is2d) {
+  const CtxPtr x = ctx_ptr(xv);
   const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   if (i > x->ide || k > kend) return;
@@ -35,8 +35,8 @@ struct BcList {
   int kend[kBcMax];
   int flags[kBcMax];  // bit 0: copy column ide, bit 1: copy row jde, bit 2: 2-D
 };
-__global__ void k_bc_batch(const DevCtx xv, BcList L) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_bc_batch(const DevCtx *xv, BcList L) {
+  const CtxPtr x = ctx_ptr(xv);
   const int a = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   const int q = (int)blockIdx.z;
@@ -80,7 +80,7 @@ __device__ __forceinline__ bool zone_point(int t, int ibe, int jbe, int &i, int 
   if (t < nj) { i = ibe; j = 2 + t; edge = 3; return true; }
   return false;
 }
-__device__ __forceinline__ float bval(const DevCtx *__restrict__ x, const float *const b4[4], int e, int a, int k, int b, int is2d) {
+__device__ __forceinline__ float bval(CtxPtr x, const float *const b4[4], int e, int a, int k, int b, int is2d) {
   if (is2d) return (e < 2) ? BY2(b4[e], a, b) : BX2(b4[e], a, b);
   return (e < 2) ? BY(b4[e], a, k, b) : BX(b4[e], a, k, b);
 }
@@ -89,8 +89,8 @@ struct BPtrs {
 };
 
 // spec_bdytend overlay: tend on the zone = boundary tendency (b = 1)
-__global__ void k_spec_overlay(const DevCtx xv, float *tend, int ibe, int jbe, int kt, int is2d, BPtrs bt) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_spec_overlay(const DevCtx *xv, float *tend, int ibe, int jbe, int kt, int is2d, BPtrs bt) {
+  const CtxPtr x = ctx_ptr(xv);
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   int i, j, e;
@@ -109,8 +109,8 @@ struct OverlayList {
   BPtrs bt[kOverlayMax];
   int ibe[kOverlayMax], jbe[kOverlayMax], kt[kOverlayMax], is2d[kOverlayMax];
 };
-__global__ void k_spec_overlay_batch(const DevCtx xv, OverlayList L) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_spec_overlay_batch(const DevCtx *xv, OverlayList L) {
+  const CtxPtr x = ctx_ptr(xv);
   const int f = (int)blockIdx.z;
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
@@ -124,8 +124,8 @@ __global__ void k_spec_overlay_batch(const DevCtx xv, OverlayList L) {
 }
 
 // spec_bdyupdate: field += dt * tend on the zone
-__global__ void k_spec_update(const DevCtx xv, float *fl, const float *tend, float dt, int ibe, int jbe, int kt, int is2d) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_spec_update(const DevCtx *xv, float *fl, const float *tend, float dt, int ibe, int jbe, int kt, int is2d) {
+  const CtxPtr x = ctx_ptr(xv);
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   int i, j, e;
@@ -135,8 +135,8 @@ __global__ void k_spec_update(const DevCtx xv, float *fl, const float *tend, flo
 }
 
 // spec_bdyupdate_ph (module_bc_em.py:1429-1560)
-__global__ void k_spec_update_ph(const DevCtx xv, float dts) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_spec_update_ph(const DevCtx *xv, float dts) {
+  const CtxPtr x = ctx_ptr(xv);
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   int i, j, e;
@@ -151,8 +151,8 @@ __global__ void k_spec_update_ph(const DevCtx xv, float dts) {
 }
 
 // zero_grad_bdy for w (zero_grad_bdy.py:21-128): rows first, then columns
-__global__ void k_zero_grad_rows(const DevCtx xv, float *w) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_zero_grad_rows(const DevCtx *xv, float *w) {
+  const CtxPtr x = ctx_ptr(xv);
   const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   const int side = (int)blockIdx.z;
@@ -162,8 +162,8 @@ __global__ void k_zero_grad_rows(const DevCtx xv, float *w) {
   if (side == 0) A3(w, i, k, 1) = A3(w, ii, k, 2);
   else A3(w, i, k, jbe) = A3(w, ii, k, jbe - 1);
 }
-__global__ void k_zero_grad_cols(const DevCtx xv, float *w) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_zero_grad_cols(const DevCtx *xv, float *w) {
+  const CtxPtr x = ctx_ptr(xv);
   const int j = 2 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   const int side = (int)blockIdx.z;
@@ -181,7 +181,7 @@ __global__ void k_zero_grad_cols(const DevCtx xv, float *w) {
 // coupled value (module_bc_em.py:561-624) formed on the spot, the field times
 // c1*mut + c2 (mw 1: half levels, c1h/c2h, k <= kde-1; mw 2: w levels,
 // c1f/c2f), zero outside the coupled range
-__device__ __forceinline__ float relax_fv(const DevCtx *__restrict__ x, const float *fld, int ii, int k, int jj, int is2d, int mw) {
+__device__ __forceinline__ float relax_fv(CtxPtr x, const float *fld, int ii, int k, int jj, int is2d, int mw) {
   if (is2d) return A2(fld, ii, jj);
   const float f = A3(fld, ii, k, jj);
   if (mw == 0) return f;
@@ -199,8 +199,8 @@ struct RelaxList {
 };
 // dt_bc_p: the time since the lateral-boundary update, read from device memory
 // (set before each step, so that a captured step reads the current value)
-__global__ void k_relax(const DevCtx xv, RelaxList R, const float *__restrict__ dt_bc_p) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_relax(const DevCtx *xv, RelaxList R, const float *__restrict__ dt_bc_p) {
+  const CtxPtr x = ctx_ptr(xv);
   const float dt_bc = *dt_bc_p;
   const int a = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
@@ -258,8 +258,8 @@ __global__ void k_relax(const DevCtx xv, RelaxList R, const float *__restrict__ 
 }
 
 // flow_dep_bdy (flow_dep_bdy.py:27-176): rows then columns
-__global__ void k_flow_dep_rows(const DevCtx xv, float *q, const float *v) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_flow_dep_rows(const DevCtx *xv, float *q, const float *v) {
+  const CtxPtr x = ctx_ptr(xv);
   const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   const int side = (int)blockIdx.z;
@@ -269,8 +269,8 @@ __global__ void k_flow_dep_rows(const DevCtx xv, float *q, const float *v) {
   if (side == 0) A3(q, i, k, 1) = A3(v, i, k, 1) < 0.f ? A3(q, ii, k, 2) : 0.f;
   else A3(q, i, k, jbe) = A3(v, i, k, jbe + 1) > 0.f ? A3(q, ii, k, jbe - 1) : 0.f;
 }
-__global__ void k_flow_dep_cols(const DevCtx xv, float *q, const float *u) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_flow_dep_cols(const DevCtx *xv, float *q, const float *u) {
+  const CtxPtr x = ctx_ptr(xv);
   const int j = 2 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   const int side = (int)blockIdx.z;
@@ -290,8 +290,8 @@ struct FinalList {
   BPtrs b[kFinalMax], bt[kFinalMax];
   int ibe[kFinalMax], jbe[kFinalMax], kt[kFinalMax], is2d[kFinalMax], msfc[kFinalMax], muc[kFinalMax];
 };
-__global__ void k_spec_final(const DevCtx xv, FinalList L, const float *__restrict__ dt_bc_p) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_spec_final(const DevCtx *xv, FinalList L, const float *__restrict__ dt_bc_p) {
+  const CtxPtr x = ctx_ptr(xv);
   const float dt_bc = *dt_bc_p;
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
@@ -311,8 +311,8 @@ __global__ void k_spec_final(const DevCtx xv, FinalList L, const float *__restri
 }
 
 // set_w_surface (module_bc_em.py:448-560) without the fill option
-__global__ void k_set_w_surface(const DevCtx xv) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_set_w_surface(const DevCtx *xv) {
+  const CtxPtr x = ctx_ptr(xv);
   const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int j = 1 + (int)blockIdx.y;
   if (i > x->ide - 1 || j > x->jde - 1) return;

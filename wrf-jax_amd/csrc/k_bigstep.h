@@ -19,8 +19,8 @@ __global__ void k_copy(float *dst, const float *src, size_t n) {
 
 // mut, muu, muv (calc_mu_uv, module_big_step_utilities_em.py:174-266) and
 // muus/muvs from muts (calc_mu_uv_1).  2-D over i [1, ide], j [1, jde].
-__global__ void k_mu_uv(const DevCtx xv, const float *mu, const float *mub, float *muu, float *muv, float *mut) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_mu_uv(const DevCtx *xv, const float *mu, const float *mub, float *muu, float *muv, float *mut) {
+  const CtxPtr x = ctx_ptr(xv);
   const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int j = 1 + (int)blockIdx.y;
   const int ide = x->ide, jde = x->jde;
@@ -46,8 +46,8 @@ __global__ void k_mu_uv(const DevCtx xv, const float *mu, const float *mub, floa
 
 // couple_momentum + calc_cq + calc_alt + calc_php over the full 3-D extent
 // (zero outside each field's range, as the reference's fresh outputs).
-__global__ void k_rk_prep3(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_rk_prep3(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned o = XI3(i, k, j), o2 = XI2(i, j);
@@ -125,8 +125,8 @@ __global__ void k_rk_prep3(const DevCtx xv, R3 r) {
 // (kde - 1) x 64 floats); the column sum and the integration then run in the
 // reference's level order, and the integration's stores never hold up a
 // load.
-__global__ void __launch_bounds__(64) k_ww_cp(const DevCtx xv, R2 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(64) k_ww_cp(const DevCtx *xv, R2 r) {
+  const CtxPtr x = ctx_ptr(xv);
   constexpr int kMaxLev = 152;  // kde <= 151 (wrfdc_create checks nz <= 150)
   __shared__ float s_c1h[kMaxLev], s_c2h[kMaxLev], s_dnw[kMaxLev];
   extern __shared__ float s_div_[];  // (kde - 1) x 64: the divergence of every level
@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(64) k_ww_cp(const DevCtx xv, R2 r) {
 // phi, the w g term and horizontal phi advection (6th/4th/2nd order with the
 // reference's specified-boundary column pattern).  k in [2, kde].
 // the phi tendency at (i,k,j), k in [2, kde], starting from `out`
-__device__ __forceinline__ float rhs_ph_val(const DevCtx *__restrict__ x, int i, int k, int j, float out) {
+__device__ __forceinline__ float rhs_ph_val(CtxPtr x, int i, int k, int j, float out) {
   const int ide = x->ide, jde = x->jde, kde = x->kde, kte = kde;
   const float *c1f = FL(c1f), *c2f = FL(c2f), *fnm = FL(fnm), *fnp = FL(fnp), *rdnw = FL(rdnw);
   const float rdx = x->rdx, rdy = x->rdy, g = x->g, cfn = x->cfn, cfn1 = x->cfn1;
@@ -321,8 +321,8 @@ __device__ __forceinline__ float rhs_ph_val(const DevCtx *__restrict__ x, int i,
   }
   return out;
 }
-__global__ void k_rhs_ph(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_rhs_ph(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   A3(FL(ph_tend), i, k, j) = rhs_ph_val(x, i, k, j, A3(FL(ph_tend), i, k, j));
 }
@@ -331,7 +331,7 @@ __global__ void k_rhs_ph(const DevCtx xv, R3 r) {
 // axis 0: u points i [2, ide-1], j [1, jde-1]; axis 1: v points i [1, ide-1], j [2, jde-1].
 // the amount the pressure gradient subtracts from the u (axis 0) or v
 // (axis 1) tendency at (i,k,j): cq * dp
-__device__ __forceinline__ float hpg_term(const DevCtx *__restrict__ x, int axis, int i, int k, int j) {
+__device__ __forceinline__ float hpg_term(CtxPtr x, int axis, int i, int k, int j) {
   const float *ph = FL(ph_2), *alt = FL(alt), *p = FL(p), *pb = FL(pb), *al = FL(al), *php = FL(php), *mu = FL(mu_2);
   const float *c1h = FL(c1h), *c2h = FL(c2h), *rdnw = FL(rdnw);
   const int di = axis == 0 ? 1 : 0, dj = axis == 0 ? 0 : 1;
@@ -359,8 +359,8 @@ __device__ __forceinline__ float hpg_term(const DevCtx *__restrict__ x, int axis
                 (A1(rdnw, k) * (dpn1 - dpn0) - 0.5f * (A1(c1h, k) * A2(mu, i - di, j - dj) + A1(c1h, k) * A2(mu, i, j)));
   return (axis == 0 ? A3(FL(cqu), i, k, j) : A3(FL(cqv), i, k, j)) * dp;
 }
-__global__ void k_hpg(const DevCtx xv, int axis, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_hpg(const DevCtx *xv, int axis, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   if (axis == 0) A3(FL(ru_tend), i, k, j) = A3(FL(ru_tend), i, k, j) - hpg_term(x, 0, i, k, j);
   else A3(FL(rv_tend), i, k, j) = A3(FL(rv_tend), i, k, j) - hpg_term(x, 1, i, k, j);
@@ -371,7 +371,7 @@ __global__ void k_hpg(const DevCtx xv, int axis, R3 r) {
 // below replaces it by 1 / (1 + cqw)
 // (cq1_out: 1 / (1 + cqw) at level min(k, kde-1), the value pg_buoy_w then
 // stores in cqw)
-__device__ __forceinline__ float buoy_w_term(const DevCtx *__restrict__ x, int i, int k, int j, float *cq1_out = nullptr) {
+__device__ __forceinline__ float buoy_w_term(CtxPtr x, int i, int k, int j, float *cq1_out = nullptr) {
   const float *p = FL(p), *mu = FL(mu_2), *mub = FL(mub), *c1f = FL(c1f), *c2f = FL(c2f);
   const int kde = x->kde, kc = imin_(k, kde - 1);  // cqw and p level: k, kde-1 at the top
   const float gm = (1.f / A2(FL(msfty), i, j)) * x->g;
@@ -387,15 +387,15 @@ __device__ __forceinline__ float buoy_w_term(const DevCtx *__restrict__ x, int i
 // cqw := 1 / (1 + cqw) (the second half of pg_buoy_w): levels [2, kde-1] in
 // the stage API; in the fused step only level kde-1 (the w kernel's top
 // level reads it, so the fused w kernel replaces levels [2, kde-2] itself)
-__global__ void k_cqw_inv(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_cqw_inv(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   float *cqw = FL(cqw);
   A3(cqw, i, k, j) = 1.f / (1.f + A3(cqw, i, k, j));
 }
 // pg_buoy_w (module_big_step_utilities_em.py:1674-1800): column kernel
-__global__ void k_pg_buoy_w(const DevCtx xv, R2 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_pg_buoy_w(const DevCtx *xv, R2 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IJ(r);
   float *rwt = FL(rw_tend), *cqw = FL(cqw);
   const float *p = FL(p), *mu = FL(mu_2), *mub = FL(mub), *c1f = FL(c1f), *c2f = FL(c2f), *rdnw = FL(rdnw), *rdn = FL(rdn);
@@ -417,7 +417,7 @@ __global__ void k_pg_buoy_w(const DevCtx xv, R2 r) {
 
 // coriolis + curvature (module_big_step_utilities_em.py:978-1120, 1214-1449)
 // for specified boundaries.  comp 0: u points; 1: v points; 2: w points.
-__device__ __forceinline__ float vxgm(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ float vxgm(CtxPtr x, int i, int k, int j) {
   const float *u = FL(u_2), *v = FL(v_2);
   return 0.5f * (A3(u, i, k, j) + A3(u, i + 1, k, j)) * (A2(FL(msfvx), i, j + 1) - A2(FL(msfvx), i, j)) * x->rdy -
          0.5f * (A3(v, i, k, j) + A3(v, i, k, j + 1)) * (A2(FL(msfuy), i + 1, j) - A2(FL(msfuy), i, j)) * x->rdx;
@@ -425,7 +425,7 @@ __device__ __forceinline__ float vxgm(const DevCtx *__restrict__ x, int i, int k
 // The terms of each component as values of their own (a kernel can issue
 // their loads with its others) and their accumulation in the reference's
 // order.
-__device__ __forceinline__ float4 cor_u_terms(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ float4 cor_u_terms(CtxPtr x, int i, int k, int j) {
   const float *rv = FL(rv), *rw = FL(rw), *u = FL(u_2);
   const float *f = FL(f), *e = FL(e), *cosa = FL(cosa);
   const float rer = x->reradius;
@@ -443,8 +443,8 @@ __device__ __forceinline__ float cor_u_add(float val, float4 c) {
   val = val - c.y;
   return val + c.z - c.w;
 }
-__device__ __forceinline__ float cor_curv_u(const DevCtx *__restrict__ x, int i, int k, int j, float val) { return cor_u_add(val, cor_u_terms(x, i, k, j)); }
-__device__ __forceinline__ float4 cor_v_terms(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ float cor_curv_u(CtxPtr x, int i, int k, int j, float val) { return cor_u_add(val, cor_u_terms(x, i, k, j)); }
+__device__ __forceinline__ float4 cor_v_terms(CtxPtr x, int i, int k, int j) {
   const float *ru = FL(ru), *rw = FL(rw), *v = FL(v_2);
   const float *f = FL(f), *e = FL(e), *sina = FL(sina);
   const float rer = x->reradius;
@@ -462,8 +462,8 @@ __device__ __forceinline__ float cor_v_add(float val, float4 c) {
   val = val + c.y;
   return val - c.z - c.w;
 }
-__device__ __forceinline__ float cor_curv_v(const DevCtx *__restrict__ x, int i, int k, int j, float val) { return cor_v_add(val, cor_v_terms(x, i, k, j)); }
-__device__ __forceinline__ float2 cor_w_terms(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ float cor_curv_v(CtxPtr x, int i, int k, int j, float val) { return cor_v_add(val, cor_v_terms(x, i, k, j)); }
+__device__ __forceinline__ float2 cor_w_terms(CtxPtr x, int i, int k, int j) {
   const float *ru = FL(ru), *rv = FL(rv), *u = FL(u_2), *v = FL(v_2);
   const float *e = FL(e), *sina = FL(sina), *cosa = FL(cosa), *fzm = FL(fnm), *fzp = FL(fnp);
   const float rer = x->reradius;
@@ -481,9 +481,9 @@ __device__ __forceinline__ float cor_w_add(float val, float2 c) {
   val = val + c.x;
   return val + c.y;
 }
-__device__ __forceinline__ float cor_curv_w(const DevCtx *__restrict__ x, int i, int k, int j, float val) { return cor_w_add(val, cor_w_terms(x, i, k, j)); }
-__global__ void k_cor_curv(const DevCtx xv, int comp, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__device__ __forceinline__ float cor_curv_w(CtxPtr x, int i, int k, int j, float val) { return cor_w_add(val, cor_w_terms(x, i, k, j)); }
+__global__ void k_cor_curv(const DevCtx *xv, int comp, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   if (comp == 0) A3(FL(ru_tend), i, k, j) = cor_curv_u(x, i, k, j, A3(FL(ru_tend), i, k, j));
   else if (comp == 1) A3(FL(rv_tend), i, k, j) = cor_curv_v(x, i, k, j, A3(FL(rv_tend), i, k, j));
@@ -510,22 +510,22 @@ __device__ __forceinline__ float tendf_fold(float *tf, unsigned o, float2 ld, fl
   }
   return v;
 }
-__device__ __forceinline__ float addtend_u(const DevCtx *__restrict__ x, int i, int k, int j, int rk, float t) {
+__device__ __forceinline__ float addtend_u(CtxPtr x, int i, int k, int j, int rk, float t) {
   const unsigned o = XI3(i, k, j);
   const float m = A2(FL(msfuy), i, j);
   return t + tendf_fold(FL(ru_tendf), o, tendf_load(FL(ru_tendf), FL(u_save), o, rk), m, rk) / m;
 }
-__device__ __forceinline__ float addtend_v(const DevCtx *__restrict__ x, int i, int k, int j, int rk, float t) {
+__device__ __forceinline__ float addtend_v(CtxPtr x, int i, int k, int j, int rk, float t) {
   const unsigned o = XI3(i, k, j);
   return t + tendf_fold(FL(rv_tendf), o, tendf_load(FL(rv_tendf), FL(v_save), o, rk), A2(FL(msfvx), i, j), rk) * A2(FL(msfvx_inv), i, j);
 }
-__device__ __forceinline__ float addtend_w(const DevCtx *__restrict__ x, int i, int k, int j, int rk, float t) {
+__device__ __forceinline__ float addtend_w(CtxPtr x, int i, int k, int j, int rk, float t) {
   const unsigned o = XI3(i, k, j);
   const float m = A2(FL(msfty), i, j);
   return t + tendf_fold(FL(rw_tendf), o, tendf_load(FL(rw_tendf), FL(w_save), o, rk), m, rk) / m;
 }
 // (the saved phi and theta tendencies carry no weight: x * 1 is x)
-__device__ __forceinline__ float addtend_ph(const DevCtx *__restrict__ x, int i, int k, int j, int rk, float t) {
+__device__ __forceinline__ float addtend_ph(CtxPtr x, int i, int k, int j, int rk, float t) {
   const unsigned o = XI3(i, k, j);
   const float m = A2(FL(msfty), i, j);
   return t + tendf_fold(FL(ph_tendf), o, tendf_load(FL(ph_tendf), FL(ph_save), o, rk), 1.f, rk) / m;
@@ -533,7 +533,7 @@ __device__ __forceinline__ float addtend_ph(const DevCtx *__restrict__ x, int i,
 // theta: also the diabatic heating, and the column's mu tendency at k = 1
 // mu_zero: mu_tend is known to be 0 here (a later stage of the fused step,
 // which does not clear it) and is formed as 0 + mu_tendf
-__device__ __forceinline__ float addtend_t(const DevCtx *__restrict__ x, int i, int k, int j, int rk, float t, bool mu_zero = false) {
+__device__ __forceinline__ float addtend_t(CtxPtr x, int i, int k, int j, int rk, float t, bool mu_zero = false) {
   const unsigned o = XI3(i, k, j);
   const float m = A2(FL(msfty), i, j);
   const float mass = A1(FL(c1h), k) * A2(FL(mut), i, j) + A1(FL(c2h), k);
@@ -543,8 +543,8 @@ __device__ __forceinline__ float addtend_t(const DevCtx *__restrict__ x, int i, 
   return t + tf / m + heating;
 }
 // comp 0 u, 1 v, 2 w/ph, 3 theta
-__global__ void k_addtend(const DevCtx xv, int comp, int rk, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_addtend(const DevCtx *xv, int comp, int rk, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const unsigned o = XI3(i, k, j);
   if (comp == 0) {
@@ -560,8 +560,8 @@ __global__ void k_addtend(const DevCtx xv, int comp, int rk, R3 r) {
 }
 
 // _calc_p_rho_phi_nonhydro_opt2 (runtime.py:12369-12537): hypsometric al, EOS p
-__global__ void k_calc_p_rho_phi(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_calc_p_rho_phi(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const float *muts = FL(muts), *ph = FL(ph_2), *phb = FL(phb), *alb = FL(alb), *pb = FL(pb), *t = FL(t_2);
   const float m = A2(muts, i, j), ptop = x->ptop;

@@ -73,9 +73,9 @@ __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? l
 // normalised inputs of every point of the range: fd = (log(|D| + 1e-7) -
 // d_shift) / d_scale and fn = (N^2 - n_shift) / n_scale (|D| as k_smag
 // stored it)
-__global__ void k_closure_feat(const DevCtx xv, R3 r, ClosureNorm nm, const float *__restrict__ defmag, float *__restrict__ fd,
+__global__ void k_closure_feat(const DevCtx *xv, R3 r, ClosureNorm nm, const float *__restrict__ defmag, float *__restrict__ fd,
                                float *__restrict__ fn) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   A3(fd, i, k, j) = (logf(A3(defmag, i, k, j) + 1e-7f) - nm.d_shift) / nm.d_scale;
   A3(fn, i, k, j) = (A3(FL(bn2), i, k, j) - nm.n_shift) / nm.n_scale;
@@ -111,9 +111,9 @@ __device__ __forceinline__ bf16x8 pack8(const float v[8]) {
   for (int q = 0; q < 8; q++) r[q] = (__bf16)v[q];
   return r;
 }
-__global__ void __launch_bounds__(256) k_closure_km(const DevCtx xv, R3 r, const float *__restrict__ theta, const __bf16 *__restrict__ wbf,
+__global__ void __launch_bounds__(256) k_closure_km(const DevCtx *xv, R3 r, const float *__restrict__ theta, const __bf16 *__restrict__ wbf,
                                                     ClosureNorm nm, const float *__restrict__ fd, const float *__restrict__ divisor) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   __shared__ __align__(16) __bf16 s_w[2][64 * kLd];
   __shared__ __align__(16) __bf16 s_h[4][16 * kLd];
   __shared__ float s_z[4][64];
@@ -232,9 +232,9 @@ __global__ void __launch_bounds__(256) k_closure_km(const DevCtx xv, R3 r, const
 // With a row per lane, in 64 two-byte stores 128 bytes apart, the kernel took
 // 254 us for 96x96x40 (353440 rows, 54 MB), 30 us this way.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_closure_rows(const DevCtx xv, R3 r, ClosureNorm nm, const float *__restrict__ fd,
+__global__ void __launch_bounds__(256) k_closure_rows(const DevCtx *xv, R3 r, ClosureNorm nm, const float *__restrict__ fd,
                                                       const float *__restrict__ fn, const float *__restrict__ divisor, __bf16 *X, float *T) {
-  const DevCtx *__restrict__ x = &xv;
+  const CtxPtr x = ctx_ptr(xv);
   // the tiles of GET_IKJ_P, with the wave's lanes shared out over its points
   const int ib = 1 + ((r.i0 - 1) & ~63);
   const unsigned gx_ = (unsigned)(r.i1 - ib + 64) / 64u;
@@ -291,8 +291,8 @@ __global__ void __launch_bounds__(256) k_closure_rows(const DevCtx xv, R3 r, Clo
 // points and of their products, t1 = (tau11 - tau22)/2, t2 = tau12 with
 // tau_ab = <a b> - <a><b>; written to columns 0 and 1 of the training rows of
 // the coarse range rc (the same row order as k_closure_rows).
-__global__ void __launch_bounds__(256) k_subgrid_stress(const DevCtx xv, R3 rc, int ratio, float *T) {
-  const DevCtx *__restrict__ x = &xv;  // the fine domain
+__global__ void __launch_bounds__(256) k_subgrid_stress(const DevCtx *xv, R3 rc, int ratio, float *T) {
+  const CtxPtr x = ctx_ptr(xv);  // the fine domain
   GET_IKJ_P(rc);                        // coarse point (i, k, j)
   const float *u = FL(u_2), *v = FL(v_2);
   double su = 0.0, sv = 0.0, suu = 0.0, svv = 0.0, suv = 0.0;

@@ -27,8 +27,8 @@
 #pragma once
 #include "wrfdc_common.h"
 
-__global__ void __launch_bounds__(64) k_tridiag_lanes_columns(const DevCtx xv, const float *rhs, float *wout) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(64) k_tridiag_lanes_columns(const DevCtx *xv, const float *rhs, float *wout) {
+  const CtxPtr x = ctx_ptr(xv);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned gx = (unsigned)(ide - 3 + 63) / 64u;
   const int i = 2 + (int)(blockIdx.x % gx) * 64 + (int)threadIdx.x, j = 2 + (int)(blockIdx.x / gx);
@@ -93,8 +93,8 @@ __device__ __forceinline__ void affine_scan(float &c, float &d, int lane, bool u
 constexpr int kTriStride = 65;  // LDS floats per level row (64 columns + 1)
 __host__ __device__ inline size_t tridiag_levels_lds(int kde) { return (size_t)4 * kde * kTriStride * sizeof(float); }
 
-__global__ void __launch_bounds__(512) k_tridiag_lanes_levels(const DevCtx xv, const float *rhs, float *wout) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(512) k_tridiag_lanes_levels(const DevCtx *xv, const float *rhs, float *wout) {
+  const CtxPtr x = ctx_ptr(xv);
   extern __shared__ float sm[];
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const int lane = (int)threadIdx.x, wv = (int)threadIdx.y;

@@ -8,15 +8,15 @@
 
 // rho = (1 + qv) / alt on mass points (phy_prep,
 // module_big_step_utilities_em.py:1823-2081, rho at :1965)
-__global__ void k_rho(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_rho(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   A3(FL(rho), i, k, j) = (1.f / A3(FL(alt), i, k, j)) * (1.f + A3(SP(moist, 0), i, k, j));
 }
 
 // compute_diff_metrics (module_diffusion_em.py:1825-2043), full extent.
-__global__ void k_diff_metrics(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_diff_metrics(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde, ktf = kde - 1;
   const float *ph = FL(ph_2), *phb = FL(phb);
@@ -55,12 +55,12 @@ __global__ void k_diff_metrics(const DevCtx xv, R3 r) {
 }
 
 // value of a staggered field scaled by a map factor
-__device__ __forceinline__ float hatv(const DevCtx *__restrict__ x, const float *f, const float *m, int i, int k, int j) {
+__device__ __forceinline__ float hatv(CtxPtr x, const float *f, const float *m, int i, int k, int j) {
   return A3(f, i, k, j) / A2(m, i, j);
 }
 // average of the two columns A and B of hat = f / m onto w level k
 // (the hatavg construction shared by the deformation components)
-__device__ __forceinline__ float hat_avg(const DevCtx *__restrict__ x, const float *f, const float *m, int ia, int ja, int ib, int jb, int k) {
+__device__ __forceinline__ float hat_avg(CtxPtr x, const float *f, const float *m, int ia, int ja, int ib, int jb, int k) {
   const int kte = x->kde, ktes1 = kte - 1, ktes2 = kte - 2;
   if (k == 1)
     return 0.5f * (x->cf1 * hatv(x, f, m, ia, 1, ja) + x->cf2 * hatv(x, f, m, ia, 2, ja) + x->cf3 * hatv(x, f, m, ia, 3, ja) +
@@ -76,8 +76,8 @@ __device__ __forceinline__ float hat_avg(const DevCtx *__restrict__ x, const flo
 
 // cal_deform_and_div (module_diffusion_em.py:366-891): D11, D22, D33 and the
 // divergence on mass points.
-__global__ void k_deform_diag(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_deform_diag(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *u = FL(u_2), *v = FL(v_2), *w = FL(w_2), *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw);
   const float *msfuy = FL(msfuy), *msfvx = FL(msfvx);
@@ -104,8 +104,8 @@ __global__ void k_deform_diag(const DevCtx xv, R3 r) {
 }
 
 // D12 at (u, v) corner points i [2, ide-1], j [2, jde-1], k [1, kde-1]
-__global__ void k_deform12(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_deform12(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *u = FL(u_2), *v = FL(v_2), *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw), *msfux = FL(msfux), *msfvy = FL(msfvy);
   const float mm = 0.25f * (A2(msfux, i, j - 1) + A2(msfux, i, j)) * (A2(msfvy, i - 1, j) + A2(msfvy, i, j));
@@ -127,8 +127,8 @@ __global__ void k_deform12(const DevCtx xv, R3 r) {
 }
 
 // D13 / D23 at (u, w) and (v, w) points i [2, ide-1], j [2, jde-1], k [1, kde]
-__global__ void k_deform13_23(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_deform13_23(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int ktf = x->kde - 1;
   float *d13 = FL(defor13), *d23 = FL(defor23);
@@ -165,8 +165,8 @@ __global__ void k_deform13_23(const DevCtx xv, R3 r) {
 
 // edge copy of whole planes: i = idst <- isrc for every (k, j) (axis 0) or
 // j = jdst <- jsrc for every (i, k) (axis 1); up to two fields per launch.
-__global__ void k_edge_copy(const DevCtx xv, float *f0, float *f1, int axis, int dst, int src, int kend) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_edge_copy(const DevCtx *xv, float *f0, float *f1, int axis, int dst, int src, int kend) {
+  const CtxPtr x = ctx_ptr(xv);
   const int a = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   if (k > kend) return;
@@ -184,8 +184,8 @@ __global__ void k_edge_copy(const DevCtx xv, float *f0, float *f1, int axis, int
 // smag2d_km (module_diffusion_em.py:1502-1646) with the slope correction;
 // i [2, ide-2], j [2, jde-2], k [1, kde-1].  With the learned closure on,
 // |D| = sqrt(def2) and the slope divisor are stored too (defmag, divisor).
-__global__ void k_smag(const DevCtx xv, R3 r, float *defmag = nullptr, float *divout = nullptr) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_smag(const DevCtx *xv, R3 r, float *defmag = nullptr, float *divout = nullptr) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *d11 = FL(defor11), *d22 = FL(defor22), *d12 = FL(defor12), *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw);
   const float dx = x->dx, dy = x->dy, c_s = x->c_s;
@@ -222,7 +222,7 @@ __global__ void k_smag(const DevCtx xv, R3 r, float *defmag = nullptr, float *di
 struct Thermo {
   float th, p, t;
 };
-__device__ __forceinline__ Thermo thermo_at(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ Thermo thermo_at(CtxPtr x, int i, int k, int j) {
   Thermo r;
   r.th = A3(FL(t_2), i, k, j) + x->t0;
   r.p = A3(FL(p), i, k, j) + A3(FL(pb), i, k, j);
@@ -235,13 +235,13 @@ __device__ __forceinline__ float qvs_of(float t, float p) {
   const float es = 1000.0f * 0.6112f * expf(17.67f * (t - 273.15f) / (t - 29.65f));
   return (float)(287.0 / 461.6) * es / (p - es);
 }
-__device__ __forceinline__ float qtot_at(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ float qtot_at(CtxPtr x, int i, int k, int j) {
   float q = A3(SP(moist, 0), i, k, j);
   if (x->nmoist > 1) q = q + A3(SP(moist, 1), i, k, j);
   if (x->nmoist > 3) q = q + A3(SP(moist, 3), i, k, j);
   return q;
 }
-__device__ __forceinline__ float qc_at(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ float qc_at(CtxPtr x, int i, int k, int j) {
   return x->nmoist > 1 ? A3(SP(moist, 1), i, k, j) : 0.f;
 }
 
@@ -250,8 +250,8 @@ __device__ __forceinline__ float qc_at(const DevCtx *__restrict__ x, int i, int 
 // surface values (pressure and temperature on w level 1 through mass levels
 // 1 and 2, linear in height), level ktf repeats ktf-1.  i [2, ide-2],
 // k [1, kde-1], j [2, jde-2]; one thread per point.
-__global__ void k_n2(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_n2(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const float G = 9.81f, R_D = 287.0f, CP = (float)(7.0 * 287.0 / 2.0), XLV = 2.5e6f, RV = 461.6f, C161 = 1.61f;
   const float *qv = SP(moist, 0), *rdz = FL(rdz), *rdzw = FL(rdzw);
@@ -316,7 +316,7 @@ __global__ void k_n2(const DevCtx xv, R3 r) {
 // diffusivity averaged to the component's point; zero outside [i0,i1]x[j0,j1]
 // (and at k = 1, kde for the 13 / 23 components).  kind 11, 12, 13, 23.
 // one stress component at (i, k, j): zero outside [i0, i1] x [j0, j1] x [1, kde-1]
-__device__ __forceinline__ float titau_val(const DevCtx *__restrict__ x, const float *xk, const float *defor, int kind, int i0, int i1,
+__device__ __forceinline__ float titau_val(CtxPtr x, const float *xk, const float *defor, int kind, int i0, int i1,
                                            int j0, int j1, int i, int k, int j) {
   const float *rho = FL(rho);
   const int ktf = x->kde - 1;
@@ -344,8 +344,8 @@ struct TitauPair {
   const float *xk[2], *defor[2];
   int kind[2], i0[2], i1[2], j0[2], j1[2];
 };
-__global__ void k_titau(const DevCtx xv, TitauPair P, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_titau(const DevCtx *xv, TitauPair P, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float v0 = titau_val(x, P.xk[0], P.defor[0], P.kind[0], P.i0[0], P.i1[0], P.j0[0], P.j1[0], i, k, j);
   const float v1 = titau_val(x, P.xk[1], P.defor[1], P.kind[1], P.i0[1], P.i1[1], P.j0[1], P.j1[1], i, k, j);
@@ -355,16 +355,16 @@ __global__ void k_titau(const DevCtx xv, TitauPair P, R3 r) {
 
 // horizontal_diffusion_u_2 (module_diffusion_em.py:2302-2532):
 // u points i [2, ide-1], j [2, jde-2], k [1, kde-1].
-__device__ __forceinline__ float hd_a1u(const DevCtx *__restrict__ x, const float *t1, int i, int k, int j) {
+__device__ __forceinline__ float hd_a1u(CtxPtr x, const float *t1, int i, int k, int j) {
   if (k == 1 || k == x->kde) return 0.f;
   return 0.5f * (A1(FL(fnm), k) * (A3(t1, i - 1, k, j) + A3(t1, i, k, j)) + A1(FL(fnp), k) * (A3(t1, i - 1, k - 1, j) + A3(t1, i, k - 1, j)));
 }
-__device__ __forceinline__ float hd_a2u(const DevCtx *__restrict__ x, const float *t2, int i, int k, int j) {
+__device__ __forceinline__ float hd_a2u(CtxPtr x, const float *t2, int i, int k, int j) {
   if (k == 1 || k == x->kde) return 0.f;
   return 0.5f * (A1(FL(fnm), k) * (A3(t2, i, k, j + 1) + A3(t2, i, k, j)) + A1(FL(fnp), k) * (A3(t2, i, k - 1, j + 1) + A3(t2, i, k - 1, j)));
 }
-__global__ void k_hdiff_u(const DevCtx xv, const float *t1, const float *t2, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_hdiff_u(const DevCtx *xv, const float *t1, const float *t2, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw);
   const float zxu = 0.5f * (A3(zx, i, k, j) + A3(zx, i, k + 1, j));
@@ -382,16 +382,16 @@ __global__ void k_hdiff_u(const DevCtx xv, const float *t1, const float *t2, R3 
 
 // horizontal_diffusion_v_2 (module_diffusion_em.py:2535-2765):
 // v points i [2, ide-2], j [2, jde-1], k [1, kde-1].
-__device__ __forceinline__ float hd_a1v(const DevCtx *__restrict__ x, const float *t1, int i, int k, int j) {
+__device__ __forceinline__ float hd_a1v(CtxPtr x, const float *t1, int i, int k, int j) {
   if (k == 1 || k == x->kde) return 0.f;
   return 0.5f * (A1(FL(fnm), k) * (A3(t1, i + 1, k, j) + A3(t1, i, k, j)) + A1(FL(fnp), k) * (A3(t1, i + 1, k - 1, j) + A3(t1, i, k - 1, j)));
 }
-__device__ __forceinline__ float hd_a2v(const DevCtx *__restrict__ x, const float *t2, int i, int k, int j) {
+__device__ __forceinline__ float hd_a2v(CtxPtr x, const float *t2, int i, int k, int j) {
   if (k == 1 || k == x->kde) return 0.f;
   return 0.5f * (A1(FL(fnm), k) * (A3(t2, i, k, j - 1) + A3(t2, i, k, j)) + A1(FL(fnp), k) * (A3(t2, i, k - 1, j - 1) + A3(t2, i, k - 1, j)));
 }
-__global__ void k_hdiff_v(const DevCtx xv, const float *t1, const float *t2, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_hdiff_v(const DevCtx *xv, const float *t1, const float *t2, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw);
   const float zxv = 0.125f * (A3(zx, i, k, j) + A3(zx, i + 1, k, j) + A3(zx, i, k, j - 1) + A3(zx, i + 1, k, j - 1) + A3(zx, i, k + 1, j) +
@@ -409,8 +409,8 @@ __global__ void k_hdiff_v(const DevCtx xv, const float *t1, const float *t2, R3 
 
 // horizontal_diffusion_w_2 (module_diffusion_em.py:2768-2985):
 // w points i [2, ide-2], j [2, jde-2], k [2, kde-1].
-__global__ void k_hdiff_w(const DevCtx xv, const float *t1, const float *t2, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_hdiff_w(const DevCtx *xv, const float *t1, const float *t2, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *zx = FL(zx), *zy = FL(zy), *rdz = FL(rdz);
 #define HA1(kk) (0.25f * (A3(t1, i + 1, (kk) + 1, j) + A3(t1, i, (kk) + 1, j) + A3(t1, i + 1, kk, j) + A3(t1, i, kk, j)))
@@ -440,11 +440,11 @@ __global__ void k_hdiff_w(const DevCtx xv, const float *t1, const float *t2, R3 
 // the values at levels k-1, k, k+1, k+2 of each column (qa[0..3], qb[0..3]):
 // at level k (surface extrapolation at k = 1) and at level k+1 (the top
 // extrapolation at kde); hs_hav's three forms with the same arithmetic.
-__device__ __forceinline__ float hs_hav_dn(const DevCtx *__restrict__ x, const float qa[4], const float qb[4], int k, float fm, float fp) {
+__device__ __forceinline__ float hs_hav_dn(CtxPtr x, const float qa[4], const float qb[4], int k, float fm, float fp) {
   if (k == 1) return 0.5f * (x->cf1 * qa[1] + x->cf2 * qa[2] + x->cf3 * qa[3] + x->cf1 * qb[1] + x->cf2 * qb[2] + x->cf3 * qb[3]);
   return 0.5f * (fm * (qb[1] + qa[1]) + fp * (qb[0] + qa[0]));
 }
-__device__ __forceinline__ float hs_hav_up(const DevCtx *__restrict__ x, const float qa[4], const float qb[4], int k, float fm, float fp,
+__device__ __forceinline__ float hs_hav_up(CtxPtr x, const float qa[4], const float qb[4], int k, float fm, float fp,
                                            float dnw1, float dn1) {
   if (k + 1 == x->kde)
     return 0.5f * (qa[1] + (qa[1] - qa[0]) * 0.5f * dnw1 / dn1 + qb[1] + (qb[1] - qb[0]) * 0.5f * dnw1 / dn1);
@@ -457,7 +457,7 @@ __device__ __forceinline__ float hs_hav_up(const DevCtx *__restrict__ x, const f
 struct HsFace {
   float c, tz, rdz;
 };
-__device__ __forceinline__ HsFace hs_face(const DevCtx *__restrict__ x, const float *zs, float msf, int ia, int ja, int ib, int jb, int k) {
+__device__ __forceinline__ HsFace hs_face(CtxPtr x, const float *zs, float msf, int ia, int ja, int ib, int jb, int k) {
   const float *xkhh = FL(xkhh), *rho = FL(rho), *rdzw = FL(rdzw);
   HsFace f;
   const float xk = 0.5f * (A3(xkhh, ib, k, jb) + A3(xkhh, ia, k, ja)) * 0.5f * (A3(rho, ib, k, jb) + A3(rho, ia, k, ja));
@@ -482,8 +482,8 @@ struct HdsList {
 // pass 1: H1 at u faces i [2, ide-1], j [2, jde-2] and H2 at v faces
 // i [2, ide-2], j [2, jde-1] of every scalar; r = i [2, ide-1], k [1, kde-1],
 // j [2, jde-1]
-__global__ void __launch_bounds__(256) k_hdiff_s_faces(const DevCtx xv, HdsList L, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(256) k_hdiff_s_faces(const DevCtx *xv, HdsList L, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int ide = x->ide, jde = x->jde;
   const bool f1 = (i <= ide - 1 && j <= jde - 2), f2 = (i <= ide - 2 && j <= jde - 1);
@@ -521,8 +521,8 @@ __global__ void __launch_bounds__(256) k_hdiff_s_faces(const DevCtx xv, HdsList 
 
 // pass 2: tendency of every scalar on mass points i [2, ide-2], j [2, jde-2],
 // k [1, kde-1] (r)
-__global__ void __launch_bounds__(256) k_hdiff_s_tend(const DevCtx xv, HdsList L, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(256) k_hdiff_s_tend(const DevCtx *xv, HdsList L, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const float *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw), *fnm = FL(fnm), *fnp = FL(fnp);
   const int ktf = x->kde - 1;

@@ -8,8 +8,8 @@
 
 // small_step_prep, 2-D part (module_small_step_em.py:272-420): stage-start
 // column masses.  i [1, ide], j [1, jde].
-__global__ void k_ssp_mass(const DevCtx xv, int rk) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_ssp_mass(const DevCtx *xv, int rk) {
+  const CtxPtr x = ctx_ptr(xv);
   const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int j = 1 + (int)blockIdx.y;
   const int ide = x->ide, jde = x->jde;
@@ -59,8 +59,8 @@ __global__ void k_ssp_mass(const DevCtx xv, int rk) {
 // full-extent fields), then the stores of the staggerings the point belongs
 // to; RK1: the first RK stage (stage-start copies, perturbations zero).
 template <bool RK1>
-__global__ void k_ssp_3d(const DevCtx xv, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_ssp_3d(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned o = XI3(i, k, j), o2 = XI2(i, j);
@@ -122,8 +122,8 @@ __global__ void k_ssp_3d(const DevCtx xv, R3 r) {
 
 // calc_p_rho, non-hydrostatic (module_small_step_em.py:720-1034) with
 // ph = ph_2, t_1 = t_save, mu = mu_2, mut = muts; mass points.
-__global__ void k_calc_p_rho(const DevCtx xv, int step, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_calc_p_rho(const DevCtx *xv, int step, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const unsigned o = XI3(i, k, j);
   // every load first (the stores below could alias them as far as the
@@ -147,8 +147,8 @@ __global__ void k_calc_p_rho(const DevCtx xv, int step, R3 r) {
 
 // calc_coef_w (module_small_step_em.py:1359-1586): LU factors of the
 // implicit w-phi system, one thread per mass column.
-__global__ void k_calc_coef_w(const DevCtx xv, float dts, R2 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_calc_coef_w(const DevCtx *xv, float dts, R2 r) {
+  const CtxPtr x = ctx_ptr(xv);
   // the column coefficients in LDS: read per level inside the recurrence, and
   // from global memory every such read would wait behind the previous level's
   // stores (the compiler cannot prove they do not alias)
@@ -219,7 +219,7 @@ __global__ void k_calc_coef_w(const DevCtx xv, float dts, R2 r) {
 }
 
 // interface pressure of a u/v face (module_small_step_em.py:1627-1645)
-__device__ __forceinline__ float uv_iface(const DevCtx *__restrict__ x, const float *p, int i, int j, int di, int dj, int level) {
+__device__ __forceinline__ float uv_iface(CtxPtr x, const float *p, int i, int j, int di, int dj, int level) {
 #define PP(kk) (A3(p, i, kk, j) + A3(p, i - di, kk, j - dj))
   if (level == 1) return 0.5f * (x->cf1 * PP(1) + x->cf2 * PP(2) + x->cf3 * PP(3));
   if (level >= 2 && level <= x->kde - 1) return 0.5f * (A1(FL(fnm), level) * PP(level) + A1(FL(fnp), level) * PP(level - 1));
@@ -229,8 +229,8 @@ __device__ __forceinline__ float uv_iface(const DevCtx *__restrict__ x, const fl
 
 // advance_uv (module_small_step_em.py:1589-1987), specified boundaries.
 // axis 0: u on i [2, ide-1], j [2, jde-2]; axis 1: v on i [2, ide-2], j [2, jde-1].
-__global__ void k_advance_uv(const DevCtx xv, int axis, float dts, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_advance_uv(const DevCtx *xv, int axis, float dts, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int di = axis == 0 ? 1 : 0, dj = axis == 0 ? 0 : 1;
   float *vel = axis == 0 ? FL(u_2) : FL(v_2);
@@ -259,7 +259,7 @@ __global__ void k_advance_uv(const DevCtx xv, int axis, float dts, R3 r) {
 }
 
 // horizontal mass divergence of one level for advance_mu_t
-__device__ __forceinline__ float mut_dvdxi(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ float mut_dvdxi(CtxPtr x, int i, int k, int j) {
   const float *u = FL(u_2), *u1 = FL(u_save), *v = FL(v_2), *v1 = FL(v_save), *muu = FL(muu), *muv = FL(muv);
   const float *msfuy = FL(msfuy), *msfvx_inv = FL(msfvx_inv);
   const float c1 = A1(FL(c1h), k), c2 = A1(FL(c2h), k);
@@ -274,8 +274,8 @@ __device__ __forceinline__ float mut_dvdxi(const DevCtx *__restrict__ x, int i, 
 // advance_mu_t (module_small_step_em.py:2024-2403) with u_1 = u_save,
 // v_1 = v_save, t_1 = t_save, t_ave = t_2ave, ft = t_tend; one thread per
 // column i [2, ide-2], j [2, jde-2].
-__global__ void k_advance_mu_t(const DevCtx xv, float dts, R2 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_advance_mu_t(const DevCtx *xv, float dts, R2 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IJ(r);
   float *ww = FL(ww), *t = FL(t_2), *t_ave = FL(t_2ave);
   const float *ww_1 = FL(ww_1), *t_1 = FL(t_save), *ft = FL(t_tend), *u = FL(u_2), *v = FL(v_2);
@@ -331,8 +331,8 @@ __global__ void k_advance_mu_t(const DevCtx xv, float dts, R2 r) {
 // ph_1 = ph_save; one thread per column i [2, ide-2], j [2, jde-2].  The
 // right-hand side of the phi equation is staged in the scratch array `rhs`
 // (w levels); the forward sweep of the tridiagonal solve runs in w itself.
-__global__ void k_advance_w(const DevCtx xv, float dts, float *__restrict__ rhs, R2 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_advance_w(const DevCtx *xv, float dts, float *__restrict__ rhs, R2 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IJ(r);
   float *w = FL(w_2), *ph = FL(ph_2), *t_2ave = FL(t_2ave);
   const float *rw_tend = FL(rw_tend), *ww = FL(ww), *u = FL(u_2), *v = FL(v_2), *t_2 = FL(t_2), *t_1 = FL(t_save);
@@ -414,8 +414,8 @@ __global__ void k_advance_w(const DevCtx xv, float dts, float *__restrict__ rhs,
 // sumflux (module_small_step_em.py:3134-3310) with ru = u_2, rv = v_2,
 // u_lin = u_save, v_lin = v_save, ww_lin = ww_1; full extent so the first
 // iteration also clears points outside the flux ranges.
-__global__ void k_sumflux(const DevCtx xv, int first, int fin, float ns, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_sumflux(const DevCtx *xv, int first, int fin, float ns, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const size_t o = XI3(i, k, j);
@@ -449,8 +449,8 @@ __global__ void k_sumflux(const DevCtx xv, int first, int fin, float ns, R3 r) {
 // (loads first, as k_ssp_3d; FINAL: the last RK stage, which also removes
 // the diabatic heating)
 template <bool FINAL>
-__global__ void k_ssf(const DevCtx xv, float dts, float nsm, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_ssf(const DevCtx *xv, float dts, float nsm, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned o = XI3(i, k, j), o2 = XI2(i, j);
@@ -490,8 +490,8 @@ __global__ void k_ssf(const DevCtx xv, float dts, float nsm, R3 r) {
 
 // rk_update_scalar_pd (module_em.py:1601-1669): last-stage physics update of
 // the old scalar with mu_old = mu_new = mu_1, then the tendency is cleared.
-__global__ void k_update_scalar_pd(const DevCtx xv, float *q_old, float *q_tend, float dt, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_update_scalar_pd(const DevCtx *xv, float *q_old, float *q_tend, float dt, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const size_t o = XI3(i, k, j);
   const float m = A1(FL(c1h), k) * (A2(FL(mu_1), i, j) + A2(FL(mub), i, j)) + A1(FL(c2h), k);
@@ -501,8 +501,8 @@ __global__ void k_update_scalar_pd(const DevCtx xv, float *q_old, float *q_tend,
 
 // rk_update_scalar (module_em.py:1437-1598): advective tendency (interior
 // only, times msfty) plus the physics tendency, mass-weighted update.
-__global__ void k_update_scalar(const DevCtx xv, float *q, float *q_old, const float *q_tend, int rk, float dt, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_update_scalar(const DevCtx *xv, float *q, float *q_old, const float *q_tend, int rk, float dt, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const size_t o = XI3(i, k, j);
   const int sz = x->spec_zone;

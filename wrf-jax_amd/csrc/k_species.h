@@ -39,7 +39,7 @@ struct UpdCoef {
   float oldm, newm, msfty;
   bool inner;
 };
-__device__ __forceinline__ UpdCoef upd_coef(const DevCtx *__restrict__ x, int i, int k, int j) {
+__device__ __forceinline__ UpdCoef upd_coef(CtxPtr x, int i, int k, int j) {
   UpdCoef c;
   const int sz = x->spec_zone;
   c.inner = (i >= 1 + sz && i <= x->ide - sz - 1 && j >= 1 + sz && j <= x->jde - sz - 1);
@@ -65,8 +65,8 @@ __device__ __forceinline__ UpdCoef upd_coef(const DevCtx *__restrict__ x, int i,
 // c2h), so the last stage finds the same q_old and a cleared tendency.  Each
 // thread reads q_old and the tendency at its own point only, so updating them
 // in place is race-free.
-__global__ void __launch_bounds__(64 * kFaceRows) k_species_update(const DevCtx xv, SpecList L, int rk, float dt, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(64 * kFaceRows) k_species_update(const DevCtx *xv, SpecList L, int rk, float dt, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   extern __shared__ float ys_[];  // L.n x kFaceRows x 64: south face flux of every species
   GET_FACE_BLOCK(r);
 #define YS(s, w) ys_[((s) * kFaceRows + (w)) * 64 + lane]
@@ -143,8 +143,8 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_species_update(const DevCtx 
 // rk_update_scalar_pd (module_em.py:1601-1669) for every species of the list:
 // last-stage physics update of q_old with mu_old = mu_new = mu_1, tendency
 // cleared.
-__global__ void k_species_pd_prep(const DevCtx xv, SpecList L, float dt, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_species_pd_prep(const DevCtx *xv, SpecList L, float dt, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const size_t o = XI3(i, k, j);
   const float m = A1(FL(c1h), k) * (A2(FL(mu_1), i, j) + A2(FL(mub), i, j)) + A1(FL(c2h), k);
@@ -162,7 +162,7 @@ struct PdFace {
   float vel, cr, muf;
   int mode;
 };
-__device__ __forceinline__ PdFace pd_face_geom(const DevCtx *__restrict__ x, int axis, int i, int k, int j, float dt) {
+__device__ __forceinline__ PdFace pd_face_geom(CtxPtr x, int axis, int i, int k, int j, float dt) {
   PdFace f{0.f, 0.f, 0.f, 0};
   const float *c1 = FL(c1h), *c2 = FL(c2h), *mut = FL(muts);
   const int ide = x->ide, jde = x->jde, ktf = x->kde - 1;
@@ -227,8 +227,8 @@ __device__ __forceinline__ void pd_vflux_sel(const PdFace &f, float qm2, float q
 // Face-sharing blocks as k_species_update: the west face comes from this
 // lane, the east face from the next lane, the south face from this wave and
 // the north face from the wave above (LDS).
-__global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_scale(const DevCtx xv, SpecList L, float dt, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_scale(const DevCtx *xv, SpecList L, float dt, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   extern __shared__ float yal_[];  // 2 x L.n x kFaceRows x 64: south antidiffusive / upwind flux of every species
   GET_FACE_BLOCK_LG(r, (unsigned)x->face_lg[2]);
 #define YA(s, w) yal_[((s) * kFaceRows + (w)) * 64 + lane]
@@ -320,8 +320,8 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_scale(const DevCt
 // fluxes are formed again as in pass 1 (face-sharing blocks over the mass
 // points, the same loads and arithmetic, so the same values); each
 // antidiffusive flux is scaled by the factor of the cell it leaves.
-__global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_update(const DevCtx xv, SpecList L, float dt, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_update(const DevCtx *xv, SpecList L, float dt, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   extern __shared__ float yal_[];  // 2 x L.n x kFaceRows x 64: south antidiffusive / upwind flux of every species
   GET_FACE_BLOCK_LG(r, (unsigned)x->face_lg[2]);
 #define YA(s, w) yal_[((s) * kFaceRows + (w)) * 64 + lane]
@@ -418,8 +418,8 @@ struct FlowList {
   float *q[kMaxSpec];
   int n;
 };
-__global__ void k_flow_dep_batch(const DevCtx xv, FlowList L) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void k_flow_dep_batch(const DevCtx *xv, FlowList L) {
+  const CtxPtr x = ctx_ptr(xv);
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = 1 + (int)blockIdx.y;
   const int s = (int)blockIdx.z;

@@ -51,8 +51,8 @@ struct CopyList {
   const float *src[kMaxCopy];
   int n;
 };
-__global__ void __launch_bounds__(256) k_copy_batch(const DevCtx xv, CopyList L, R3 r) {
-  const DevCtx *__restrict__ x = &xv;
+__global__ void __launch_bounds__(256) k_copy_batch(const DevCtx *xv, CopyList L, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
   const unsigned gi = (unsigned)(r.i1 - r.i0 + 256) / 256u;
   const int i0 = r.i0 + (int)(blockIdx.x % gi) * 256 + 4 * (int)threadIdx.x;
   const int k = r.k0 + (int)(blockIdx.x / gi) * 4 + (int)threadIdx.y;
@@ -115,6 +115,7 @@ __device__ __forceinline__ void ck_block_sum(const double s[CK_N], double *out) 
     out[threadIdx.x] = v;
   }
 }
+// (the context by value: wrfdc_checksums_noalloc has none in device memory)
 __global__ void __launch_bounds__(CK_BLOCK) k_checksum_partial(const DevCtx xv, double *part) {
   const DevCtx *__restrict__ x = &xv;
   constexpr int NW = CK_BLOCK / 64;
@@ -193,6 +194,13 @@ struct DtbcList {
   float v[kMaxMembers];
   int n;
 };
+// a context into device memory (by value: no host memory to outlive the launch,
+// and a capture records it like any kernel)
+__global__ void k_put_ctx(DevCtx v, DevCtx *dst) {
+  static_assert(sizeof(DevCtx) % 4 == 0, "copied in words");
+  const unsigned *src = reinterpret_cast<const unsigned *>(&v);
+  for (unsigned q = threadIdx.x; q < sizeof(DevCtx) / 4; q += blockDim.x) reinterpret_cast<unsigned *>(dst)[q] = src[q];
+}
 __global__ void k_put_dtbc(DtbcList L) {
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m < L.n) *L.p[m] = L.v[m];
@@ -256,6 +264,12 @@ struct wrfdc_ctx {
   int rec_n = 0, rec_i = 0;
   int rk = 1, nsmall = 1, iteration = 1;
   double dt_rk = 0.0, dts_rk = 0.0, dtbc = 0.0;
+  // the contexts kernels read: [0] for eager work, [1] for captured work,
+  // each with the species in the caller's buffers and in the library's second
+  // ones; up: what [0] holds (Run::put_ctx)
+  DevCtx *ctx_dev = nullptr;
+  DevCtx up[2];
+  bool up_ok = false;
   Xfer xfer;
   float *dtbc_dev = nullptr;  // dtbc as the boundary kernels read it (one float)
   bool capturing = false;     // a step being captured into a graph leaves dtbc_dev to the replayer
@@ -277,10 +291,9 @@ inline unsigned cdiv(int a, int b) { return (unsigned)((a + b - 1) / b); }
 
 struct Run {
   wrfdc_ctx *X;
-  // passed by value to every kernel: kernels read the field pointers from
-  // kernel arguments.  The moist / scalar entries point at whichever species
-  // buffer holds the current stage's values (the caller's or the library's
-  // second buffer, see species_stage).
+  // host copy of the context the kernels get (D()).  The moist / scalar
+  // entries point at whichever species buffer holds the current stage's
+  // values (the caller's or the library's second buffer, see species_stage).
   mutable DevCtx d;
   hipStream_t s;
   int ide, jde, kde;
@@ -292,7 +305,38 @@ struct Run {
   mutable bool fold_pd_prep = false, pd_prepped = false;
   explicit Run(wrfdc_ctx *x)
       : X(x), d(x->h), s(x->s), ide(x->ide), jde(x->jde), kde(x->kde), user_moist(x->h.F[F_moist]), user_scalar(x->h.F[F_scalar]),
-        alt_moist(x->spec_alt), alt_scalar(x->spec_alt + x->n3 * (size_t)x->c.nmoist) {}
+        alt_moist(x->spec_alt), alt_scalar(x->spec_alt + x->n3 * (size_t)x->c.nmoist) {
+    put_ctx();
+  }
+
+  // Brings the device contexts up to date.  Eager work has a pair of its own,
+  // written when something changed since the last call (a field bound
+  // elsewhere, a tile setting).  Captured work writes another pair at its
+  // start, so that a graph replays with what it was captured with, whatever
+  // eager calls have set in between.
+  const DevCtx *dev_ctx;  // the pair in use
+  void put_ctx() {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!X->capturing && hipStreamIsCapturing(s, &st) != hipSuccess) {
+      (void)hipGetLastError();  // the legacy stream while another one captures: not part of that capture
+      st = hipStreamCaptureStatusNone;
+    }
+    const bool capture = X->capturing || st != hipStreamCaptureStatusNone;
+    DevCtx alt = d;
+    alt.F[F_moist] = alt_moist;
+    alt.F[F_scalar] = (X->c.nscalar > 0) ? alt_scalar : nullptr;
+    DevCtx *pair = X->ctx_dev + (capture ? 2 : 0);
+    dev_ctx = pair;
+    if (!capture && X->up_ok && memcmp(&X->up[0], &d, sizeof d) == 0 && memcmp(&X->up[1], &alt, sizeof alt) == 0) return;
+    k_put_ctx<<<1, 256, 0, s>>>(d, pair);
+    k_put_ctx<<<1, 256, 0, s>>>(alt, pair + 1);
+    if (capture) return;
+    X->up[0] = d;
+    X->up[1] = alt;
+    X->up_ok = true;
+  }
+  // the context of the current species buffers, for a launch
+  const DevCtx *D() const { return dev_ctx + (species_in_alt() ? 1 : 0); }
 
   float *F(int id) const { return d.F[id]; }
   float *Sp(int id, int s_) const { return d.F[id] + (size_t)s_ * X->n3; }
@@ -342,7 +386,7 @@ struct Run {
     void flush() {
       if (n == 0) return;
       const int along = r->ide > r->jde ? r->ide : r->jde;
-      k_bc_batch<<<dim3(cdiv(along, 64), kmax, n), 64, 0, r->s>>>(r->d, L);
+      k_bc_batch<<<dim3(cdiv(along, 64), kmax, n), 64, 0, r->s>>>(r->D(), L);
       n = 0;
       kmax = 1;
     }
@@ -371,12 +415,12 @@ struct Run {
   void bc3(float *fl, char var) const {
     const bool full_k = (var == 'e' || var == 'f' || var == 'w');
     const int kend = full_k ? kde : kde - 1;
-    if (!(var == 'u' || var == 'x')) k_bc_x<<<dim3(cdiv(jde, 64), kend), 64, 0, s>>>(d, fl, kend, 0);
-    if (!(var == 'v' || var == 'y')) k_bc_y<<<dim3(cdiv(ide, 64), kend), 64, 0, s>>>(d, fl, kend, 0);
+    if (!(var == 'u' || var == 'x')) k_bc_x<<<dim3(cdiv(jde, 64), kend), 64, 0, s>>>(D(), fl, kend, 0);
+    if (!(var == 'v' || var == 'y')) k_bc_y<<<dim3(cdiv(ide, 64), kend), 64, 0, s>>>(D(), fl, kend, 0);
   }
   void bc2(float *fl, char var) const {
-    if (!(var == 'u' || var == 'x')) k_bc_x<<<dim3(cdiv(jde, 64), 1), 64, 0, s>>>(d, fl, 1, 1);
-    if (!(var == 'v' || var == 'y')) k_bc_y<<<dim3(cdiv(ide, 64), 1), 64, 0, s>>>(d, fl, 1, 1);
+    if (!(var == 'u' || var == 'x')) k_bc_x<<<dim3(cdiv(jde, 64), 1), 64, 0, s>>>(D(), fl, 1, 1);
+    if (!(var == 'v' || var == 'y')) k_bc_y<<<dim3(cdiv(ide, 64), 1), 64, 0, s>>>(D(), fl, 1, 1);
   }
 
   // ---- specified / relaxation zones --------------------------------------
@@ -395,11 +439,11 @@ struct Run {
 
   void spec_overlay(float *tend, char var, bool ktop, bool is2d, BPtrs bt) const {
     Z z = zd(var, ktop, is2d);
-    k_spec_overlay<<<dim3(cdiv(zone_n(z), 64), z.kt), 64, 0, s>>>(d, tend, z.ibe, z.jbe, z.kt, is2d ? 1 : 0, bt);
+    k_spec_overlay<<<dim3(cdiv(zone_n(z), 64), z.kt), 64, 0, s>>>(D(), tend, z.ibe, z.jbe, z.kt, is2d ? 1 : 0, bt);
   }
   void spec_update(float *fl, const float *tend, double dt, char var, bool is2d) const {
     Z z = zd(var, var == 'm' || var == 'h', is2d);
-    k_spec_update<<<dim3(cdiv(zone_n(z), 64), z.kt), 64, 0, s>>>(d, fl, tend, (float)dt, z.ibe, z.jbe, z.kt, is2d ? 1 : 0);
+    k_spec_update<<<dim3(cdiv(zone_n(z), 64), z.kt), 64, 0, s>>>(D(), fl, tend, (float)dt, z.ibe, z.jbe, z.kt, is2d ? 1 : 0);
   }
   // relax_bdytend of fld (mw 0), or of its mass-weighted value (mw 1: half
   // levels, 2: w levels), formed by the relaxation kernel on the zone points
@@ -429,7 +473,7 @@ struct Run {
     void flush() {
       if (n == 0) return;
       const int rz = r->X->c.relax_zone;
-      k_relax<<<dim3(cdiv(along, 64), kmax, n * 4 * (rz - 1)), 64, 0, r->s>>>(r->d, L, r->X->dtbc_dev);
+      k_relax<<<dim3(cdiv(along, 64), kmax, n * 4 * (rz - 1)), 64, 0, r->s>>>(r->D(), L, r->X->dtbc_dev);
       n = 0;
       along = kmax = 1;
     }
@@ -469,7 +513,7 @@ struct Run {
     }
     void flush() {
       if (n == 0) return;
-      k_spec_final<<<dim3(cdiv(nmax, 64), kmax, n), 64, 0, r->s>>>(r->d, L, r->X->dtbc_dev);
+      k_spec_final<<<dim3(cdiv(nmax, 64), kmax, n), 64, 0, r->s>>>(r->D(), L, r->X->dtbc_dev);
       n = 0;
       nmax = kmax = 1;
     }
@@ -477,16 +521,16 @@ struct Run {
   };
   void edge_copy(float *f0, float *f1, int axis, int dst, int src_, int kend) const {
     const int n = axis == 0 ? jde : ide;
-    k_edge_copy<<<dim3(cdiv(n, 64), kend), 64, 0, s>>>(d, f0, f1, axis, dst, src_, kend);
+    k_edge_copy<<<dim3(cdiv(n, 64), kend), 64, 0, s>>>(D(), f0, f1, axis, dst, src_, kend);
   }
 
   // ---- RK-stage pieces -----------------------------------------------------
   void rk_step_prep() const {
-    k_mu_uv<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(d, F(F_mu_2), F(F_mub), F(F_muu), F(F_muv), F(F_mut));
+    k_mu_uv<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D(), F(F_mu_2), F(F_mub), F(F_muu), F(F_muv), F(F_mut));
     R3 r = full3();
-    k_rk_prep3<<<g3(r), b3(), 0, s>>>(d, r);
+    k_rk_prep3<<<g3(r), b3(), 0, s>>>(D(), r);
     R2 c = mass2();
-    k_ww_cp<<<g2(c), 64, sizeof(float) * 64 * (size_t)(kde - 1), s>>>(d, c);
+    k_ww_cp<<<g2(c), 64, sizeof(float) * 64 * (size_t)(kde - 1), s>>>(D(), c);
   }
   void first_rk_step_part1() const {
     const size_t n3 = X->n3;
@@ -494,23 +538,23 @@ struct Run {
                {F(F_mu_tendf), X->n2}, {F(F_moist_tend), n3 * (size_t)X->c.nmoist},
                {F(F_scalar_tend), n3 * (size_t)X->c.nscalar}});
     R3 m = mass3();
-    k_rho<<<g3p(m), b3(), 0, s>>>(d, m);
+    k_rho<<<g3p(m), b3(), 0, s>>>(D(), m);
   }
   void compute_diff_metrics() const {
     R3 r = full3();
-    k_diff_metrics<<<g3(r), b3(), 0, s>>>(d, r);
+    k_diff_metrics<<<g3(r), b3(), 0, s>>>(D(), r);
   }
   void cal_deform_and_div() const {
     R3 m = mass3();
-    k_deform_diag<<<g3(m), b3(), 0, s>>>(d, m);
+    k_deform_diag<<<g3(m), b3(), 0, s>>>(D(), m);
     R3 r12{2, ide - 1, 1, kde - 1, 2, jde - 1};
-    k_deform12<<<g3(r12), b3(), 0, s>>>(d, r12);
+    k_deform12<<<g3(r12), b3(), 0, s>>>(D(), r12);
     edge_copy(F(F_defor12), nullptr, 0, 1, 2, kde);
     edge_copy(F(F_defor12), nullptr, 1, 1, 2, kde);
     edge_copy(F(F_defor12), nullptr, 0, ide, ide - 1, kde);
     edge_copy(F(F_defor12), nullptr, 1, jde, jde - 1, kde);
     R3 r13{2, ide - 1, 1, kde, 2, jde - 1};
-    k_deform13_23<<<g3(r13), b3(), 0, s>>>(d, r13);
+    k_deform13_23<<<g3(r13), b3(), 0, s>>>(D(), r13);
     edge_copy(F(F_defor13), F(F_defor23), 0, 1, 2, kde);
     edge_copy(F(F_defor13), F(F_defor23), 1, 1, 2, kde);
     edge_copy(F(F_defor13), F(F_defor23), 0, ide, ide - 1, kde);
@@ -518,13 +562,13 @@ struct Run {
   }
   void smag2d_km() const {
     R3 r{2, ide - 2, 1, kde - 1, 2, jde - 2};
-    k_smag<<<g3(r), b3(), 0, s>>>(d, r);
+    k_smag<<<g3(r), b3(), 0, s>>>(D(), r);
   }
   // N^2 of calculate_km_kh (read by no later stage of the km_opt 4 path
   // itself; the learned closure takes it as an input)
   void calculate_n2() const {
     R3 r{2, ide - 2, 1, kde - 1, 2, jde - 2};
-    k_n2<<<g3p(r), b3(), 0, s>>>(d, r);
+    k_n2<<<g3p(r), b3(), 0, s>>>(D(), r);
   }
   // Smagorinsky km storing |D| and the slope divisor in the scratch arrays
   // S_T1 and S_T2 (free until the diffusion's stresses), then the learned km
@@ -533,13 +577,13 @@ struct Run {
   // per-field positive-definite advection stage)
   void smag_for_closure(const ClosureNorm &nm) const {
     R3 r{2, ide - 2, 1, kde - 1, 2, jde - 2};
-    k_smag<<<g3(r), b3(), 0, s>>>(d, r, Scr(S_T1), Scr(S_T2));
-    k_closure_feat<<<g3p(r), b3(), 0, s>>>(d, r, nm, Scr(S_T1), Scr(S_FQX), Scr(S_FQY));
+    k_smag<<<g3(r), b3(), 0, s>>>(D(), r, Scr(S_T1), Scr(S_T2));
+    k_closure_feat<<<g3p(r), b3(), 0, s>>>(D(), r, nm, Scr(S_T1), Scr(S_FQX), Scr(S_FQY));
   }
   void closure_km() const {
     R3 r{2, ide - 2, 1, kde - 1, 2, jde - 2};
     static_assert(S_FQY == S_FQX + 1, "the network's two input arrays are adjacent scratch slots");
-    k_closure_km<<<g3p(r), b3(), 0, s>>>(d, r, X->cl_theta, X->cl_wbf, X->cl_norm, Scr(S_FQX), Scr(S_T2));
+    k_closure_km<<<g3p(r), b3(), 0, s>>>(D(), r, X->cl_theta, X->cl_wbf, X->cl_norm, Scr(S_FQX), Scr(S_T2));
   }
   // training rows of the current state (features, s1, s2, divisor, km)
   void closure_rows(const ClosureNorm &nm, __bf16 *Xr, float *T) const {
@@ -549,7 +593,7 @@ struct Run {
     calculate_n2();
     smag_for_closure(nm);
     R3 r{2, ide - 2, 1, kde - 1, 2, jde - 2};
-    k_closure_rows<<<g3p(r), b3(), 0, s>>>(d, r, nm, Scr(S_FQX), Scr(S_FQY), Scr(S_T2), Xr, T);
+    k_closure_rows<<<g3p(r), b3(), 0, s>>>(D(), r, nm, Scr(S_FQX), Scr(S_FQY), Scr(S_T2), Xr, T);
   }
   // two stress components (t1, t2 of one diffusion kernel) in one launch;
   // each entry: xk, defor, kind, i0, i1, j0, j1
@@ -568,7 +612,7 @@ struct Run {
       P.j1[n] = (*e[n])[6];
     }
     R3 r = full3();
-    k_titau<<<g3(r), b3(), 0, s>>>(d, P, r);
+    k_titau<<<g3(r), b3(), 0, s>>>(D(), P, r);
   }
   // horizontal_diffusion_s of theta and every species: faces, then tendencies
   void hdiff_scalars() const {
@@ -585,21 +629,21 @@ struct Run {
     for (int q = 0; q < X->c.nmoist; q++) add(Sp(F_moist, q), Sp(F_moist_tend, q));
     for (int q = 0; q < X->c.nscalar; q++) add(Sp(F_scalar, q), Sp(F_scalar_tend, q));
     const R3 rf{2, ide - 1, 1, kde - 1, 2, jde - 1};
-    k_hdiff_s_faces<<<g3(rf), b3(), 0, s>>>(d, L, rf);
+    k_hdiff_s_faces<<<g3(rf), b3(), 0, s>>>(D(), L, rf);
     const R3 rt{2, ide - 2, 1, kde - 1, 2, jde - 2};
-    k_hdiff_s_tend<<<g3(rt), b3(), 0, s>>>(d, L, rt);
+    k_hdiff_s_tend<<<g3(rt), b3(), 0, s>>>(D(), L, rt);
   }
   void horizontal_diffusion_2() const {
     float *t1 = Scr(S_T1), *t2 = Scr(S_T2);
     titau(t1, t2, {F_xkmh, F_defor11, 11, 1, ide - 1, 2, jde - 1}, {F_xkmh, F_defor12, 12, 2, ide - 1, 2, jde});
     R3 ru{2, ide - 1, 1, kde - 1, 2, jde - 2};
-    k_hdiff_u<<<g3(ru), b3(), 0, s>>>(d, t1, t2, ru);
+    k_hdiff_u<<<g3(ru), b3(), 0, s>>>(D(), t1, t2, ru);
     titau(t1, t2, {F_xkmh, F_defor12, 12, 2, ide, 2, jde - 1}, {F_xkmh, F_defor22, 11, 2, ide - 1, 1, jde - 1});
     R3 rv{2, ide - 2, 1, kde - 1, 2, jde - 1};
-    k_hdiff_v<<<g3(rv), b3(), 0, s>>>(d, t1, t2, rv);
+    k_hdiff_v<<<g3(rv), b3(), 0, s>>>(D(), t1, t2, rv);
     titau(t1, t2, {F_xkmv, F_defor13, 13, 2, ide, 2, jde - 2}, {F_xkmv, F_defor23, 23, 2, ide - 2, 2, jde});
     R3 rw{2, ide - 2, 2, kde - 1, 2, jde - 2};
-    k_hdiff_w<<<g3(rw), b3(), 0, s>>>(d, t1, t2, rw);
+    k_hdiff_w<<<g3(rw), b3(), 0, s>>>(D(), t1, t2, rw);
     hdiff_scalars();
   }
   // with_n2: also N^2 (the stage API always, the step when the learned
@@ -623,48 +667,48 @@ struct Run {
   }
   void advect_u() const {
     R3 r{2, ide - 1, 1, kde - 1, 1, jde - 1};
-    k_advect_u<false><<<dim3(face_tiles(r, d.face_lg[0]).count()), bf(), 0, s>>>(d, F(F_u_2), F(F_ru_tend), F(F_ru), F(F_rv), F(F_ww), r, 0);
+    k_advect_u<false><<<dim3(face_tiles(r, d.face_lg[0]).count()), bf(), 0, s>>>(D(), F(F_u_2), F(F_ru_tend), F(F_ru), F(F_rv), F(F_ww), r, 0);
   }
   void advect_v() const {
     R3 r{1, ide - 1, 1, kde - 1, 2, jde - 1};
-    k_advect_v<false><<<dim3(face_tiles(r, d.face_lg[0]).count()), bf(), 0, s>>>(d, F(F_v_2), F(F_rv_tend), F(F_ru), F(F_rv), F(F_ww), r, 0);
+    k_advect_v<false><<<dim3(face_tiles(r, d.face_lg[0]).count()), bf(), 0, s>>>(D(), F(F_v_2), F(F_rv_tend), F(F_ru), F(F_rv), F(F_ww), r, 0);
   }
   void advect_w() const {
     R3 r{1, ide - 1, 2, kde, 1, jde - 1};
-    k_advect_w<false><<<dim3(face_tiles(r, d.face_lg[1]).count()), bf(), 0, s>>>(d, F(F_w_2), F(F_rw_tend), F(F_ru), F(F_rv), F(F_ww), r, 0);
+    k_advect_w<false><<<dim3(face_tiles(r, d.face_lg[1]).count()), bf(), 0, s>>>(D(), F(F_w_2), F(F_rw_tend), F(F_ru), F(F_rv), F(F_ww), r, 0);
   }
   void advect_scalar(const float *q, float *tend, const float *ru, const float *rv, const float *rom) const {
     R3 m = mass3();
-    k_advect_scalar<kAdvAdd><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(d, q, tend, ru, rv, rom, m, 0, TransportUpd{});
+    k_advect_scalar<kAdvAdd><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(D(), q, tend, ru, rv, rom, m, 0, TransportUpd{});
   }
   void advect_scalar_pd(const float *q, const float *q_old, float *tend, double dt) const {
     R3 r = full3();
-    k_pd_fluxes<<<g3(r), b3(), 0, s>>>(d, q, q_old, F(F_ru_m), F(F_rv_m), F(F_ww_m), F(F_muts), (float)dt, r);
-    k_pd_scale<<<g3(r), b3(), 0, s>>>(d, q_old, F(F_mub), F(F_mu_1), (float)dt, r);
+    k_pd_fluxes<<<g3(r), b3(), 0, s>>>(D(), q, q_old, F(F_ru_m), F(F_rv_m), F(F_ww_m), F(F_muts), (float)dt, r);
+    k_pd_scale<<<g3(r), b3(), 0, s>>>(D(), q_old, F(F_mub), F(F_mu_1), (float)dt, r);
     R3 m = mass3();
-    k_pd_tend<<<g3(m), b3(), 0, s>>>(d, tend, m);
+    k_pd_tend<<<g3(m), b3(), 0, s>>>(D(), tend, m);
   }
   void rhs_ph() const {
     R3 r{1, ide - 1, 2, kde, 1, jde - 1};
-    k_rhs_ph<<<g3(r), b3(), 0, s>>>(d, r);
+    k_rhs_ph<<<g3(r), b3(), 0, s>>>(D(), r);
   }
   void horizontal_pressure_gradient() const {
     R3 rv{1, ide - 1, 1, kde - 1, 2, jde - 1};
-    k_hpg<<<g3(rv), b3(), 0, s>>>(d, 1, rv);
+    k_hpg<<<g3(rv), b3(), 0, s>>>(D(), 1, rv);
     R3 ru{2, ide - 1, 1, kde - 1, 1, jde - 1};
-    k_hpg<<<g3(ru), b3(), 0, s>>>(d, 0, ru);
+    k_hpg<<<g3(ru), b3(), 0, s>>>(D(), 0, ru);
   }
   void pg_buoy_w() const {
     R2 c = mass2();
-    k_pg_buoy_w<<<g2(c), 64, 0, s>>>(d, c);
+    k_pg_buoy_w<<<g2(c), 64, 0, s>>>(D(), c);
   }
   void coriolis_curvature() const {
     R3 ru{2, ide - 1, 1, kde - 1, 1, jde - 1};
-    k_cor_curv<<<g3(ru), b3(), 0, s>>>(d, 0, ru);
+    k_cor_curv<<<g3(ru), b3(), 0, s>>>(D(), 0, ru);
     R3 rv{1, ide - 1, 1, kde - 1, 2, jde - 1};
-    k_cor_curv<<<g3(rv), b3(), 0, s>>>(d, 1, rv);
+    k_cor_curv<<<g3(rv), b3(), 0, s>>>(D(), 1, rv);
     R3 rw{1, ide - 1, 2, kde - 1, 1, jde - 1};
-    k_cor_curv<<<g3(rw), b3(), 0, s>>>(d, 2, rw);
+    k_cor_curv<<<g3(rw), b3(), 0, s>>>(D(), 2, rw);
   }
   // the RK tendencies and the saved tendencies start from zero each stage.
   // The first stage clears every tendency and saved tendency.  Later stages
@@ -703,16 +747,16 @@ struct Run {
     clear_tendencies(rk == 1);
     if (rk == 1) lateral_relax();
     const R3 ru{1, ide, 1, kde - 1, 1, jde - 1};
-    k_advect_u<true><<<dim3(face_tiles(ru, d.face_lg[0]).count()), bf(), 0, s>>>(d, F(F_u_2), F(F_ru_tend), F(F_ru), F(F_rv), F(F_ww), ru, rk);
+    k_advect_u<true><<<dim3(face_tiles(ru, d.face_lg[0]).count()), bf(), 0, s>>>(D(), F(F_u_2), F(F_ru_tend), F(F_ru), F(F_rv), F(F_ww), ru, rk);
     const R3 rv{1, ide - 1, 1, kde - 1, 1, jde};
-    k_advect_v<true><<<dim3(face_tiles(rv, d.face_lg[0]).count()), bf(), 0, s>>>(d, F(F_v_2), F(F_rv_tend), F(F_ru), F(F_rv), F(F_ww), rv, rk);
+    k_advect_v<true><<<dim3(face_tiles(rv, d.face_lg[0]).count()), bf(), 0, s>>>(D(), F(F_v_2), F(F_rv_tend), F(F_ru), F(F_rv), F(F_ww), rv, rk);
     const R3 rw{1, ide - 1, 1, kde, 1, jde - 1};
-    k_advect_w<true><<<dim3(face_tiles(rw, d.face_lg[1]).count()), bf(), 0, s>>>(d, F(F_w_2), F(F_rw_tend), F(F_ru), F(F_rv), F(F_ww), rw, rk);
+    k_advect_w<true><<<dim3(face_tiles(rw, d.face_lg[1]).count()), bf(), 0, s>>>(D(), F(F_w_2), F(F_rw_tend), F(F_ru), F(F_rv), F(F_ww), rw, rk);
     const R3 rq{1, ide - 1, kde - 1, kde - 1, 1, jde - 1};  // levels [2, kde-2]: k_advect_w<true>
-    k_cqw_inv<<<g3p(rq), b3(), 0, s>>>(d, rq);
+    k_cqw_inv<<<g3p(rq), b3(), 0, s>>>(D(), rq);
     const R3 m = mass3();
-    k_advect_scalar<kAdvTend><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(d, F(F_t_2), F(F_t_tend), F(F_ru), F(F_rv), F(F_ww), m, rk, TransportUpd{});
-    k_tend_ph<<<g3(rw), b3(), 0, s>>>(d, rw, rk);
+    k_advect_scalar<kAdvTend><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(D(), F(F_t_2), F(F_t_tend), F(F_ru), F(F_rv), F(F_ww), m, rk, TransportUpd{});
+    k_tend_ph<<<g3(rw), b3(), 0, s>>>(D(), rw, rk);
     spec_overlays();
   }
   // relax_bdy_dry at the first stage (physics tendencies of u, v, ph, theta, mu)
@@ -749,19 +793,19 @@ struct Run {
     add(F(F_ph_tend), 'h', true, false, bp(F_ph_btys, F_ph_btye, F_ph_btxs, F_ph_btxe));
     add(F(F_t_tend), 't', false, false, bp(F_t_btys, F_t_btye, F_t_btxs, F_t_btxe));
     add(F(F_mu_tend), 'm', true, true, bp(F_mu_btys, F_mu_btye, F_mu_btxs, F_mu_btxe));
-    k_spec_overlay_batch<<<dim3(cdiv(nmax, 64), kmax, n), 64, 0, s>>>(d, L);
+    k_spec_overlay_batch<<<dim3(cdiv(nmax, 64), kmax, n), 64, 0, s>>>(D(), L);
   }
   // rk_addtend_dry: the physics tendencies into the RK tendencies
   void rk_addtend_dry() const {
     const int rk = X->rk;
     R3 r0{1, ide, 1, kde - 1, 1, jde - 1};
-    k_addtend<<<g3p(r0), b3(), 0, s>>>(d, 0, rk, r0);
+    k_addtend<<<g3p(r0), b3(), 0, s>>>(D(), 0, rk, r0);
     R3 r1{1, ide - 1, 1, kde - 1, 1, jde};
-    k_addtend<<<g3p(r1), b3(), 0, s>>>(d, 1, rk, r1);
+    k_addtend<<<g3p(r1), b3(), 0, s>>>(D(), 1, rk, r1);
     R3 r2{1, ide - 1, 1, kde, 1, jde - 1};
-    k_addtend<<<g3p(r2), b3(), 0, s>>>(d, 2, rk, r2);
+    k_addtend<<<g3p(r2), b3(), 0, s>>>(D(), 2, rk, r2);
     R3 r3 = mass3();
-    k_addtend<<<g3p(r3), b3(), 0, s>>>(d, 3, rk, r3);
+    k_addtend<<<g3p(r3), b3(), 0, s>>>(D(), 3, rk, r3);
   }
   // relax_bdy_dry (first stage) + rk_addtend_dry + spec_bdy_dry
   void dry_boundary_tendency() const {
@@ -770,45 +814,45 @@ struct Run {
     spec_overlays();
   }
   void small_step_prep() const {
-    k_ssp_mass<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(d, X->rk);
+    k_ssp_mass<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D(), X->rk);
     R3 r = full3();
-    if (X->rk == 1) k_ssp_3d<true><<<g3p(r), b3(), 0, s>>>(d, r);
-    else k_ssp_3d<false><<<g3p(r), b3(), 0, s>>>(d, r);
+    if (X->rk == 1) k_ssp_3d<true><<<g3p(r), b3(), 0, s>>>(D(), r);
+    else k_ssp_3d<false><<<g3p(r), b3(), 0, s>>>(D(), r);
   }
   void calc_p_rho(int step) const {
     R3 m = mass3();
-    k_calc_p_rho<<<g3p(m), b3(), 0, s>>>(d, step, m);
+    k_calc_p_rho<<<g3p(m), b3(), 0, s>>>(D(), step, m);
   }
   void calc_coef_w() const {
     R2 c = mass2();
-    k_calc_coef_w<<<g2(c), 64, 0, s>>>(d, (float)X->dts_rk, c);
+    k_calc_coef_w<<<g2(c), 64, 0, s>>>(D(), (float)X->dts_rk, c);
   }
   void advance_uv() const {
     const int sz = X->c.spec_zone;
     R3 ru{1 + sz, ide - sz, 1, kde - 1, 1 + sz, jde - sz - 1};
-    k_advance_uv<<<g3(ru), b3(), 0, s>>>(d, 0, (float)X->dts_rk, ru);
+    k_advance_uv<<<g3(ru), b3(), 0, s>>>(D(), 0, (float)X->dts_rk, ru);
     R3 rv{1 + sz, ide - sz - 1, 1, kde - 1, 1 + sz, jde - sz};
-    k_advance_uv<<<g3(rv), b3(), 0, s>>>(d, 1, (float)X->dts_rk, rv);
+    k_advance_uv<<<g3(rv), b3(), 0, s>>>(D(), 1, (float)X->dts_rk, rv);
   }
   void advance_mu_t() const {
     R2 c{2, ide - 2, 2, jde - 2};
-    k_advance_mu_t<<<g2(c), 64, 0, s>>>(d, (float)X->dts_rk, c);
+    k_advance_mu_t<<<g2(c), 64, 0, s>>>(D(), (float)X->dts_rk, c);
   }
   void advance_w() const {
     R2 c{2, ide - 2, 2, jde - 2};
-    k_advance_w<<<g2(c), 64, 0, s>>>(d, (float)X->dts_rk, Scr(S_HAT2), c);
+    k_advance_w<<<g2(c), 64, 0, s>>>(D(), (float)X->dts_rk, Scr(S_HAT2), c);
   }
   void sumflux() const {
     R3 r = full3();
-    k_sumflux<<<g3p(r), b3(), 0, s>>>(d, X->iteration == 1, X->iteration == X->nsmall, (float)X->nsmall, r);
+    k_sumflux<<<g3p(r), b3(), 0, s>>>(D(), X->iteration == 1, X->iteration == X->nsmall, (float)X->nsmall, r);
   }
   void spec_bdyupdate_ph() const {
     Z z = zd('h', true, false);
-    k_spec_update_ph<<<dim3(cdiv(zone_n(z), 64), kde), 64, 0, s>>>(d, (float)X->dts_rk);
+    k_spec_update_ph<<<dim3(cdiv(zone_n(z), 64), kde), 64, 0, s>>>(D(), (float)X->dts_rk);
   }
   void zero_grad_bdy_w() const {
-    k_zero_grad_rows<<<dim3(cdiv(ide - 1, 64), kde, 2), 64, 0, s>>>(d, F(F_w_2));
-    k_zero_grad_cols<<<dim3(cdiv(jde - 1, 64), kde, 2), 64, 0, s>>>(d, F(F_w_2));
+    k_zero_grad_rows<<<dim3(cdiv(ide - 1, 64), kde, 2), 64, 0, s>>>(D(), F(F_w_2));
+    k_zero_grad_cols<<<dim3(cdiv(jde - 1, 64), kde, 2), 64, 0, s>>>(D(), F(F_w_2));
   }
   // one fused acoustic substep: u/v, the column kernel, zero_grad_bdy of w;
   // all_outputs: also the intermediate t_2ave (a substep called on its own)
@@ -816,14 +860,14 @@ struct Run {
     X->iteration = it;
     const float dts = (float)X->dts_rk;
     R3 r{1, ide, 1, kde - 1, 1, jde};
-    k_uv_substep<<<g3(r), b3(), 0, s>>>(d, dts, r);
-    launch_acoustic_col(d, s, dts, it == 1, it == X->nsmall, (float)X->nsmall, all_outputs || it == X->nsmall);
+    k_uv_substep<<<g3(r), b3(), 0, s>>>(D(), dts, r);
+    launch_acoustic_col(d, D(), s, dts, it == 1, it == X->nsmall, (float)X->nsmall, all_outputs || it == X->nsmall);
     Z z = zd('w', true, false);
-    k_zero_grad_w<<<dim3(cdiv(zone_n(z), 64), kde), 64, 0, s>>>(d);
+    k_zero_grad_w<<<dim3(cdiv(zone_n(z), 64), kde), 64, 0, s>>>(D());
   }
   // calc_mu_uv_1: the staggered column masses of muts
   void calc_mu_uv_1() const {
-    k_mu_uv<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(d, F(F_muts), nullptr, F(F_muus), F(F_muvs), nullptr);
+    k_mu_uv<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D(), F(F_muts), nullptr, F(F_muus), F(F_muvs), nullptr);
   }
   void small_step_finish() const {
     calc_mu_uv_1();
@@ -833,16 +877,16 @@ struct Run {
   // the calc_mu_uv_1 that the RK stage runs before it
   void recouple() const {
     R3 r = full3();
-    if (X->rk == 3) k_ssf<true><<<g3(r), b3(), 0, s>>>(d, (float)X->dts_rk, (float)X->nsmall, r);
-    else k_ssf<false><<<g3(r), b3(), 0, s>>>(d, (float)X->dts_rk, (float)X->nsmall, r);
+    if (X->rk == 3) k_ssf<true><<<g3(r), b3(), 0, s>>>(D(), (float)X->dts_rk, (float)X->nsmall, r);
+    else k_ssf<false><<<g3(r), b3(), 0, s>>>(D(), (float)X->dts_rk, (float)X->nsmall, r);
   }
   void calc_p_rho_phi() const {
     R3 m = mass3();
-    k_calc_p_rho_phi<<<g3p(m), b3(), 0, s>>>(d, m);
+    k_calc_p_rho_phi<<<g3p(m), b3(), 0, s>>>(D(), m);
   }
   void update_scalar_pd(float *q_old, float *q_tend) const {
     R3 m = mass3();
-    k_update_scalar_pd<<<g3p(m), b3(), 0, s>>>(d, q_old, q_tend, (float)X->dt_rk, m);
+    k_update_scalar_pd<<<g3p(m), b3(), 0, s>>>(D(), q_old, q_tend, (float)X->dt_rk, m);
   }
   void species_advance(float *q, float *q_old, float *q_tend, bool is_qv, bool is_moist, bool pd) const {
     float *adv = F(F_advect_tend);
@@ -854,10 +898,10 @@ struct Run {
       relax(q, q_tend, 'q', false, false, bp(F_qv_bys, F_qv_bye, F_qv_bxs, F_qv_bxe), bp(F_qv_btys, F_qv_btye, F_qv_btxs, F_qv_btxe), 1);
       spec_overlay(q_tend, 't', false, false, bp(F_qv_btys, F_qv_btye, F_qv_btxs, F_qv_btxe));
     }
-    k_update_scalar<<<g3p(m), b3(), 0, s>>>(d, q, q_old, q_tend, X->rk, (float)X->dt_rk, m);
+    k_update_scalar<<<g3p(m), b3(), 0, s>>>(D(), q, q_old, q_tend, X->rk, (float)X->dt_rk, m);
     if (is_moist && !is_qv) {
-      k_flow_dep_rows<<<dim3(cdiv(ide - 1, 64), kde - 1, 2), 64, 0, s>>>(d, q, F(F_rv_m));
-      k_flow_dep_cols<<<dim3(cdiv(jde - 1, 64), kde - 1, 2), 64, 0, s>>>(d, q, F(F_ru_m));
+      k_flow_dep_rows<<<dim3(cdiv(ide - 1, 64), kde - 1, 2), 64, 0, s>>>(D(), q, F(F_rv_m));
+      k_flow_dep_cols<<<dim3(cdiv(jde - 1, 64), kde - 1, 2), 64, 0, s>>>(D(), q, F(F_ru_m));
     }
   }
 
@@ -878,7 +922,7 @@ struct Run {
   void copy_batch(const CopyList &L, R3 r) const {
     if (L.n == 0) return;
     const unsigned gi = (unsigned)(r.i1 - r.i0 + 256) / 256u, gk = (unsigned)(r.k1 - r.k0 + 4) / 4u;
-    k_copy_batch<<<dim3(gi * gk, (unsigned)(r.j1 - r.j0 + 1), (unsigned)L.n), dim3(64, 4), 0, s>>>(d, L, r);
+    k_copy_batch<<<dim3(gi * gk, (unsigned)(r.j1 - r.j0 + 1), (unsigned)L.n), dim3(64, 4), 0, s>>>(D(), L, r);
   }
   void copy_species(R3 r, bool to_alt) const {
     const size_t n = X->n3;
@@ -963,16 +1007,16 @@ struct Run {
       for (int q = 0; q < pd.n; q++) {
         pd.scale[q] = X->spec_scale + (size_t)q * n3;
       }
-      if (!pd_prepped) k_species_pd_prep<<<g3p(m), b3(), 0, s>>>(d, pd, dt, m);
+      if (!pd_prepped) k_species_pd_prep<<<g3p(m), b3(), 0, s>>>(D(), pd, dt, m);
       {
         BcBatch bc(this);
         for (int q = 0; q < pd.n; q++) bc.add3(pd.old[q], 'p');
       }
       R3 r = full3();
-      k_species_pd_scale<<<dim3(face_tiles(r, d.face_lg[2]).count()), bf(), sizeof(float) * 2 * 64 * kFaceRows * pd.n, s>>>(d, pd, dt, r);
-      k_species_pd_update<<<dim3(face_tiles(m, d.face_lg[2]).count()), bf(), sizeof(float) * 2 * 64 * kFaceRows * pd.n, s>>>(d, pd, dt, m);
+      k_species_pd_scale<<<dim3(face_tiles(r, d.face_lg[2]).count()), bf(), sizeof(float) * 2 * 64 * kFaceRows * pd.n, s>>>(D(), pd, dt, r);
+      k_species_pd_update<<<dim3(face_tiles(m, d.face_lg[2]).count()), bf(), sizeof(float) * 2 * 64 * kFaceRows * pd.n, s>>>(D(), pd, dt, m);
     }
-    if (plain.n > 0) k_species_update<<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), sizeof(float) * 64 * kFaceRows * plain.n, s>>>(d, plain, rk, dt, m);
+    if (plain.n > 0) k_species_update<<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), sizeof(float) * 64 * kFaceRows * plain.n, s>>>(D(), plain, rk, dt, m);
     // outputs become the current species
     use_species(out_alt);
     if (rk == 3) {
@@ -986,7 +1030,7 @@ struct Run {
       memset(&fl, 0, sizeof(fl));
       for (int q = 1; q < nm; q++) fl.q[fl.n++] = Sp(F_moist, q);
       Z z = zd('t', false, false);
-      k_flow_dep_batch<<<dim3(cdiv(zone_n(z), 64), kde - 1, fl.n), 64, 0, s>>>(d, fl);
+      k_flow_dep_batch<<<dim3(cdiv(zone_n(z), 64), kde - 1, fl.n), 64, 0, s>>>(D(), fl);
     }
   }
 
@@ -994,14 +1038,14 @@ struct Run {
   // forward) and its adjoint; rk sets dt_rk (set_rk before)
   void transport_stage(const float *const *st, const float *q_in, const float *q_old, float *q_out) const {
     R3 m = mass3();
-    k_advect_scalar<kAdvTransport><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(d, q_in, q_out, st[0], st[1], st[2], m, 0,
+    k_advect_scalar<kAdvTransport><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(D(), q_in, q_out, st[0], st[1], st[2], m, 0,
                                                                                             TransportUpd{q_old, st[3], st[4], (float)X->dt_rk});
   }
   void transport_stage_adjoint(const float *const *st, const float *qbar_out, float *qbar_old, float *qbar_in) const {
     float *tbar = Scr(S_T1);
     R3 m = mass3();
-    k_ad_update<<<g3p(m), b3(), 0, s>>>(d, m, StageMass{st[3], st[4]}, qbar_out, qbar_old, tbar, (float)X->dt_rk, 0);
-    k_ad_advect<kAdAdd><<<g3(m), b3(), 0, s>>>(d, m, tbar, st[0], st[1], st[2], qbar_in, AdNext{});
+    k_ad_update<<<g3p(m), b3(), 0, s>>>(D(), m, StageMass{st[3], st[4]}, qbar_out, qbar_old, tbar, (float)X->dt_rk, 0);
+    k_ad_advect<kAdAdd><<<g3(m), b3(), 0, s>>>(D(), m, tbar, st[0], st[1], st[2], qbar_in, AdNext{});
   }
   // the adjoint of nsteps whole steps (stages: 5 pointers for each of their
   // 3 * nsteps stages, in forward order): qbar_begin = M^T qbar_end on the
@@ -1016,14 +1060,14 @@ struct Run {
     };
     float *tbar = Scr(S_T1), *other = Scr(S_T2);
     const int last = 3 * nsteps - 1;
-    k_ad_update<<<g3p(m), b3(), 0, s>>>(d, m, StageMass{st(last)[3], st(last)[4]}, qbar_end, qbar_begin, tbar, dt(last), 1);
+    k_ad_update<<<g3p(m), b3(), 0, s>>>(D(), m, StageMass{st(last)[3], st(last)[4]}, qbar_end, qbar_begin, tbar, dt(last), 1);
     for (int n = last; n >= 0; n--) {
       const float *const *f = st(n);
       AdNext nx{};
       if (n > 0) nx = AdNext{StageMass{st(n - 1)[3], st(n - 1)[4]}, other, dt(n - 1)};
-      if (n == 0) k_ad_advect<kAdAdd><<<g3(m), b3(), 0, s>>>(d, m, tbar, f[0], f[1], f[2], qbar_begin, nx);
-      else if (n % 3 == 0) k_ad_advect<kAdStep><<<g3(m), b3(), 0, s>>>(d, m, tbar, f[0], f[1], f[2], qbar_begin, nx);
-      else k_ad_advect<kAdNext><<<g3(m), b3(), 0, s>>>(d, m, tbar, f[0], f[1], f[2], qbar_begin, nx);
+      if (n == 0) k_ad_advect<kAdAdd><<<g3(m), b3(), 0, s>>>(D(), m, tbar, f[0], f[1], f[2], qbar_begin, nx);
+      else if (n % 3 == 0) k_ad_advect<kAdStep><<<g3(m), b3(), 0, s>>>(D(), m, tbar, f[0], f[1], f[2], qbar_begin, nx);
+      else k_ad_advect<kAdNext><<<g3(m), b3(), 0, s>>>(D(), m, tbar, f[0], f[1], f[2], qbar_begin, nx);
       std::swap(tbar, other);
     }
   }
@@ -1083,7 +1127,7 @@ struct Run {
                      bp(F_qv_btys, F_qv_btye, F_qv_btxs, F_qv_btxe));
     }
   }
-  void set_w_surface() const { k_set_w_surface<<<dim3(cdiv(ide - 1, 64), jde - 1), 64, 0, s>>>(d); }
+  void set_w_surface() const { k_set_w_surface<<<dim3(cdiv(ide - 1, 64), jde - 1), 64, 0, s>>>(D()); }
 
   void rk_stage() const {
     rk_step_prep();
@@ -1356,6 +1400,7 @@ int wrfdc_create(const wrfdc_config *cfg, wrfdc_ctx **out) {
     hchk(hipMalloc((void **)&x->scratch, sizeof(float) * x->n3 * NSCRATCH), "hipMalloc scratch");
     hchk(hipMalloc((void **)&x->ck, sizeof(double) * (kCkBlocks * CK_N + CK_N)), "hipMalloc checksum");
     hchk(hipMalloc((void **)&x->dtbc_dev, sizeof(float) * 64), "hipMalloc dtbc");
+    hchk(hipMalloc((void **)&x->ctx_dev, sizeof(DevCtx) * 4), "hipMalloc context");
     hchk(hipMalloc((void **)&x->spec_alt, sizeof(float) * x->n3 * (size_t)(cfg->nmoist + cfg->nscalar)), "hipMalloc species");
     hchk(hipMalloc((void **)&x->spec_scale, sizeof(float) * x->n3 * (size_t)(cfg->nmoist + cfg->nscalar)), "hipMalloc species scale");
     hchk(hipMalloc((void **)&x->hds, sizeof(float) * x->n3 * 2 * (size_t)(1 + cfg->nmoist + cfg->nscalar)), "hipMalloc diffusion fluxes");
@@ -1364,6 +1409,7 @@ int wrfdc_create(const wrfdc_config *cfg, wrfdc_ctx **out) {
     if (x->scratch) (void)hipFree(x->scratch);
     if (x->ck) (void)hipFree(x->ck);
     if (x->dtbc_dev) (void)hipFree(x->dtbc_dev);
+    if (x->ctx_dev) (void)hipFree(x->ctx_dev);
     if (x->spec_alt) (void)hipFree(x->spec_alt);
     if (x->spec_scale) (void)hipFree(x->spec_scale);
     if (x->hds) (void)hipFree(x->hds);
@@ -1389,6 +1435,7 @@ void wrfdc_destroy(wrfdc_ctx *x) {
   if (x->scratch) (void)hipFree(x->scratch);
   if (x->ck) (void)hipFree(x->ck);
   if (x->dtbc_dev) (void)hipFree(x->dtbc_dev);
+  if (x->ctx_dev) (void)hipFree(x->ctx_dev);
   if (x->spec_alt) (void)hipFree(x->spec_alt);
   if (x->spec_scale) (void)hipFree(x->spec_scale);
   if (x->hds) (void)hipFree(x->hds);
@@ -1808,9 +1855,9 @@ int wrfdc_stage(wrfdc_ctx *x, const char *name, int rk_step, int iteration) {
       x->iteration = iteration < 1 ? 1 : iteration;
       if (n == "acoustic_uv") {
         R3 r{1, run.ide, 1, run.kde - 1, 1, run.jde};
-        k_uv_substep<<<Run::g3(r), Run::b3(), 0, x->s>>>(x->h, dts, r);
+        k_uv_substep<<<Run::g3(r), Run::b3(), 0, x->s>>>(run.D(), dts, r);
       } else {
-        launch_acoustic_col(x->h, x->s, dts, x->iteration == 1, x->iteration == x->nsmall, (float)x->nsmall, 1);
+        launch_acoustic_col(run.d, run.D(), x->s, dts, x->iteration == 1, x->iteration == x->nsmall, (float)x->nsmall, 1);
       }
     }
     else if (n == "w_solve:columns" || n == "w_solve:levels") {
@@ -1819,14 +1866,14 @@ int wrfdc_stage(wrfdc_ctx *x, const char *name, int rk_step, int iteration) {
       const unsigned nb = (unsigned)((x->ide - 3 + 63) / 64) * (unsigned)(x->jde - 3);
       float *w = x->h.F[F_w_2];
       if (n == "w_solve:columns") {
-        k_tridiag_lanes_columns<<<nb, 64, 0, x->s>>>(x->h, w, w);
+        k_tridiag_lanes_columns<<<nb, 64, 0, x->s>>>(run.D(), w, w);
       } else {
         if (x->kde > 64) return set_err(x, WRFDC_EINVAL, "w_solve:levels needs kde <= 64 (one level per lane)");
         const size_t lds = tridiag_levels_lds(x->kde);
         if (lds > 65536)
           hchk(hipFuncSetAttribute((const void *)k_tridiag_lanes_levels, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                "w_solve LDS");
-        k_tridiag_lanes_levels<<<nb, dim3(64, 8), lds, x->s>>>(x->h, w, w);
+        k_tridiag_lanes_levels<<<nb, dim3(64, 8), lds, x->s>>>(run.D(), w, w);
       }
     }
     else if (n == "acoustic_substep") {
@@ -2137,7 +2184,8 @@ int wrfdc_subgrid_stress(wrfdc_ctx *fine, int nx_coarse, int ny_coarse, int rati
   if (nx_coarse < 12 || ny_coarse < 12) return set_err(fine, WRFDC_EINVAL, "coarse grid below 12 x 12");
   return guarded(fine, [&]() {
     R3 rc{2, nx_coarse - 1, 1, fine->kde - 1, 2, ny_coarse - 1};
-    k_subgrid_stress<<<Run::g3p(rc), Run::b3(), 0, fine->s>>>(fine->h, rc, ratio, rows_t);
+    Run run(fine);
+    k_subgrid_stress<<<Run::g3p(rc), Run::b3(), 0, fine->s>>>(run.D(), rc, ratio, rows_t);
     return WRFDC_OK;
   });
 }

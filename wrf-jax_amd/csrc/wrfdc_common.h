@@ -60,8 +60,8 @@ enum {
 // Library-owned scratch arrays (3-D, same layout as fields).
 enum { S_T1, S_T2, S_FQX, S_FQY, S_FQZ, S_FQXL, S_FQYL, S_FQZL, S_SCALE, S_HAT2, S_VXGM, NSCRATCH };
 
-// View of one domain (dimensions, scalars, pointers), passed to every kernel
-// by value (about 1.7 KB of kernel arguments).
+// View of one domain (dimensions, scalars, pointers), 1.7 KB in device memory.
+// Every kernel gets its address and reads it with scalar loads (CtxPtr).
 struct DevCtx {
   int ide, jde, kde, ip;
   int nmoist, nscalar, spec_zone, relax_zone, spec_bdy_width, top_lid;
@@ -76,6 +76,17 @@ struct DevCtx {
   float *F[NFIELDS];
   float *S[NSCRATCH];
 };
+
+// The context as kernels read it: through the constant address space (scalar
+// loads), and its field pointers cast through the global one (FL, SP, SCR),
+// without which a pointer read from memory makes every access a flat one.
+// Passed by value instead, its 27 cache lines were written for every launch
+// and read cold, a line at a time as a kernel came to need them:
+// a step of 24x20x10 (127 launches) took 600 us, 550 us this way, 100x100x45
+// 1307 and 1252, 400x400x60 14.62 and 14.54 ms.
+typedef const __attribute__((address_space(4))) DevCtx *CtxPtr;
+__device__ __forceinline__ CtxPtr ctx_ptr(const DevCtx *p) { return (CtxPtr)p; }
+__device__ __forceinline__ float *gmem(float *p) { return (float *)(__attribute__((address_space(1))) float *)p; }
 
 // Element offsets in 32-bit arithmetic, scaled to byte offsets in 32-bit
 // arithmetic too (a 3-D field holds < 2^30 elements, so its byte offsets fit;
@@ -118,9 +129,9 @@ __device__ __forceinline__ void pin1(float v) { asm volatile("" : : "v"(v)); }
 #define BY(fl, i, k, b) ((fl)[(unsigned)((((b) - 1) * x->kde + ((k) - 1)) * x->ip + ((i) - 1))])
 #define BX2(fl, j, b) ((fl)[(unsigned)(((b) - 1) * x->jde + ((j) - 1))])
 #define BY2(fl, i, b) ((fl)[(unsigned)(((b) - 1) * x->ip + ((i) - 1))])
-#define FL(name) (x->F[F_##name])
-#define SP(name, s) (x->F[F_##name] + (size_t)(s) * x->n3)
-#define SCR(id) (x->S[id])
+#define FL(name) gmem(x->F[F_##name])
+#define SP(name, s) (gmem(x->F[F_##name]) + (size_t)(s) * x->n3)
+#define SCR(id) gmem(x->S[id])
 
 // Inclusive Fortran index ranges of a launch.
 struct R3 {
