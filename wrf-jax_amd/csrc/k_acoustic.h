@@ -7,12 +7,14 @@
 //                   advance_w (implicit w-phi solve), sumflux,
 //                   spec_bdyupdate_ph, calc_p_rho and the physical-boundary
 //                   copies of ph/al/p/mu_2/muts/mudf (the owner of column
-//                   ide-1 / row jde-1 also writes its copy);
-//   k_zero_grad_w   zero_grad_bdy of w, rows and columns in one launch.
+//                   ide-1 / row jde-1 also writes its copy) and
+//                   zero_grad_bdy of w (the owner of a column beside the
+//                   zone ring writes the ring points that copy it).
 //
 // The column kernel runs 64 columns (one j row, lanes = i) per block of
-// eight waves.  Work that is pointwise in k is spread over the waves (wave w
-// owns levels w+1, w+1+8, ...) with loads coalesced along i; every phase first
+// eight waves (sixteen on small domains).  Work that is pointwise in k is
+// spread over the waves (wave w owns levels w+1, w+1+8, ...) with loads
+// coalesced along i; every phase first
 // loads the inputs of a group of its levels into registers, then computes and
 // stores, so a wave keeps a group's worth of loads in flight.  The two k
 // recurrences (column sum + omega, tridiagonal sweeps) run in wave 0 over
@@ -21,6 +23,7 @@
 #pragma once
 #include "wrfdc_common.h"
 #include "k_small.h"
+#include <type_traits>
 
 // ---------------------------------------------------------------------------
 // vertical pressure difference of advance_uv, rdnw(k) * (P(k+1) - P(k)) with
@@ -92,58 +95,40 @@ __global__ void __launch_bounds__(256) k_uv_substep(const DevCtx *xv, float dts,
   if (vpt) elem(FL(v_2), o) = vin ? vn_in : vn_z;
 }
 
-// zero_grad_bdy of w: every destination (the zone ring of the mass grid)
-// copies an interior point, so rows and columns go in one race-free pass.
-__global__ void k_zero_grad_w(const DevCtx *xv) {
-  const CtxPtr x = ctx_ptr(xv);
-  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int k = 1 + (int)blockIdx.y;
-  const int ibe = x->ide - 1, jbe = x->jde - 1;
-  int i, j, e;
-  if (k > x->kde || !zone_point(t, ibe, jbe, i, j, e)) return;
-  float *w = FL(w_2);
-  if (e < 2) {
-    const int ii = imin_(imax_(i, 2), ibe - 1);
-    A3(w, i, k, j) = A3(w, ii, k, e == 0 ? 2 : jbe - 1);
-  } else {
-    const int jj = imin_(imax_(j, 2), jbe - 1);
-    A3(w, e == 2 ? 1 : ibe, k, j) = A3(w, e == 2 ? 2 : ibe - 1, k, jj);
-  }
-}
-
 // ---------------------------------------------------------------------------
-// waves per block of k_acoustic_col, and levels per register group of each
-// phase (the loads of one group are issued together).  The group sizes trade
-// memory round trips against registers: phases with few loads per level take
-// larger groups (phase 3: 2 loads per level, all 8 levels of a wave at once;
-// phases 5, 6, 10: 4 levels), phases 1, 4 and 9 stay at 2 so the kernel keeps
-// 6 waves per SIMD (at most 80 VGPRs, the LDS limit being 3 blocks per CU).
-#ifndef WRFDC_COL_WAVES
-#define WRFDC_COL_WAVES 8
-#endif
-#ifndef WRFDC_COL_GROUP
-#define WRFDC_COL_GROUP 2
-#endif
-constexpr int kColG1 = WRFDC_COL_GROUP, kColG3 = 4 * WRFDC_COL_GROUP, kColG4 = WRFDC_COL_GROUP, kColG5 = 2 * WRFDC_COL_GROUP,
-              kColG6 = 2 * WRFDC_COL_GROUP, kColG9 = WRFDC_COL_GROUP, kColG10 = 2 * WRFDC_COL_GROUP;
-constexpr int kColWaves = WRFDC_COL_WAVES;
-
+// Levels per register group of each phase (the loads of one group are issued
+// together).  The group sizes trade memory round trips against registers:
+// phases with few loads per level take larger groups (phase 3: 2 loads per
+// level, all 8 levels of a wave at once; phases 5, 6, 10: 4 levels), phases 1,
+// 4 and 9 stay at 2 so the kernel keeps 6 waves per SIMD (at most 80 VGPRs,
+// the LDS limit being 3 blocks of 8 waves per CU).  A block of 16 waves has a
+// CU to itself and registers to spare: its waves load all their levels at
+// once up to 4.
+//
+// With every CU full the kernel runs at the rate its bytes move (430 us at
+// 400x400x60, 1.79 GB of HBM traffic): loads issued ahead of the serial
+// parts, and divisions taken out of them, change it by less than 1 %.  With
+// CUs idle the time is one block's latency, and there they count.
+template <int NW, int NPW>
+struct ColGroups {
+  static constexpr bool kWide = NW > 8;
+  static constexpr int w = NPW <= 4 ? NPW : 2;
+  static constexpr int G1 = kWide ? w : 2, G3 = kWide ? NPW : (NPW < 8 ? NPW : 8), G4 = kWide ? w : 2, G5 = kWide ? w : 4, G6 = kWide ? w : 4,
+                       G9 = kWide ? w : 2, G10 = kWide ? w : 4;
+};
 constexpr int kColMaxLev = 152;  // levels the column kernel holds (nz <= 150)
 // bytes of dynamic LDS of k_acoustic_col for kde levels
 __host__ __device__ inline size_t acoustic_col_lds(int kde) { return (size_t)3 * (kde + 1) * 64 * sizeof(float); }
-// levels per wave the kernel is instantiated for (kde <= kColWaves * NPW)
-inline int acoustic_col_npw(int kde) {
-  const int need = (kde + kColWaves - 1) / kColWaves;
-  return need <= 4 ? 4 : need <= 8 ? 8 : need <= 12 ? 12 : need <= 16 ? 16 : 20;
-}
 
-template <int NPW>
-__global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *xv, float dts, int first, int fin, float ns, int store_tav) {
+// ring: also zero_grad_bdy of w (the owner of a column next to the zone ring
+// of the mass grid writes its w to the ring points that copy it)
+template <int NW, int NPW>
+__global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const DevCtx *xv, float dts, int first, int fin, float ns, int store_tav, int ring) {
   const CtxPtr x = ctx_ptr(xv);
-  constexpr int NW = kColWaves;
-  constexpr int G1 = kColG1, G3 = kColG3, G4 = kColG4, G5 = kColG5, G6 = kColG6, G9 = kColG9, G10 = kColG10;
+  using G = ColGroups<NW, NPW>;
+  constexpr int G1 = G::G1, G3 = G::G3, G4 = G::G4, G5 = G::G5, G6 = G::G6, G9 = G::G9, G10 = G::G10;
   extern __shared__ float sm[];
-  __shared__ float c_mts[64], c_mav[64];
+  __shared__ float c_mts[64], c_mav[64], c_dmdt[64], c_mtend[64];
   // dnw and c1h in LDS for the serial column sum and omega recurrence (their
   // global loads would otherwise sit on the recurrence's critical path)
   __shared__ float c_dnw[kColMaxLev], c_c1h[kColMaxLev];
@@ -219,19 +204,41 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
       }
     }
   }
+  // phase 3's loads, in flight over the barriers and the serial part before it
+  float r3_w1[G3], r3_wm[G3];
+  auto load3 = [&](int gq) {
+    const float *ww_1 = FL(ww_1);
+#pragma unroll
+    for (int q = 0; q < G3; q++) {
+      const int k = imin_(LEV(gq + q), kend);
+      r3_w1[q] = A3(ww_1, i, k, j);
+      r3_wm[q] = first ? 0.f : A3(ww_m, i, k, j);
+    }
+  };
+  if (interior) load3(0);
   __syncthreads();
-  // ---- 2. column sum, column-mass update and the omega recurrence (wave 0)
+  // ---- 2. column sum and column-mass update (wave 0), the level terms of the
+  // omega recurrence (all waves: the division is off the recurrence's chain),
+  // then the recurrence itself
   if (wv == 0 && interior) {
     // column mass tendency: FP32 level terms summed in FP64, rounded once
-    double dmdt_acc = 0.0;
-    for (int k = 1; k <= kend; k++) dmdt_acc += (double)(c_dnw[k - 1] * LS(B0, k));
-    const float dmdt = (float)dmdt_acc;
     float *mu = FL(mu_2);
     const float old = A2(mu, i, j);
     const float mtend = A2(FL(mu_tend), i, j);
+    const float mut = A2(FL(mut), i, j);
+    double dmdt_acc = 0.0;
+    for (int k0 = 1; k0 <= kend; k0 += 8) {  // 8 levels' operands ahead of the chain
+      float r[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) r[q] = c_dnw[imin_(k0 + q, kend) - 1] * LS(B0, imin_(k0 + q, kend));
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        if (k0 + q <= kend) dmdt_acc += (double)r[q];
+    }
+    const float dmdt = (float)dmdt_acc;
     const float tend = dmdt + mtend;
     const float nmu = old + dts * tend;
-    const float mts = A2(FL(mut), i, j) + nmu;
+    const float mts = mut + nmu;
     const float mav = 0.5f * ((1.f + epssm) * nmu + (1.f - epssm) * old);
     A2(mu, i, j) = nmu;
     A2(FL(mudf), i, j) = tend;
@@ -239,15 +246,8 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
     A2(FL(muave), i, j) = mav;
     c_mts[lane] = mts;
     c_mav[lane] = mav;
-    float prev = A3(ww, i, 1, j);
-    LS(B1, 1) = prev;
-    for (int k = 2; k <= kend; k++) {
-      float integ = c_c1h[k - 2] * dmdt + LS(B0, k - 1);
-      integ = integ + c_c1h[k - 2] * mtend;
-      const float cur = prev - (c_dnw[k - 2] * integ) / msfty;
-      LS(B1, k) = cur;
-      prev = cur;
-    }
+    c_dmdt[lane] = dmdt;
+    c_mtend[lane] = mtend;
   }
   if (wv == 0 && zone) {
     const float mt = A2(FL(mu_tend), i, j);
@@ -257,28 +257,47 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
     c_mts[lane] = mts;
   }
   __syncthreads();
+  if (interior) {
+    const float dmdt = c_dmdt[lane], mtend = c_mtend[lane];
+    for (int k = 1 + wv; k < kend; k += NW) {
+      float integ = c_c1h[k - 1] * dmdt + LS(B0, k);
+      integ = integ + c_c1h[k - 1] * mtend;
+      LS(B1, k + 1) = (c_dnw[k - 1] * integ) / msfty;
+    }
+  }
+  __syncthreads();
+  if (wv == 0 && interior) {
+    float prev = A3(ww, i, 1, j);
+    LS(B1, 1) = prev;
+    for (int k0 = 2; k0 <= kend; k0 += 8) {
+      float r[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) r[q] = LS(B1, imin_(k0 + q, kend));
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        if (k0 + q <= kend) {
+          prev = prev - r[q];
+          LS(B1, k0 + q) = prev;
+        }
+    }
+  }
+  __syncthreads();
   // ---- 3. omega minus the stage-start omega (B1 = final omega, k = 1..kde),
   // and sumflux of the column's w points
   if (interior) {
     const float *ww_1 = FL(ww_1);
 #pragma unroll
     for (int gq = 0; gq < NPW; gq += G3) {
-      float r[G3], r_wwm[G3];
-#pragma unroll
-      for (int q = 0; q < G3; q++) {
-        const int k = imin_(LEV(gq + q), kend);
-        r[q] = A3(ww_1, i, k, j);
-        r_wwm[q] = first ? 0.f : A3(ww_m, i, k, j);
-      }
+      if (gq > 0) load3(gq);
 #pragma unroll
       for (int q = 0; q < G3; q++) {
         const int k = LEV(gq + q);
         if (k > kend) break;
-        const float vv = LS(B1, k) - r[q];
+        const float vv = LS(B1, k) - r3_w1[q];
         A3(ww, i, k, j) = vv;
         LS(B1, k) = vv;
-        float aw = r_wwm[q] + vv;
-        if (fin) aw = aw / ns + r[q];
+        float aw = r3_wm[q] + vv;
+        if (fin) aw = aw / ns + r3_w1[q];
         A3(ww_m, i, k, j) = aw;
       }
     }
@@ -453,6 +472,21 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
   // so their latency overlaps it).  Meanwhile the other waves copy gamma of
   // every level into B2 (free between phase 6 and phase 9), so the backward
   // sweep reads it from LDS.
+  // phase 10's loads (its inputs that no later phase writes), in flight over the sweeps
+  float r_alt[G10], r_t1[G10], r_t2[G10], r_c2a[G10], r_pm1[G10];
+  auto load10 = [&](int gq) {
+    const float *alt = FL(alt), *t_2 = FL(t_2), *c2a = FL(c2a), *pm1 = FL(pm1);
+#pragma unroll
+    for (int q = 0; q < G10; q++) {
+      const unsigned o = XI3(i, imin_(LEV(gq + q), kend), j);
+      r_alt[q] = elem(alt, o);
+      r_t1[q] = elem(t_1, o);
+      r_t2[q] = elem(t_2, o);
+      r_c2a[q] = elem(c2a, o);
+      r_pm1[q] = elem(pm1, o);
+    }
+  };
+  if (mass) load10(0);
   const int sk = x->ip;  // element stride between levels
   const unsigned o1 = XI3(ic, 1, jc);
   float wprev = 0.f;
@@ -463,7 +497,7 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
     // forward: levels 2..kde
     {
       const int n = kde - 1;
-      float ca[C], cl[C], na[C], nl[C];
+      float ca[C], cl[C], na[C], nl[C], rb[C];
 #pragma unroll
       for (int q = 0; q < C; q++) {
         const int k = imin_(2 + q, kde);
@@ -478,10 +512,12 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
           nl[q] = alpha[o1 + (unsigned)((k - 1) * sk)];
         }
 #pragma unroll
+        for (int q = 0; q < C; q++) rb[q] = LS(B3, imin_(2 + c0 + q, kde));
+#pragma unroll
         for (int q = 0; q < C; q++) {
           const int k = 2 + c0 + q;
           if (k <= kde) {
-            const float wl = (LS(B3, k) - ca[q] * wprev) * cl[q];
+            const float wl = (rb[q] - ca[q] * wprev) * cl[q];
             LS(B3, k) = wl;
             wprev = wl;
           }
@@ -500,11 +536,20 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
   __syncthreads();
   // backward: levels kend..2
   if (wv == 0 && interior) {
-#pragma unroll 8
-    for (int k = kend; k >= 2; k--) {
-      const float wl = LS(B3, k) - LS(B2, k) * wprev;
-      LS(B3, k) = wl;
-      wprev = wl;
+    for (int k0 = kend; k0 >= 2; k0 -= 8) {
+      float rb[8], rg[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        rb[q] = LS(B3, imax_(k0 - q, 2));
+        rg[q] = LS(B2, imax_(k0 - q, 2));
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        if (k0 - q >= 2) {
+          const float wl = rb[q] - rg[q] * wprev;
+          LS(B3, k0 - q) = wl;
+          wprev = wl;
+        }
     }
   }
   __syncthreads();
@@ -514,9 +559,13 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
     const float mts = c_mts[lane];
     const float pcoef = (((msfty * 0.5f) * dts) * g) * ope;
     float *w = FL(w_2);
+    const int ri = !ring ? 0 : i == 2 ? 1 : i == ide - 2 ? ide - 1 : 0, rj = !ring ? 0 : j == 2 ? 1 : j == jde - 2 ? jde - 1 : 0;
     for (int k = 1 + wv; k <= kde; k += NW) {
       const float wl = LS(B3, k);
       A3(w, i, k, j) = wl;
+      if (ri) A3(w, ri, k, j) = wl;
+      if (rj) A3(w, i, k, rj) = wl;
+      if (ri && rj) A3(w, ri, k, rj) = wl;
       float phn;
       if (k == 1) phn = A3(php2, i, 1, j);
       else {
@@ -615,20 +664,10 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
   if (mass) {
     const float mts = c_mts[lane], mu2 = A2(FL(mu_2), i, j);
     const bool gx = (i == ide - 1), gy = (j == jde - 1);
-    const float *alt = FL(alt), *t_2 = FL(t_2), *c2a = FL(c2a);
     float *al = FL(al), *p = FL(p), *pm1 = FL(pm1);
 #pragma unroll
     for (int gq = 0; gq < NPW; gq += G10) {
-      float r_alt[G10], r_t1[G10], r_t2[G10], r_c2a[G10], r_pm1[G10];
-#pragma unroll
-      for (int q = 0; q < G10; q++) {
-        const size_t o = XI3(i, imin_(LEV(gq + q), kend), j);
-        r_alt[q] = alt[o];
-        r_t1[q] = t_1[o];
-        r_t2[q] = t_2[o];
-        r_c2a[q] = c2a[o];
-        r_pm1[q] = pm1[o];
-      }
+      if (gq > 0) load10(gq);
 #pragma unroll
       for (int q = 0; q < G10; q++) {
         const int k = LEV(gq + q);
@@ -683,29 +722,43 @@ __global__ void __launch_bounds__(64 * kColWaves) k_acoustic_col(const DevCtx *x
 #undef LEV
 }
 
-// host launcher: instantiation by levels per wave
-// store_tav: write the acoustic theta average to t_2ave (only its last
-// substep's value is read outside the kernel)
-inline void launch_acoustic_col(const DevCtx &d, const DevCtx *dev, hipStream_t s, float dts, int first, int fin, float ns, int store_tav) {
-  const dim3 grid((unsigned)((d.ide + 63) / 64) * (unsigned)d.jde), block(64, kColWaves);
-  const size_t lds = acoustic_col_lds(d.kde);
-  switch (acoustic_col_npw(d.kde)) {
-    case 4: k_acoustic_col<4><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
-    case 8: k_acoustic_col<8><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
-    case 12: k_acoustic_col<12><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
-    case 16: k_acoustic_col<16><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
-    default: k_acoustic_col<20><<<grid, block, lds, s>>>(dev, dts, first, fin, ns, store_tav); break;
+// A domain of at most kColWideBlocks blocks leaves CUs idle, so its substep
+// takes as long as one block does: 16 waves, each with half the levels
+// (a substep's column kernel at 100x100x45, 202 blocks: 44 us with 8 waves, 33
+// with 16; at 24x20x10 14 and 12).  From there on 8 waves: three such blocks
+// share a CU, one of 16.
+constexpr unsigned kColWideBlocks = 256;
+inline unsigned acoustic_col_blocks(const DevCtx &d) { return (unsigned)((d.ide + 63) / 64) * (unsigned)d.jde; }
+// one instantiation per levels-per-wave range: fn(std::integral_constant<NW>, <NPW>)
+template <class Fn>
+inline auto acoustic_col_pick(int kde, bool wide, Fn fn) {
+#define PICK(nw, npw) fn(std::integral_constant<int, nw>(), std::integral_constant<int, npw>())
+  if (wide) {
+    const int need = (kde + 15) / 16;
+    return need <= 2 ? PICK(16, 2) : need <= 4 ? PICK(16, 4) : need <= 6 ? PICK(16, 6) : PICK(16, 10);
   }
+  const int need = (kde + 7) / 8;
+  return need <= 4 ? PICK(8, 4) : need <= 8 ? PICK(8, 8) : need <= 12 ? PICK(8, 12) : need <= 16 ? PICK(8, 16) : PICK(8, 20);
+#undef PICK
 }
-// raise the dynamic-LDS limit of the instantiation kde needs (beyond 64 KB)
+// store_tav: write the acoustic theta average to t_2ave (only its last
+// substep's value is read outside the kernel); ring: zero_grad_bdy of w too
+inline void launch_acoustic_col(const DevCtx &d, const DevCtx *dev, hipStream_t s, float dts, int first, int fin, float ns, int store_tav, int ring) {
+  const unsigned nb = acoustic_col_blocks(d);
+  acoustic_col_pick(d.kde, nb <= kColWideBlocks, [&](auto nw, auto npw) {
+    k_acoustic_col<nw(), npw()><<<nb, dim3(64, nw()), acoustic_col_lds(d.kde), s>>>(dev, dts, first, fin, ns, store_tav, ring);
+    return 0;
+  });
+}
+// raise the dynamic-LDS limit of the instantiations kde can need (beyond 64 KB)
 inline hipError_t acoustic_col_allow_lds(int kde) {
   const int lds = (int)acoustic_col_lds(kde);
   if (lds <= 65536) return hipSuccess;
-  switch (acoustic_col_npw(kde)) {
-    case 4: return hipFuncSetAttribute((const void *)k_acoustic_col<4>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    case 8: return hipFuncSetAttribute((const void *)k_acoustic_col<8>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    case 12: return hipFuncSetAttribute((const void *)k_acoustic_col<12>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    case 16: return hipFuncSetAttribute((const void *)k_acoustic_col<16>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    default: return hipFuncSetAttribute((const void *)k_acoustic_col<20>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  for (const bool wide : {false, true}) {
+    const hipError_t e = acoustic_col_pick(kde, wide, [&](auto nw, auto npw) {
+      return hipFuncSetAttribute((const void *)k_acoustic_col<nw(), npw()>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    });
+    if (e != hipSuccess) return e;
   }
+  return hipSuccess;
 }

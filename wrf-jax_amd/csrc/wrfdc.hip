@@ -854,16 +854,14 @@ struct Run {
     k_zero_grad_rows<<<dim3(cdiv(ide - 1, 64), kde, 2), 64, 0, s>>>(D(), F(F_w_2));
     k_zero_grad_cols<<<dim3(cdiv(jde - 1, 64), kde, 2), 64, 0, s>>>(D(), F(F_w_2));
   }
-  // one fused acoustic substep: u/v, the column kernel, zero_grad_bdy of w;
+  // one fused acoustic substep: u/v, then the column kernel;
   // all_outputs: also the intermediate t_2ave (a substep called on its own)
   void acoustic_substep(int it, bool all_outputs) const {
     X->iteration = it;
     const float dts = (float)X->dts_rk;
     R3 r{1, ide, 1, kde - 1, 1, jde};
     k_uv_substep<<<g3(r), b3(), 0, s>>>(D(), dts, r);
-    launch_acoustic_col(d, D(), s, dts, it == 1, it == X->nsmall, (float)X->nsmall, all_outputs || it == X->nsmall);
-    Z z = zd('w', true, false);
-    k_zero_grad_w<<<dim3(cdiv(zone_n(z), 64), kde), 64, 0, s>>>(D());
+    launch_acoustic_col(d, D(), s, dts, it == 1, it == X->nsmall, (float)X->nsmall, all_outputs || it == X->nsmall, 1);
   }
   // calc_mu_uv_1: the staggered column masses of muts
   void calc_mu_uv_1() const {
@@ -1857,7 +1855,7 @@ int wrfdc_stage(wrfdc_ctx *x, const char *name, int rk_step, int iteration) {
         R3 r{1, run.ide, 1, run.kde - 1, 1, run.jde};
         k_uv_substep<<<Run::g3(r), Run::b3(), 0, x->s>>>(run.D(), dts, r);
       } else {
-        launch_acoustic_col(run.d, run.D(), x->s, dts, x->iteration == 1, x->iteration == x->nsmall, (float)x->nsmall, 1);
+        launch_acoustic_col(run.d, run.D(), x->s, dts, x->iteration == 1, x->iteration == x->nsmall, (float)x->nsmall, 1, 0);
       }
     }
     else if (n == "w_solve:columns" || n == "w_solve:levels") {
