@@ -8,14 +8,18 @@
 
 // rho = (1 + qv) / alt on mass points (phy_prep,
 // module_big_step_utilities_em.py:1823-2081, rho at :1965)
+__device__ __forceinline__ void rho_pt(CtxPtr x, int i, int k, int j) {
+  A3(FL(rho), i, k, j) = (1.f / A3(FL(alt), i, k, j)) * (1.f + A3(SP(moist, 0), i, k, j));
+}
 __global__ void k_rho(const DevCtx *xv, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
-  A3(FL(rho), i, k, j) = (1.f / A3(FL(alt), i, k, j)) * (1.f + A3(SP(moist, 0), i, k, j));
+  rho_pt(x, i, k, j);
 }
 
-// compute_diff_metrics (module_diffusion_em.py:1825-2043), full extent.
-__global__ void k_diff_metrics(const DevCtx *xv, R3 r) {
+// compute_diff_metrics (module_diffusion_em.py:1825-2043), full extent; with
+// rho too where the step has not formed it yet.
+__global__ void k_diff_metrics(const DevCtx *xv, R3 r, int rho) {
   const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde, ktf = kde - 1;
@@ -51,6 +55,7 @@ __global__ void k_diff_metrics(const DevCtx *xv, R3 r) {
     s = s + A3(ph, i, k + 1, j);
     s = s + A3(phb, i, k + 1, j);
     A3(FL(z), i, k, j) = (0.5f * s) / g;
+    if (rho) rho_pt(x, i, k, j);
   }
 }
 
@@ -76,9 +81,7 @@ __device__ __forceinline__ float hat_avg(CtxPtr x, const float *f, const float *
 
 // cal_deform_and_div (module_diffusion_em.py:366-891): D11, D22, D33 and the
 // divergence on mass points.
-__global__ void k_deform_diag(const DevCtx *xv, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+__device__ __forceinline__ void deform_diag(CtxPtr x, int i, int k, int j) {
   const float *u = FL(u_2), *v = FL(v_2), *w = FL(w_2), *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw);
   const float *msfuy = FL(msfuy), *msfvx = FL(msfvx);
   const float mm = A2(FL(msftx), i, j) * A2(FL(msfty), i, j);
@@ -103,10 +106,24 @@ __global__ void k_deform_diag(const DevCtx *xv, R3 r) {
   A3(FL(div), i, k, j) = dv;
 }
 
-// D12 at (u, v) corner points i [2, ide-1], j [2, jde-1], k [1, kde-1]
-__global__ void k_deform12(const DevCtx *xv, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+// v at (i, k, j) of i [2, ide-1], j [2, jde-1], and at the edge points that
+// copy it: column 1 and ide, row 1 and jde take the nearest of the range (the
+// reference's copies of whole planes one after another end with the same)
+__device__ __forceinline__ void store_edges(CtxPtr x, float *f, int i, int k, int j, float v) {
+  const int ie = i == 2 ? 1 : i == x->ide - 1 ? x->ide : 0, je = j == 2 ? 1 : j == x->jde - 1 ? x->jde : 0;
+  A3(f, i, k, j) = v;
+  if (ie) A3(f, ie, k, j) = v;
+  if (je) A3(f, i, k, je) = v;
+  if (ie && je) A3(f, ie, k, je) = v;
+}
+
+// D12 at (u, v) corner points i [2, ide-1], j [2, jde-1], k [1, kde-1] (level
+// kde, which nothing forms, takes part in the copies to the edges)
+__device__ __forceinline__ void deform12(CtxPtr x, int i, int k, int j) {
+  if (k == x->kde) {
+    store_edges(x, FL(defor12), i, k, j, A3(FL(defor12), i, k, j));
+    return;
+  }
   const float *u = FL(u_2), *v = FL(v_2), *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw), *msfux = FL(msfux), *msfvy = FL(msfvy);
   const float mm = 0.25f * (A2(msfux, i, j - 1) + A2(msfux, i, j)) * (A2(msfvy, i - 1, j) + A2(msfvy, i, j));
   float d;
@@ -123,18 +140,16 @@ __global__ void k_deform12(const DevCtx *xv, R3 r) {
     const float second = mm * (x->rdx * (hatv(x, v, msfvy, i, k, j) - hatv(x, v, msfvy, i - 1, k, j)) - t1);
     d = d + second;
   }
-  A3(FL(defor12), i, k, j) = d;
+  store_edges(x, FL(defor12), i, k, j, d);
 }
 
 // D13 / D23 at (u, w) and (v, w) points i [2, ide-1], j [2, jde-1], k [1, kde]
-__global__ void k_deform13_23(const DevCtx *xv, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+__device__ __forceinline__ void deform13_23(CtxPtr x, int i, int k, int j) {
   const int ktf = x->kde - 1;
   float *d13 = FL(defor13), *d23 = FL(defor23);
   if (k == 1 || k == ktf + 1) {
-    A3(d13, i, k, j) = 0.f;
-    A3(d23, i, k, j) = 0.f;
+    store_edges(x, d13, i, k, j, 0.f);
+    store_edges(x, d23, i, k, j, 0.f);
     return;
   }
   const float *w = FL(w_2), *u = FL(u_2), *v = FL(v_2), *zx = FL(zx), *zy = FL(zy), *rdz = FL(rdz);
@@ -146,7 +161,7 @@ __global__ void k_deform13_23(const DevCtx *xv, R3 r) {
     const float t1 = (AV13(k) - AV13(k - 1)) * A3(zx, i, k, j) * 0.5f * (A3(rdz, i, k, j) + A3(rdz, i - 1, k, j));
     float d = mm * (x->rdx * (H13(i, k) - H13(i - 1, k)) - t1);
     const float val = (A3(u, i, k, j) - A1(ub, k) - A3(u, i, k - 1, j) + A1(ub, k - 1)) * 0.5f * (A3(rdz, i, k, j) + A3(rdz, i - 1, k, j));
-    A3(d13, i, k, j) = d + val;
+    store_edges(x, d13, i, k, j, d + val);
 #undef AV13
 #undef H13
   }
@@ -157,27 +172,32 @@ __global__ void k_deform13_23(const DevCtx *xv, R3 r) {
     const float t1 = (AV23(k) - AV23(k - 1)) * A3(zy, i, k, j) * 0.5f * (A3(rdz, i, k, j) + A3(rdz, i, k, j - 1));
     float d = mm * (x->rdy * (H23(j, k) - H23(j - 1, k)) - t1);
     const float val = (A3(v, i, k, j) - A1(vb, k) - A3(v, i, k - 1, j) + A1(vb, k - 1)) * 0.5f * (A3(rdz, i, k, j) + A3(rdz, i, k, j - 1));
-    A3(d23, i, k, j) = d + val;
+    store_edges(x, d23, i, k, j, d + val);
 #undef AV23
 #undef H23
   }
 }
 
-// edge copy of whole planes: i = idst <- isrc for every (k, j) (axis 0) or
-// j = jdst <- jsrc for every (i, k) (axis 1); up to two fields per launch.
-__global__ void k_edge_copy(const DevCtx *xv, float *f0, float *f1, int axis, int dst, int src, int kend) {
+// cal_deform_and_div in one launch: the three groups of components, which
+// read the same winds and metrics and not each other, over three ranges of
+// blocks (first = first block of each range, first[3] the grid).  With the
+// edge copies in launches of their own they were eleven (400x400x60: 375 us
+// of kernels and the eight copies, 320 us this way; 24x20x10 33 and 7 us).
+struct DeformRanges {
+  R3 r[3];
+  unsigned first[4];
+};
+__global__ void __launch_bounds__(256) k_deform(const DevCtx *xv, DeformRanges R) {
   const CtxPtr x = ctx_ptr(xv);
-  const int a = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int k = 1 + (int)blockIdx.y;
-  if (k > kend) return;
-  if (axis == 0) {
-    if (a > x->jde) return;
-    A3(f0, dst, k, a) = A3(f0, src, k, a);
-    if (f1) A3(f1, dst, k, a) = A3(f1, src, k, a);
+  if (blockIdx.x < R.first[1]) {
+    GET_IKJ_B(R.r[0], blockIdx.x, R.first[1]);
+    deform_diag(x, i, k, j);
+  } else if (blockIdx.x < R.first[2]) {
+    GET_IKJ_B(R.r[1], blockIdx.x - R.first[1], R.first[2] - R.first[1]);
+    deform12(x, i, k, j);
   } else {
-    if (a > x->ide) return;
-    A3(f0, a, k, dst) = A3(f0, a, k, src);
-    if (f1) A3(f1, a, k, dst) = A3(f1, a, k, src);
+    GET_IKJ_B(R.r[2], blockIdx.x - R.first[2], R.first[3] - R.first[2]);
+    deform13_23(x, i, k, j);
   }
 }
 
@@ -338,15 +358,22 @@ __device__ __forceinline__ float titau_val(CtxPtr x, const float *xk, const floa
   }
   return val;
 }
-// the two stress components one diffusion kernel reads, in one pass
+// the two stress components a momentum diffusion reads, and those of all
+// three in one launch (nb: blocks of one of them)
 struct TitauPair {
   float *tt[2];
   const float *xk[2], *defor[2];
   int kind[2], i0[2], i1[2], j0[2], j1[2];
 };
-__global__ void k_titau(const DevCtx *xv, TitauPair P, R3 r) {
+struct TitauList {
+  TitauPair p[3];
+  unsigned nb;
+};
+__global__ void k_titau(const DevCtx *xv, TitauList L, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+  const unsigned q = blockIdx.x / L.nb;
+  const TitauPair &P = L.p[q];
+  GET_IKJ_B(r, blockIdx.x - q * L.nb, L.nb);
   const float v0 = titau_val(x, P.xk[0], P.defor[0], P.kind[0], P.i0[0], P.i1[0], P.j0[0], P.j1[0], i, k, j);
   const float v1 = titau_val(x, P.xk[1], P.defor[1], P.kind[1], P.i0[1], P.i1[1], P.j0[1], P.j1[1], i, k, j);
   A3(P.tt[0], i, k, j) = v0;
@@ -363,9 +390,7 @@ __device__ __forceinline__ float hd_a2u(CtxPtr x, const float *t2, int i, int k,
   if (k == 1 || k == x->kde) return 0.f;
   return 0.5f * (A1(FL(fnm), k) * (A3(t2, i, k, j + 1) + A3(t2, i, k, j)) + A1(FL(fnp), k) * (A3(t2, i, k - 1, j + 1) + A3(t2, i, k - 1, j)));
 }
-__global__ void k_hdiff_u(const DevCtx *xv, const float *t1, const float *t2, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+__device__ __forceinline__ void hdiff_u(CtxPtr x, const float *t1, const float *t2, int i, int k, int j) {
   const float *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw);
   const float zxu = 0.5f * (A3(zx, i, k, j) + A3(zx, i, k + 1, j));
   const float zyu = 0.125f * (A3(zy, i - 1, k, j) + A3(zy, i, k, j) + A3(zy, i - 1, k, j + 1) + A3(zy, i, k, j + 1) + A3(zy, i - 1, k + 1, j) +
@@ -390,9 +415,7 @@ __device__ __forceinline__ float hd_a2v(CtxPtr x, const float *t2, int i, int k,
   if (k == 1 || k == x->kde) return 0.f;
   return 0.5f * (A1(FL(fnm), k) * (A3(t2, i, k, j - 1) + A3(t2, i, k, j)) + A1(FL(fnp), k) * (A3(t2, i, k - 1, j - 1) + A3(t2, i, k - 1, j)));
 }
-__global__ void k_hdiff_v(const DevCtx *xv, const float *t1, const float *t2, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+__device__ __forceinline__ void hdiff_v(CtxPtr x, const float *t1, const float *t2, int i, int k, int j) {
   const float *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw);
   const float zxv = 0.125f * (A3(zx, i, k, j) + A3(zx, i + 1, k, j) + A3(zx, i, k, j - 1) + A3(zx, i + 1, k, j - 1) + A3(zx, i, k + 1, j) +
                               A3(zx, i + 1, k + 1, j) + A3(zx, i, k + 1, j - 1) + A3(zx, i + 1, k + 1, j - 1));
@@ -409,9 +432,7 @@ __global__ void k_hdiff_v(const DevCtx *xv, const float *t1, const float *t2, R3
 
 // horizontal_diffusion_w_2 (module_diffusion_em.py:2768-2985):
 // w points i [2, ide-2], j [2, jde-2], k [2, kde-1].
-__global__ void k_hdiff_w(const DevCtx *xv, const float *t1, const float *t2, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+__device__ __forceinline__ void hdiff_w(CtxPtr x, const float *t1, const float *t2, int i, int k, int j) {
   const float *zx = FL(zx), *zy = FL(zy), *rdz = FL(rdz);
 #define HA1(kk) (0.25f * (A3(t1, i + 1, (kk) + 1, j) + A3(t1, i, (kk) + 1, j) + A3(t1, i + 1, kk, j) + A3(t1, i, kk, j)))
 #define HA2(kk) (0.25f * (A3(t2, i, (kk) + 1, j + 1) + A3(t2, i, (kk) + 1, j) + A3(t2, i, kk, j + 1) + A3(t2, i, kk, j)))
@@ -425,6 +446,25 @@ __global__ void k_hdiff_w(const DevCtx *xv, const float *t1, const float *t2, R3
 #undef HA1
 #undef HA2
   A3(FL(rw_tendf), i, k, j) = A3(FL(rw_tendf), i, k, j) + inc;
+}
+
+// the momentum diffusions (u, v, w) from their stresses in one launch.  With
+// a pair of stress arrays used in turn, six launches, horizontal_diffusion_2
+// took 34 us at 24x20x10 and 1253 us at 400x400x60, with six arrays 22 and
+// 1238 us.
+struct HdiffList {
+  const float *t1[3], *t2[3];
+  R3 r[3];
+  unsigned first[4];
+};
+__global__ void __launch_bounds__(256) k_hdiff(const DevCtx *xv, HdiffList L) {
+  const CtxPtr x = ctx_ptr(xv);
+  const int q = blockIdx.x < L.first[1] ? 0 : blockIdx.x < L.first[2] ? 1 : 2;
+  const float *t1 = L.t1[q], *t2 = L.t2[q];
+  GET_IKJ_B(L.r[q], blockIdx.x - L.first[q], L.first[q + 1] - L.first[q]);
+  if (q == 0) hdiff_u(x, t1, t2, i, k, j);
+  else if (q == 1) hdiff_v(x, t1, t2, i, k, j);
+  else hdiff_w(x, t1, t2, i, k, j);
 }
 
 // horizontal_diffusion_s (module_diffusion_em.py:2046-2291) of every

@@ -519,11 +519,6 @@ struct Run {
     }
     ~FinalBatch() { flush(); }
   };
-  void edge_copy(float *f0, float *f1, int axis, int dst, int src_, int kend) const {
-    const int n = axis == 0 ? jde : ide;
-    k_edge_copy<<<dim3(cdiv(n, 64), kend), 64, 0, s>>>(D(), f0, f1, axis, dst, src_, kend);
-  }
-
   // ---- RK-stage pieces -----------------------------------------------------
   void rk_step_prep() const {
     k_mu_uv<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D(), F(F_mu_2), F(F_mub), F(F_muu), F(F_muv), F(F_mut));
@@ -532,33 +527,26 @@ struct Run {
     R2 c = mass2();
     k_ww_cp<<<g2(c), 64, sizeof(float) * 64 * (size_t)(kde - 1), s>>>(D(), c);
   }
-  void first_rk_step_part1() const {
+  void first_rk_step_part1(bool with_rho = true) const {
     const size_t n3 = X->n3;
     fill_many({{F(F_ru_tendf), n3}, {F(F_rv_tendf), n3}, {F(F_rw_tendf), n3}, {F(F_ph_tendf), n3}, {F(F_t_tendf), n3},
                {F(F_mu_tendf), X->n2}, {F(F_moist_tend), n3 * (size_t)X->c.nmoist},
                {F(F_scalar_tend), n3 * (size_t)X->c.nscalar}});
+    if (!with_rho) return;  // the step forms rho with the diffusion metrics
     R3 m = mass3();
     k_rho<<<g3p(m), b3(), 0, s>>>(D(), m);
   }
-  void compute_diff_metrics() const {
+  void compute_diff_metrics(bool with_rho = false) const {
     R3 r = full3();
-    k_diff_metrics<<<g3(r), b3(), 0, s>>>(D(), r);
+    k_diff_metrics<<<g3(r), b3(), 0, s>>>(D(), r, with_rho ? 1 : 0);
   }
   void cal_deform_and_div() const {
-    R3 m = mass3();
-    k_deform_diag<<<g3(m), b3(), 0, s>>>(D(), m);
-    R3 r12{2, ide - 1, 1, kde - 1, 2, jde - 1};
-    k_deform12<<<g3(r12), b3(), 0, s>>>(D(), r12);
-    edge_copy(F(F_defor12), nullptr, 0, 1, 2, kde);
-    edge_copy(F(F_defor12), nullptr, 1, 1, 2, kde);
-    edge_copy(F(F_defor12), nullptr, 0, ide, ide - 1, kde);
-    edge_copy(F(F_defor12), nullptr, 1, jde, jde - 1, kde);
-    R3 r13{2, ide - 1, 1, kde, 2, jde - 1};
-    k_deform13_23<<<g3(r13), b3(), 0, s>>>(D(), r13);
-    edge_copy(F(F_defor13), F(F_defor23), 0, 1, 2, kde);
-    edge_copy(F(F_defor13), F(F_defor23), 1, 1, 2, kde);
-    edge_copy(F(F_defor13), F(F_defor23), 0, ide, ide - 1, kde);
-    edge_copy(F(F_defor13), F(F_defor23), 1, jde, jde - 1, kde);
+    DeformRanges R;
+    R.r[0] = mass3();
+    R.r[1] = R.r[2] = R3{2, ide - 1, 1, kde, 2, jde - 1};
+    R.first[0] = 0;
+    for (int q = 0; q < 3; q++) R.first[q + 1] = R.first[q] + g3(R.r[q]).x;
+    k_deform<<<R.first[3], b3(), 0, s>>>(D(), R);
   }
   void smag2d_km() const {
     R3 r{2, ide - 2, 1, kde - 1, 2, jde - 2};
@@ -595,9 +583,9 @@ struct Run {
     R3 r{2, ide - 2, 1, kde - 1, 2, jde - 2};
     k_closure_rows<<<g3p(r), b3(), 0, s>>>(D(), r, nm, Scr(S_FQX), Scr(S_FQY), Scr(S_T2), Xr, T);
   }
-  // two stress components (t1, t2 of one diffusion kernel) in one launch;
-  // each entry: xk, defor, kind, i0, i1, j0, j1
-  void titau(float *t1, float *t2, std::array<int, 7> a, std::array<int, 7> b) const {
+  // two stress components (t1, t2 of one diffusion); each entry: xk, defor,
+  // kind, i0, i1, j0, j1
+  TitauPair titau(float *t1, float *t2, std::array<int, 7> a, std::array<int, 7> b) const {
     TitauPair P;
     P.tt[0] = t1;
     P.tt[1] = t2;
@@ -611,8 +599,7 @@ struct Run {
       P.j0[n] = (*e[n])[5];
       P.j1[n] = (*e[n])[6];
     }
-    R3 r = full3();
-    k_titau<<<g3(r), b3(), 0, s>>>(D(), P, r);
+    return P;
   }
   // horizontal_diffusion_s of theta and every species: faces, then tendencies
   void hdiff_scalars() const {
@@ -634,22 +621,31 @@ struct Run {
     k_hdiff_s_tend<<<g3(rt), b3(), 0, s>>>(D(), L, rt);
   }
   void horizontal_diffusion_2() const {
-    float *t1 = Scr(S_T1), *t2 = Scr(S_T2);
-    titau(t1, t2, {F_xkmh, F_defor11, 11, 1, ide - 1, 2, jde - 1}, {F_xkmh, F_defor12, 12, 2, ide - 1, 2, jde});
-    R3 ru{2, ide - 1, 1, kde - 1, 2, jde - 2};
-    k_hdiff_u<<<g3(ru), b3(), 0, s>>>(D(), t1, t2, ru);
-    titau(t1, t2, {F_xkmh, F_defor12, 12, 2, ide, 2, jde - 1}, {F_xkmh, F_defor22, 11, 2, ide - 1, 1, jde - 1});
-    R3 rv{2, ide - 2, 1, kde - 1, 2, jde - 1};
-    k_hdiff_v<<<g3(rv), b3(), 0, s>>>(D(), t1, t2, rv);
-    titau(t1, t2, {F_xkmv, F_defor13, 13, 2, ide, 2, jde - 2}, {F_xkmv, F_defor23, 23, 2, ide - 2, 2, jde});
-    R3 rw{2, ide - 2, 2, kde - 1, 2, jde - 2};
-    k_hdiff_w<<<g3(rw), b3(), 0, s>>>(D(), t1, t2, rw);
+    const R3 full = full3();
+    const R3 r[3] = {{2, ide - 1, 1, kde - 1, 2, jde - 2}, {2, ide - 2, 1, kde - 1, 2, jde - 1}, {2, ide - 2, 2, kde - 1, 2, jde - 2}};
+    float *const t[6] = {Scr(S_T1), Scr(S_T2), Scr(S_FQX), Scr(S_FQY), Scr(S_FQZ), Scr(S_FQXL)};
+    TitauList T;
+    memset(&T, 0, sizeof(T));
+    T.nb = g3(full).x;
+    T.p[0] = titau(t[0], t[1], {F_xkmh, F_defor11, 11, 1, ide - 1, 2, jde - 1}, {F_xkmh, F_defor12, 12, 2, ide - 1, 2, jde});
+    T.p[1] = titau(t[2], t[3], {F_xkmh, F_defor12, 12, 2, ide, 2, jde - 1}, {F_xkmh, F_defor22, 11, 2, ide - 1, 1, jde - 1});
+    T.p[2] = titau(t[4], t[5], {F_xkmv, F_defor13, 13, 2, ide, 2, jde - 2}, {F_xkmv, F_defor23, 23, 2, ide - 2, 2, jde});
+    HdiffList H;
+    memset(&H, 0, sizeof(H));
+    for (int q = 0; q < 3; q++) {
+      H.t1[q] = t[2 * q];
+      H.t2[q] = t[2 * q + 1];
+      H.r[q] = r[q];
+      H.first[q + 1] = H.first[q] + g3(r[q]).x;
+    }
+    k_titau<<<3u * T.nb, b3(), 0, s>>>(D(), T, full);
+    k_hdiff<<<H.first[3], b3(), 0, s>>>(D(), H);
     hdiff_scalars();
   }
   // with_n2: also N^2 (the stage API always, the step when the learned
   // closure reads it)
-  void first_rk_step_part2(bool with_n2) const {
-    compute_diff_metrics();
+  void first_rk_step_part2(bool with_n2, bool with_rho = false) const {
+    compute_diff_metrics(with_rho);
     BcBatch(this).add3(F(F_rdzw), 'w').add3(F(F_rdz), 'w').add3(F(F_z), 'w').add3(F(F_zx), 'e').add3(F(F_zy), 'f').flush();
     cal_deform_and_div();
     if (with_n2 || X->cl_theta) calculate_n2();
@@ -1134,8 +1130,8 @@ struct Run {
       phys_bc_dry_1(b).add3(F(F_al), 'p').add3(F(F_ph_2), 'w');
     }
     if (X->rk == 1) {
-      first_rk_step_part1();
-      first_rk_step_part2(false);
+      first_rk_step_part1(false);
+      first_rk_step_part2(false, true);
     }
     fused_tendency();
     small_step_prep();

@@ -167,11 +167,14 @@ __device__ __forceinline__ unsigned wave_y() { return (unsigned)__builtin_amdgcn
 // then 4 consecutive rows, then k, then groups of 4 rows, in XCD-contiguous
 // order: the j+-1 rows of a stencil were read a few blocks earlier by the
 // same XCD and are still in its L2.
-#define GET_IKJ(r)                                                                           \
+#define GET_IKJ(r) GET_IKJ_B(r, blockIdx.x, gridDim.x)
+// the same over blocks [0, nb) of a launch that holds several ranges: b is the
+// block's number in its range
+#define GET_IKJ_B(r, b, nb)                                                                  \
   const int ib_ = 1 + (((r).i0 - 1) & ~63);                                                  \
   const unsigned gx_ = (unsigned)((r).i1 - ib_ + 64) / 64u;                                  \
   const unsigned gy_ = (unsigned)((r).k1 - (r).k0 + 4) / 4u;                                 \
-  const unsigned t_ = xcd_tile(blockIdx.x, gridDim.x);                                       \
+  const unsigned t_ = xcd_tile(b, nb);                                                       \
   const unsigned u_ = t_ / gx_;                                                              \
   const int i = ib_ + (int)((t_ % gx_) * 64u + threadIdx.x);                                 \
   const int k = (r).k0 + (int)(((u_ / 4u) % gy_) * 4u + wave_y());                           \
