@@ -128,11 +128,13 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
   using G = ColGroups<NW, NPW>;
   constexpr int G1 = G::G1, G3 = G::G3, G4 = G::G4, G5 = G::G5, G6 = G::G6, G9 = G::G9, G10 = G::G10;
   extern __shared__ float sm[];
-  __shared__ float c_mts[64], c_mav[64], c_dmdt[64], c_mtend[64];
+  __shared__ float c_mts[64], c_mav[64], c_dmdt[64], c_mtend[64], c_mu[64];
   // dnw and c1h in LDS for the serial column sum and omega recurrence (their
   // global loads would otherwise sit on the recurrence's critical path)
   __shared__ float c_dnw[kColMaxLev], c_c1h[kColMaxLev];
-  const int lane = (int)threadIdx.x, wv = (int)threadIdx.y;
+  // (the wave's number as a scalar, and with it every level and coefficient:
+  // with 8 waves it cost registers that three blocks per CU need)
+  const int lane = (int)threadIdx.x, wv = G::kWide ? (int)wave_y() : (int)threadIdx.y;
   const unsigned gx = (unsigned)(x->ide + 63) / 64u, t = xcd_tile(blockIdx.x, gridDim.x);
   const int i = (int)(t % gx) * 64 + lane + 1, j = (int)(t / gx) + 1;
   const int ide = x->ide, jde = x->jde, kde = x->kde, kend = kde - 1;
@@ -147,8 +149,8 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
   const bool zone = mass && !interior;
   const float g = x->g, t0 = x->t0, epssm = x->epssm;
   const float ope = 1.f + epssm, ome = 1.f - epssm;
-  const float *c1h = FL(c1h), *c2h = FL(c2h), *c1f = FL(c1f), *c2f = FL(c2f), *dnw = FL(dnw), *fnm = FL(fnm), *fnp = FL(fnp);
-  const float *rdnw = FL(rdnw), *rdn = FL(rdn);
+  const CoefPtr c1h = coef(FL(c1h)), c2h = coef(FL(c2h)), c1f = coef(FL(c1f)), c2f = coef(FL(c2f)), dnw = coef(FL(dnw));
+  const CoefPtr fnm = coef(FL(fnm)), fnp = coef(FL(fnp)), rdnw = coef(FL(rdnw)), rdn = coef(FL(rdn));
   const float *t_1 = FL(t_save), *u = FL(u_2), *v = FL(v_2);
   float *ww = FL(ww);
   const int ic = mass ? i : 1, jc = mass ? j : 1;  // clamped column for address arithmetic
@@ -159,31 +161,137 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
     c_dnw[q] = dnw[q];
     c_c1h[q] = c1h[q];
   }
+  // The loads of each phase's group of levels.  None of them reads what this
+  // launch writes but the thread's own earlier stores, so a group may be
+  // issued any time before its phase: with 8 waves at the phase (the first
+  // groups of phases 3 and 10 ahead of the serial parts), with 16 as early as
+  // the registers allow (kTop: all of a wave's levels at the start).
+  constexpr bool kWide = G::kWide, kTop = kWide && NPW <= 2;
+  float r_ue[G1], r_uw[G1], r_use[G1], r_usw[G1], r_vn[G1], r_vs[G1], r_vsn[G1], r_vss[G1], r_rum[G1], r_rvm[G1];
+  auto load1 = [&](int gq) {
+    const float *us = FL(u_save), *vs = FL(v_save);
+#pragma unroll
+    for (int q = 0; q < G1; q++) {
+      const int k = imin_(LEV(gq + q), kend);
+      r_rum[q] = first ? 0.f : A3(ru_m, i, k, j);
+      r_rvm[q] = first ? 0.f : A3(rv_m, i, k, j);
+      r_ue[q] = A3(u, i + 1, k, j);
+      r_uw[q] = A3(u, i, k, j);
+      r_use[q] = A3(us, i + 1, k, j);
+      r_usw[q] = A3(us, i, k, j);
+      r_vn[q] = A3(v, i, k, j + 1);
+      r_vs[q] = A3(v, i, k, j);
+      r_vsn[q] = A3(vs, i, k, j + 1);
+      r_vss[q] = A3(vs, i, k, j);
+    }
+  };
+  float r3_w1[G3], r3_wm[G3];
+  auto load3 = [&](int gq) {
+    const float *ww_1 = FL(ww_1);
+#pragma unroll
+    for (int q = 0; q < G3; q++) {
+      const int k = imin_(LEV(gq + q), kend);
+      r3_w1[q] = A3(ww_1, i, k, j);
+      r3_wm[q] = first ? 0.f : A3(ww_m, i, k, j);
+    }
+  };
+  float r4_t1[G4], r4_t1m[G4], r4_t1p[G4], r4_t1e[G4], r4_t1w[G4], r4_t1n[G4], r4_t1s[G4], r4_ue[G4], r4_uw[G4], r4_vn[G4], r4_vs[G4], r4_t[G4],
+      r4_ft[G4];
+  auto load4 = [&](int gq) {
+    const float *ft = FL(t_tend), *t = FL(t_2);
+#pragma unroll
+    for (int q = 0; q < G4; q++) {
+      const int k = imin_(LEV(gq + q), kend);
+      r4_t1[q] = A3(t_1, i, k, j);
+      r4_t1m[q] = A3(t_1, i, imax_(k - 1, 1), j);
+      r4_t1p[q] = A3(t_1, i, imin_(k + 1, kend), j);
+      r4_t1e[q] = A3(t_1, i + 1, k, j);
+      r4_t1w[q] = A3(t_1, i - 1, k, j);
+      r4_t1n[q] = A3(t_1, i, k, j + 1);
+      r4_t1s[q] = A3(t_1, i, k, j - 1);
+      r4_ue[q] = A3(u, i + 1, k, j);
+      r4_uw[q] = A3(u, i, k, j);
+      r4_vn[q] = A3(v, i, k, j + 1);
+      r4_vs[q] = A3(v, i, k, j);
+      r4_t[q] = A3(t, i, k, j);
+      r4_ft[q] = A3(ft, i, k, j);
+    }
+  };
+  const float *ph = FL(ph_2);
+  float r5_pt[G5], r5_w[G5], r5_p1[G5], r5_p1m[G5], r5_p1p[G5], r5_pb[G5], r5_pbm[G5], r5_pbp[G5], r5_ph[G5];
+  auto load5 = [&](int gq) {
+    const float *ph_1 = FL(ph_save), *phb = FL(phb), *ph_tend = FL(ph_tend), *w = FL(w_2);
+#pragma unroll
+    for (int q = 0; q < G5; q++) {
+      const int k = imax_(imin_(LEV(gq + q), kde), 2);
+      r5_pt[q] = A3(ph_tend, i, k, j);
+      r5_w[q] = A3(w, i, k, j);
+      r5_p1[q] = A3(ph_1, i, k, j);
+      r5_p1m[q] = A3(ph_1, i, k - 1, j);
+      r5_p1p[q] = A3(ph_1, i, imin_(k + 1, kde), j);
+      r5_pb[q] = A3(phb, i, k, j);
+      r5_pbm[q] = A3(phb, i, k - 1, j);
+      r5_pbp[q] = A3(phb, i, imin_(k + 1, kde), j);
+      r5_ph[q] = A3(ph, i, k, j);
+    }
+  };
+  float r6_c2a[G6], r6_c2am[G6], r6_alt[G6], r6_altm[G6], r6_ph[G6], r6_phm[G6], r6_php[G6], r6_w[G6], r6_rwt[G6], r6_cqw[G6];
+  auto load6 = [&](int gq) {
+    const float *w = FL(w_2), *rw_tend = FL(rw_tend), *c2a = FL(c2a), *cqw = FL(cqw), *alt = FL(alt);
+#pragma unroll
+    for (int q = 0; q < G6; q++) {
+      const int k = imax_(imin_(LEV(gq + q), kde), 2);
+      r6_c2a[q] = A3(c2a, i, imin_(k, kend), j);
+      r6_c2am[q] = A3(c2a, i, k - 1, j);
+      r6_alt[q] = A3(alt, i, imin_(k, kend), j);
+      r6_altm[q] = A3(alt, i, k - 1, j);
+      r6_ph[q] = A3(ph, i, k, j);
+      r6_phm[q] = A3(ph, i, k - 1, j);
+      r6_php[q] = A3(ph, i, imin_(k + 1, kde), j);
+      r6_w[q] = A3(w, i, k, j);
+      r6_rwt[q] = A3(rw_tend, i, k, j);
+      r6_cqw[q] = A3(cqw, i, k, j);
+    }
+  };
+  // the column's 2-D values of phase 2 (wave 0): old mu, its tendency, mut,
+  // muts and mudf
+  float mu0 = 0.f, mu_tnd = 0.f, mut0 = 0.f, muts0 = 0.f, mudf0 = 0.f;
+  auto load2 = [&]() {
+    mu0 = A2(FL(mu_2), i, j);
+    mu_tnd = A2(FL(mu_tend), i, j);
+    mut0 = A2(FL(mut), i, j);
+    muts0 = A2(FL(muts), i, j);
+    mudf0 = A2(FL(mudf), i, j);
+  };
+  if (kWide && mass && wv == 0) load2();
+  if (kWide && interior) {
+    load1(0);
+    load3(0);
+    load4(0);
+    if (kTop) {
+      load5(0);
+      load6(0);
+    }
+  }
+  if (kWide && zone) {
+    const float *ft = FL(t_tend), *t = FL(t_2);
+#pragma unroll
+    for (int q = 0; q < G4; q++) {
+      r4_t[q] = A3(t, i, imin_(LEV(q), kend), j);
+      r4_ft[q] = A3(ft, i, imin_(LEV(q), kend), j);
+    }
+  }
   // ---- 1. advance_mu_t: horizontal mass divergence per level -> B0; with
   // the same loads, sumflux of the column's u and v points (levels 1..kde-1)
   if (interior) {
-    const float *us = FL(u_save), *vs = FL(v_save), *muu = FL(muu), *muv = FL(muv);
+    const float *muu = FL(muu), *muv = FL(muv);
     const float muu0 = A2(muu, i, j), muu1 = A2(muu, i + 1, j), muv0 = A2(muv, i, j), muv1 = A2(muv, i, j + 1);
     const float iuy0 = A2(FL(msfuy), i, j), iuy1 = A2(FL(msfuy), i + 1, j);
     const float vx0 = A2(FL(msfvx_inv), i, j), vx1 = A2(FL(msfvx_inv), i, j + 1);
     const float mm = msftx * msfty;
 #pragma unroll
     for (int gq = 0; gq < NPW; gq += G1) {
-      float r_ue[G1], r_uw[G1], r_use[G1], r_usw[G1], r_vn[G1], r_vs[G1], r_vsn[G1], r_vss[G1], r_rum[G1], r_rvm[G1];
-#pragma unroll
-      for (int q = 0; q < G1; q++) {
-        const int k = imin_(LEV(gq + q), kend);
-        r_rum[q] = first ? 0.f : A3(ru_m, i, k, j);
-        r_rvm[q] = first ? 0.f : A3(rv_m, i, k, j);
-        r_ue[q] = A3(u, i + 1, k, j);
-        r_uw[q] = A3(u, i, k, j);
-        r_use[q] = A3(us, i + 1, k, j);
-        r_usw[q] = A3(us, i, k, j);
-        r_vn[q] = A3(v, i, k, j + 1);
-        r_vs[q] = A3(v, i, k, j);
-        r_vsn[q] = A3(vs, i, k, j + 1);
-        r_vss[q] = A3(vs, i, k, j);
-      }
+      if (gq > 0 || !kWide) load1(gq);
 #pragma unroll
       for (int q = 0; q < G1; q++) {
         const int k = LEV(gq + q);
@@ -204,28 +312,14 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
       }
     }
   }
-  // phase 3's loads, in flight over the barriers and the serial part before it
-  float r3_w1[G3], r3_wm[G3];
-  auto load3 = [&](int gq) {
-    const float *ww_1 = FL(ww_1);
-#pragma unroll
-    for (int q = 0; q < G3; q++) {
-      const int k = imin_(LEV(gq + q), kend);
-      r3_w1[q] = A3(ww_1, i, k, j);
-      r3_wm[q] = first ? 0.f : A3(ww_m, i, k, j);
-    }
-  };
-  if (interior) load3(0);
+  if (interior && !kWide) load3(0);
   __syncthreads();
   // ---- 2. column sum and column-mass update (wave 0), the level terms of the
   // omega recurrence (all waves: the division is off the recurrence's chain),
   // then the recurrence itself
+  if (!kWide && mass && wv == 0) load2();
   if (wv == 0 && interior) {
     // column mass tendency: FP32 level terms summed in FP64, rounded once
-    float *mu = FL(mu_2);
-    const float old = A2(mu, i, j);
-    const float mtend = A2(FL(mu_tend), i, j);
-    const float mut = A2(FL(mut), i, j);
     double dmdt_acc = 0.0;
     for (int k0 = 1; k0 <= kend; k0 += 8) {  // 8 levels' operands ahead of the chain
       float r[8];
@@ -236,23 +330,27 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
         if (k0 + q <= kend) dmdt_acc += (double)r[q];
     }
     const float dmdt = (float)dmdt_acc;
-    const float tend = dmdt + mtend;
-    const float nmu = old + dts * tend;
-    const float mts = mut + nmu;
-    const float mav = 0.5f * ((1.f + epssm) * nmu + (1.f - epssm) * old);
-    A2(mu, i, j) = nmu;
+    const float tend = dmdt + mu_tnd;
+    const float nmu = mu0 + dts * tend;
+    const float mts = mut0 + nmu;
+    const float mav = 0.5f * ((1.f + epssm) * nmu + (1.f - epssm) * mu0);
+    A2(FL(mu_2), i, j) = nmu;
     A2(FL(mudf), i, j) = tend;
     A2(FL(muts), i, j) = mts;
     A2(FL(muave), i, j) = mav;
     c_mts[lane] = mts;
     c_mav[lane] = mav;
     c_dmdt[lane] = dmdt;
-    c_mtend[lane] = mtend;
+    c_mtend[lane] = mu_tnd;
+    c_mu[lane] = nmu;
+    mudf0 = tend;
   }
   if (wv == 0 && zone) {
-    const float mt = A2(FL(mu_tend), i, j);
-    A2(FL(mu_2), i, j) = A2(FL(mu_2), i, j) + dts * mt;
-    const float mts = A2(FL(muts), i, j) + dts * mt;
+    const float nmu = mu0 + dts * mu_tnd;
+    const float mts = muts0 + dts * mu_tnd;
+    c_mtend[lane] = mu_tnd;
+    A2(FL(mu_2), i, j) = nmu;
+    c_mu[lane] = nmu;
     A2(FL(muts), i, j) = mts;
     c_mts[lane] = mts;
   }
@@ -314,48 +412,31 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
   // (phase 10 reads the new theta back: the same thread wrote it)
   if (interior) {
     const float mts = c_mts[lane], mav = c_mav[lane];
-    const float *ft = FL(t_tend);
     float *t = FL(t_2), *tav_out = FL(t_2ave);
+    if (kWide && !kTop) load5(0);
 #pragma unroll
     for (int gq = 0; gq < NPW; gq += G4) {
-      float r_t1[G4], r_t1m[G4], r_t1p[G4], r_t1e[G4], r_t1w[G4], r_t1n[G4], r_t1s[G4], r_ue[G4], r_uw[G4], r_vn[G4], r_vs[G4], r_t[G4], r_ft[G4];
-#pragma unroll
-      for (int q = 0; q < G4; q++) {
-        const int k = imin_(LEV(gq + q), kend);
-        r_t1[q] = A3(t_1, i, k, j);
-        r_t1m[q] = A3(t_1, i, imax_(k - 1, 1), j);
-        r_t1p[q] = A3(t_1, i, imin_(k + 1, kend), j);
-        r_t1e[q] = A3(t_1, i + 1, k, j);
-        r_t1w[q] = A3(t_1, i - 1, k, j);
-        r_t1n[q] = A3(t_1, i, k, j + 1);
-        r_t1s[q] = A3(t_1, i, k, j - 1);
-        r_ue[q] = A3(u, i + 1, k, j);
-        r_uw[q] = A3(u, i, k, j);
-        r_vn[q] = A3(v, i, k, j + 1);
-        r_vs[q] = A3(v, i, k, j);
-        r_t[q] = A3(t, i, k, j);
-        r_ft[q] = A3(ft, i, k, j);
-      }
+      if (gq > 0 || !kWide) load4(gq);
 #pragma unroll
       for (int q = 0; q < G4; q++) {
         const int k = LEV(gq + q);
         if (k > kend) break;
-        const float wlo = (k >= 2) ? LS(B1, k) * (A1(fnm, k) * r_t1[q] + A1(fnp, k) * r_t1m[q]) : 0.f;
-        const float whi = (k + 1 <= kend) ? LS(B1, k + 1) * (A1(fnm, k + 1) * r_t1p[q] + A1(fnp, k + 1) * r_t1[q]) : 0.f;
-        const float tk = r_t[q];
-        const float ta = tk + (msfty * dts) * r_ft[q];
-        const float vnorth = r_vn[q] * (r_t1n[q] + r_t1[q]);
-        const float vsouth = r_vs[q] * (r_t1[q] + r_t1s[q]);
+        const float wlo = (k >= 2) ? LS(B1, k) * (A1(fnm, k) * r4_t1[q] + A1(fnp, k) * r4_t1m[q]) : 0.f;
+        const float whi = (k + 1 <= kend) ? LS(B1, k + 1) * (A1(fnm, k + 1) * r4_t1p[q] + A1(fnp, k + 1) * r4_t1[q]) : 0.f;
+        const float tk = r4_t[q];
+        const float ta = tk + (msfty * dts) * r4_ft[q];
+        const float vnorth = r4_vn[q] * (r4_t1n[q] + r4_t1[q]);
+        const float vsouth = r4_vs[q] * (r4_t1[q] + r4_t1s[q]);
         const float vft = (0.5f * x->rdy) * (vnorth - vsouth);
-        const float ueast = r_ue[q] * (r_t1e[q] + r_t1[q]);
-        const float uwest = r_uw[q] * (r_t1[q] + r_t1w[q]);
+        const float ueast = r4_ue[q] * (r4_t1e[q] + r4_t1[q]);
+        const float uwest = r4_uw[q] * (r4_t1[q] + r4_t1w[q]);
         const float uft = (0.5f * x->rdx) * (ueast - uwest);
         const float horiz = msftx * (vft + uft);
         const float vert = A1(rdnw, k) * (whi - wlo);
         const float tnew = ta - (dts * msfty) * (horiz + vert);
         A3(t, i, k, j) = tnew;
         float tav = 0.5f * (ope * tnew + ome * tk);
-        tav = (tav + (A1(c1h, k) * mav) * t0) / ((A1(c1h, k) * mts + A1(c2h, k)) * (t0 + r_t1[q]));
+        tav = (tav + (A1(c1h, k) * mav) * t0) / ((A1(c1h, k) * mts + A1(c2h, k)) * (t0 + r4_t1[q]));
         if (store_tav) A3(tav_out, i, k, j) = tav;
         LS(B2, k) = tav;
       }
@@ -363,31 +444,22 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
   } else if (zone) {
     float *t = FL(t_2);
     const float *ft = FL(t_tend);
-    for (int k = 1 + wv; k <= kend; k += NW) A3(t, i, k, j) = A3(t, i, k, j) + dts * A3(ft, i, k, j);
+    if (kWide) {
+#pragma unroll
+      for (int q = 0; q < G4; q++)
+        if (LEV(q) <= kend) A3(t, i, LEV(q), j) = r4_t[q] + dts * r4_ft[q];
+    }
+    for (int k = kWide ? LEV(G4) : LEV(0); k <= kend; k += NW) A3(t, i, k, j) = A3(t, i, k, j) + dts * A3(ft, i, k, j);
   }
   // (no barrier: phase 5 reads omega (final since the barrier above), phi and
   // w, and writes B0; phase 4 writes theta, its average and B2 only)
   // ---- 5. advance_w: right-hand side of the phi equation (levels 2..kde) -> B0
-  const float *ph = FL(ph_2);
   const float m = A2(FL(mut), ic, jc);
   if (interior) {
-    const float *ph_1 = FL(ph_save), *phb = FL(phb), *ph_tend = FL(ph_tend), *w = FL(w_2);
+    if (kWide && !kTop) load6(0);
 #pragma unroll
     for (int gq = 0; gq < NPW; gq += G5) {
-      float r_pt[G5], r_w[G5], r_p1[G5], r_p1m[G5], r_p1p[G5], r_pb[G5], r_pbm[G5], r_pbp[G5], r_ph[G5];
-#pragma unroll
-      for (int q = 0; q < G5; q++) {
-        const int k = imax_(imin_(LEV(gq + q), kde), 2);
-        r_pt[q] = A3(ph_tend, i, k, j);
-        r_w[q] = A3(w, i, k, j);
-        r_p1[q] = A3(ph_1, i, k, j);
-        r_p1m[q] = A3(ph_1, i, k - 1, j);
-        r_p1p[q] = A3(ph_1, i, imin_(k + 1, kde), j);
-        r_pb[q] = A3(phb, i, k, j);
-        r_pbm[q] = A3(phb, i, k - 1, j);
-        r_pbp[q] = A3(phb, i, imin_(k + 1, kde), j);
-        r_ph[q] = A3(ph, i, k, j);
-      }
+      if (gq > 0 || !kWide) load5(gq);
 #pragma unroll
       for (int q = 0; q < G5; q++) {
         const int k = LEV(gq + q);
@@ -396,13 +468,13 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
           LS(B0, 1) = 0.f;
           continue;
         }
-        float rk = dts * (r_pt[q] + ((0.5f * g) * ome) * r_w[q]);
+        float rk = dts * (r5_pt[q] + ((0.5f * g) * ome) * r5_w[q]);
         if (k <= kend) {
-          const float wdn_k = ((0.5f * (LS(B1, k) + LS(B1, k - 1))) * A1(rdnw, k - 1)) * (r_p1[q] - r_p1m[q] + r_pb[q] - r_pbm[q]);
-          const float wdn_kp = ((0.5f * (LS(B1, k + 1) + LS(B1, k))) * A1(rdnw, k)) * (r_p1p[q] - r_p1[q] + r_pbp[q] - r_pb[q]);
+          const float wdn_k = ((0.5f * (LS(B1, k) + LS(B1, k - 1))) * A1(rdnw, k - 1)) * (r5_p1[q] - r5_p1m[q] + r5_pb[q] - r5_pbm[q]);
+          const float wdn_kp = ((0.5f * (LS(B1, k + 1) + LS(B1, k))) * A1(rdnw, k)) * (r5_p1p[q] - r5_p1[q] + r5_pbp[q] - r5_pb[q]);
           rk = rk - dts * (A1(fnm, k) * wdn_kp + A1(fnp, k) * wdn_k);
         }
-        rk = r_ph[q] + (msfty * rk) / (A1(c1f, k) * m + A1(c2f, k));
+        rk = r5_ph[q] + (msfty * rk) / (A1(c1f, k) * m + A1(c2f, k));
         LS(B0, k) = rk;
       }
     }
@@ -410,25 +482,10 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
   __syncthreads();
   // ---- 6. explicit w (raw right-hand side of the tridiagonal system) -> B3
   if (interior) {
-    const float *w = FL(w_2), *rw_tend = FL(rw_tend), *c2a = FL(c2a), *cqw = FL(cqw), *alt = FL(alt);
     const float mav = c_mav[lane], msft_inv = 1.f / msfty;
 #pragma unroll
     for (int gq = 0; gq < NPW; gq += G6) {
-      float r_c2a[G6], r_c2am[G6], r_alt[G6], r_altm[G6], r_ph[G6], r_phm[G6], r_php[G6], r_w[G6], r_rwt[G6], r_cqw[G6];
-#pragma unroll
-      for (int q = 0; q < G6; q++) {
-        const int k = imax_(imin_(LEV(gq + q), kde), 2);
-        r_c2a[q] = A3(c2a, i, imin_(k, kend), j);
-        r_c2am[q] = A3(c2a, i, k - 1, j);
-        r_alt[q] = A3(alt, i, imin_(k, kend), j);
-        r_altm[q] = A3(alt, i, k - 1, j);
-        r_ph[q] = A3(ph, i, k, j);
-        r_phm[q] = A3(ph, i, k - 1, j);
-        r_php[q] = A3(ph, i, imin_(k + 1, kde), j);
-        r_w[q] = A3(w, i, k, j);
-        r_rwt[q] = A3(rw_tend, i, k, j);
-        r_cqw[q] = A3(cqw, i, k, j);
-      }
+      if (gq > 0 || !kWide) load6(gq);
 #pragma unroll
       for (int q = 0; q < G6; q++) {
         const int k = LEV(gq + q);
@@ -444,21 +501,21 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
           wl = ((msfty * 0.5f) * x->rdy) * lv + ((msftx * 0.5f) * x->rdx) * lu;
         } else if (k <= kend) {
           const float rkp = LS(B0, k + 1), rk0 = LS(B0, k), rkm = LS(B0, k - 1);
-          const float pu = ((r_c2a[q] * A1(rdnw, k)) / (A1(c1h, k) * m + A1(c2h, k))) * (ope * (rkp - rk0) + ome * (r_php[q] - r_ph[q]));
-          const float pl = ((r_c2am[q] * A1(rdnw, k - 1)) / (A1(c1h, k - 1) * m + A1(c2h, k - 1))) * (ope * (rk0 - rkm) + ome * (r_ph[q] - r_phm[q]));
+          const float pu = ((r6_c2a[q] * A1(rdnw, k)) / (A1(c1h, k) * m + A1(c2h, k))) * (ope * (rkp - rk0) + ome * (r6_php[q] - r6_ph[q]));
+          const float pl = ((r6_c2am[q] * A1(rdnw, k - 1)) / (A1(c1h, k - 1) * m + A1(c2h, k - 1))) * (ope * (rk0 - rkm) + ome * (r6_ph[q] - r6_phm[q]));
           const float ppart = (((0.5f * dts) * g) * A1(rdn, k)) * (pu - pl);
-          const float tu = (r_c2a[q] * r_alt[q]) * LS(B2, k);
-          const float tl = (r_c2am[q] * r_altm[q]) * LS(B2, k - 1);
+          const float tu = (r6_c2a[q] * r6_alt[q]) * LS(B2, k);
+          const float tl = (r6_c2am[q] * r6_altm[q]) * LS(B2, k - 1);
           const float bpart = A1(rdn, k) * (tu - tl) - A1(c1f, k) * mav;
-          wl = ((r_w[q] + dts * r_rwt[q]) + (msft_inv * r_cqw[q]) * ppart) + ((dts * g) * msft_inv) * bpart;
+          wl = ((r6_w[q] + dts * r6_rwt[q]) + (msft_inv * r6_cqw[q]) * ppart) + ((dts * g) * msft_inv) * bpart;
         } else {
           float fac = ((-0.5f * dts) * g) / (A1(c1h, k - 1) * m + A1(c2h, k - 1));
           fac = fac * (A1(rdnw, k - 1) * A1(rdnw, k - 1));
           fac = fac * 2.f;
-          fac = fac * r_c2am[q];
-          const float ptop = fac * (ope * (LS(B0, k) - LS(B0, k - 1)) + ome * (r_ph[q] - r_phm[q]));
-          const float btop = (-dts * g) * (((2.f * A1(rdnw, k - 1)) * r_c2am[q]) * r_altm[q] * LS(B2, k - 1) + A1(c1f, k) * mav);
-          wl = r_w[q] + dts * r_rwt[q] + (1.f / msfty) * (ptop + btop);
+          fac = fac * r6_c2am[q];
+          const float ptop = fac * (ope * (LS(B0, k) - LS(B0, k - 1)) + ome * (r6_ph[q] - r6_phm[q]));
+          const float btop = (-dts * g) * (((2.f * A1(rdnw, k - 1)) * r6_c2am[q]) * r6_altm[q] * LS(B2, k - 1) + A1(c1f, k) * mav);
+          wl = r6_w[q] + dts * r6_rwt[q] + (1.f / msfty) * (ptop + btop);
           if (x->top_lid) wl = 0.f;
         }
         LS(B3, k) = wl;
@@ -487,6 +544,39 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
     }
   };
   if (mass) load10(0);
+  // the zone's phi update and the edge columns' mass-flux sums (phase 9)
+  const bool edge = !interior && i <= ide && j <= jde;
+  const bool upt = (j <= jde - 1), vpt = (i <= ide - 1);
+  float z_ph[G9], z_pt[G9], z_ps[G9], z_rum[G9], z_rvm[G9], z_wwm[G9], z_u[G9], z_v[G9], z_ww[G9], z_us[G9], z_vs[G9], z_ww1[G9];
+  auto loadz = [&](int gq) {
+    const float *ph_tend = FL(ph_tend), *ph_save = FL(ph_save);
+#pragma unroll
+    for (int q = 0; q < G9; q++) {
+      const unsigned o = XI3(i, imin_(LEV(gq + q), kde), j);
+      z_ph[q] = mass ? elem(ph, o) : 0.f;
+      z_pt[q] = mass ? elem(ph_tend, o) : 0.f;
+      z_ps[q] = mass ? elem(ph_save, o) : 0.f;
+    }
+  };
+  auto loads = [&](int gq) {
+#pragma unroll
+    for (int q = 0; q < G9; q++) {
+      const unsigned o = XI3(i, imin_(LEV(gq + q), kde), j);
+      z_rum[q] = first ? 0.f : elem(ru_m, o);
+      z_rvm[q] = first ? 0.f : elem(rv_m, o);
+      z_wwm[q] = first ? 0.f : elem(ww_m, o);
+      z_u[q] = upt ? elem(u, o) : 0.f;
+      z_v[q] = vpt ? elem(v, o) : 0.f;
+      z_ww[q] = mass ? elem(ww, o) : 0.f;
+      z_us[q] = (fin && upt) ? elem(FL(u_save), o) : 0.f;
+      z_vs[q] = (fin && vpt) ? elem(FL(v_save), o) : 0.f;
+      z_ww1[q] = (fin && mass) ? elem(FL(ww_1), o) : 0.f;
+    }
+  };
+  if (kWide && edge) {
+    loadz(0);
+    loads(0);
+  }
   const int sk = x->ip;  // element stride between levels
   const unsigned o1 = XI3(ic, 1, jc);
   float wprev = 0.f;
@@ -576,26 +666,17 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
     }
   } else if (zone) {
     const float mts = c_mts[lane];
-    const float mtend = A2(FL(mu_tend), i, j);
-    const float mu_old = mts - dts * mtend;
-    const float *ph_tend = FL(ph_tend), *ph_save = FL(ph_save);
+    const float mu_old = mts - dts * c_mtend[lane];
 #pragma unroll
     for (int gq = 0; gq < NPW; gq += G9) {
-      float r_ph[G9], r_pt[G9], r_ps[G9];
-#pragma unroll
-      for (int q = 0; q < G9; q++) {
-        const int k = imin_(LEV(gq + q), kde);
-        r_ph[q] = A3(php2, i, k, j);
-        r_pt[q] = A3(ph_tend, i, k, j);
-        r_ps[q] = A3(ph_save, i, k, j);
-      }
+      if (gq > 0 || !kWide) loadz(gq);
 #pragma unroll
       for (int q = 0; q < G9; q++) {
         const int k = LEV(gq + q);
         if (k > kde) break;
         const float den = A1(c1f, k) * mts + A1(c2f, k);
         const float ratio = (A1(c1f, k) * mu_old + A1(c2f, k)) / den;
-        const float phn = r_ph[q] * ratio + dts * r_pt[q] / den + r_ps[q] * (ratio - 1.f);
+        const float phn = z_ph[q] * ratio + dts * z_pt[q] / den + z_ps[q] * (ratio - 1.f);
         A3(php2, i, k, j) = phn;
         LS(B2, k) = phn;
       }
@@ -609,49 +690,34 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
       A3(ru_m, i, kde, j) = 0.f;
       A3(rv_m, i, kde, j) = 0.f;
     }
-  } else if (i <= ide && j <= jde) {
-    const bool upt = (j <= jde - 1), vpt = (i <= ide - 1);
+  } else if (edge) {
     const float cmu_u = upt ? A2(FL(muu), i, j) : 0.f, cmsf_u = upt ? A2(FL(msfuy), i, j) : 1.f;
     const float cmu_v = vpt ? A2(FL(muv), i, j) : 0.f, cmsf_v = vpt ? A2(FL(msfvx_inv), i, j) : 1.f;
 #pragma unroll
     for (int gq = 0; gq < NPW; gq += G9) {
-      float r_rum[G9], r_rvm[G9], r_wwm[G9], r_u[G9], r_v[G9], r_ww[G9], r_us[G9], r_vs[G9], r_ww1[G9];
-#pragma unroll
-      for (int q = 0; q < G9; q++) {
-        const int k = imin_(LEV(gq + q), kde);
-        const size_t o = XI3(i, k, j);
-        r_rum[q] = first ? 0.f : ru_m[o];
-        r_rvm[q] = first ? 0.f : rv_m[o];
-        r_wwm[q] = first ? 0.f : ww_m[o];
-        r_u[q] = upt ? u[o] : 0.f;
-        r_v[q] = vpt ? v[o] : 0.f;
-        r_ww[q] = mass ? ww[o] : 0.f;
-        r_us[q] = (fin && upt) ? FL(u_save)[o] : 0.f;
-        r_vs[q] = (fin && vpt) ? FL(v_save)[o] : 0.f;
-        r_ww1[q] = (fin && mass) ? FL(ww_1)[o] : 0.f;
-      }
+      if (gq > 0 || !kWide) loads(gq);
 #pragma unroll
       for (int q = 0; q < G9; q++) {
         const int k = LEV(gq + q);
         if (k > kde) break;
         const size_t o = XI3(i, k, j);
         if (upt && k <= kend) {
-          float acc = r_rum[q] + r_u[q];
-          if (fin) acc = acc / ns + ((A1(c1h, k) * cmu_u + A1(c2h, k)) * r_us[q]) / cmsf_u;
+          float acc = z_rum[q] + z_u[q];
+          if (fin) acc = acc / ns + ((A1(c1h, k) * cmu_u + A1(c2h, k)) * z_us[q]) / cmsf_u;
           ru_m[o] = acc;
         } else if (first) {
           ru_m[o] = 0.f;
         }
         if (vpt && k <= kend) {
-          float acc = r_rvm[q] + r_v[q];
-          if (fin) acc = acc / ns + ((A1(c1h, k) * cmu_v + A1(c2h, k)) * r_vs[q]) * cmsf_v;
+          float acc = z_rvm[q] + z_v[q];
+          if (fin) acc = acc / ns + ((A1(c1h, k) * cmu_v + A1(c2h, k)) * z_vs[q]) * cmsf_v;
           rv_m[o] = acc;
         } else if (first) {
           rv_m[o] = 0.f;
         }
         if (mass) {
-          float acc = r_wwm[q] + r_ww[q];
-          if (fin) acc = acc / ns + r_ww1[q];
+          float acc = z_wwm[q] + z_ww[q];
+          if (fin) acc = acc / ns + z_ww1[q];
           ww_m[o] = acc;
         } else if (first) {
           ww_m[o] = 0.f;
@@ -662,7 +728,7 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
   __syncthreads();
   // ---- 10. calc_p_rho (iteration >= 1) and the physical-boundary copies
   if (mass) {
-    const float mts = c_mts[lane], mu2 = A2(FL(mu_2), i, j);
+    const float mts = c_mts[lane], mu2 = c_mu[lane];
     const bool gx = (i == ide - 1), gy = (j == jde - 1);
     float *al = FL(al), *p = FL(p), *pm1 = FL(pm1);
 #pragma unroll
@@ -706,7 +772,7 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
         if (gx && gy) A3(php2, ide, k, jde) = vv;
       }
       if (wv == 0) {
-        const float a2 = A2(FL(muts), i, j), b2 = A2(FL(mu_2), i, j), c2 = A2(FL(mudf), i, j);
+        const float a2 = mts, b2 = mu2, c2 = mudf0;
         const int is[3] = {ide, i, ide}, js[3] = {j, jde, jde};
         const bool on[3] = {gx, gy, gx && gy};
         for (int q = 0; q < 3; q++)
@@ -724,8 +790,8 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
 
 // A domain of at most kColWideBlocks blocks leaves CUs idle, so its substep
 // takes as long as one block does: 16 waves, each with half the levels
-// (a substep's column kernel at 100x100x45, 202 blocks: 44 us with 8 waves, 33
-// with 16; at 24x20x10 14 and 12).  From there on 8 waves: three such blocks
+// (a substep's column kernel at 100x100x45, 202 blocks: 44 us with 8 waves, 30
+// with 16; at 24x20x10 14 and 11).  From there on 8 waves: three such blocks
 // share a CU, one of 16.
 constexpr unsigned kColWideBlocks = 256;
 inline unsigned acoustic_col_blocks(const DevCtx &d) { return (unsigned)((d.ide + 63) / 64) * (unsigned)d.jde; }

@@ -133,6 +133,12 @@ __device__ __forceinline__ void pin1(float v) { asm volatile("" : : "v"(v)); }
 #define SP(name, s) (gmem(x->F[F_##name]) + (size_t)(s) * x->n3)
 #define SCR(id) gmem(x->S[id])
 
+// A column array ([k] coefficients, which no kernel writes) through the
+// constant address space: its loads may pass the stores around them, and are
+// scalar where the level is.
+typedef const __attribute__((address_space(4))) float *CoefPtr;
+__device__ __forceinline__ CoefPtr coef(const float *p) { return (CoefPtr)p; }
+
 // Inclusive Fortran index ranges of a launch.
 struct R3 {
   int i0, i1, k0, k1, j0, j1;
