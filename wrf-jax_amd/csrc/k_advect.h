@@ -71,9 +71,11 @@ __host__ __device__ inline FaceTiles face_tiles(const R3 &r, unsigned lg = kFace
 // whole; waves past the last row (jrow false) still take part in the block's
 // barrier and form their south face.  The launch's grid is
 // face_tiles(r, LG).count() blocks with the kernel's LG.
-#define GET_FACE_BLOCK_LG(r, LG)                                                         \
+// (b of nb: the block's number where a launch holds several ranges)
+#define GET_FACE_BLOCK_LG(r, LG) GET_FACE_BLOCK_B(r, LG, blockIdx.x, gridDim.x)
+#define GET_FACE_BLOCK_B(r, LG, b, nb)                                                   \
   const FaceTiles T_ = face_tiles(r, LG);                                                \
-  const unsigned t_ = xcd_tile(blockIdx.x, gridDim.x);                                   \
+  const unsigned t_ = xcd_tile(b, nb);                                   \
   const int lane = (int)threadIdx.x, wv = (int)wave_y();                                 \
   const unsigned u_ = t_ / T_.ni;                                                        \
   const int i = (r).i0 + (int)(t_ % T_.ni) * 63 + lane;                                  \
@@ -224,11 +226,9 @@ struct TransportUpd {
   float dt;
 };
 template <int MODE>
-__global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx *xv, const float *q, float *tend, const float *ru, const float *rv,
-                                                       const float *rom, R3 r, int rk, TransportUpd tu) {
-  const CtxPtr x = ctx_ptr(xv);
-  __shared__ float ys[kFaceRows][64];
-  GET_FACE_BLOCK(r);
+__device__ __forceinline__ void advect_scalar(CtxPtr x, float (*ys)[64], unsigned b, unsigned nblk, const float *q, float *tend, const float *ru,
+                                         const float *rv, const float *rom, const R3 &r, int rk, TransportUpd tu) {
+  GET_FACE_BLOCK_B(r, (unsigned)x->face_lg[0], b, nblk);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned nb = (unsigned)x->n3, sj = (unsigned)(kde * x->ip), sk = (unsigned)x->ip;
   const BufF bq = bufv(q, nb), bv = bufv(rv, nb);
@@ -277,7 +277,10 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx *
   if (j >= 2 && j <= jde - 2) t -= msf * x->rdy * (fn - fs);
   if (ic >= 2 && ic <= ide - 2) t -= msf * x->rdx * (fe - fw);
   t -= rdz * (zflux_br(wz[1], wz[2], wz[3], wz[4], wt, k + 1, kde, fm1, fp1) - zflux_br(wz[0], wz[1], wz[2], wz[3], wb, k, kde, fm0, fp0));
-  if (MODE == kAdvTend) t = addtend_t(x, ic, k, j, rk, t, rk > 1);
+  if (MODE == kAdvTend) {
+    t = addtend_t(x, ic, k, j, rk, t, rk > 1, true);
+    if (on_ring(i, j, ide - 1, jde - 1)) t = RING_TEND(t, i, k, j, jde - 1);
+  }
   if (MODE == kAdvTransport) {
     const int sz = x->spec_zone;
     const bool inner = i >= 1 + sz && i <= ide - sz - 1 && j >= 1 + sz && j <= jde - sz - 1;
@@ -287,6 +290,13 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx *
   }
   elem(tend, o) = t;
 }
+template <int MODE>
+__global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx *xv, const float *q, float *tend, const float *ru, const float *rv,
+                                                       const float *rom, R3 r, int rk, TransportUpd tu) {
+  __shared__ float ys[kFaceRows][64];
+  advect_scalar<MODE>(ctx_ptr(xv), ys, blockIdx.x, gridDim.x, q, tend, ru, rv, rom, r, rk, tu);
+}
+
 
 // ---------------- u momentum (u points i in [2, ide-1]) ---------------------
 // advect_u (module_advect_em.py:762-1034); r covers i [2, ide-1], j [1, jde-1]
@@ -298,11 +308,9 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_scalar(const DevCtx *
 // a column clamped into [2, ide-1], so their loads stay in the field) and
 // used where they apply.
 template <bool TEND>
-__global__ void __launch_bounds__(64 * kFaceRows) k_advect_u(const DevCtx *xv, const float *u, float *tend, const float *ru, const float *rv,
-                                                  const float *rom, R3 r, int rk) {
-  const CtxPtr x = ctx_ptr(xv);
-  __shared__ float ys[kFaceRows][64];
-  GET_FACE_BLOCK(r);
+__device__ __forceinline__ void advect_u(CtxPtr x, float (*ys)[64], unsigned b, unsigned nblk, const float *u, float *tend, const float *ru,
+                                         const float *rv, const float *rom, const R3 &r, int rk) {
+  GET_FACE_BLOCK_B(r, (unsigned)x->face_lg[0], b, nblk);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned nb = (unsigned)x->n3, sj = (unsigned)(kde * x->ip), sk = (unsigned)x->ip;
   const BufF bq = bufv(u, nb), bv = bufv(rv, nb);
@@ -362,9 +370,19 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_u(const DevCtx *xv, c
       t = cor_u_add(t, cc);
     }
   }
-  if (TEND) t = t + tendf_fold(FL(ru_tendf), o, tfl, mt, rk) / mt;
+  if (TEND) {
+    t = t + tendf_fold(FL(ru_tendf), o, tfl, mt, rk) / mt;
+    if (on_ring(i, j, ide, jde - 1)) t = RING_TEND(u, i, k, j, jde - 1);
+  }
   elem(tend, o) = t;
 }
+template <bool TEND>
+__global__ void __launch_bounds__(64 * kFaceRows) k_advect_u(const DevCtx *xv, const float *u, float *tend, const float *ru, const float *rv,
+                                                       const float *rom, R3 r, int rk) {
+  __shared__ float ys[kFaceRows][64];
+  advect_u<TEND>(ctx_ptr(xv), ys, blockIdx.x, gridDim.x, u, tend, ru, rv, rom, r, rk);
+}
+
 
 // ---------------- v momentum (v rows j in [2, jde-1]) -----------------------
 // advect_v (module_advect_em.py:1037-1354); r covers i [1, ide-1], j [2, jde-1]
@@ -373,11 +391,9 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_u(const DevCtx *xv, c
 // gradient, Coriolis/curvature at j [2, jde-1], then rk_addtend_dry); the
 // pressure-gradient and Coriolis terms at a row clamped into [2, jde-1].
 template <bool TEND>
-__global__ void __launch_bounds__(64 * kFaceRows) k_advect_v(const DevCtx *xv, const float *v, float *tend, const float *ru, const float *rv,
-                                                  const float *rom, R3 r, int rk) {
-  const CtxPtr x = ctx_ptr(xv);
-  __shared__ float ys[kFaceRows][64];
-  GET_FACE_BLOCK(r);
+__device__ __forceinline__ void advect_v(CtxPtr x, float (*ys)[64], unsigned b, unsigned nblk, const float *v, float *tend, const float *ru,
+                                         const float *rv, const float *rom, const R3 &r, int rk) {
+  GET_FACE_BLOCK_B(r, (unsigned)x->face_lg[0], b, nblk);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned nb = (unsigned)x->n3, sj = (unsigned)(kde * x->ip), sk = (unsigned)x->ip;
   const BufF bq = bufv(v, nb), bv = bufv(rv, nb);
@@ -438,9 +454,19 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_v(const DevCtx *xv, c
       t = cor_v_add(t, cc);
     }
   }
-  if (TEND) t = t + tendf_fold(FL(rv_tendf), o, tfl, mvx, rk) * mvxi;
+  if (TEND) {
+    t = t + tendf_fold(FL(rv_tendf), o, tfl, mvx, rk) * mvxi;
+    if (on_ring(i, j, ide - 1, jde)) t = RING_TEND(v, i, k, j, jde);
+  }
   elem(tend, o) = t;
 }
+template <bool TEND>
+__global__ void __launch_bounds__(64 * kFaceRows) k_advect_v(const DevCtx *xv, const float *v, float *tend, const float *ru, const float *rv,
+                                                       const float *rom, R3 r, int rk) {
+  __shared__ float ys[kFaceRows][64];
+  advect_v<TEND>(ctx_ptr(xv), ys, blockIdx.x, gridDim.x, v, tend, ru, rv, rom, r, rk);
+}
+
 
 // ---------------- w momentum (levels k in [2, kde]) -------------------------
 // advect_w (module_advect_em.py:1357-1640); r covers i [1, ide-1], k [2, kde], j [1, jde-1]
@@ -450,11 +476,9 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_v(const DevCtx *xv, c
 // the top, Coriolis/curvature at k [2, kde]; then rk_addtend_dry.  Buoyancy
 // and Coriolis terms at a level clamped into the range they apply to.
 template <bool TEND>
-__global__ void __launch_bounds__(64 * kFaceRows) k_advect_w(const DevCtx *xv, const float *w, float *tend, const float *ru, const float *rv,
-                                                  const float *rom, R3 r, int rk) {
-  const CtxPtr x = ctx_ptr(xv);
-  __shared__ float ys[kFaceRows][64];
-  GET_FACE_BLOCK_LG(r, (unsigned)x->face_lg[1]);
+__device__ __forceinline__ void advect_w(CtxPtr x, float (*ys)[64], unsigned b, unsigned nblk, const float *w, float *tend, const float *ru,
+                                         const float *rv, const float *rom, const R3 &r, int rk) {
+  GET_FACE_BLOCK_B(r, (unsigned)x->face_lg[1], b, nblk);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned nb = (unsigned)x->n3, sj = (unsigned)(kde * x->ip), sk = (unsigned)x->ip;
   const BufF bq = bufv(w, nb), bv = bufv(rv, nb);
@@ -521,13 +545,19 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_w(const DevCtx *xv, c
   // replaced after this kernel)
   if (TEND && k >= 2 && k <= kde - 2) elem(FL(cqw), o) = cq1;
 }
+template <bool TEND>
+__global__ void __launch_bounds__(64 * kFaceRows) k_advect_w(const DevCtx *xv, const float *w, float *tend, const float *ru, const float *rv,
+                                                       const float *rom, R3 r, int rk) {
+  __shared__ float ys[kFaceRows][64];
+  advect_w<TEND>(ctx_ptr(xv), ys, blockIdx.x, gridDim.x, w, tend, ru, rv, rom, r, rk);
+}
+
 
 // the phi tendency of the RK step over k [1, kde]: rhs_ph at k [2, kde] from
 // zero (the cleared array), then rk_addtend_dry; r = i [1, ide-1], k [1, kde],
 // j [1, jde-1]
-__global__ void __launch_bounds__(256) k_tend_ph(const DevCtx *xv, R3 r, int rk) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+__device__ __forceinline__ void tend_ph(CtxPtr x, unsigned b, unsigned nblk, const R3 &r, int rk) {
+  GET_IKJ_B(r, b, nblk);
   const unsigned o = XI3(i, k, j);
   // rk_addtend_dry's loads go out first (addtend_ph in two parts)
   const float2 tfl = tendf_load(FL(ph_tendf), FL(ph_save), o, rk);
@@ -535,7 +565,40 @@ __global__ void __launch_bounds__(256) k_tend_ph(const DevCtx *xv, R3 r, int rk)
   float t = 0.f;
   if (k >= 2) t = rhs_ph_val(x, i, k, j, t);
   t = t + tendf_fold(FL(ph_tendf), o, tfl, 1.f, rk) / m;
+  if (on_ring(i, j, x->ide - 1, x->jde - 1)) t = RING_TEND(ph, i, k, j, x->jde - 1);
   elem(FL(ph_tend), o) = t;
+}
+
+// The RK tendencies of the fused step: the five components, which read the
+// same winds and each write their own arrays, over five ranges of blocks
+// (first: first block of each range), or one of them (only >= 0) in a launch
+// of its own with its own registers.
+struct TendRanges {
+  R3 r[5];  // u, v, w, theta, phi
+  unsigned first[6];
+};
+template <int C>
+__device__ __forceinline__ void tendency(CtxPtr x, float (*ys)[64], const TendRanges &T, int rk) {
+  const unsigned b = blockIdx.x - T.first[C], nb = T.first[C + 1] - T.first[C];
+  if (C == 0) advect_u<true>(x, ys, b, nb, FL(u_2), FL(ru_tend), FL(ru), FL(rv), FL(ww), T.r[0], rk);
+  if (C == 1) advect_v<true>(x, ys, b, nb, FL(v_2), FL(rv_tend), FL(ru), FL(rv), FL(ww), T.r[1], rk);
+  if (C == 2) advect_w<true>(x, ys, b, nb, FL(w_2), FL(rw_tend), FL(ru), FL(rv), FL(ww), T.r[2], rk);
+  if (C == 3) advect_scalar<kAdvTend>(x, ys, b, nb, FL(t_2), FL(t_tend), FL(ru), FL(rv), FL(ww), T.r[3], rk, TransportUpd{});
+  if (C == 4) tend_ph(x, b, nb, T.r[4], rk);
+}
+__global__ void __launch_bounds__(64 * kFaceRows) k_tendencies(const DevCtx *xv, TendRanges T, int rk) {
+  const CtxPtr x = ctx_ptr(xv);
+  __shared__ float ys[kFaceRows][64];
+  if (blockIdx.x < T.first[1]) tendency<0>(x, ys, T, rk);
+  else if (blockIdx.x < T.first[2]) tendency<1>(x, ys, T, rk);
+  else if (blockIdx.x < T.first[3]) tendency<2>(x, ys, T, rk);
+  else if (blockIdx.x < T.first[4]) tendency<3>(x, ys, T, rk);
+  else tendency<4>(x, ys, T, rk);
+}
+template <int C>
+__global__ void __launch_bounds__(64 * kFaceRows) k_tendency(const DevCtx *xv, TendRanges T, int rk) {
+  __shared__ float ys[kFaceRows][64];
+  tendency<C>(ctx_ptr(xv), ys, T, rk);
 }
 // ---------------- positive-definite scalar advection ------------------------
 // pass 1: high-order minus upwind (antidiffusive) and upwind fluxes

@@ -490,6 +490,17 @@ __global__ void k_cor_curv(const DevCtx *xv, int comp, R3 r) {
   else A3(FL(rw_tend), i, k, j) = cor_curv_w(x, i, k, j, A3(FL(rw_tend), i, k, j));
 }
 
+// spec_bdytend: on the ring of its grid (columns 1 and ibe, rows 1 and jbe) a
+// variable's RK tendency is its boundary tendency (boundary row 1 of the
+// arrays ys, ye, xs, xe; rows before columns at the corners)
+__device__ __forceinline__ bool on_ring(int i, int j, int ibe, int jbe) { return i == 1 || j == 1 || i == ibe || j == jbe; }
+__device__ __forceinline__ float ring_tend(CtxPtr x, const float *ys, const float *ye, const float *xs, const float *xe, int i, int k, int j, int jbe) {
+  if (j == 1) return BY(ys, i, k, 1);
+  if (j == jbe) return BY(ye, i, k, 1);
+  return i == 1 ? BX(xs, j, k, 1) : BX(xe, j, k, 1);
+}
+#define RING_TEND(v, i, k, j, jbe) ring_tend(x, FL(v##_btys), FL(v##_btye), FL(v##_btxs), FL(v##_btxe), i, k, j, jbe)
+
 // rk_addtend_dry (module_em.py:959-1148), one component at one point: the
 // physics / boundary tendency (scaled by the map factor) added to the RK
 // tendency t, which is returned; at the first stage the saved tendency is
@@ -532,14 +543,23 @@ __device__ __forceinline__ float addtend_ph(CtxPtr x, int i, int k, int j, int r
 }
 // theta: also the diabatic heating, and the column's mu tendency at k = 1
 // mu_zero: mu_tend is known to be 0 here (a later stage of the fused step,
-// which does not clear it) and is formed as 0 + mu_tendf
-__device__ __forceinline__ float addtend_t(CtxPtr x, int i, int k, int j, int rk, float t, bool mu_zero = false) {
+// which does not clear it) and is formed as 0 + mu_tendf; spec: the column's
+// spec_bdytend too
+__device__ __forceinline__ float addtend_t(CtxPtr x, int i, int k, int j, int rk, float t, bool mu_zero = false, bool spec = false) {
   const unsigned o = XI3(i, k, j);
   const float m = A2(FL(msfty), i, j);
   const float mass = A1(FL(c1h), k) * A2(FL(mut), i, j) + A1(FL(c2h), k);
   const float tf = tendf_fold(FL(t_tendf), o, tendf_load(FL(t_tendf), FL(t_save), o, rk), 1.f, rk);
   const float heating = mass * elem(FL(h_diabatic), o) / m;
-  if (k == 1) A2(FL(mu_tend), i, j) = (mu_zero ? 0.f : A2(FL(mu_tend), i, j)) + A2(FL(mu_tendf), i, j);
+  if (k == 1) {
+    float mt = (mu_zero ? 0.f : A2(FL(mu_tend), i, j)) + A2(FL(mu_tendf), i, j);
+    if (spec && on_ring(i, j, x->ide - 1, x->jde - 1)) {
+      if (j == 1) mt = BY2(FL(mu_btys), i, 1);
+      else if (j == x->jde - 1) mt = BY2(FL(mu_btye), i, 1);
+      else mt = i == 1 ? BX2(FL(mu_btxs), j, 1) : BX2(FL(mu_btxe), j, 1);
+    }
+    A2(FL(mu_tend), i, j) = mt;
+  }
   return t + tf / m + heating;
 }
 // comp 0 u, 1 v, 2 w/ph, 3 theta

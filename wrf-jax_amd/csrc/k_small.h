@@ -7,48 +7,46 @@
 #include "wrfdc_common.h"
 
 // small_step_prep, 2-D part (module_small_step_em.py:272-420): stage-start
-// column masses.  i [1, ide], j [1, jde].
-__global__ void k_ssp_mass(const DevCtx *xv, int rk) {
-  const CtxPtr x = ctx_ptr(xv);
-  const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int j = 1 + (int)blockIdx.y;
+// column masses of the column (i, j), i [1, ide], j [1, jde].  Every value is
+// formed from mub, mu_1 and mu_2 of the launch's start and written by the
+// column's own thread; mu_1 changes at the first stage only, where nothing
+// else of the launch reads it.
+__device__ __forceinline__ float ssp_muus(CtxPtr x, int i, int j) {
+  const float *mub = FL(mub), *mu_1 = FL(mu_1);
+  const int iw = (i == 1) ? 1 : i - 1;
+  float s = A2(mub, i, j) + A2(mu_1, i, j);
+  s = s + A2(mub, iw, j);
+  s = s + A2(mu_1, iw, j);
+  return 0.5f * s;
+}
+__device__ __forceinline__ float ssp_muvs(CtxPtr x, int i, int j) {
+  const float *mub = FL(mub), *mu_1 = FL(mu_1);
+  const int js = (j == 1) ? 1 : j - 1;
+  float s = A2(mub, i, j) + A2(mu_1, i, j);
+  s = s + A2(mub, i, js);
+  s = s + A2(mu_1, i, js);
+  return 0.5f * s;
+}
+template <bool RK1>
+__device__ __forceinline__ void ssp_mass(CtxPtr x, int i, int j) {
   const int ide = x->ide, jde = x->jde;
-  if (i > ide || j > jde) return;
   const float *mub = FL(mub), *mu_1 = FL(mu_1);
   float *mu_2 = FL(mu_2);
-  const bool mass = (i <= ide - 1 && j <= jde - 1);
-  if (rk == 1) {
-    if (j <= jde - 1) A2(FL(muus), i, j) = A2(FL(muu), i, j);
-    if (i <= ide - 1) A2(FL(muvs), i, j) = A2(FL(muv), i, j);
-    if (mass) {
-      const float m2 = A2(mu_2, i, j);
-      A2(FL(mu_1), i, j) = m2;
-      A2(FL(mudf), i, j) = 0.f;
-      A2(FL(muts), i, j) = A2(mub, i, j) + m2;
-      A2(FL(mu_save), i, j) = m2;
-      A2(mu_2, i, j) = 0.f;
-    }
+  if (j <= jde - 1) A2(FL(muus), i, j) = RK1 ? A2(FL(muu), i, j) : ssp_muus(x, i, j);
+  if (i <= ide - 1) A2(FL(muvs), i, j) = RK1 ? A2(FL(muv), i, j) : ssp_muvs(x, i, j);
+  if (i > ide - 1 || j > jde - 1) return;
+  const float m2 = A2(mu_2, i, j), mb = A2(mub, i, j);
+  if (RK1) {
+    A2(FL(mu_1), i, j) = m2;
+    A2(FL(mudf), i, j) = 0.f;
+    A2(FL(muts), i, j) = mb + m2;
+    A2(FL(mu_save), i, j) = m2;
+    A2(mu_2, i, j) = 0.f;
   } else {
-    if (j <= jde - 1) {
-      const int iw = (i == 1) ? 1 : i - 1;
-      float s = A2(mub, i, j) + A2(mu_1, i, j);
-      s = s + A2(mub, iw, j);
-      s = s + A2(mu_1, iw, j);
-      A2(FL(muus), i, j) = 0.5f * s;
-    }
-    if (i <= ide - 1) {
-      const int js = (j == 1) ? 1 : j - 1;
-      float s = A2(mub, i, j) + A2(mu_1, i, j);
-      s = s + A2(mub, i, js);
-      s = s + A2(mu_1, i, js);
-      A2(FL(muvs), i, j) = 0.5f * s;
-    }
-    if (mass) {
-      A2(FL(muts), i, j) = A2(mub, i, j) + A2(mu_1, i, j);
-      const float m2 = A2(mu_2, i, j);
-      A2(FL(mu_save), i, j) = m2;
-      A2(mu_2, i, j) = A2(mu_1, i, j) - m2;
-    }
+    const float m1 = A2(mu_1, i, j);
+    A2(FL(muts), i, j) = mb + m1;
+    A2(FL(mu_save), i, j) = m2;
+    A2(mu_2, i, j) = m1 - m2;
   }
 }
 
@@ -57,9 +55,12 @@ __global__ void k_ssp_mass(const DevCtx *xv, int rk) {
 // Full extent i [1, ide], k [1, kde], j [1, jde].
 // Every field of the point is loaded first (all addresses are points of the
 // full-extent fields), then the stores of the staggerings the point belongs
-// to; RK1: the first RK stage (stage-start copies, perturbations zero).
+// to; RK1: the first RK stage (stage-start copies, perturbations zero).  The
+// threads of level 1 also do the 2-D part, whose column masses the others
+// form for themselves: a launch less.  cqw_top: level kde-1 of cqw :=
+// 1/(1+cqw), left over by the fused step's w tendency.
 template <bool RK1>
-__global__ void k_ssp_3d(const DevCtx *xv, R3 r) {
+__global__ void k_ssp_3d(const DevCtx *xv, R3 r, int cqw_top) {
   const CtxPtr x = ctx_ptr(xv);
   GET_IKJ_P(r);
   const int ide = x->ide, jde = x->jde, kde = x->kde;
@@ -79,19 +80,21 @@ __global__ void k_ssp_3d(const DevCtx *xv, R3 r) {
     t1 = elem(FL(t_1), o);
     w1 = elem(FL(w_1), o);
     ph1 = elem(FL(ph_1), o);
-    muus = elem(FL(muus), o2);
+    muus = up ? ssp_muus(x, i, j) : 0.f;
     muu = elem(FL(muu), o2);
     msfuy = elem(FL(msfuy), o2);
-    muvs = elem(FL(muvs), o2);
+    muvs = vp ? ssp_muvs(x, i, j) : 0.f;
     muv = elem(FL(muv), o2);
     msfvxi = elem(FL(msfvx_inv), o2);
-    mts = elem(FL(muts), o2);
+    mts = elem(FL(mub), o2) + elem(FL(mu_1), o2);
     mt = elem(FL(mut), o2);
     msfty = elem(FL(msfty), o2);
   }
   pin1(pb);
   pin1(pp);
   pin1(alt);
+  if (k == 1) ssp_mass<RK1>(x, i, j);
+  if (tp && cqw_top && k == kde - 1) elem(FL(cqw), o) = 1.f / (1.f + elem(FL(cqw), o));
   if (tp) elem(FL(c2a), o) = (x->cpovcv * (pb + pp)) / alt;
   if (up) {  // u points
     if (RK1) elem(FL(u_1), o) = u2;

@@ -289,6 +289,14 @@ inline void hchk(hipError_t e, const char *what) {
 
 inline unsigned cdiv(int a, int b) { return (unsigned)((a + b - 1) / b); }
 
+// Elements of a 3-D field up to which the five RK tendencies share a launch.
+// Together they take the registers of the largest (102: 4 waves per SIMD
+// where theta and phi run with 7 and 8), which a domain that fills the chip
+// pays for: a step of 24x20x10 457 us apart and 404 together, 100x100x45
+// (0.5 M elements) 1052 and 1031, 257x131x37 (1.4 M) 1868 and 1889,
+// 400x400x60 14.52 and 14.96 ms.
+constexpr size_t kTendTogether = (size_t)1 << 20;
+
 struct Run {
   wrfdc_ctx *X;
   // host copy of the context the kernels get (D()).  The moist / scalar
@@ -735,25 +743,37 @@ struct Run {
   }
   // rk_tendency + dry_boundary_tendency as the RK step runs them: the
   // lateral relaxation first (it only writes the physics tendencies, which the
-  // tendency terms do not read), then one kernel per tendency that forms all
-  // its terms in the reference's order and adds the physics tendency
-  // (rk_addtend_dry), then the specified-zone overlay.
+  // tendency terms do not read), then per tendency one pass that forms all its
+  // terms in the reference's order, adds the physics tendency
+  // (rk_addtend_dry) and on the specified zone's ring puts the boundary
+  // tendency instead (spec_bdy_dry).
   void fused_tendency() const {
     const int rk = X->rk;
     clear_tendencies(rk == 1);
     if (rk == 1) lateral_relax();
-    const R3 ru{1, ide, 1, kde - 1, 1, jde - 1};
-    k_advect_u<true><<<dim3(face_tiles(ru, d.face_lg[0]).count()), bf(), 0, s>>>(D(), F(F_u_2), F(F_ru_tend), F(F_ru), F(F_rv), F(F_ww), ru, rk);
-    const R3 rv{1, ide - 1, 1, kde - 1, 1, jde};
-    k_advect_v<true><<<dim3(face_tiles(rv, d.face_lg[0]).count()), bf(), 0, s>>>(D(), F(F_v_2), F(F_rv_tend), F(F_ru), F(F_rv), F(F_ww), rv, rk);
-    const R3 rw{1, ide - 1, 1, kde, 1, jde - 1};
-    k_advect_w<true><<<dim3(face_tiles(rw, d.face_lg[1]).count()), bf(), 0, s>>>(D(), F(F_w_2), F(F_rw_tend), F(F_ru), F(F_rv), F(F_ww), rw, rk);
-    const R3 rq{1, ide - 1, kde - 1, kde - 1, 1, jde - 1};  // levels [2, kde-2]: k_advect_w<true>
-    k_cqw_inv<<<g3p(rq), b3(), 0, s>>>(D(), rq);
-    const R3 m = mass3();
-    k_advect_scalar<kAdvTend><<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), 0, s>>>(D(), F(F_t_2), F(F_t_tend), F(F_ru), F(F_rv), F(F_ww), m, rk, TransportUpd{});
-    k_tend_ph<<<g3(rw), b3(), 0, s>>>(D(), rw, rk);
-    spec_overlays();
+    TendRanges T;
+    T.r[0] = R3{1, ide, 1, kde - 1, 1, jde - 1};
+    T.r[1] = R3{1, ide - 1, 1, kde - 1, 1, jde};
+    T.r[2] = T.r[4] = R3{1, ide - 1, 1, kde, 1, jde - 1};
+    T.r[3] = mass3();
+    const unsigned nb[5] = {face_tiles(T.r[0], d.face_lg[0]).count(), face_tiles(T.r[1], d.face_lg[0]).count(),
+                            face_tiles(T.r[2], d.face_lg[1]).count(), face_tiles(T.r[3], d.face_lg[0]).count(), g3(T.r[4]).x};
+    if (X->n3 <= kTendTogether) {
+      T.first[0] = 0;
+      for (int c = 0; c < 5; c++) T.first[c + 1] = T.first[c] + nb[c];
+      k_tendencies<<<T.first[5], bf(), 0, s>>>(D(), T, rk);
+    } else {
+      auto one = [&](int c, void (*kernel)(const DevCtx *, TendRanges, int)) {
+        T.first[c] = 0;
+        T.first[c + 1] = nb[c];
+        kernel<<<nb[c], bf(), 0, s>>>(D(), T, rk);
+      };
+      one(0, k_tendency<0>);
+      one(1, k_tendency<1>);
+      one(2, k_tendency<2>);
+      one(3, k_tendency<3>);
+      one(4, k_tendency<4>);
+    }
   }
   // relax_bdy_dry at the first stage (physics tendencies of u, v, ph, theta, mu)
   void lateral_relax() const {
@@ -809,11 +829,12 @@ struct Run {
     rk_addtend_dry();
     spec_overlays();
   }
-  void small_step_prep() const {
-    k_ssp_mass<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D(), X->rk);
+  // cqw_top: the fused step's cqw := 1/(1+cqw) on level kde-1 (its w tendency
+  // does the levels below, and reads this one twice)
+  void small_step_prep(bool cqw_top = false) const {
     R3 r = full3();
-    if (X->rk == 1) k_ssp_3d<true><<<g3p(r), b3(), 0, s>>>(D(), r);
-    else k_ssp_3d<false><<<g3p(r), b3(), 0, s>>>(D(), r);
+    if (X->rk == 1) k_ssp_3d<true><<<g3p(r), b3(), 0, s>>>(D(), r, cqw_top ? 1 : 0);
+    else k_ssp_3d<false><<<g3p(r), b3(), 0, s>>>(D(), r, cqw_top ? 1 : 0);
   }
   void calc_p_rho(int step) const {
     R3 m = mass3();
@@ -1134,7 +1155,7 @@ struct Run {
       first_rk_step_part2(false, true);
     }
     fused_tendency();
-    small_step_prep();
+    small_step_prep(true);
     calc_p_rho(0);
     calc_coef_w();
     BcBatch(this)
