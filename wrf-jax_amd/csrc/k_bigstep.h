@@ -17,35 +17,54 @@ __global__ void k_copy(float *dst, const float *src, size_t n) {
   for (; t < n; t += stride) dst[t] = src[t];
 }
 
-// mut, muu, muv (calc_mu_uv, module_big_step_utilities_em.py:174-266) and
-// muus/muvs from muts (calc_mu_uv_1).  2-D over i [1, ide], j [1, jde].
-__global__ void k_mu_uv(const DevCtx *xv, const float *mu, const float *mub, float *muu, float *muv, float *mut) {
+// muu, muv (calc_mu_uv, module_big_step_utilities_em.py:174-266) of one point
+// from the column masses mu + mub (u points i [1, ide], j [1, jde-1], v points
+// i [1, ide-1], j [1, jde]); mub nullptr: calc_mu_uv_1 on the full column mass
+// (adding the zero base state of the reference form leaves every sum
+// unchanged)
+__device__ __forceinline__ float mu_u(CtxPtr x, const float *mu, const float *mub, int i, int j) {
+  const int ide = x->ide;
+  const int ia = (i == ide) ? ide - 1 : i, ib = (i == 1) ? 1 : ((i == ide) ? ide - 1 : i - 1);
+  float s = A2(mu, ia, j) + A2(mu, ib, j);
+  if (mub) s = s + A2(mub, ia, j) + A2(mub, ib, j);
+  return 0.5f * s;
+}
+__device__ __forceinline__ float mu_v(CtxPtr x, const float *mu, const float *mub, int i, int j) {
+  const int jde = x->jde;
+  const int ja = (j == jde) ? jde - 1 : j, jb = (j == 1) ? 1 : ((j == jde) ? jde - 1 : j - 1);
+  float s = A2(mu, i, ja) + A2(mu, i, jb);
+  if (mub) s = s + A2(mub, i, ja) + A2(mub, i, jb);
+  return 0.5f * s;
+}
+// calc_mu_uv: mut, muu and muv.  2-D over i [1, ide], j [1, jde].
+__global__ void k_mu_uv(const DevCtx *xv) {
   const CtxPtr x = ctx_ptr(xv);
   const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int j = 1 + (int)blockIdx.y;
   const int ide = x->ide, jde = x->jde;
   if (i > ide || j > jde) return;
-  // mub == nullptr: calc_mu_uv_1 on the full column mass (adding the zero
-  // base state of the reference form leaves every sum unchanged)
-  if (mut) A2(mut, i, j) = A2(mub, i, j) + A2(mu, i, j);
-  if (j <= jde - 1) {
-    int ia = (i == ide) ? ide - 1 : i;
-    int ib = (i == 1) ? 1 : ((i == ide) ? ide - 1 : i - 1);
-    float s = A2(mu, ia, j) + A2(mu, ib, j);
-    if (mub) s = s + A2(mub, ia, j) + A2(mub, ib, j);
-    A2(muu, i, j) = 0.5f * s;
-  }
-  if (i <= ide - 1) {
-    int ja = (j == jde) ? jde - 1 : j;
-    int jb = (j == 1) ? 1 : ((j == jde) ? jde - 1 : j - 1);
-    float s = A2(mu, i, ja) + A2(mu, i, jb);
-    if (mub) s = s + A2(mub, i, ja) + A2(mub, i, jb);
-    A2(muv, i, j) = 0.5f * s;
-  }
+  const float *mu = FL(mu_2), *mub = FL(mub);
+  A2(FL(mut), i, j) = A2(mub, i, j) + A2(mu, i, j);
+  if (j <= jde - 1) A2(FL(muu), i, j) = mu_u(x, mu, mub, i, j);
+  if (i <= ide - 1) A2(FL(muv), i, j) = mu_v(x, mu, mub, i, j);
+}
+// calc_mu_uv_1: muus / muvs from muts.  2-D over i [1, ide], j [1, jde].
+__global__ void k_mu_uv_1(const DevCtx *xv) {
+  const CtxPtr x = ctx_ptr(xv);
+  const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  const int j = 1 + (int)blockIdx.y;
+  const int ide = x->ide, jde = x->jde;
+  if (i > ide || j > jde) return;
+  if (j <= jde - 1) A2(FL(muus), i, j) = mu_u(x, FL(muts), nullptr, i, j);
+  if (i <= ide - 1) A2(FL(muvs), i, j) = mu_v(x, FL(muts), nullptr, i, j);
 }
 
 // couple_momentum + calc_cq + calc_alt + calc_php over the full 3-D extent
-// (zero outside each field's range, as the reference's fresh outputs).
+// (zero outside each field's range, as the reference's fresh outputs).  MUV:
+// calc_mu_uv too: every thread forms the column masses it needs, those of
+// level 1 store mut, muu and muv (a launch of 4 us less, 24 us more for the
+// kernel at 400x400x60: kPrepMuv).
+template <bool MUV>
 __global__ void k_rk_prep3(const DevCtx *xv, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
@@ -56,7 +75,10 @@ __global__ void k_rk_prep3(const DevCtx *xv, R3 r) {
   const float c1h = A1(FL(c1h), kh), c2h = A1(FL(c2h), kh), c1f = A1(FL(c1f), k), c2f = A1(FL(c2f), k);
   // every load of the point first (the moist species follow in groups)
   const float u = elem(FL(u_2), o), v = elem(FL(v_2), o), w = elem(FL(w_2), o);
-  const float muu = elem(FL(muu), o2), muv = elem(FL(muv), o2), mut = elem(FL(mut), o2);
+  const float *mu = FL(mu_2), *mub = FL(mub);
+  const float muu = MUV ? mu_u(x, mu, mub, i, imin_(j, jde - 1)) : elem(FL(muu), o2);
+  const float muv = MUV ? mu_v(x, mu, mub, imin_(i, ide - 1), j) : elem(FL(muv), o2);
+  const float mut = MUV ? elem(mub, o2) + elem(mu, o2) : elem(FL(mut), o2);
   const float msfuy = elem(FL(msfuy), o2), msfvxi = elem(FL(msfvx_inv), o2), msfty = elem(FL(msfty), o2);
   const float al = elem(FL(al), o), alb = elem(FL(alb), o);
   const float phb0 = elem(FL(phb), o), phb1 = elem(FL(phb), ok1), ph0 = elem(FL(ph_2), o), ph1 = elem(FL(ph_2), ok1);
@@ -69,6 +91,11 @@ __global__ void k_rk_prep3(const DevCtx *xv, R3 r) {
   pin1(phb1);
   pin1(ph0);
   pin1(ph1);
+  if (MUV && k == 1) {
+    elem(FL(mut), o2) = mut;
+    if (j <= jde - 1) elem(FL(muu), o2) = muu;
+    if (i <= ide - 1) elem(FL(muv), o2) = muv;
+  }
   // ru / rv / rw
   elem(FL(ru), o) = (j <= jde - 1 && k <= kde - 1) ? u * (c1h * muu + c2h) / msfuy : 0.f;
   elem(FL(rv), o) = (i <= ide - 1 && k <= kde - 1) ? v * (c1h * muv + c2h) * msfvxi : 0.f;
@@ -580,9 +607,7 @@ __global__ void k_addtend(const DevCtx *xv, int comp, int rk, R3 r) {
 }
 
 // _calc_p_rho_phi_nonhydro_opt2 (runtime.py:12369-12537): hypsometric al, EOS p
-__global__ void k_calc_p_rho_phi(const DevCtx *xv, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ_P(r);
+__device__ __forceinline__ void calc_p_rho_phi_pt(CtxPtr x, int i, int k, int j) {
   const float *muts = FL(muts), *ph = FL(ph_2), *phb = FL(phb), *alb = FL(alb), *pb = FL(pb), *t = FL(t_2);
   const float m = A2(muts, i, j), ptop = x->ptop;
   const float pfu = A1(FL(c3f), k + 1) * m + A1(FL(c4f), k + 1) + ptop;
@@ -607,4 +632,9 @@ __global__ void k_calc_p_rho_phi(const DevCtx *xv, R3 r) {
   const float qvf = 1.f + x->rvovrd * qv;
   const float temp = (x->r_d * (x->t0 + tv) * qvf) / (x->p0 * (alv + albv));
   elem(FL(p), o) = (float)f64_pow((double)temp, (double)x->cpovcv) * x->p0 - pbv;
+}
+__global__ void k_calc_p_rho_phi(const DevCtx *xv, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
+  GET_IKJ_P(r);
+  calc_p_rho_phi_pt(x, i, k, j);
 }

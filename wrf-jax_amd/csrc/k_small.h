@@ -5,6 +5,7 @@
 // argument mapping of the stage adapters in src/wrf_jax/runtime.py.
 #pragma once
 #include "wrfdc_common.h"
+#include "k_bigstep.h"
 
 // small_step_prep, 2-D part (module_small_step_em.py:272-420): stage-start
 // column masses of the column (i, j), i [1, ide], j [1, jde].  Every value is
@@ -125,9 +126,7 @@ __global__ void k_ssp_3d(const DevCtx *xv, R3 r, int cqw_top) {
 
 // calc_p_rho, non-hydrostatic (module_small_step_em.py:720-1034) with
 // ph = ph_2, t_1 = t_save, mu = mu_2, mut = muts; mass points.
-__global__ void k_calc_p_rho(const DevCtx *xv, int step, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ_P(r);
+__device__ __forceinline__ void calc_p_rho_pt(CtxPtr x, int step, int i, int k, int j) {
   const unsigned o = XI3(i, k, j);
   // every load first (the stores below could alias them as far as the
   // compiler knows)
@@ -148,17 +147,22 @@ __global__ void k_calc_p_rho(const DevCtx *xv, int step, R3 r) {
   elem(FL(pm1), o) = pr;
 }
 
+__global__ void k_calc_p_rho(const DevCtx *xv, int step, R3 r) {
+  const CtxPtr x = ctx_ptr(xv);
+  GET_IKJ_P(r);
+  calc_p_rho_pt(x, step, i, k, j);
+}
+
 // calc_coef_w (module_small_step_em.py:1359-1586): LU factors of the
 // implicit w-phi system, one thread per mass column.
-__global__ void k_calc_coef_w(const DevCtx *xv, float dts, R2 r) {
-  const CtxPtr x = ctx_ptr(xv);
+__device__ __forceinline__ void calc_coef_w(CtxPtr x, float dts, const R2 &r, unsigned b, unsigned nb) {
   // the column coefficients in LDS: read per level inside the recurrence, and
   // from global memory every such read would wait behind the previous level's
   // stores (the compiler cannot prove they do not alias)
   constexpr int kMaxLev = 152;  // kde <= 151 (wrfdc_create checks nz <= 150)
   __shared__ float c1h[kMaxLev], c2h[kMaxLev], c1f[kMaxLev], c2f[kMaxLev], rdn[kMaxLev], rdnw[kMaxLev];
   const int kde = x->kde;
-  for (int q = (int)threadIdx.x; q < kde; q += (int)blockDim.x) {
+  for (int q = (int)(threadIdx.y * 64u + threadIdx.x); q < kde; q += (int)(blockDim.x * blockDim.y)) {
     c1h[q] = FL(c1h)[q];
     c2h[q] = FL(c2h)[q];
     c1f[q] = FL(c1f)[q];
@@ -167,7 +171,7 @@ __global__ void k_calc_coef_w(const DevCtx *xv, float dts, R2 r) {
     rdnw[q] = FL(rdnw)[q];
   }
   __syncthreads();
-  GET_IJ(r);
+  GET_IJ_B(r, b, nb);
   float *a = FL(a), *alpha = FL(alpha), *gamma = FL(gamma);
   const float *cqw = FL(cqw), *c2a = FL(c2a);
   const float lid = x->top_lid ? 0.f : 1.f;
@@ -219,6 +223,23 @@ __global__ void k_calc_coef_w(const DevCtx *xv, float dts, R2 r) {
                                ((A1(c1h, kde - 1) * m + A1(c2h, kde - 1)) * (A1(c1f, kde) * m + A1(c2f, kde)));
   A3(alpha, i, kde, j) = 1.f / (btop - atop * gprev);
   A3(gamma, i, kde, j) = 0.f;
+}
+__global__ void __launch_bounds__(64) k_calc_coef_w(const DevCtx *xv, float dts, R2 r) {
+  calc_coef_w(ctx_ptr(xv), dts, r, blockIdx.x, gridDim.x);
+}
+// both, which share their inputs and not their outputs, in one launch: the
+// first nc blocks the columns (4 waves, a tile of 64 columns each: a chain of
+// divisions that waits on little), the others the points, which wait on
+// memory.  400x400x60: 52 and 80 us one after the other, 126 us together;
+// 24x20x10 6 and 3, then 7.
+__global__ void __launch_bounds__(256) k_coef_p_rho(const DevCtx *xv, float dts, R2 c, unsigned nc, R3 m) {
+  const CtxPtr x = ctx_ptr(xv);
+  if (blockIdx.x < nc) {
+    calc_coef_w(x, dts, c, blockIdx.x * 4u + wave_y(), nc * 4u);
+    return;
+  }
+  GET_IKJ_PB(m, blockIdx.x - nc);
+  calc_p_rho_pt(x, 0, i, k, j);
 }
 
 // interface pressure of a u/v face (module_small_step_em.py:1627-1645)
@@ -450,8 +471,9 @@ __global__ void k_sumflux(const DevCtx *xv, int first, int fin, float ns, R3 r) 
 // small_step_finish (module_small_step_em.py:1119-1332): recouple the
 // acoustic perturbations onto the stage-start state.  Full extent.
 // (loads first, as k_ssp_3d; FINAL: the last RK stage, which also removes
-// the diabatic heating)
-template <bool FINAL>
+// the diabatic heating; MUV: calc_mu_uv_1 too: every thread forms its own
+// staggered masses of muts, those of level 1 store them)
+template <bool FINAL, bool MUV>
 __global__ void k_ssf(const DevCtx *xv, float dts, float nsm, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
@@ -463,8 +485,17 @@ __global__ void k_ssf(const DevCtx *xv, float dts, float nsm, R3 r) {
   const float w2 = elem(FL(w_2), o), ws = elem(FL(w_save), o), ph2 = elem(FL(ph_2), o), phs = elem(FL(ph_save), o);
   const float wwv = elem(FL(ww), o), ww1 = elem(FL(ww_1), o), t2 = elem(FL(t_2), o), ts = elem(FL(t_save), o);
   const float hd = FINAL ? elem(FL(h_diabatic), o) : 0.f;
-  const float muv = elem(FL(muv), o2), muvs = elem(FL(muvs), o2), msfvx = elem(FL(msfvx), o2);
-  const float muu = elem(FL(muu), o2), muus = elem(FL(muus), o2), msfuy = elem(FL(msfuy), o2);
+  const float muv = elem(FL(muv), o2), msfvx = elem(FL(msfvx), o2), muu = elem(FL(muu), o2), msfuy = elem(FL(msfuy), o2);
+  float muus, muvs;
+  if (MUV) {
+    muus = mu_u(x, FL(muts), nullptr, i, imin_(j, jde - 1));
+    muvs = mu_v(x, FL(muts), nullptr, imin_(i, ide - 1), j);
+    if (k == 1 && j <= jde - 1) elem(FL(muus), o2) = muus;
+    if (k == 1 && i <= ide - 1) elem(FL(muvs), o2) = muvs;
+  } else {
+    muus = elem(FL(muus), o2);
+    muvs = elem(FL(muvs), o2);
+  }
   const float mt = elem(FL(mut), o2), mts = elem(FL(muts), o2), msfty = elem(FL(msfty), o2);
   if (i <= ide - 1 && k <= kde - 1) {
     const float old = c1h * muv + c2h, nw = c1h * muvs + c2h;

@@ -418,14 +418,13 @@ struct FlowList {
   float *q[kMaxSpec];
   int n;
 };
-__global__ void k_flow_dep_batch(const DevCtx *xv, FlowList L) {
-  const CtxPtr x = ctx_ptr(xv);
-  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int k = 1 + (int)blockIdx.y;
-  const int s = (int)blockIdx.z;
+// point n of the list: zone point, level, species
+__device__ __forceinline__ void flow_dep(CtxPtr x, const FlowList &L, unsigned n) {
   const int ibe = x->ide - 1, jbe = x->jde - 1;
+  const unsigned zn = (unsigned)(2 * ibe + 2 * (jbe - 2)), nk = (unsigned)(x->kde - 1);
+  const int k = 1 + (int)(n / zn % nk), s = (int)(n / zn / nk);
   int i, j, e;
-  if (k > x->kde - 1 || !zone_point(t, ibe, jbe, i, j, e)) return;
+  if (s >= L.n || !zone_point((int)(n % zn), ibe, jbe, i, j, e)) return;
   float *q = L.q[s];
   const float *u = FL(ru_m), *v = FL(rv_m);
   if (e == 0) {
@@ -441,4 +440,15 @@ __global__ void k_flow_dep_batch(const DevCtx *xv, FlowList L) {
     const int jj = imin_(imax_(j, 2), jbe - 1);
     A3(q, ibe, k, j) = A3(u, ibe + 1, k, j) > 0.f ? A3(q, ibe - 1, k, jj) : 0.f;
   }
+}
+// calc_p_rho_phi over the mass points m (the first nm blocks), which of the
+// species reads QV, and flow_dep_bdy of the others, in one launch
+__global__ void __launch_bounds__(256) k_p_rho_phi_flow(const DevCtx *xv, R3 m, unsigned nm, FlowList L) {
+  const CtxPtr x = ctx_ptr(xv);
+  if (blockIdx.x >= nm) {
+    flow_dep(x, L, (blockIdx.x - nm) * 256u + wave_y() * 64u + threadIdx.x);
+    return;
+  }
+  GET_IKJ_PB(m, blockIdx.x);
+  calc_p_rho_phi_pt(x, i, k, j);
 }

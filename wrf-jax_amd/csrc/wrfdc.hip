@@ -296,6 +296,10 @@ inline unsigned cdiv(int a, int b) { return (unsigned)((a + b - 1) / b); }
 // (0.5 M elements) 1052 and 1031, 257x131x37 (1.4 M) 1868 and 1889,
 // 400x400x60 14.52 and 14.96 ms.
 constexpr size_t kTendTogether = (size_t)1 << 20;
+// Elements up to which rk_step_prep's 3-D kernel forms the column masses
+// itself: the launch saved (4 us) against 24 us for the 25 M elements of
+// 400x400x60.
+constexpr size_t kPrepMuv = (size_t)4 << 20;
 
 struct Run {
   wrfdc_ctx *X;
@@ -529,9 +533,13 @@ struct Run {
   };
   // ---- RK-stage pieces -----------------------------------------------------
   void rk_step_prep() const {
-    k_mu_uv<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D(), F(F_mu_2), F(F_mub), F(F_muu), F(F_muv), F(F_mut));
     R3 r = full3();
-    k_rk_prep3<<<g3(r), b3(), 0, s>>>(D(), r);
+    if (X->n3 <= kPrepMuv) {
+      k_rk_prep3<true><<<g3(r), b3(), 0, s>>>(D(), r);
+    } else {
+      k_mu_uv<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D());
+      k_rk_prep3<false><<<g3(r), b3(), 0, s>>>(D(), r);
+    }
     R2 c = mass2();
     k_ww_cp<<<g2(c), 64, sizeof(float) * 64 * (size_t)(kde - 1), s>>>(D(), c);
   }
@@ -844,6 +852,13 @@ struct Run {
     R2 c = mass2();
     k_calc_coef_w<<<g2(c), 64, 0, s>>>(D(), (float)X->dts_rk, c);
   }
+  // calc_p_rho(0) and calc_coef_w in one launch
+  void coef_p_rho() const {
+    R2 c = mass2();
+    R3 m = mass3();
+    const unsigned nc = (g2(c).x + 3u) / 4u;
+    k_coef_p_rho<<<nc + g3p(m).x, b3(), 0, s>>>(D(), (float)X->dts_rk, c, nc, m);
+  }
   void advance_uv() const {
     const int sz = X->c.spec_zone;
     R3 ru{1 + sz, ide - sz, 1, kde - 1, 1 + sz, jde - sz - 1};
@@ -882,18 +897,17 @@ struct Run {
   }
   // calc_mu_uv_1: the staggered column masses of muts
   void calc_mu_uv_1() const {
-    k_mu_uv<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D(), F(F_muts), nullptr, F(F_muus), F(F_muvs), nullptr);
+    k_mu_uv_1<<<dim3(cdiv(ide, 64), jde), 64, 0, s>>>(D());
   }
-  void small_step_finish() const {
-    calc_mu_uv_1();
-    recouple();
-  }
-  // small_step_finish proper (module_small_step_em.py:1119-1332), without
-  // the calc_mu_uv_1 that the RK stage runs before it
-  void recouple() const {
+  // calc_mu_uv_1 and small_step_finish proper, as the RK stage runs them
+  void small_step_finish() const { finish<true>(); }
+  // small_step_finish proper (module_small_step_em.py:1119-1332)
+  void recouple() const { finish<false>(); }
+  template <bool MUV>
+  void finish() const {
     R3 r = full3();
-    if (X->rk == 3) k_ssf<true><<<g3(r), b3(), 0, s>>>(D(), (float)X->dts_rk, (float)X->nsmall, r);
-    else k_ssf<false><<<g3(r), b3(), 0, s>>>(D(), (float)X->dts_rk, (float)X->nsmall, r);
+    if (X->rk == 3) k_ssf<true, MUV><<<g3(r), b3(), 0, s>>>(D(), (float)X->dts_rk, (float)X->nsmall, r);
+    else k_ssf<false, MUV><<<g3(r), b3(), 0, s>>>(D(), (float)X->dts_rk, (float)X->nsmall, r);
   }
   void calc_p_rho_phi() const {
     R3 m = mass3();
@@ -1040,13 +1054,15 @@ struct Run {
       copy_species(R3{ide, ide, 1, kde - 1, 1, jde}, false);
       copy_species(R3{1, ide, 1, kde - 1, jde, jde}, false);
     }
-    if (nm > 1) {
-      FlowList fl;
-      memset(&fl, 0, sizeof(fl));
-      for (int q = 1; q < nm; q++) fl.q[fl.n++] = Sp(F_moist, q);
-      Z z = zd('t', false, false);
-      k_flow_dep_batch<<<dim3(cdiv(zone_n(z), 64), kde - 1, fl.n), 64, 0, s>>>(D(), fl);
-    }
+  }
+  // flow_dep_bdy of the species beyond QV, with calc_p_rho_phi
+  void p_rho_phi_and_flow() const {
+    FlowList fl;
+    memset(&fl, 0, sizeof(fl));
+    for (int q = 1; q < X->c.nmoist; q++) fl.q[fl.n++] = Sp(F_moist, q);
+    R3 m = mass3();
+    const unsigned nm = g3p(m).x, points = (unsigned)zone_n(zd('t', false, false)) * (unsigned)(kde - 1) * (unsigned)fl.n;
+    k_p_rho_phi_flow<<<nm + (points + 255u) / 256u, b3(), 0, s>>>(D(), m, nm, fl);
   }
 
   // one stage of scalar transport with recorded dynamics (tangent-linear =
@@ -1156,8 +1172,7 @@ struct Run {
     }
     fused_tendency();
     small_step_prep(true);
-    calc_p_rho(0);
-    calc_coef_w();
+    coef_p_rho();
     BcBatch(this)
         .add3(F(F_ru_tend), 'u').add3(F(F_rv_tend), 'v').add3(F(F_ph_2), 'w').add3(F(F_al), 'p').add3(F(F_p), 'p')
         .add3(F(F_t_1), 'p').add3(F(F_t_save), 't').add2(F(F_mu_1), 't').add2(F(F_mu_2), 't').add2(F(F_mudf), 't')
@@ -1169,7 +1184,7 @@ struct Run {
     const int nm = X->c.nmoist, nsc = X->c.nscalar;
     record_stage();
     species_stage();
-    calc_p_rho_phi();
+    p_rho_phi_and_flow();
     if (X->rk < 3) {
       BcBatch bc(this);
       phys_bc_dry_2(bc);

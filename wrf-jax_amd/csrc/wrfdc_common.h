@@ -189,19 +189,21 @@ __device__ __forceinline__ unsigned wave_y() { return (unsigned)__builtin_amdgcn
 // Pointwise kernels (no neighbour in j): the same block shape and i tiles, a
 // 1-D grid of ceil((i1 - ib + 1)/64) * ceil(nk/4) * nj blocks in plain order
 // (i, then k, then j).
-#define GET_IKJ_P(r)                                                                         \
+#define GET_IKJ_P(r) GET_IKJ_PB(r, blockIdx.x)
+#define GET_IKJ_PB(r, b)                                                                     \
   const int ib_ = 1 + (((r).i0 - 1) & ~63);                                                  \
   const unsigned gx_ = (unsigned)((r).i1 - ib_ + 64) / 64u;                                  \
-  const unsigned gy_ = (unsigned)((r).k1 - (r).k0 + 4) / 4u;                                 \
-  const int i = ib_ + (int)((blockIdx.x % gx_) * 64u + threadIdx.x);                         \
-  const int k = (r).k0 + (int)(((blockIdx.x / gx_) % gy_) * 4u + wave_y());                  \
-  const int j = (r).j0 + (int)(blockIdx.x / (gx_ * gy_));                                    \
+  const unsigned gy_ = (unsigned)((r).k1 - (r).k0 + 4) / 4u, bp_ = (b);                      \
+  const int i = ib_ + (int)((bp_ % gx_) * 64u + threadIdx.x);                                \
+  const int k = (r).k0 + (int)(((bp_ / gx_) % gy_) * 4u + wave_y());                         \
+  const int j = (r).j0 + (int)(bp_ / (gx_ * gy_));                                           \
   if (i < (r).i0 || i > (r).i1 || k > (r).k1 || j > (r).j1) return
 // thread -> (i, j) for column kernels: blockDim (64, 1, 1), 1-D grid of
 // ceil(ni/64) * nj blocks
-#define GET_IJ(r)                                                                            \
+#define GET_IJ(r) GET_IJ_B(r, blockIdx.x, gridDim.x)
+#define GET_IJ_B(r, b, nb)                                                                   \
   const unsigned gx_ = (unsigned)((r).i1 - (r).i0 + 64) / 64u;                               \
-  const unsigned t_ = xcd_tile(blockIdx.x, gridDim.x);                                       \
+  const unsigned t_ = xcd_tile(b, nb);                                                       \
   const int i = (r).i0 + (int)((t_ % gx_) * 64u + threadIdx.x);                              \
   const int j = (r).j0 + (int)(t_ / gx_);                                                    \
   if (i > (r).i1 || j > (r).j1) return
