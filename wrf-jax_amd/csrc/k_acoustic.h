@@ -23,6 +23,7 @@
 #pragma once
 #include "wrfdc_common.h"
 #include "k_small.h"
+#include "k_bc.h"
 #include <type_traits>
 
 // ---------------------------------------------------------------------------
@@ -76,9 +77,8 @@ __device__ __forceinline__ float uv_interior(CtxPtr x, int axis, int i, int k, i
 // (its own where they apply) and the zone formula, with no branch around the
 // loads, so all of them are in flight together; the results are selected
 // and stored at the end.
-__global__ void __launch_bounds__(256) k_uv_substep(const DevCtx *xv, float dts, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ(r);
+__device__ __forceinline__ void uv_substep(CtxPtr x, float dts, const R3 &r, unsigned b, unsigned nb) {
+  GET_IKJ_B(r, b, nb);
   const int ide = x->ide, jde = x->jde;
   const unsigned o = XI3(i, k, j);
   const bool upt = (j <= jde - 1), vpt = (i <= ide - 1);
@@ -93,6 +93,23 @@ __global__ void __launch_bounds__(256) k_uv_substep(const DevCtx *xv, float dts,
   const float vn_in = uv_interior(x, 1, imin_(imax_(i, 2), ide - 2), k, imin_(imax_(j, 2), jde - 1), dts, vn_z);
   if (upt) elem(FL(u_2), o) = uin ? un_in : un_z;
   if (vpt) elem(FL(v_2), o) = vin ? vn_in : vn_z;
+}
+__global__ void __launch_bounds__(256) k_uv_substep(const DevCtx *xv, float dts, R3 r) {
+  uv_substep(ctx_ptr(xv), dts, r, blockIdx.x, gridDim.x);
+}
+// The first substep of a stage, with the physical-boundary copies between
+// small_step_prep and the loop (column ide, row jde).  The u and v points read
+// no mass column of that edge, and the tendencies of u in row jde and of v in
+// column ide, which are copied, belong to no point that is stored.  The copies
+// have the nbc blocks before u and v: they are few threads that wait for one
+// load each, and after u and v they trailed alone (257x131x37 step: 1831 us
+// after, 1819 before, 1822 as a launch of their own; with the fills of
+// k_fill_bc 24x20x10 378 -> 367, 100x100x45 981 -> 971, 400x400x60 14466 ->
+// 14434 us a step).
+__global__ void __launch_bounds__(256) k_uv_first(const DevCtx *xv, float dts, R3 r, unsigned nbc, BcPart B) {
+  const CtxPtr x = ctx_ptr(xv);
+  if (blockIdx.x < nbc) bc_part(x, B, blockIdx.x * 256u + wave_y() * 64u + threadIdx.x);
+  else uv_substep(x, dts, r, blockIdx.x - nbc, gridDim.x - nbc);
 }
 
 // ---------------------------------------------------------------------------

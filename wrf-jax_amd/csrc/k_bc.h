@@ -35,11 +35,7 @@ struct BcList {
   int kend[kBcMax];
   int flags[kBcMax];  // bit 0: copy column ide, bit 1: copy row jde, bit 2: 2-D
 };
-__global__ void k_bc_batch(const DevCtx *xv, BcList L) {
-  const CtxPtr x = ctx_ptr(xv);
-  const int a = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int k = 1 + (int)blockIdx.y;
-  const int q = (int)blockIdx.z;
+__device__ __forceinline__ void bc_copy(CtxPtr x, const BcList &L, int a, int k, int q) {
   const int fl = L.flags[q];
   if (k > L.kend[q]) return;
   float *f = L.f[q];
@@ -53,9 +49,28 @@ __global__ void k_bc_batch(const DevCtx *xv, BcList L) {
   if (cy && a <= ide && !(a == ide && cx)) AT(a, jde) = AT(a, jde - 1);
 #undef AT
 }
+__global__ void k_bc_batch(const DevCtx *xv, BcList L) {
+  bc_copy(ctx_ptr(xv), L, 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x), 1 + (int)blockIdx.y, (int)blockIdx.z);
+}
+// The same as part of another launch: thread t of n fields over kmax levels
+// and the longer edge.  The fields' copies must not be read by that launch's
+// other work, nor read what it writes.
+struct BcPart {
+  BcList L;
+  int n, kmax;
+};
+__device__ __forceinline__ unsigned bc_part_threads(CtxPtr x, const BcPart &B) {
+  return (unsigned)(x->ide > x->jde ? x->ide : x->jde) * (unsigned)(B.kmax * B.n);
+}
+__device__ __forceinline__ void bc_part(CtxPtr x, const BcPart &B, unsigned t) {
+  const unsigned along = (unsigned)(x->ide > x->jde ? x->ide : x->jde);
+  const int q = (int)(t / along / (unsigned)B.kmax);
+  if (q >= B.n) return;
+  bc_copy(x, B.L, 1 + (int)(t % along), 1 + (int)(t / along % (unsigned)B.kmax), q);
+}
 
 // Batched fills: blockIdx.y = field, grid-stride over its elements.
-constexpr int kFillMax = 16;
+constexpr int kFillMax = 24;
 struct FillList {
   float *p[kFillMax];
   size_t n[kFillMax];
@@ -64,6 +79,21 @@ __global__ void k_fill_batch(FillList L) {
   float *p = L.p[blockIdx.y];
   const size_t n = L.n[blockIdx.y];
   for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) p[t] = 0.f;
+}
+// The first stage's boundary copies (blockIdx.y = 0) and fills (blockIdx.y - 1
+// = field) in one launch instead of three, each of which left the chip idle
+// for its 4 us on a small domain.
+__global__ void __launch_bounds__(256) k_fill_bc(const DevCtx *xv, FillList L, BcPart B) {
+  const CtxPtr x = ctx_ptr(xv);
+  const unsigned step = gridDim.x * blockDim.x;
+  if (blockIdx.y == 0) {
+    const unsigned nt = bc_part_threads(x, B);
+    for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < nt; t += step) bc_part(x, B, t);
+    return;
+  }
+  float *p = L.p[blockIdx.y - 1];
+  const size_t n = L.n[blockIdx.y - 1];
+  for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += step) p[t] = 0.f;
 }
 
 // ---- specified zone (spec_zone = 1): ring of the variable's grid ----------

@@ -441,14 +441,14 @@ __device__ __forceinline__ void flow_dep(CtxPtr x, const FlowList &L, unsigned n
     A3(q, ibe, k, j) = A3(u, ibe + 1, k, j) > 0.f ? A3(q, ibe - 1, k, jj) : 0.f;
   }
 }
-// calc_p_rho_phi over the mass points m (the first nm blocks), which of the
-// species reads QV, and flow_dep_bdy of the others, in one launch
-__global__ void __launch_bounds__(256) k_p_rho_phi_flow(const DevCtx *xv, R3 m, unsigned nm, FlowList L) {
+// calc_p_rho_phi over the mass points m, which of the species reads QV, and
+// (the first nf blocks) flow_dep_bdy of the others, in one launch
+__global__ void __launch_bounds__(256) k_p_rho_phi_flow(const DevCtx *xv, R3 m, unsigned nf, FlowList L) {
   const CtxPtr x = ctx_ptr(xv);
-  if (blockIdx.x >= nm) {
-    flow_dep(x, L, (blockIdx.x - nm) * 256u + wave_y() * 64u + threadIdx.x);
+  if (blockIdx.x < nf) {
+    flow_dep(x, L, blockIdx.x * 256u + wave_y() * 64u + threadIdx.x);
     return;
   }
-  GET_IKJ_PB(m, blockIdx.x);
+  GET_IKJ_PB(m, blockIdx.x - nf);
   calc_p_rho_phi_pt(x, i, k, j);
 }

@@ -402,6 +402,19 @@ struct Run {
       n = 0;
       kmax = 1;
     }
+    // the batch as part of another launch (its blocks of 256 threads)
+    BcPart take() {
+      BcPart B;
+      B.L = L;
+      B.n = n;
+      B.kmax = kmax;
+      n = 0;
+      kmax = 1;
+      return B;
+    }
+    static unsigned blocks(const Run *r, const BcPart &B) {
+      return ((unsigned)std::max(r->ide, r->jde) * (unsigned)(B.n * B.kmax) + 255u) / 256u;
+    }
     ~BcBatch() { flush(); }
   };
   void fill_many(std::initializer_list<std::pair<float *, size_t>> items) const {
@@ -543,12 +556,33 @@ struct Run {
     R2 c = mass2();
     k_ww_cp<<<g2(c), 64, sizeof(float) * 64 * (size_t)(kde - 1), s>>>(D(), c);
   }
-  void first_rk_step_part1(bool with_rho = true) const {
+  // the first stage of the fused step: what first_rk_step_part1 and
+  // clear_tendencies clear (nothing between them reads or writes the RK and
+  // saved tendencies) and the boundary copies b, in one launch
+  void first_stage_clears(const BcPart &B) const {
+    const size_t n3 = X->n3;
+    FillList L;
+    memset(&L, 0, sizeof(L));
+    int n = 0;
+    auto add = [&](float *p, size_t count) {
+      if (count == 0) return;
+      L.p[n] = p;
+      L.n[n++] = count;
+    };
+    for (int f : {F_ru_tendf, F_rv_tendf, F_rw_tendf, F_ph_tendf, F_t_tendf, F_ru_tend, F_rv_tend, F_rw_tend, F_t_tend, F_ph_tend, F_u_save,
+                  F_v_save, F_w_save, F_ph_save, F_t_save})
+      add(F(f), n3);
+    for (int f : {F_mu_tendf, F_mu_tend, F_mu_save}) add(F(f), X->n2);
+    add(F(F_moist_tend), n3 * (size_t)X->c.nmoist);
+    add(F(F_scalar_tend), n3 * (size_t)X->c.nscalar);
+    const size_t nmax = std::max(n3, n3 * (size_t)std::max(X->c.nmoist, X->c.nscalar));
+    k_fill_bc<<<dim3((unsigned)std::min<size_t>((nmax + 255) / 256, 2048), n + 1), 256, 0, s>>>(D(), L, B);
+  }
+  void first_rk_step_part1() const {
     const size_t n3 = X->n3;
     fill_many({{F(F_ru_tendf), n3}, {F(F_rv_tendf), n3}, {F(F_rw_tendf), n3}, {F(F_ph_tendf), n3}, {F(F_t_tendf), n3},
                {F(F_mu_tendf), X->n2}, {F(F_moist_tend), n3 * (size_t)X->c.nmoist},
                {F(F_scalar_tend), n3 * (size_t)X->c.nscalar}});
-    if (!with_rho) return;  // the step forms rho with the diffusion metrics
     R3 m = mass3();
     k_rho<<<g3p(m), b3(), 0, s>>>(D(), m);
   }
@@ -723,23 +757,22 @@ struct Run {
     k_cor_curv<<<g3(rw), b3(), 0, s>>>(D(), 2, rw);
   }
   // the RK tendencies and the saved tendencies start from zero each stage.
-  // The first stage clears every tendency and saved tendency.  Later stages
-  // of the fused step (first = false) clear nothing: the fused tendency
+  // The first stage of the fused step clears every tendency and saved tendency
+  // (first_stage_clears).  Its later stages clear nothing: the fused tendency
   // kernels write every point of their ranges from 0 (the points outside
   // stay 0 from the first stage's clear), the zone overlay writes its
   // points, mu_tend is formed as 0 + mu_tendf by the theta kernel at rk > 1,
   // and the saved tendencies keep their values - nothing reads them before
   // small_step_prep writes them again over the same points, and the first
   // stage's addtend fold is their only earlier reader.
-  void clear_tendencies(bool first) const {
+  void clear_tendencies() const {
     const size_t n3 = X->n3, n2 = X->n2;
-    if (first)
-      fill_many({{F(F_ru_tend), n3}, {F(F_rv_tend), n3}, {F(F_rw_tend), n3}, {F(F_t_tend), n3}, {F(F_ph_tend), n3},
-                 {F(F_u_save), n3}, {F(F_v_save), n3}, {F(F_w_save), n3}, {F(F_ph_save), n3}, {F(F_t_save), n3},
-                 {F(F_mu_tend), n2}, {F(F_mu_save), n2}});
+    fill_many({{F(F_ru_tend), n3}, {F(F_rv_tend), n3}, {F(F_rw_tend), n3}, {F(F_t_tend), n3}, {F(F_ph_tend), n3},
+               {F(F_u_save), n3}, {F(F_v_save), n3}, {F(F_w_save), n3}, {F(F_ph_save), n3}, {F(F_t_save), n3},
+               {F(F_mu_tend), n2}, {F(F_mu_save), n2}});
   }
   void rk_tendency() const {
-    clear_tendencies(true);
+    clear_tendencies();
     advect_u();
     advect_v();
     advect_w();
@@ -757,7 +790,6 @@ struct Run {
   // tendency instead (spec_bdy_dry).
   void fused_tendency() const {
     const int rk = X->rk;
-    clear_tendencies(rk == 1);
     if (rk == 1) lateral_relax();
     TendRanges T;
     T.r[0] = R3{1, ide, 1, kde - 1, 1, jde - 1};
@@ -888,11 +920,14 @@ struct Run {
   }
   // one fused acoustic substep: u/v, then the column kernel;
   // all_outputs: also the intermediate t_2ave (a substep called on its own)
-  void acoustic_substep(int it, bool all_outputs) const {
+  // bc: boundary copies to do along with u and v
+  void acoustic_substep(int it, bool all_outputs, const BcPart *bc = nullptr) const {
     X->iteration = it;
     const float dts = (float)X->dts_rk;
     R3 r{1, ide, 1, kde - 1, 1, jde};
-    k_uv_substep<<<g3(r), b3(), 0, s>>>(D(), dts, r);
+    const unsigned nuv = g3(r).x;
+    if (bc) k_uv_first<<<nuv + BcBatch::blocks(this, *bc), b3(), 0, s>>>(D(), dts, r, BcBatch::blocks(this, *bc), *bc);
+    else k_uv_substep<<<nuv, b3(), 0, s>>>(D(), dts, r);
     launch_acoustic_col(d, D(), s, dts, it == 1, it == X->nsmall, (float)X->nsmall, all_outputs || it == X->nsmall, 1);
   }
   // calc_mu_uv_1: the staggered column masses of muts
@@ -1061,8 +1096,8 @@ struct Run {
     memset(&fl, 0, sizeof(fl));
     for (int q = 1; q < X->c.nmoist; q++) fl.q[fl.n++] = Sp(F_moist, q);
     R3 m = mass3();
-    const unsigned nm = g3p(m).x, points = (unsigned)zone_n(zd('t', false, false)) * (unsigned)(kde - 1) * (unsigned)fl.n;
-    k_p_rho_phi_flow<<<nm + (points + 255u) / 256u, b3(), 0, s>>>(D(), m, nm, fl);
+    const unsigned nf = ((unsigned)zone_n(zd('t', false, false)) * (unsigned)(kde - 1) * (unsigned)fl.n + 255u) / 256u;
+    k_p_rho_phi_flow<<<nf + g3p(m).x, b3(), 0, s>>>(D(), m, nf, fl);
   }
 
   // one stage of scalar transport with recorded dynamics (tangent-linear =
@@ -1162,22 +1197,22 @@ struct Run {
 
   void rk_stage() const {
     rk_step_prep();
-    {
-      BcBatch b(this);
-      phys_bc_dry_1(b).add3(F(F_al), 'p').add3(F(F_ph_2), 'w');
-    }
+    BcBatch b1(this);
+    phys_bc_dry_1(b1).add3(F(F_al), 'p').add3(F(F_ph_2), 'w');
     if (X->rk == 1) {
-      first_rk_step_part1(false);
-      first_rk_step_part2(false, true);
+      first_stage_clears(b1.take());
+      first_rk_step_part2(false, true);  // rho comes with the diffusion metrics
+    } else {
+      b1.flush();
     }
     fused_tendency();
     small_step_prep(true);
     coef_p_rho();
-    BcBatch(this)
-        .add3(F(F_ru_tend), 'u').add3(F(F_rv_tend), 'v').add3(F(F_ph_2), 'w').add3(F(F_al), 'p').add3(F(F_p), 'p')
-        .add3(F(F_t_1), 'p').add3(F(F_t_save), 't').add2(F(F_mu_1), 't').add2(F(F_mu_2), 't').add2(F(F_mudf), 't')
-        .flush();
-    for (int it = 1; it <= X->nsmall; it++) acoustic_substep(it, false);
+    BcBatch b2(this);
+    b2.add3(F(F_ru_tend), 'u').add3(F(F_rv_tend), 'v').add3(F(F_ph_2), 'w').add3(F(F_al), 'p').add3(F(F_p), 'p')
+        .add3(F(F_t_1), 'p').add3(F(F_t_save), 't').add2(F(F_mu_1), 't').add2(F(F_mu_2), 't').add2(F(F_mudf), 't');
+    const BcPart part = b2.take();
+    for (int it = 1; it <= X->nsmall; it++) acoustic_substep(it, false, it == 1 ? &part : nullptr);
     small_step_finish();
     if (X->rk == 3)
       BcBatch(this).add3(F(F_ru_m), 'u').add3(F(F_rv_m), 'v').add3(F(F_ww_m), 'w').add2(F(F_mut), 't').add2(F(F_muts), 't').flush();
