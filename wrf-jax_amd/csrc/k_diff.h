@@ -522,9 +522,10 @@ struct HdsList {
 // pass 1: H1 at u faces i [2, ide-1], j [2, jde-2] and H2 at v faces
 // i [2, ide-2], j [2, jde-1] of every scalar; r = i [2, ide-1], k [1, kde-1],
 // j [2, jde-1]
-__global__ void __launch_bounds__(256) k_hdiff_s_faces(const DevCtx *xv, HdsList L, R3 r) {
+__global__ void __launch_bounds__(256) k_hdiff_s_faces(const DevCtx *xv, HdsList L, int per, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
+  SPECIES_RANGE;
   const int ide = x->ide, jde = x->jde;
   const bool f1 = (i <= ide - 1 && j <= jde - 2), f2 = (i <= ide - 2 && j <= jde - 1);
   const unsigned o = XI3(i, k, j);
@@ -535,7 +536,7 @@ __global__ void __launch_bounds__(256) k_hdiff_s_faces(const DevCtx *xv, HdsList
   const float fm0 = A1(FL(fnm), k), fp0 = A1(FL(fnp), k), fm1 = A1(FL(fnm), k1), fp1 = A1(FL(fnp), k1);
   const float dnw1 = A1(FL(dnw), kde - 1), dn1 = A1(FL(dn), kde - 1);
   const unsigned nb = (unsigned)x->n3, sk = (unsigned)x->ip, sj = (unsigned)(kde * x->ip);
-  for (int s = 0; s < L.n; s++) {
+  for (int s = sp0; s < sp1; s++) {
     // levels k-1 .. k+2 of the point's column and of its west and south
     // neighbours, all loaded first (buffer loads: the levels outside the
     // column read 0 and are not used)
@@ -561,9 +562,10 @@ __global__ void __launch_bounds__(256) k_hdiff_s_faces(const DevCtx *xv, HdsList
 
 // pass 2: tendency of every scalar on mass points i [2, ide-2], j [2, jde-2],
 // k [1, kde-1] (r)
-__global__ void __launch_bounds__(256) k_hdiff_s_tend(const DevCtx *xv, HdsList L, R3 r) {
+__global__ void __launch_bounds__(256) k_hdiff_s_tend(const DevCtx *xv, HdsList L, int per, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
   GET_IKJ(r);
+  SPECIES_RANGE;
   const float *zx = FL(zx), *zy = FL(zy), *rdzw = FL(rdzw), *fnm = FL(fnm), *fnp = FL(fnp);
   const int ktf = x->kde - 1;
   const float zxm = 0.25f * (A3(zx, i, k, j) + A3(zx, i + 1, k, j) + A3(zx, i, k + 1, j) + A3(zx, i + 1, k + 1, j));
@@ -577,7 +579,7 @@ __global__ void __launch_bounds__(256) k_hdiff_s_tend(const DevCtx *xv, HdsList 
   const float fm0 = A1(fnm, k), fp0 = A1(fnp, k), fm1 = A1(fnm, k + 1), fp1 = A1(fnp, k + 1);
   const unsigned o = XI3(i, k, j), sk = (unsigned)x->ip, sj = (unsigned)(x->kde * x->ip);
   const unsigned nb = (unsigned)x->n3;
-  for (int s = 0; s < L.n; s++) {
+  for (int s = sp0; s < sp1; s++) {
     // every load of this scalar first (buffer loads: the level below 1 and
     // above kde-1 read 0 and are not used)
     const BufF b1 = bufv(L.h1[s], nb), b2 = bufv(L.h2[s], nb);

@@ -65,11 +65,12 @@ __device__ __forceinline__ UpdCoef upd_coef(CtxPtr x, int i, int k, int j) {
 // c2h), so the last stage finds the same q_old and a cleared tendency.  Each
 // thread reads q_old and the tendency at its own point only, so updating them
 // in place is race-free.
-__global__ void __launch_bounds__(64 * kFaceRows) k_species_update(const DevCtx *xv, SpecList L, int rk, float dt, R3 r) {
+__global__ void __launch_bounds__(64 * kFaceRows) k_species_update(const DevCtx *xv, SpecList L, int per, int rk, float dt, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
-  extern __shared__ float ys_[];  // L.n x kFaceRows x 64: south face flux of every species
+  extern __shared__ float ys_[];  // per x kFaceRows x 64: south face flux of every species
   GET_FACE_BLOCK(r);
-#define YS(s, w) ys_[((s) * kFaceRows + (w)) * 64 + lane]
+  SPECIES_RANGE;
+#define YS(s, w) ys_[(((s) - sp0) * kFaceRows + (w)) * 64 + lane]
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const float *ru = FL(ru_m), *rv = FL(rv_m), *rom = FL(ww_m);
   const unsigned nb = (unsigned)x->n3, sj = (unsigned)(kde * x->ip), sk = (unsigned)x->ip;
@@ -79,7 +80,7 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_species_update(const DevCtx 
     const bool yf = (j >= 2 && j <= jde - 1);
     const float vs = yf ? A3(rv, ic, k, j) : 0.f;
     const unsigned os = XI3(ic, k, j);
-    for (int s = 0; s < L.n; s++) {
+    for (int s = sp0; s < sp1; s++) {
       float w[6];
       win6b(bufv(L.in[s], nb), os, sj, w);
       pin6(w);
@@ -99,7 +100,7 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_species_update(const DevCtx 
   const unsigned o = XI3(ic, k, j), ox = XI3(i, k, j);
   const int k1 = imin_(k + 1, kde);
   const float fm0 = A1(FL(fnm), k), fp0 = A1(FL(fnp), k), fm1 = A1(FL(fnm), k1), fp1 = A1(FL(fnp), k1);
-  for (int s = 0; s < L.n; s++) {
+  for (int s = sp0; s < sp1; s++) {
     const BufF bq = bufv(L.in[s], nb);
     // every load of this species first: x stencil of the west face, the
     // column window k-2 .. k+2 of both vertical faces, tendency and old
@@ -227,12 +228,13 @@ __device__ __forceinline__ void pd_vflux_sel(const PdFace &f, float qm2, float q
 // Face-sharing blocks as k_species_update: the west face comes from this
 // lane, the east face from the next lane, the south face from this wave and
 // the north face from the wave above (LDS).
-__global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_scale(const DevCtx *xv, SpecList L, float dt, R3 r) {
+__global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_scale(const DevCtx *xv, SpecList L, int per, float dt, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
-  extern __shared__ float yal_[];  // 2 x L.n x kFaceRows x 64: south antidiffusive / upwind flux of every species
+  extern __shared__ float yal_[];  // 2 x per x kFaceRows x 64: south antidiffusive / upwind flux of every species
   GET_FACE_BLOCK_LG(r, (unsigned)x->face_lg[2]);
-#define YA(s, w) yal_[((s) * kFaceRows + (w)) * 64 + lane]
-#define YL(s, w) yal_[((L.n + (s)) * kFaceRows + (w)) * 64 + lane]
+  SPECIES_RANGE;
+#define YA(s, w) yal_[(((s) - sp0) * kFaceRows + (w)) * 64 + lane]
+#define YL(s, w) yal_[((per + (s) - sp0) * kFaceRows + (w)) * 64 + lane]
   const int ide = x->ide, jde = x->jde, kde = x->kde;
   const unsigned nb = (unsigned)x->n3, sj = (unsigned)(kde * x->ip), sk = (unsigned)x->ip;
   {
@@ -240,7 +242,7 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_scale(const DevCt
     // it); its window may fall outside the field, the face is then 0
     const PdFace fs = pd_face_geom(x, 1, ic, k, j, dt);
     const unsigned os = XI3(ic, k, j);
-    for (int s = 0; s < L.n; s++) {
+    for (int s = sp0; s < sp1; s++) {
       const BufF bo = bufv(L.old[s], nb);
       float w[6], a, l;
       win6b(bufv(L.in[s], nb), os, sj, w);
@@ -265,7 +267,7 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_scale(const DevCt
   const int k1 = imin_(k + 1, kde);
   const float fm0 = A1(FL(fnm), k), fp0 = A1(FL(fnp), k), fm1 = A1(FL(fnm), k1), fp1 = A1(FL(fnp), k1);
   const unsigned ox = XI3(i, k, j);
-  for (int s = 0; s < L.n; s++) {
+  for (int s = sp0; s < sp1; s++) {
     const BufF bq = bufv(L.in[s], nb), bo = bufv(L.old[s], nb);
     // every load of this species first: x stencil of the west face, the
     // column windows of both vertical faces and the north face stencil (top
@@ -320,18 +322,19 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_scale(const DevCt
 // fluxes are formed again as in pass 1 (face-sharing blocks over the mass
 // points, the same loads and arithmetic, so the same values); each
 // antidiffusive flux is scaled by the factor of the cell it leaves.
-__global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_update(const DevCtx *xv, SpecList L, float dt, R3 r) {
+__global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_update(const DevCtx *xv, SpecList L, int per, float dt, R3 r) {
   const CtxPtr x = ctx_ptr(xv);
-  extern __shared__ float yal_[];  // 2 x L.n x kFaceRows x 64: south antidiffusive / upwind flux of every species
+  extern __shared__ float yal_[];  // 2 x per x kFaceRows x 64: south antidiffusive / upwind flux of every species
   GET_FACE_BLOCK_LG(r, (unsigned)x->face_lg[2]);
-#define YA(s, w) yal_[((s) * kFaceRows + (w)) * 64 + lane]
-#define YL(s, w) yal_[((L.n + (s)) * kFaceRows + (w)) * 64 + lane]
+  SPECIES_RANGE;
+#define YA(s, w) yal_[(((s) - sp0) * kFaceRows + (w)) * 64 + lane]
+#define YL(s, w) yal_[((per + (s) - sp0) * kFaceRows + (w)) * 64 + lane]
   const int kde = x->kde;
   const unsigned nb = (unsigned)x->n3, sj = (unsigned)(kde * x->ip), sk = (unsigned)x->ip;
   {
     const PdFace fs = pd_face_geom(x, 1, ic, k, j, dt);
     const unsigned os = XI3(ic, k, j);
-    for (int s = 0; s < L.n; s++) {
+    for (int s = sp0; s < sp1; s++) {
       const BufF bo = bufv(L.old[s], nb);
       float w[6], a, l;
       win6b(bufv(L.in[s], nb), os, sj, w);
@@ -353,7 +356,7 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_species_pd_update(const DevC
   const PdFace fz0 = pd_face_geom(x, 2, ic, k, j, dt), fz1 = pd_face_geom(x, 2, ic, k + 1, j, dt);
   const int k1 = imin_(k + 1, kde);
   const float fm0 = A1(FL(fnm), k), fp0 = A1(FL(fnp), k), fm1 = A1(FL(fnm), k1), fp1 = A1(FL(fnp), k1);
-  for (int s = 0; s < L.n; s++) {
+  for (int s = sp0; s < sp1; s++) {
     const BufF bq = bufv(L.in[s], nb), bo = bufv(L.old[s], nb), bs = bufv(L.scale[s], nb);
     float xw[6], yw[6], zw[5], zo[3];
     win6b(bq, ox, 1u, xw);

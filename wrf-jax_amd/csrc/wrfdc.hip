@@ -666,9 +666,11 @@ struct Run {
     for (int q = 0; q < X->c.nmoist; q++) add(Sp(F_moist, q), Sp(F_moist_tend, q));
     for (int q = 0; q < X->c.nscalar; q++) add(Sp(F_scalar, q), Sp(F_scalar_tend, q));
     const R3 rf{2, ide - 1, 1, kde - 1, 2, jde - 1};
-    k_hdiff_s_faces<<<g3(rf), b3(), 0, s>>>(D(), L, rf);
+    const int pf = species_per(g3(rf).x, L.n);
+    k_hdiff_s_faces<<<dim3(g3(rf).x, cdiv(L.n, pf)), b3(), 0, s>>>(D(), L, pf, rf);
     const R3 rt{2, ide - 2, 1, kde - 1, 2, jde - 2};
-    k_hdiff_s_tend<<<g3(rt), b3(), 0, s>>>(D(), L, rt);
+    const int pt = species_per(g3(rt).x, L.n);
+    k_hdiff_s_tend<<<dim3(g3(rt).x, cdiv(L.n, pt)), b3(), 0, s>>>(D(), L, pt, rt);
   }
   void horizontal_diffusion_2() const {
     const R3 full = full3();
@@ -1077,10 +1079,16 @@ struct Run {
         for (int q = 0; q < pd.n; q++) bc.add3(pd.old[q], 'p');
       }
       R3 r = full3();
-      k_species_pd_scale<<<dim3(face_tiles(r, d.face_lg[2]).count()), bf(), sizeof(float) * 2 * 64 * kFaceRows * pd.n, s>>>(D(), pd, dt, r);
-      k_species_pd_update<<<dim3(face_tiles(m, d.face_lg[2]).count()), bf(), sizeof(float) * 2 * 64 * kFaceRows * pd.n, s>>>(D(), pd, dt, m);
+      const unsigned ts = face_tiles(r, d.face_lg[2]).count(), tu = face_tiles(m, d.face_lg[2]).count();
+      const int ps = species_per(ts, pd.n), pu = species_per(tu, pd.n);
+      k_species_pd_scale<<<dim3(ts, cdiv(pd.n, ps)), bf(), sizeof(float) * 2 * 64 * kFaceRows * ps, s>>>(D(), pd, ps, dt, r);
+      k_species_pd_update<<<dim3(tu, cdiv(pd.n, pu)), bf(), sizeof(float) * 2 * 64 * kFaceRows * pu, s>>>(D(), pd, pu, dt, m);
     }
-    if (plain.n > 0) k_species_update<<<dim3(face_tiles(m, d.face_lg[0]).count()), bf(), sizeof(float) * 64 * kFaceRows * plain.n, s>>>(D(), plain, rk, dt, m);
+    if (plain.n > 0) {
+      const unsigned t = face_tiles(m, d.face_lg[0]).count();
+      const int per = species_per(t, plain.n);
+      k_species_update<<<dim3(t, cdiv(plain.n, per)), bf(), sizeof(float) * 64 * kFaceRows * per, s>>>(D(), plain, per, rk, dt, m);
+    }
     // outputs become the current species
     use_species(out_alt);
     if (rk == 3) {

@@ -245,3 +245,19 @@ __device__ __forceinline__ float div_const(float xv, float c, float rc) {
 }
 __device__ __forceinline__ int imin_(int a, int b) { return a < b ? a : b; }
 __device__ __forceinline__ int imax_(int a, int b) { return a > b ? a : b; }
+
+// The species of a block of the species kernels and of the scalar diffusion:
+// blockIdx.y's share of per of the list.  One share where the tiles fill the
+// chip, so that the geometry of a point is formed once for all species.  On a
+// small domain the species follow one another in each of a few blocks, about
+// 1 us apiece, and are dealt to blocks of their own until there are
+// kSpeciesBlocks.  The line is at 8 blocks per CU: a 24x20x10 step takes 323 us
+// with 2048 (367 undealt), 325 with 512; 100x100x45 (2250 tiles) 971 undealt,
+// 996 dealt to 9000, 1070 to 18000; 257x131x37 1822 against 1847 dealt.
+#define SPECIES_RANGE const int sp0 = (int)blockIdx.y * per, sp1 = imin_(sp0 + per, L.n)
+constexpr int kSpeciesBlocks = 2048;
+__host__ inline int species_per(unsigned tiles, int n) {
+  const int fit = tiles > 0 ? kSpeciesBlocks / (int)tiles : 1;  // shares that still fit
+  const int shares = fit < 1 ? 1 : fit < n ? fit : n;
+  return shares > 0 ? (n + shares - 1) / shares : 1;
+}
