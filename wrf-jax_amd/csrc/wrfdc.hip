@@ -69,6 +69,18 @@ __global__ void __launch_bounds__(256) k_copy_batch(const DevCtx *xv, CopyList L
   }
 }
 
+// column ide and row jde only, k <= kde-1: blockIdx.x over the longer edge,
+// y the level, z the pair
+__global__ void __launch_bounds__(64) k_copy_ring(const DevCtx *xv, CopyList L) {
+  const CtxPtr x = ctx_ptr(xv);
+  const int ide = x->ide, jde = x->jde;
+  const int a = 1 + (int)(blockIdx.x * 64u + threadIdx.x), k = 1 + (int)blockIdx.y;
+  float *dst = L.dst[blockIdx.z];
+  const float *src = L.src[blockIdx.z];
+  if (a <= jde) A3(dst, ide, k, a) = A3(src, ide, k, a);
+  if (a < ide) A3(dst, a, k, jde) = A3(src, a, k, jde);
+}
+
 // FP64 checksums over mass points (WRFDC_NCHECKSUMS values):
 // [0] sum(mu_2 + mub), [1] sum(t_2), [2] sum of all moist species,
 // [3] count of non-finite prognostic values,
@@ -981,7 +993,7 @@ struct Run {
   // k <= kde-1, j <= jde) into the other buffer and switch to it
   void species_to(bool alt) const {
     if (species_in_alt() == alt) return;
-    copy_species(R3{1, ide, 1, kde - 1, 1, jde}, alt);
+    copy_batch(species_copies(alt), R3{1, ide, 1, kde - 1, 1, jde});
     use_species(alt);
   }
   // one launch of k_copy_batch over r for the pairs of L
@@ -990,7 +1002,7 @@ struct Run {
     const unsigned gi = (unsigned)(r.i1 - r.i0 + 256) / 256u, gk = (unsigned)(r.k1 - r.k0 + 4) / 4u;
     k_copy_batch<<<dim3(gi * gk, (unsigned)(r.j1 - r.j0 + 1), (unsigned)L.n), dim3(64, 4), 0, s>>>(D(), L, r);
   }
-  void copy_species(R3 r, bool to_alt) const {
+  CopyList species_copies(bool to_alt) const {
     const size_t n = X->n3;
     const float *sm = to_alt ? user_moist : alt_moist, *ss = to_alt ? user_scalar : alt_scalar;
     float *dm = to_alt ? alt_moist : user_moist, *ds = to_alt ? alt_scalar : user_scalar;
@@ -1004,7 +1016,7 @@ struct Run {
       L.dst[L.n] = ds + q * n;
       L.src[L.n++] = ss + q * n;
     }
-    copy_batch(L, r);
+    return L;
   }
   void fill_copy(float *dst, const float *src, size_t n) const {
     unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, 8192);
@@ -1073,10 +1085,10 @@ struct Run {
       for (int q = 0; q < pd.n; q++) {
         pd.scale[q] = X->spec_scale + (size_t)q * n3;
       }
-      if (!pd_prepped) k_species_pd_prep<<<g3p(m), b3(), 0, s>>>(D(), pd, dt, m);
-      {
+      if (!pd_prepped) {
+        k_species_pd_prep<<<g3p(m), b3(), 0, s>>>(D(), pd, dt, m);
         BcBatch bc(this);
-        for (int q = 0; q < pd.n; q++) bc.add3(pd.old[q], 'p');
+        add_pd_old(bc);
       }
       R3 r = full3();
       const unsigned ts = face_tiles(r, d.face_lg[2]).count(), tu = face_tiles(m, d.face_lg[2]).count();
@@ -1094,8 +1106,8 @@ struct Run {
     if (rk == 3) {
       // the physical-boundary ring (column ide, row jde) is last written by
       // the second stage's copies, which went to the other buffer
-      copy_species(R3{ide, ide, 1, kde - 1, 1, jde}, false);
-      copy_species(R3{1, ide, 1, kde - 1, jde, jde}, false);
+      const CopyList L = species_copies(false);
+      if (L.n > 0) k_copy_ring<<<dim3(cdiv(std::max(ide, jde), 64), kde - 1, L.n), 64, 0, s>>>(D(), L);
     }
   }
   // flow_dep_bdy of the species beyond QV, with calc_p_rho_phi
@@ -1203,11 +1215,23 @@ struct Run {
   }
   void set_w_surface() const { k_set_w_surface<<<dim3(cdiv(ide - 1, 64), jde - 1), 64, 0, s>>>(D()); }
 
-  void rk_stage() const {
+  // the old species of the last stage's PD list
+  void add_pd_old(BcBatch &b) const {
+    for (int q = 0; q < X->c.nmoist; q++)
+      if (X->c.pd_moist) b.add3(Sp(F_moist_old, q), 'p');
+    for (int q = 0; q < X->c.nscalar; q++)
+      if (X->c.pd_scalar) b.add3(Sp(F_scalar_old, q), 'p');
+  }
+
+  // moist_old_bc: the first stage does the boundary copies of the old moist
+  // species too, along with its own (nothing before them reads those points)
+  void rk_stage(bool moist_old_bc = false) const {
     rk_step_prep();
     BcBatch b1(this);
     phys_bc_dry_1(b1).add3(F(F_al), 'p').add3(F(F_ph_2), 'w');
     if (X->rk == 1) {
+      if (moist_old_bc)
+        for (int q = 0; q < X->c.nmoist; q++) b1.add3(Sp(F_moist_old, q), 'p');
       first_stage_clears(b1.take());
       first_rk_step_part2(false, true);  // rho comes with the diffusion metrics
     } else {
@@ -1222,8 +1246,11 @@ struct Run {
     const BcPart part = b2.take();
     for (int it = 1; it <= X->nsmall; it++) acoustic_substep(it, false, it == 1 ? &part : nullptr);
     small_step_finish();
-    if (X->rk == 3)
-      BcBatch(this).add3(F(F_ru_m), 'u').add3(F(F_rv_m), 'v').add3(F(F_ww_m), 'w').add2(F(F_mut), 't').add2(F(F_muts), 't').flush();
+    if (X->rk == 3) {
+      BcBatch b(this);
+      b.add3(F(F_ru_m), 'u').add3(F(F_rv_m), 'v').add3(F(F_ww_m), 'w').add2(F(F_mut), 't').add2(F(F_muts), 't');
+      if (pd_prepped) add_pd_old(b);  // formed by the second stage's update
+    }
     const int nm = X->c.nmoist, nsc = X->c.nscalar;
     record_stage();
     species_stage();
@@ -1246,12 +1273,9 @@ struct Run {
     if (species_in_alt()) species_to(false);
     // initialize_moist_old (module_big_step_utilities_em.py:935-975); the
     // scalars' q_old <- q of the first-stage update is done here as well
-    // (one copy launch), then the moist q_old's boundary update
+    // (one copy launch); the moist q_old's boundary update comes with the
+    // first stage's
     sync_old(true, true);
-    {
-      BcBatch bc(this);
-      for (int q = 0; q < X->c.nmoist; q++) bc.add3(Sp(F_moist_old, q), 'p');
-    }
     old_synced = true;
     struct FoldScope {  // cleared however the stages end
       const Run *r;
@@ -1260,7 +1284,7 @@ struct Run {
     } fold(this);
     for (int rk = 1; rk <= 3; rk++) {
       set_rk(rk);
-      rk_stage();
+      rk_stage(rk == 1);
     }
     {
       BcBatch b(this);
