@@ -80,7 +80,7 @@ KERNELS = {
                                 writes=("al", "p", "pm1")),
     "k_rhs_ph": KernelModel("k_rhs_ph", "rhs_ph", 2, 0, reads=("u_2", "v_2", "ww", "ph_2", "phb", "w_2", "ph_tend"),
                             writes=("ph_tend",)),
-    # kernels of the step's fused path (a stage name only where one launches
+    # kernels of the step's fused path; k_tendency<0> to <4> are u, v, w, theta and phi (a stage name only where one launches
     # the kernel alone); the species kernels carry every species of a stage
     # q in, q_old, tendency, q out; at rk 2 also q_old' and the cleared
     # tendency of every PD species (the last stage's rk_update_scalar_pd):
@@ -93,30 +93,30 @@ KERNELS = {
     "k_species_pd_update": KernelModel("k_species_pd_update", "", 3, 0, reads=("ru_m", "rv_m", "ww_m"), writes=(),
                                        per_species=4),  # q in, q_old, factor, q out
     "k_advect_u": KernelModel("k_advect_u", "advect_u", 2, 0, reads=("u_2", "ru", "rv", "ww", "ru_tend"), writes=("ru_tend",)),
-    "k_advect_u<true>": KernelModel("k_advect_u<true>", "", 2, 0,
+    "k_tendency<0>": KernelModel("k_tendency<0>", "", 2, 0,
                                     reads=("u_2", "ru", "rv", "ww", "ph_2", "php", "alt", "al", "p", "pb", "v_2", "w_2", "ru_tendf",
                                            "u_save"), writes=("ru_tend",)),
-    "k_advect_v<true>": KernelModel("k_advect_v<true>", "", 2, 0,
+    "k_tendency<1>": KernelModel("k_tendency<1>", "", 2, 0,
                                     reads=("v_2", "ru", "rv", "ww", "ph_2", "php", "alt", "al", "p", "pb", "u_2", "w_2", "rv_tendf",
                                            "v_save"), writes=("rv_tend",)),
-    "k_advect_w<true>": KernelModel("k_advect_w<true>", "", 2, 0,
+    "k_tendency<2>": KernelModel("k_tendency<2>", "", 2, 0,
                                     reads=("w_2", "ru", "rv", "ww", "t_2", "t_save", "alt", "al", "p", "pb", "cqw", "u_2", "v_2",
                                            "rw_tendf", "w_save"), writes=("rw_tend", "cqw")),
-    "k_advect_scalar<true>": KernelModel("k_advect_scalar<true>", "", 2, 0, reads=("t_2", "ru", "rv", "ww", "t_tendf", "t_save"),
+    "k_tendency<3>": KernelModel("k_tendency<3>", "", 2, 0, reads=("t_2", "ru", "rv", "ww", "t_tendf", "t_save"),
                                          writes=("t_tend",)),
-    "k_tend_ph": KernelModel("k_tend_ph", "", 2, 0, reads=("u_2", "v_2", "ww", "ph_2", "phb", "w_2", "ph_tendf", "ph_save"),
+    "k_tendency<4>": KernelModel("k_tendency<4>", "", 2, 0, reads=("u_2", "v_2", "ww", "ph_2", "phb", "w_2", "ph_tendf", "ph_save"),
                              writes=("ph_tend",)),
-    "k_rk_prep3": KernelModel("k_rk_prep3", "", 2, 0, reads=("u_2", "v_2", "w_2", "al", "alb", "phb", "ph_2"),
+    "k_rk_prep3<false>": KernelModel("k_rk_prep3<false>", "", 2, 0, reads=("u_2", "v_2", "w_2", "al", "alb", "phb", "ph_2"),
                               writes=("ru", "rv", "rw", "alt", "php", "cqu", "cqv", "cqw"), per_moist=1),
     "k_ssp_3d<false>": KernelModel("k_ssp_3d<false>", "", 2, 0,
                                    reads=("pb", "p", "alt", "u_2", "v_2", "t_2", "w_2", "ph_2", "ww", "u_1", "v_1", "t_1", "w_1",
                                           "ph_1"),
                                    writes=("c2a", "u_save", "u_2", "v_save", "v_2", "t_save", "t_2", "w_save", "w_2", "ph_save",
                                            "ph_2", "ww_1")),
-    "k_ssf<false>": KernelModel("k_ssf<false>", "", 2, 0,
+    "k_ssf<false, false>": KernelModel("k_ssf<false, false>", "", 2, 0,
                                 reads=("u_2", "u_save", "v_2", "v_save", "w_2", "w_save", "ph_2", "ph_save", "ww", "ww_1", "t_2",
                                        "t_save"), writes=("u_2", "v_2", "w_2", "ph_2", "ww", "t_2")),
-    "k_calc_p_rho_phi": KernelModel("k_calc_p_rho_phi", "calc_p_rho_phi", 2, 0, reads=("ph_2", "phb", "alb", "pb", "t_2"),
+    "k_p_rho_phi_flow": KernelModel("k_p_rho_phi_flow", "calc_p_rho_phi", 2, 0, reads=("ph_2", "phb", "alb", "pb", "t_2"),
                                     writes=("al", "p"), per_moist=0),
     "k_hdiff_s_faces": KernelModel("k_hdiff_s_faces", "", 1, 0, reads=("xkhh", "rho", "zx", "zy", "rdzw"), writes=(),
                                    per_scalar_diffused=3),  # q in, H1 and H2 out
