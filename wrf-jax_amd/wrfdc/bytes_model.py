@@ -113,7 +113,7 @@ KERNELS = {
                                           "ph_1"),
                                    writes=("c2a", "u_save", "u_2", "v_save", "v_2", "t_save", "t_2", "w_save", "w_2", "ph_save",
                                            "ph_2", "ww_1")),
-    "k_ssf<false, false>": KernelModel("k_ssf<false, false>", "", 2, 0,
+    "k_ssf<false, true>": KernelModel("k_ssf<false, true>", "", 2, 0,
                                 reads=("u_2", "u_save", "v_2", "v_save", "w_2", "w_save", "ph_2", "ph_save", "ww", "ww_1", "t_2",
                                        "t_save"), writes=("u_2", "v_2", "w_2", "ph_2", "ww", "t_2")),
     "k_p_rho_phi_flow": KernelModel("k_p_rho_phi_flow", "calc_p_rho_phi", 2, 0, reads=("ph_2", "phb", "alb", "pb", "t_2"),
