@@ -84,9 +84,12 @@ __device__ __forceinline__ void ad_face(const float t[7], const float ms[7], con
     fb = 0.f;
     if (f <= e - 2) fb += hi;
     if (f - 1 >= 2) fb -= lo;
-    const float c2 = (M == -1 || M == 0) ? 0.5f : 0.f;
-    coef = (f >= 4 && f <= e - 3) ? coef : ((f == 2 || f == e - 1) ? c2 : coef3<M>(up));
-    if (f < 2 || f > e - 1) return;
+    const bool five = f >= 4 && f <= e - 3, two = f == 2 || f == e - 1;
+    constexpr bool in2 = M == -1 || M == 0, in3 = M >= -2 && M <= 1;  // cells a 2nd- / 3rd-order flux reads
+    coef = five ? coef : two ? 0.5f : coef3<M>(up);
+    // a face whose flux does not read c adds nothing: 0 times its values would
+    // not be 0 where they are infinite or NaN
+    if (f < 2 || f > e - 1 || !(five || (two ? in2 : in3))) return;
   }
   acc += vel * coef * fb;
 }
