@@ -286,6 +286,42 @@ wrfdc_ctx *make_ctx(int nx, int ny, int nz, int nmoist = 3, int nscalar = 1) {
   return x;
 }
 
+// The kernels' context in device memory: uploaded when it changed, on the stream
+// that reads it, and again after an upload that could not be launched.
+void context_upload() {
+  wrfdc_ctx *x = make_ctx(24, 20, 10);
+  hipStream_t other;
+  CHECK(hipStreamCreateWithFlags(&other, hipStreamNonBlocking) == hipSuccess);
+  auto uploads = [&](hipStream_t s) {
+    rt::log_.clear();
+    const int rc = wrfdc_step(x, 1, 0.0);
+    const bool first = !rt::log_.empty() && rt::log_[0].name == "k_put_ctx";
+    const long n = rt::count("k_put_ctx", s);
+    CHECK(n == 0 || first);
+    return rc == WRFDC_OK ? n : -1;
+  };
+  CHECK(uploads(nullptr) == 2);
+  CHECK(uploads(nullptr) == 0);
+  wrfdc_bind(x, "t_2", g_field + 1);
+  CHECK(uploads(nullptr) == 2);
+  for (long n : {0, 1}) {  // the first or the second of the two
+    wrfdc_bind(x, "t_2", g_field + 2 + n);
+    rt::fail_name = "k_put_ctx";
+    rt::fail_left = n;
+    CHECK(uploads(nullptr) == -1);
+    CHECK(rt::count("k_uv_first", nullptr) == 0);  // nothing ran on the stale context
+    CHECK(uploads(nullptr) == 2);
+  }
+  CHECK(wrfdc_set_stream(x, other) == WRFDC_OK);
+  CHECK(uploads(other) == 2);
+  CHECK(wrfdc_set_stream(x, other) == WRFDC_OK);
+  CHECK(uploads(other) == 0);
+  CHECK(wrfdc_set_stream(x, nullptr) == WRFDC_OK);
+  CHECK(uploads(nullptr) == 2);
+  CHECK(hipStreamSynchronize(other) == hipSuccess && hipStreamDestroy(other) == hipSuccess);
+  wrfdc_destroy(x);
+}
+
 // An ensemble's streams, events and graph: each created once, used while
 // it lives, destroyed once, after its work has been waited for.
 void ensemble_lifecycle() {
@@ -337,7 +373,9 @@ void ensemble_create_failures() {
 const struct {
   const char *name;
   void (*fn)();
-} kChecks[] = {{"ensemble_lifecycle", ensemble_lifecycle}, {"ensemble_create_failures", ensemble_create_failures}};
+} kChecks[] = {{"context_upload", context_upload},
+               {"ensemble_lifecycle", ensemble_lifecycle},
+               {"ensemble_create_failures", ensemble_create_failures}};
 }  // namespace
 
 int main(int argc, char **argv) {

@@ -337,7 +337,8 @@ struct Run {
 
   // Brings the device contexts up to date.  Eager work has a pair of its own,
   // written when something changed since the last call (a field bound
-  // elsewhere, a tile setting).  Captured work writes another pair at its
+  // elsewhere, a tile setting, the stream, which orders the upload before its
+  // readers).  Captured work writes another pair at its
   // start, so that a graph replays with what it was captured with, whatever
   // eager calls have set in between.
   const DevCtx *dev_ctx;  // the pair in use
@@ -354,8 +355,10 @@ struct Run {
     DevCtx *pair = X->ctx_dev + (capture ? 2 : 0);
     dev_ctx = pair;
     if (!capture && X->up_ok && memcmp(&X->up[0], &d, sizeof d) == 0 && memcmp(&X->up[1], &alt, sizeof alt) == 0) return;
+    if (!capture) X->up_ok = false;  // until both are on their way
     k_put_ctx<<<1, 256, 0, s>>>(d, pair);
     k_put_ctx<<<1, 256, 0, s>>>(alt, pair + 1);
+    hchk(hipGetLastError(), "context upload");
     if (capture) return;
     X->up[0] = d;
     X->up[1] = alt;
@@ -1729,6 +1732,7 @@ int wrfdc_bind(wrfdc_ctx *x, const char *name, void *device_ptr) {
 
 int wrfdc_set_stream(wrfdc_ctx *x, void *hip_stream) {
   if (!x) return WRFDC_EINVAL;
+  if (x->s != (hipStream_t)hip_stream) x->up_ok = false;  // Run::put_ctx ordered the last upload on the old stream only
   x->s = (hipStream_t)hip_stream;
   return WRFDC_OK;
 }
