@@ -22,8 +22,9 @@
 
 // ---- allocation failures -----------------------------------------------------
 static std::atomic<long> g_alloc_left{-1};  // the allocation that throws (counted down), -1 none
+static thread_local int t_inside = 0;           // in the runtime below, whose own allocations do not count
 void *operator new(size_t n) {
-  if (g_alloc_left.load() >= 0 && g_alloc_left.fetch_sub(1) == 0) throw std::bad_alloc();
+  if (!t_inside && g_alloc_left.load() >= 0 && g_alloc_left.fetch_sub(1) == 0) throw std::bad_alloc();
   if (void *p = std::malloc(n ? n : 1)) return p;
   throw std::bad_alloc();
 }
@@ -37,6 +38,10 @@ struct Launch {
   hipStream_t s;
 };
 std::recursive_mutex mu;
+struct Guard {
+  Guard() { mu.lock(), t_inside++; }
+  ~Guard() { t_inside--, mu.unlock(); }
+};
 std::map<const void *, std::string> kernels;
 std::vector<Launch> log_;
 std::map<void *, std::string> live;      // device and pinned memory, streams, events, graphs
@@ -45,13 +50,17 @@ std::map<hipEvent_t, hipStream_t> recorded;
 std::vector<std::string> errors;
 hipError_t last = hipSuccess;
 std::string fail_name;  // the call (or kernel) that fails ...
-long fail_left = -1;    // ... after this many successes, once
+long fail_left = -1;    // ... after this many successes
+long fail_times = 1;    // ... this many times
 long fail_any = -1;     // any call at all, after this many
 
 void error(const std::string &s) { errors.push_back(s); }
 bool fails(const std::string &name) {
   bool f = false;
-  if (fail_left >= 0 && name == fail_name) f = fail_left-- == 0;
+  if (fail_left >= 0 && name == fail_name) {
+    f = fail_left == 0;
+    if (fail_left > 0 || --fail_times <= 0) fail_left--;
+  }
   if (fail_any >= 0 && fail_any-- == 0) f = true;
   return f;
 }
@@ -94,8 +103,8 @@ long count(const std::string &name, hipStream_t s) {
   return std::count_if(log_.begin(), log_.end(), [&](const Launch &l) { return l.name == name && l.s == s; });
 }
 }  // namespace rt
-#define RT(name)                                       \
-  std::lock_guard<std::recursive_mutex> guard(rt::mu); \
+#define RT(name)   \
+  rt::Guard guard; \
   if (rt::fails(name)) return rt::fail()
 
 extern "C" {
@@ -121,7 +130,7 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **, size_t, hipStream_t s) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   const std::string name = rt::kernels.at(f);
   if (rt::fails(name)) return rt::fail(hipErrorLaunchFailure);
   if (!rt::stream_ok(s)) return rt::fail(hipErrorInvalidHandle);
@@ -131,13 +140,17 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **, size_t, hipStre
   return hipSuccess;
 }
 hipError_t hipGetLastError(void) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   const hipError_t e = rt::last;
   rt::last = hipSuccess;
   return e;
 }
 const char *hipGetErrorString(hipError_t) { return "failed"; }
-hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
+hipError_t hipGetDevice(int *d) {
+  RT("hipGetDevice");
+  *d = 0;
+  return hipSuccess;
+}
 hipError_t hipSetDevice(int) { RT("hipSetDevice"); return hipSuccess; }
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { RT("hipFuncSetAttribute"); return hipSuccess; }
 hipError_t hipGetSymbolAddress(void **, const void *) { return rt::fail(); }
@@ -147,7 +160,7 @@ hipError_t hipMalloc(void **p, size_t n) {
   return hipSuccess;
 }
 hipError_t hipFree(void *p) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   return p ? rt::drop(p, "device memory") : hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
@@ -156,7 +169,7 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   return hipSuccess;
 }
 hipError_t hipHostFree(void *p) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   return rt::drop(p, "pinned memory");
 }
 hipError_t hipMemcpyAsync(void *d, const void *h, size_t n, hipMemcpyKind, hipStream_t s) {
@@ -168,20 +181,20 @@ hipError_t hipMemcpyAsync(void *d, const void *h, size_t n, hipMemcpyKind, hipSt
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { RT("hipStreamCreateWithFlags"); return rt::make(s, "stream"); }
 hipError_t hipStreamDestroy(hipStream_t s) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   if (rt::busy.count(s)) rt::error("stream destroyed with work in flight");
   if (rt::capturing.count(s)) rt::error("stream destroyed while it captures");
   return rt::drop(s, "stream");
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   rt::busy.erase(s);
   if (rt::fails("hipStreamSynchronize")) return rt::fail();
   if (rt::capturing.count(s)) rt::error("synchronised a stream that captures");
   return rt::stream_ok(s) ? hipSuccess : rt::fail();
 }
 hipError_t hipDeviceSynchronize(void) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   rt::busy.clear();
   return rt::fails("hipDeviceSynchronize") ? rt::fail() : hipSuccess;
 }
@@ -196,7 +209,7 @@ hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
   return rt::stream_ok(s) ? hipSuccess : rt::fail();
 }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   if (!rt::capturing.count(s)) rt::error("ended a capture that was not begun");
   rt::capturing.clear();  // the streams that joined too
   *g = nullptr;
@@ -212,7 +225,7 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { RT("hipEventCreateWithFlags"); return rt::make(e, "event"); }
 hipError_t hipEventDestroy(hipEvent_t e) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   rt::recorded.erase(e);
   return rt::drop(e, "event");
 }
@@ -244,12 +257,12 @@ hipError_t hipGraphLaunch(hipGraphExec_t x, hipStream_t s) {
   return hipSuccess;
 }
 hipError_t hipGraphExecDestroy(hipGraphExec_t x) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   if (!rt::busy.empty()) rt::error("graph exec destroyed with work in flight");
   return rt::drop(x, "graph exec");
 }
 hipError_t hipGraphDestroy(hipGraph_t g) {
-  std::lock_guard<std::recursive_mutex> guard(rt::mu);
+  rt::Guard guard;
   return rt::drop(g, "graph");
 }
 }  // extern "C"
@@ -308,6 +321,7 @@ void context_upload() {
     wrfdc_bind(x, "t_2", g_field + 2 + n);
     rt::fail_name = "k_put_ctx";
     rt::fail_left = n;
+    rt::fail_times = 1;
     CHECK(uploads(nullptr) == -1);
     CHECK(rt::count("k_uv_first", nullptr) == 0);  // nothing ran on the stale context
     CHECK(uploads(nullptr) == 2);
@@ -319,6 +333,82 @@ void context_upload() {
   CHECK(wrfdc_set_stream(x, nullptr) == WRFDC_OK);
   CHECK(uploads(nullptr) == 2);
   CHECK(hipStreamSynchronize(other) == hipSuccess && hipStreamDestroy(other) == hipSuccess);
+  wrfdc_destroy(x);
+}
+
+// The transfers of host arrays: whatever fails, the call returns an error or
+// does without, nothing is in flight when it returns, and the next call works.
+struct Arrays {
+  std::vector<std::vector<float>> a;
+  std::vector<int> fields;
+  std::vector<void *> p;
+  Arrays(wrfdc_ctx *x) {
+    for (const char *name : {"moist", "u_2", "mu_2", "c1h", "t_bxs"})
+      for (int f = 0; f < wrfdc_field_count(); f++)
+        if (name == std::string(wrfdc_field_name(f))) {
+          const LayoutSeg g = layout_of(x, f);
+          fields.push_back(f);
+          a.emplace_back((size_t)g.ni * g.si);
+        }
+    for (auto &v : a) p.push_back(v.data());
+  }
+  int put(wrfdc_ctx *x) { return wrfdc_put_reference(x, (int)p.size(), fields.data(), p.data()); }
+  int get(wrfdc_ctx *x) { return wrfdc_get_reference(x, (int)p.size(), fields.data(), p.data()); }
+};
+void transfer_call_failures() {
+  for (int up = 0; up < 2; up++)
+    for (long n = 0;; n++) {
+      wrfdc_ctx *x = make_ctx(400, 90, 33, 6, 1);  // 35 MB of moist: a chunk for each worker
+      Arrays A(x);
+      rt::busy.clear();
+      rt::fail_any = n;
+      const int rc = up ? A.put(x) : A.get(x);
+      const bool failed = rt::fail_any < 0;
+      rt::fail_any = -1;
+      rt::last = hipSuccess;
+      CHECK(rc == WRFDC_OK || (failed && rc == WRFDC_EHIP));
+      CHECK(rt::busy.empty());
+      CHECK(A.put(x) == WRFDC_OK && A.get(x) == WRFDC_OK);
+      wrfdc_destroy(x);
+      if (!failed || n > 1000) break;
+    }
+}
+// No pinned memory, memory for one worker, memory for one small chunk: the
+// transfers work all the same; none at all: an error.
+void transfer_short_memory() {
+  const struct {
+    const char *call;
+    long after;
+    int rc;
+  } kinds[] = {{"hipHostMalloc", 0, WRFDC_OK}, {"hipMalloc", 1, WRFDC_OK}, {"hipMalloc", 0, WRFDC_OK}, {"hipMalloc", -1, WRFDC_EHIP}};
+  for (auto &k : kinds) {
+    wrfdc_ctx *x = make_ctx(400, 90, 33, 6, 1);
+    Arrays A(x);
+    rt::fail_name = k.call;
+    rt::fail_left = std::max(k.after, 0L);
+    rt::fail_times = k.after < 0 ? 2 : k.call == std::string("hipHostMalloc") ? 4 : 1;
+    CHECK(A.put(x) == k.rc);
+    rt::fail_left = -1;
+    rt::fail_times = 1;
+    rt::last = hipSuccess;
+    CHECK(A.put(x) == WRFDC_OK && A.get(x) == WRFDC_OK);
+    wrfdc_destroy(x);
+  }
+}
+// Every allocation of a transfer failing in turn, those of its threads among
+// them: an error or fewer threads, and no way out but the return.
+void transfer_allocation_failures() {
+  wrfdc_ctx *x = make_ctx(400, 90, 33, 6, 1);
+  Arrays A(x);
+  for (long n = 0;; n++) {
+    g_alloc_left = n;
+    const int rc = n % 2 ? A.put(x) : A.get(x);
+    const bool failed = g_alloc_left < 0;
+    g_alloc_left = -1;
+    CHECK(rc == WRFDC_OK || (failed && rc == WRFDC_EHIP));
+    CHECK(rt::busy.empty());
+    if (!failed || n > 1000) break;
+  }
   wrfdc_destroy(x);
 }
 
@@ -374,6 +464,9 @@ const struct {
   const char *name;
   void (*fn)();
 } kChecks[] = {{"context_upload", context_upload},
+               {"transfer_call_failures", transfer_call_failures},
+               {"transfer_short_memory", transfer_short_memory},
+               {"transfer_allocation_failures", transfer_allocation_failures},
                {"ensemble_lifecycle", ensemble_lifecycle},
                {"ensemble_create_failures", ensemble_create_failures}};
 }  // namespace

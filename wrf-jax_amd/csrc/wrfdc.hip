@@ -13,12 +13,13 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <initializer_list>
 #include <mutex>
 #include <utility>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -243,15 +244,17 @@ static const int kCkBlocks = 512;
 // device with that device current (noalloc_scratch below).
 static __device__ __align__(256) double scratch[kCkBlocks * CK_N];
 
-// Pinned and device chunks of the reference-layout transfers: one of each and
-// an event per worker thread, allocated at the first transfer of a context
-// and kept with it (4 x 8 MB each side, or the largest i row of an array if
-// that is more).
+// Host and device chunks of the reference-layout transfers: one of each and an
+// event per worker thread, allocated at the first transfer of a context and
+// kept with it (4 x 8 MB each side, or the largest i row of an array if that
+// is more; fewer workers or smaller chunks where memory is short).
 constexpr int kXferWorkers = 4;
 constexpr size_t kXferFloats = (size_t)2 << 20;
 struct Xfer {
-  size_t cap = 0;  // floats per chunk
-  float *pin[kXferWorkers] = {}, *dev[kXferWorkers] = {};
+  size_t cap = 0;   // floats per chunk
+  int workers = 0;  // that have their chunks
+  float *host[kXferWorkers] = {}, *dev[kXferWorkers] = {};
+  bool pinned[kXferWorkers] = {};
   hipEvent_t ev[kXferWorkers] = {};
 };
 
@@ -1472,13 +1475,48 @@ int wrfdc_field_count(void) { return NFIELDS; }
 const char *wrfdc_field_name(int index) { return (index >= 0 && index < NFIELDS) ? kNames[index] : nullptr; }
 int wrfdc_field_kind(int index) { return (index >= 0 && index < NFIELDS) ? (int)kKinds[index] : 0; }
 
-static void xfer_free(wrfdc_ctx *x) {
-  for (int w = 0; w < kXferWorkers; w++) {
-    if (x->xfer.pin[w]) (void)hipHostFree(x->xfer.pin[w]);
-    if (x->xfer.dev[w]) (void)hipFree(x->xfer.dev[w]);
-    if (x->xfer.ev[w]) (void)hipEventDestroy(x->xfer.ev[w]);
+static void xfer_free_worker(Xfer &X, int w) {
+  if (X.host[w] && X.pinned[w]) (void)hipHostFree(X.host[w]);
+  else std::free(X.host[w]);
+  if (X.dev[w]) (void)hipFree(X.dev[w]);
+  if (X.ev[w]) (void)hipEventDestroy(X.ev[w]);
+  X.host[w] = X.dev[w] = nullptr;
+  X.ev[w] = nullptr;
+}
+static void xfer_free(Xfer &X) {
+  for (int w = 0; w < X.workers; w++) xfer_free_worker(X, w);
+  X = Xfer{};
+}
+
+// Chunks of cap floats for as many workers as there is memory for, at least
+// one; pageable host memory where no pinned is to be had (slower transfers).
+static hipError_t xfer_alloc(Xfer &X, size_t cap) {
+  hipError_t e = hipSuccess;
+  for (int w = 0; w < kXferWorkers && e == hipSuccess; w++) {
+    e = hipMalloc((void **)&X.dev[w], cap * sizeof(float));
+    if (e != hipSuccess) X.dev[w] = nullptr;
+    if (e == hipSuccess) {
+      e = hipEventCreateWithFlags(&X.ev[w], hipEventDisableTiming);
+      if (e != hipSuccess) X.ev[w] = nullptr;
+    }
+    if (e == hipSuccess) {
+      X.pinned[w] = hipHostMalloc((void **)&X.host[w], cap * sizeof(float), hipHostMallocDefault) == hipSuccess;
+      if (!X.pinned[w]) {
+        (void)hipGetLastError();
+        X.host[w] = static_cast<float *>(std::malloc(cap * sizeof(float)));
+        if (!X.host[w]) e = hipErrorOutOfMemory;
+      }
+    }
+    if (e == hipSuccess) {
+      X.workers = w + 1;
+    } else {
+      (void)hipGetLastError();
+      xfer_free_worker(X, w);
+    }
   }
-  x->xfer = Xfer{};
+  if (X.workers == 0) return e;
+  X.cap = cap;
+  return hipSuccess;
 }
 
 int wrfdc_create(const wrfdc_config *cfg, wrfdc_ctx **out) {
@@ -1541,7 +1579,7 @@ void wrfdc_destroy(wrfdc_ctx *x) {
   if (x->spec_alt) (void)hipFree(x->spec_alt);
   if (x->spec_scale) (void)hipFree(x->spec_scale);
   if (x->hds) (void)hipFree(x->hds);
-  xfer_free(x);
+  xfer_free(x->xfer);
   delete x;
 }
 
@@ -1599,29 +1637,22 @@ static int xfer_reference(wrfdc_ctx *x, int n, const int *fields, void *const *h
   };
   return guarded(x, [&]() {
     try {
-      size_t cap = kXferFloats;
+      size_t need = 1;  // floats of the largest i row
       for (int q = 0; q < n; q++) {
         if (fields[q] < 0 || fields[q] >= NFIELDS) return set_err(x, WRFDC_EINVAL, "unknown field index");
         if (!host[q]) return set_err(x, WRFDC_EINVAL, std::string("null host array: ") + kNames[fields[q]]);
-        cap = std::max<size_t>(cap, layout_of(x, fields[q]).si);
+        need = std::max<size_t>(need, layout_of(x, fields[q]).si);
       }
       Xfer &X = x->xfer;
-      if (X.cap < cap) {
+      auto wait = [&]() { return x->s ? hipStreamSynchronize(x->s) : hipDeviceSynchronize(); };
+      if (X.cap < need) {
         if (X.cap) {
-          hchk(x->s ? hipStreamSynchronize(x->s) : hipDeviceSynchronize(), "transfer buffers");
-          xfer_free(x);
+          hchk(wait(), "transfer buffers");
+          xfer_free(X);
         }
-        try {
-          for (int w = 0; w < kXferWorkers; w++) {
-            hchk(hipHostMalloc((void **)&X.pin[w], cap * sizeof(float), hipHostMallocDefault), "hipHostMalloc transfer");
-            hchk(hipMalloc((void **)&X.dev[w], cap * sizeof(float)), "hipMalloc transfer");
-            hchk(hipEventCreateWithFlags(&X.ev[w], hipEventDisableTiming), "transfer event");
-          }
-        } catch (const HipError &) {
-          xfer_free(x);
-          throw;
-        }
-        X.cap = cap;
+        hipError_t e = xfer_alloc(X, std::max(need, kXferFloats));
+        if (e != hipSuccess && need < kXferFloats) e = xfer_alloc(X, need);
+        hchk(e, "transfer buffers");
       }
       std::vector<Piece> pieces;
       std::vector<Chunk> chunks;
@@ -1661,12 +1692,12 @@ static int xfer_reference(wrfdc_ctx *x, int n, const int *fields, void *const *h
         }
         return hipGetLastError();
       };
-      auto copy = [&](const Chunk &c, float *pin) {
+      auto copy = [&](const Chunk &c, float *chunk) {
         for (size_t q = c.p0; q < c.p1; q++) {
           const Piece &p = pieces[q];
           const size_t bytes = (size_t)p.g.ni * p.g.si * sizeof(float);
-          if (UP) memcpy(pin + p.g.ref, p.host, bytes);
-          else memcpy(p.host, pin + p.g.ref, bytes);
+          if (UP) memcpy(chunk + p.g.ref, p.host, bytes);
+          else memcpy(p.host, chunk + p.g.ref, bytes);
         }
       };
       auto work = [&](int w) {
@@ -1678,35 +1709,36 @@ static int xfer_reference(wrfdc_ctx *x, int n, const int *fields, void *const *h
           if (UP) {
             if (used) e = hipEventSynchronize(X.ev[w]);  // this worker's last chunk has left its buffers
             if (e != hipSuccess) break;
-            copy(c, X.pin[w]);
-            e = hipMemcpyAsync(X.dev[w], X.pin[w], bytes, hipMemcpyHostToDevice, x->s);
+            copy(c, X.host[w]);
+            e = hipMemcpyAsync(X.dev[w], X.host[w], bytes, hipMemcpyHostToDevice, x->s);
             if (e == hipSuccess) e = turn(c, X.dev[w]);
             if (e == hipSuccess) e = hipEventRecord(X.ev[w], x->s);
             used = true;
           } else {
             e = turn(c, X.dev[w]);
-            if (e == hipSuccess) e = hipMemcpyAsync(X.pin[w], X.dev[w], bytes, hipMemcpyDeviceToHost, x->s);
+            if (e == hipSuccess) e = hipMemcpyAsync(X.host[w], X.dev[w], bytes, hipMemcpyDeviceToHost, x->s);
             if (e == hipSuccess) e = hipEventRecord(X.ev[w], x->s);
             if (e == hipSuccess) e = hipEventSynchronize(X.ev[w]);
-            if (e == hipSuccess) copy(c, X.pin[w]);
+            if (e == hipSuccess) copy(c, X.host[w]);
           }
         }
         // the buffers are free when the call returns
         if (UP && e == hipSuccess && used) e = hipEventSynchronize(X.ev[w]);
         if (e != hipSuccess) failed.store((int)e);
       };
-      const int helpers = (int)std::min<size_t>(kXferWorkers, chunks.size()) - 1;
+      const int helpers = (int)std::min<size_t>((size_t)X.workers, chunks.size()) - 1;
       std::thread pool[kXferWorkers];
       for (int w = 1; w <= helpers; w++) {
         try {
           pool[w] = std::thread(work, w);
-        } catch (const std::system_error &) {
-          break;  // no more threads to be had: the ones that run do it all
+        } catch (const std::exception &) {
+          break;  // no more threads, or no memory for one: the ones that run do it all
         }
       }
       work(0);
       for (auto &t : pool)
         if (t.joinable()) t.join();
+      if (failed.load() != (int)hipSuccess) (void)wait();  // the next call finds the buffers idle
       hchk((hipError_t)failed.load(), UP ? "upload" : "download");
       return WRFDC_OK;
     } catch (const std::bad_alloc &) {
