@@ -34,15 +34,16 @@ void operator delete(void *p, size_t) noexcept { std::free(p); }
 // ---- the runtime ---------------------------------------------------------------
 namespace rt {
 struct Launch {
-  std::string name;
+  std::string name, mangled;
   hipStream_t s;
+  dim3 block;
 };
 std::recursive_mutex mu;
 struct Guard {
   Guard() { mu.lock(), t_inside++; }
   ~Guard() { t_inside--, mu.unlock(); }
 };
-std::map<const void *, std::string> kernels;
+std::map<const void *, std::string> kernels;  // mangled names
 std::vector<Launch> log_;
 std::map<void *, std::string> live;      // device and pinned memory, streams, events, graphs
 std::set<hipStream_t> capturing, busy;   // busy: work that nothing has waited for
@@ -114,7 +115,7 @@ void **__hipRegisterFatBinary(const void *) {
 }
 void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, void *, void *, int *) {
-  rt::kernels[f] = rt::base(name);
+  rt::kernels[f] = name;
 }
 void __hipRegisterVar(void **, void *, char *, const char *, int, size_t, int, int) {}
 static thread_local struct { dim3 g, b; size_t lds; hipStream_t s; } g_cfg;
@@ -129,13 +130,13 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
   *s = g_cfg.s;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **, size_t, hipStream_t s) {
   rt::Guard guard;
-  const std::string name = rt::kernels.at(f);
+  const std::string mangled = rt::kernels.at(f), name = rt::base(mangled.c_str());
   if (rt::fails(name)) return rt::fail(hipErrorLaunchFailure);
   if (!rt::stream_ok(s)) return rt::fail(hipErrorInvalidHandle);
   if (!g.x || !g.y || !g.z) return rt::fail(hipErrorInvalidConfiguration);
-  rt::log_.push_back({name, s});
+  rt::log_.push_back({name, mangled, s, b});
   if (!rt::capturing.count(s)) rt::busy.insert(s);
   return hipSuccess;
 }
@@ -336,6 +337,26 @@ void context_upload() {
   wrfdc_destroy(x);
 }
 
+// The phi tendency's index arithmetic takes blocks of four waves, whatever the
+// rows of the face blocks it shares its launch with (WRFDC_FACE_ROWS).
+void phi_tendency_blocks() {
+  for (int nx : {24, 300}) {
+    wrfdc_ctx *x = make_ctx(nx, 200, 40);
+    rt::log_.clear();
+    CHECK(wrfdc_step(x, 1, 0.0) == WRFDC_OK);
+    int phi = 0;
+    for (auto &l : rt::log_)
+      if (l.name == "k_tendencies" || l.mangled.find("k_tendencyILi4E") != std::string::npos) {
+        phi++;
+        CHECK(l.block.x == 64 && l.block.y == 4);
+      } else if (l.name == "k_tendency") {
+        CHECK(l.block.x == 64 && (int)l.block.y == kFaceRows);
+      }
+    CHECK(phi == 3);
+    wrfdc_destroy(x);
+  }
+}
+
 // The transfers of host arrays: whatever fails, the call returns an error or
 // does without, nothing is in flight when it returns, and the next call works.
 struct Arrays {
@@ -464,6 +485,7 @@ const struct {
   const char *name;
   void (*fn)();
 } kChecks[] = {{"context_upload", context_upload},
+               {"phi_tendency_blocks", phi_tendency_blocks},
                {"transfer_call_failures", transfer_call_failures},
                {"transfer_short_memory", transfer_short_memory},
                {"transfer_allocation_failures", transfer_allocation_failures},

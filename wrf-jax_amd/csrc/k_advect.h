@@ -572,7 +572,9 @@ __device__ __forceinline__ void tend_ph(CtxPtr x, unsigned b, unsigned nblk, con
 // The RK tendencies of the fused step: the five components, which read the
 // same winds and each write their own arrays, over five ranges of blocks
 // (first: first block of each range), or one of them (only >= 0) in a launch
-// of its own with its own registers.
+// of its own with its own registers.  phi's blocks are of four waves (GET_IKJ_B),
+// the others' of kFaceRows: together only where that is the same.
+constexpr bool kTendSameBlocks = kFaceRows == 4;
 struct TendRanges {
   R3 r[5];  // u, v, w, theta, phi
   unsigned first[6];
@@ -596,7 +598,7 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_tendencies(const DevCtx *xv,
   else tendency<4>(x, ys, T, rk);
 }
 template <int C>
-__global__ void __launch_bounds__(64 * kFaceRows) k_tendency(const DevCtx *xv, TendRanges T, int rk) {
+__global__ void __launch_bounds__(C == 4 ? 256 : 64 * kFaceRows) k_tendency(const DevCtx *xv, TendRanges T, int rk) {
   __shared__ float ys[kFaceRows][64];
   tendency<C>(ctx_ptr(xv), ys, T, rk);
 }

@@ -820,7 +820,7 @@ struct Run {
     T.r[3] = mass3();
     const unsigned nb[5] = {face_tiles(T.r[0], d.face_lg[0]).count(), face_tiles(T.r[1], d.face_lg[0]).count(),
                             face_tiles(T.r[2], d.face_lg[1]).count(), face_tiles(T.r[3], d.face_lg[0]).count(), g3(T.r[4]).x};
-    if (X->n3 <= kTendTogether) {
+    if (kTendSameBlocks && X->n3 <= kTendTogether) {
       T.first[0] = 0;
       for (int c = 0; c < 5; c++) T.first[c + 1] = T.first[c] + nb[c];
       k_tendencies<<<T.first[5], bf(), 0, s>>>(D(), T, rk);
@@ -828,7 +828,7 @@ struct Run {
       auto one = [&](int c, void (*kernel)(const DevCtx *, TendRanges, int)) {
         T.first[c] = 0;
         T.first[c + 1] = nb[c];
-        kernel<<<nb[c], bf(), 0, s>>>(D(), T, rk);
+        kernel<<<nb[c], c == 4 ? b3() : bf(), 0, s>>>(D(), T, rk);
       };
       one(0, k_tendency<0>);
       one(1, k_tendency<1>);
