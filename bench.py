@@ -10,7 +10,7 @@ species, lateral boundaries).
 Forms (``--forms``, all three by default; the headline ``value`` is plain):
 ``forms.batched`` runs the 32-member ensemble of uneven domains (100^2..300^2
 columns, 45..60 levels, dx 1..9 km) with one RK3 step of every member
-captured in one HIP graph over the autotuned streams; ``forms.learned`` runs
+captured in one HIP graph over 16 streams; ``forms.learned`` runs
 1000x1000x60 at dx 3 km with the bf16 MLP eddy viscosity (trained first on a
 coarse-grained 1 km run of this dycore) and the same domain with
 Smagorinsky.  Each reports Mpoint-steps/s and its ratio to plain.
@@ -115,12 +115,12 @@ def _log(msg: str) -> None:
 def batched_form(steps: int, plain_value: float) -> dict:
     """32 seeded members of uneven domains (100^2..300^2 columns, 45..60
     levels, dx 1..9 km, 6 moist species), one RK3 step of all of them
-    captured in one HIP graph over concurrent streams, the stream layout
-    and the face-block tile shape chosen by the autotuner; value = sum of N_mass x steps / s."""
+    captured in one HIP graph over 16 concurrent streams, each member on the
+    least loaded one, longest first; value = sum of N_mass x steps / s."""
     import torch
 
     from wrfdc.device import Domain
-    from wrfdc.ensemble import Ensemble, autotune, c2_members, eager_step_time, member_case, n_mass
+    from wrfdc.ensemble import Ensemble, assign_longest_first, c2_members, eager_step_time, member_case, member_times, n_mass
 
     t0 = time.perf_counter()
     specs = c2_members()
@@ -134,9 +134,8 @@ def batched_form(steps: int, plain_value: float) -> dict:
     nm = n_mass(doms)
     _log(f"batched: {len(doms)} members, {nm / 1e6:.1f} M mass points, built in {time.perf_counter() - t0:.1f} s")
     eager = eager_step_time(doms, reps=2)
-    nb, assign, table, tiles = autotune(doms, candidates=(1, 2, 4, 8, 16), reps=2,
-                                        log=lambda m: _log("batched autotune: " + m))
-    face_levels = min(tiles, key=lambda e: e[1])[0]
+    nb = 16  # of 1, 2, 4, 8 and 16 the fastest here
+    assign = assign_longest_first(member_times(doms, reps=2), nb)
     ens = Ensemble(doms, assign, nb)
     ens.step(1, 0.0)
     ens.synchronize()
@@ -154,8 +153,6 @@ def batched_form(steps: int, plain_value: float) -> dict:
     return {"value": value, "unit": "Mpoint-steps/s", "ms_per_step": 1e3 * sec / steps, "steps": steps, "n_mass": nm,
             "members": len(doms), "streams": nb, "eager_ms_per_step": 1e3 * eager, "graph_vs_eager": eager / (sec / steps),
             "vs_plain": value / plain_value, "nonfinite": bad,
-            "face_levels": face_levels, "autotune_ms": {str(b): 1e3 * t for b, t in table},
-            "autotune_face_levels_ms": {str(lg): 1e3 * t for lg, t in tiles},
             "workload": "32 seeded members, 100^2..300^2 x 45..60, dx 1..9 km, 6 moist species, PD on, FP32, "
                         "one captured RK3 step per replay"}
 

@@ -111,8 +111,7 @@ int wrfdc_stage(wrfdc_ctx *ctx, const char *name, int rk_step, int iteration);
  * calls read it (wrfdc_step sets it to dtbc0 + (n+1) dt itself). */
 int wrfdc_set_dtbc(wrfdc_ctx *ctx, double dtbc);
 int wrfdc_checksums(wrfdc_ctx *ctx, double out[WRFDC_NCHECKSUMS]);
-/* No counterpart in the reference (the batched ensemble's autotuner uses
- * it): a launch-shape setting of the context.  "face_levels": levels per
+/* No counterpart in the reference: a launch-shape setting of the context.  "face_levels": levels per
  * level group in the tile order of the face-sharing stencil kernels
  * (advection, species), 1..32, or 0 for the per-kernel defaults (4, and 8
  * for advect_w and the positive-definite species passes).  Results do not
@@ -152,7 +151,11 @@ int wrfdc_ensemble_step(wrfdc_ensemble *ens, int nsteps, double dtbc0);
 int wrfdc_ensemble_sync(wrfdc_ensemble *ens);
 void *wrfdc_ensemble_stream(wrfdc_ensemble *ens);
 long long wrfdc_ensemble_nodes(wrfdc_ensemble *ens);
-void wrfdc_ensemble_destroy(wrfdc_ensemble *ens);
+/* Waits for the replays and destroys the graph, its streams and events (NULL:
+ * nothing to do).  WRFDC_EHIP, named by wrfdc_last_error(NULL), if one of these
+ * calls failed; after a failed wait nothing is destroyed.  The handle is gone
+ * in either case. */
+int wrfdc_ensemble_destroy(wrfdc_ensemble *ens);
 
 /* ---- tangent-linear and adjoint scalar transport (north-star extension: the
  * adjoint of advect_scalar, src/wrf_jax/dyn_em/module_advect_em_fast.py:1437-1769,

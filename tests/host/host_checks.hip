@@ -185,7 +185,8 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   rt::Guard guard;
   if (rt::busy.count(s)) rt::error("stream destroyed with work in flight");
   if (rt::capturing.count(s)) rt::error("stream destroyed while it captures");
-  return rt::drop(s, "stream");
+  const hipError_t e_ = rt::drop(s, "stream");
+  return rt::fails("hipStreamDestroy") ? rt::fail() : e_;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
   rt::Guard guard;
@@ -228,7 +229,8 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { RT("hipEventCreate
 hipError_t hipEventDestroy(hipEvent_t e) {
   rt::Guard guard;
   rt::recorded.erase(e);
-  return rt::drop(e, "event");
+  const hipError_t e_ = rt::drop(e, "event");
+  return rt::fails("hipEventDestroy") ? rt::fail() : e_;
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   RT("hipEventRecord");
@@ -260,11 +262,13 @@ hipError_t hipGraphLaunch(hipGraphExec_t x, hipStream_t s) {
 hipError_t hipGraphExecDestroy(hipGraphExec_t x) {
   rt::Guard guard;
   if (!rt::busy.empty()) rt::error("graph exec destroyed with work in flight");
-  return rt::drop(x, "graph exec");
+  const hipError_t e_ = rt::drop(x, "graph exec");
+  return rt::fails("hipGraphExecDestroy") ? rt::fail() : e_;
 }
 hipError_t hipGraphDestroy(hipGraph_t g) {
   rt::Guard guard;
-  return rt::drop(g, "graph");
+  const hipError_t e_ = rt::drop(g, "graph");
+  return rt::fails("hipGraphDestroy") ? rt::fail() : e_;
 }
 }  // extern "C"
 
@@ -447,10 +451,37 @@ void ensemble_lifecycle() {
     CHECK(wrfdc_ensemble_step(e, 3, 5.0) == WRFDC_OK);
     CHECK(wrfdc_ensemble_sync(e) == WRFDC_OK);
     for (auto x : m) CHECK(x->s == nullptr && !x->capturing);
-    wrfdc_ensemble_destroy(e);
+    CHECK(wrfdc_ensemble_destroy(e) == WRFDC_OK);
     CHECK(rt::live.size() == base);
   }
   for (auto x : m) wrfdc_destroy(x);
+}
+
+// A destruction that fails is reported, and the rest is destroyed all the same;
+// replays that cannot be waited for leave everything as it is.
+void ensemble_destroy_failures() {
+  wrfdc_ctx *x = make_ctx(24, 20, 10);
+  const auto before = rt::live;
+  for (const char *call : {"hipStreamSynchronize", "hipGraphExecDestroy", "hipGraphDestroy", "hipEventDestroy", "hipStreamDestroy"}) {
+    wrfdc_ensemble *e = nullptr;
+    CHECK(wrfdc_ensemble_create(&x, 1, nullptr, 2, &e) == WRFDC_OK);
+    const size_t all = rt::live.size();
+    CHECK(wrfdc_ensemble_step(e, 1, 0.0) == WRFDC_OK && wrfdc_ensemble_sync(e) == WRFDC_OK);
+    rt::fail_name = call;
+    rt::fail_left = 0;
+    rt::fail_times = 1;
+    CHECK(wrfdc_ensemble_destroy(e) == WRFDC_EHIP);
+    rt::last = hipSuccess;
+    if (call == std::string("hipStreamSynchronize")) {
+      CHECK(rt::live.size() == all);
+      for (auto &l : rt::live)
+        if (!before.count(l.first)) std::free(l.first);
+      rt::live = before;
+    }
+    CHECK(rt::live.size() == before.size());
+  }
+  CHECK(wrfdc_ensemble_destroy(nullptr) == WRFDC_OK);
+  wrfdc_destroy(x);
 }
 
 // Every runtime call of the creation failing in turn: an error, the members
@@ -490,6 +521,7 @@ const struct {
                {"transfer_short_memory", transfer_short_memory},
                {"transfer_allocation_failures", transfer_allocation_failures},
                {"ensemble_lifecycle", ensemble_lifecycle},
+               {"ensemble_destroy_failures", ensemble_destroy_failures},
                {"ensemble_create_failures", ensemble_create_failures}};
 }  // namespace
 

@@ -6,7 +6,7 @@ uneven members, csrc/wrfdc.hip wrfdc_ensemble_*).
   each replay must see the current boundary time;
 * every member matches the FP32 oracle after the replays (relative L2 1e-5),
   also the smallest members of the 32-member batched workload;
-* the autotuner returns a valid layout and tile shape.
+* the autotuner returns a valid layout and tile shape (skipped: it is off).
 """
 
 import numpy as np
@@ -111,7 +111,7 @@ def test_workload_members_match_oracle(gpu):
 
 
 @pytest.mark.skip(reason="ended in a segmentation fault (once SIGABRT) inside wrfdc_ensemble_destroy, no GPU fault: seven graphs "
-                         "created and each destroyed right after its last replay; no cause shown")
+                         "created and each destroyed right after its last replay; no cause shown, and autotune raises an error until there is one")
 def test_autotune_returns_a_layout(gpu):
     from wrfdc.ensemble import Ensemble, autotune
 

@@ -13,7 +13,8 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.environ.get("HIPCC", os.path.join(ROCM, "bin", "hipcc"))
-CHECKS = ["context_upload", "phi_tendency_blocks", "transfer_call_failures", "transfer_short_memory", "transfer_allocation_failures", "ensemble_lifecycle", "ensemble_create_failures"]
+CHECKS = ["context_upload", "phi_tendency_blocks", "transfer_call_failures", "transfer_short_memory", "transfer_allocation_failures", "ensemble_lifecycle", "ensemble_create_failures",
+          "ensemble_destroy_failures"]
 
 pytestmark = pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not found")
 

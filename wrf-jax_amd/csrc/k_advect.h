@@ -44,7 +44,7 @@ __device__ __forceinline__ float lane_next(float v, int lane) {
 // LG is a launch setting of the domain (DevCtx::face_lg, wrfdc_set_tile):
 // by default 4 for most kernels and 8 for the PD species passes and
 // advect_w, which measured fastest at 400x400x60 (each kernel timed with LG
-// 2, 4, 8 and 16); the ensemble's autotuner tries others per layout.
+// 2, 4, 8 and 16).
 #ifndef WRFDC_FACE_LG
 #define WRFDC_FACE_LG 4
 #endif

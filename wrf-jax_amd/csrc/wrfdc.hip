@@ -2084,18 +2084,29 @@ struct wrfdc_ensemble {
   size_t nodes = 0;
 };
 
-static void ensemble_free(wrfdc_ensemble *e) {
-  if (!e) return;
-  if (e->root) (void)hipStreamSynchronize(e->root);
-  if (e->exec) (void)hipGraphExecDestroy(e->exec);
-  if (e->graph) (void)hipGraphDestroy(e->graph);
+// Destroys what the ensemble holds, the graph first, once its replays have been
+// waited for; where that wait fails, its graph, streams and events are left to
+// the process (they may be in use).  The first error and its call.
+static HipError ensemble_free(wrfdc_ensemble *e) {
+  HipError first{hipSuccess, ""};
+  auto note = [&](hipError_t rc, const char *what) {
+    if (rc != hipSuccess && first.e == hipSuccess) first = HipError{rc, what};
+  };
+  if (e->root) note(hipStreamSynchronize(e->root), "replays");
+  if (first.e != hipSuccess) {
+    delete e;
+    return first;
+  }
+  if (e->exec) note(hipGraphExecDestroy(e->exec), "graph exec");
+  if (e->graph) note(hipGraphDestroy(e->graph), "graph");
   for (hipEvent_t v : e->join)
-    if (v) (void)hipEventDestroy(v);
-  if (e->fork) (void)hipEventDestroy(e->fork);
+    if (v) note(hipEventDestroy(v), "event");
+  if (e->fork) note(hipEventDestroy(e->fork), "event");
   for (hipStream_t st : e->streams)
-    if (st) (void)hipStreamDestroy(st);
-  if (e->root) (void)hipStreamDestroy(e->root);
+    if (st) note(hipStreamDestroy(st), "stream");
+  if (e->root) note(hipStreamDestroy(e->root), "stream");
   delete e;
+  return first;
 }
 
 int wrfdc_ensemble_create(wrfdc_ctx *const *members, int n, const int *branch_of, int nbranches, wrfdc_ensemble **out) {
@@ -2163,7 +2174,7 @@ int wrfdc_ensemble_create(wrfdc_ctx *const *members, int n, const int *branch_of
       members[q]->s = saved[q];
       members[q]->capturing = false;
     }
-    ensemble_free(e);
+    (void)ensemble_free(e);
     return set_err(nullptr, WRFDC_EHIP, std::string("ensemble: ") + err.what + ": " + hipGetErrorString(err.e));
   }
   // replays run on the root stream; the members' own streams wait for it
@@ -2205,7 +2216,12 @@ int wrfdc_ensemble_sync(wrfdc_ensemble *e) {
 
 void *wrfdc_ensemble_stream(wrfdc_ensemble *e) { return e ? (void *)e->root : nullptr; }
 long long wrfdc_ensemble_nodes(wrfdc_ensemble *e) { return e ? (long long)e->nodes : -1; }
-void wrfdc_ensemble_destroy(wrfdc_ensemble *e) { ensemble_free(e); }
+int wrfdc_ensemble_destroy(wrfdc_ensemble *e) {
+  if (!e) return WRFDC_OK;
+  const HipError err = ensemble_free(e);
+  if (err.e == hipSuccess) return WRFDC_OK;
+  return set_err(nullptr, WRFDC_EHIP, std::string("ensemble teardown: ") + err.what + ": " + hipGetErrorString(err.e));
+}
 
 // ---------------------------------------------------------------------------
 // tangent-linear / adjoint scalar transport

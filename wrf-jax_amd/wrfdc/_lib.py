@@ -45,7 +45,7 @@ SIGNATURES = {
     "wrfdc_ensemble_sync": (ctypes.c_int, [ctypes.c_void_p]),
     "wrfdc_ensemble_stream": (ctypes.c_void_p, [ctypes.c_void_p]),
     "wrfdc_ensemble_nodes": (ctypes.c_longlong, [ctypes.c_void_p]),
-    "wrfdc_ensemble_destroy": (None, [ctypes.c_void_p]),
+    "wrfdc_ensemble_destroy": (ctypes.c_int, [ctypes.c_void_p]),
     "wrfdc_record_stages": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int]),
     "wrfdc_recorded_stages": (ctypes.c_int, [ctypes.c_void_p]),
     "wrfdc_transport_stage": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,

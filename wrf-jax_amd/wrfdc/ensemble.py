@@ -5,14 +5,11 @@ species) and the HIP graph in which one RK3 step of every member was
 captured (``wrfdc_ensemble_create``): members on the same stream run one
 after another, the streams concurrently, and each replay
 (``wrfdc_ensemble_step``) launches the whole ensemble's step at once.
-``autotune`` picks how many streams to use, which member goes on which and
-the tile shape of the face-block stencil kernels: it times each member's
-step on its own, assigns members longest first to the least loaded stream
-for each candidate stream count, times the captured ensemble step of each
-layout and keeps the fastest; then, on that layout, it times each candidate
-level-group size of the face-block tiles (``Domain.set_tile("face_levels",
-n)``, 0 = the per-kernel defaults) and leaves the members set to the
-fastest.  Neither choice changes any result bit.
+The layout is the caller's: ``assign_longest_first(member_times(domains), n)``
+puts the members, longest first, on the least loaded of n streams, and
+``Domain.set_tile("face_levels", n)`` sets the tile shape of the face-block
+kernels before the capture.  Neither changes any result bit.  ``autotune``,
+which searched over both with one captured graph after another, is off.
 
 ``c2_members`` draws the seeded members of the batched workload: 32
 domains of 100^2..300^2 columns and 45..60 levels, dx 1..9 km, dt = 6 s per
@@ -90,8 +87,8 @@ class Ensemble:
 
     def close(self) -> None:
         if getattr(self, "h", None):
-            self.lib.wrfdc_ensemble_destroy(self.h)
-            self.h = None
+            h, self.h = self.h, None
+            _lib.raise_for(self.lib.wrfdc_ensemble_destroy(h), self.lib, None, "wrfdc_ensemble_destroy")
 
     def __del__(self):
         try:
@@ -153,41 +150,14 @@ def graph_step_time(ens: Ensemble, reps: int = 5) -> float:
 
 
 def autotune(domains, candidates=(1, 2, 4, 8), reps: int = 3, log=None, face_levels=(0, 2, 8, 16)):
-    """(best stream count, member -> stream, table of (streams, s/step),
-    table of (face_levels, s/step)); the members are left set to the best
-    face_levels, so an Ensemble captured afterwards uses it."""
-    times = member_times(domains, reps)
-    table = []
-    best = None
-    for nb in candidates:
-        nb = min(nb, len(domains))
-        if any(t[0] == nb for t in table):
-            continue
-        assign = assign_longest_first(times, nb)
-        ens = Ensemble(domains, assign, nb)
-        t = graph_step_time(ens, reps)
-        ens.close()
-        table.append((nb, t))
-        if log:
-            log(f"{nb} stream(s): {1e3 * t:.2f} ms per ensemble step")
-        if best is None or t < best[1]:
-            best = (nb, t, assign)
-    nb, assign = best[0], best[2]
-    tiles = []
-    for lg in face_levels:
-        for d in domains:
-            d.set_tile("face_levels", lg)
-        ens = Ensemble(domains, assign, nb)
-        t = graph_step_time(ens, reps)
-        ens.close()
-        tiles.append((lg, t))
-        if log:
-            log(f"{nb} stream(s), face_levels {lg}: {1e3 * t:.2f} ms per ensemble step")
-    if tiles:
-        lg = min(tiles, key=lambda e: e[1])[0]
-        for d in domains:
-            d.set_tile("face_levels", lg)
-    return nb, assign, table, tiles
+    """Off: raises RuntimeError.  It captured, replayed and destroyed one graph
+    per candidate layout, and two such searches ended the process inside the
+    destruction of a graph (a host fault, after its replays had been waited
+    for).  The library's part of that path runs clean on the CPU under address
+    and undefined-behaviour sanitizers, and no cause is known, so the search
+    stays off; one ensemble kept for a run is not concerned."""
+    raise RuntimeError("wrfdc.ensemble.autotune is off (a search over captured graphs has ended the process in a graph's destruction, "
+                       "cause unknown): give Ensemble a layout, for instance assign_longest_first(member_times(domains), 16)")
 
 
 __all__ = ["Ensemble", "MemberSpec", "assign_longest_first", "autotune", "c2_members", "eager_step_time", "graph_step_time",
