@@ -472,7 +472,7 @@ __global__ void __launch_bounds__(64 * kFaceRows) k_advect_v(const DevCtx *xv, c
 // advect_w (module_advect_em.py:1357-1640); r covers i [1, ide-1], k [2, kde], j [1, jde-1]
 // (face-sharing blocks: x faces i in [2, ide-1], y faces j in [2, jde-1]).
 // TEND: the w tendency of the RK step over k [1, kde]: advection, buoyancy
-// and pressure (pg_buoy_w, reading cqw before k_cqw_inv replaces it) and, below
+// and pressure (pg_buoy_w, reading cqw before 1 / (1 + cqw) replaces it) and, below
 // the top, Coriolis/curvature at k [2, kde]; then rk_addtend_dry.  Buoyancy
 // and Coriolis terms at a level clamped into the range they apply to.
 template <bool TEND>
@@ -542,7 +542,7 @@ __device__ __forceinline__ void advect_w(CtxPtr x, float (*ys)[64], unsigned b, 
   elem(tend, o) = t;
   // pg_buoy_w's cqw := 1 / (1 + cqw) at this point (read only by this
   // thread here; level kde-1, which the top level's thread also reads, is
-  // replaced after this kernel)
+  // replaced by small_step_prep, k_ssp_3d's cqw_top)
   if (TEND && k >= 2 && k <= kde - 2) elem(FL(cqw), o) = cq1;
 }
 template <bool TEND>

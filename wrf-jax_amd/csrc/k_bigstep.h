@@ -411,15 +411,6 @@ __device__ __forceinline__ float buoy_w_term(CtxPtr x, int i, int k, int j, floa
   const float mid = gm * (cq1 * A1(FL(rdn), kc) * (pk - pkm) - (A1(c1f, k) * A2(mu, i, j)) - cq2 * (A1(c1f, k) * A2(mub, i, j) + A1(c2f, k)));
   return k == kde ? top : mid;
 }
-// cqw := 1 / (1 + cqw) (the second half of pg_buoy_w): levels [2, kde-1] in
-// the stage API; in the fused step only level kde-1 (the w kernel's top
-// level reads it, so the fused w kernel replaces levels [2, kde-2] itself)
-__global__ void k_cqw_inv(const DevCtx *xv, R3 r) {
-  const CtxPtr x = ctx_ptr(xv);
-  GET_IKJ_P(r);
-  float *cqw = FL(cqw);
-  A3(cqw, i, k, j) = 1.f / (1.f + A3(cqw, i, k, j));
-}
 // pg_buoy_w (module_big_step_utilities_em.py:1674-1800): column kernel
 __global__ void k_pg_buoy_w(const DevCtx *xv, R2 r) {
   const CtxPtr x = ctx_ptr(xv);

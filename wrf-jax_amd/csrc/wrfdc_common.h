@@ -61,7 +61,8 @@ enum {
 enum { S_T1, S_T2, S_FQX, S_FQY, S_FQZ, S_FQXL, S_FQYL, S_FQZL, S_SCALE, S_HAT2, S_VXGM, NSCRATCH };
 
 // View of one domain (dimensions, scalars, pointers), 1.7 KB in device memory.
-// Every kernel gets its address and reads it with scalar loads (CtxPtr).
+// The step's kernels get its address and read it with scalar loads (CtxPtr);
+// k_checksum_partial, which also runs without a context, gets it by value.
 struct DevCtx {
   int ide, jde, kde, ip;
   int nmoist, nscalar, spec_zone, relax_zone, spec_bdy_width, top_lid;
