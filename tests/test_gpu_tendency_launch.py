@@ -1,6 +1,6 @@
-"""The five RK tendencies in one launch and in five: one step against the oracle on both sides of the line (2^20
-elements of a 3-D field: jde * kde * pitch), with boundary tendencies that the ring takes.  Tolerance of the one-step
-parity tests: relative L2 1e-5 per field."""
+"""The five RK tendencies in one launch and in five: one step against the oracle on both sides of the line (5 * 2^17
+elements of a 3-D field, jde * kde * pitch: 80 and 81 rows of 64 levels at a pitch of 128) and of 2^20, with boundary
+tendencies that the ring takes.  Tolerance of the one-step parity tests: relative L2 1e-5 per field."""
 
 import numpy as np
 import pytest
@@ -10,7 +10,7 @@ from parity import REL_L2_STEP, STEP_DIAGNOSTICS, compare
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,ny,nz", [(12, 12, 6), (127, 127, 63), (127, 128, 63)])
+@pytest.mark.parametrize("nx,ny,nz", [(12, 12, 6), (127, 79, 63), (127, 80, 63), (127, 127, 63), (127, 128, 63)])
 def test_step_matches_oracle(gpu, nx, ny, nz):
     from oracle import Oracle
     from wrfdc.cases import make_case

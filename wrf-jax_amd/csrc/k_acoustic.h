@@ -808,8 +808,9 @@ __global__ void __launch_bounds__(64 * NW, NW > 8 ? 4 : 6) k_acoustic_col(const 
 // A domain of at most kColWideBlocks blocks leaves CUs idle, so its substep
 // takes as long as one block does: 16 waves, each with half the levels
 // (a substep's column kernel at 100x100x45, 202 blocks: 44 us with 8 waves, 30
-// with 16; at 24x20x10 14 and 11).  From there on 8 waves: three such blocks
-// share a CU, one of 16.
+// with 16; at 24x20x10 14 and 11; a step of 63x255x45, 256 blocks: 1140 and
+// 1050 us).  From there on 8 waves: three such blocks share a CU, one of 16
+// (63x299x45, 300 blocks: 1349 us with 8 waves, 1375 with 16).
 constexpr unsigned kColWideBlocks = 256;
 inline unsigned acoustic_col_blocks(const DevCtx &d) { return (unsigned)((d.ide + 63) / 64) * (unsigned)d.jde; }
 // one instantiation per levels-per-wave range: fn(std::integral_constant<NW>, <NPW>)

@@ -309,13 +309,16 @@ inline unsigned cdiv(int a, int b) { return (unsigned)((a + b - 1) / b); }
 // Elements of a 3-D field up to which the five RK tendencies share a launch.
 // Together they take the registers of the largest (102: 4 waves per SIMD
 // where theta and phi run with 7 and 8), which a domain that fills the chip
-// pays for: a step of 24x20x10 457 us apart and 404 together, 100x100x45
-// (0.5 M elements) 1052 and 1031, 257x131x37 (1.4 M) 1868 and 1889,
-// 400x400x60 14.52 and 14.96 ms.
-constexpr size_t kTendTogether = (size_t)1 << 20;
+// pays for.  A step, apart and together: 24x20x10 457 and 404 us, 111x100x49
+// (0.54 * 2^20 elements) 1057 and 1033, 127x110x49 (0.68) 1232 and 1232,
+// 143x120x49 (0.83) 1606 and 1614, 143x141x49 (0.98) 1796 and 1818, 159x160x49
+// (1.23) 2015 and 2045, 400x400x60 14.52 and 14.96 ms.
+constexpr size_t kTendTogether = (size_t)5 << 17;
 // Elements up to which rk_step_prep's 3-D kernel forms the column masses
 // itself: the launch saved (4 us) against 24 us for the 25 M elements of
-// 400x400x60.
+// 400x400x60.  A step with and without is within 0.2 % from 1.8 * 2^20
+// (191x200x49, 2943 and 2941 us) to 3.8 * 2^20 elements (255x320x48, 5808 and
+// 5805), 6394 and 6375 us beyond the line (255x400x49, 4.9 * 2^20).
 constexpr size_t kPrepMuv = (size_t)4 << 20;
 
 struct Run {
