@@ -1,8 +1,8 @@
 """Checksums at the sizes where the column walk can go wrong, against NumPy in FP64.
 
-One short tile, a tile that ends on column 64 and one that goes past it, level runs of exactly 16 and with one left
-over.  The sums are FP64 of the same FP32 values: the order of at most 1e6 terms and a few roundings per term give
-1e-12 relative.  A non-finite pressure must show in the energy and nowhere else, a non-finite wind in the count.
+One short tile, a tile that ends on column 64 and one that goes past it, runs of one level; then enough columns for
+runs of 2 for the state and 3 for the species, of 5 and 9, and of 16 with one level left over.  The sums are FP64 of
+the same FP32 values: the order of at most 1e6 terms and a few roundings per term give 1e-12 relative.  A non-finite pressure must show in the energy and nowhere else, a non-finite wind in the count.
 """
 
 import numpy as np
@@ -29,7 +29,7 @@ def _numpy(case):
     return [mt.sum(), at("t_2").sum(), A["moist"][:, :ny, :nz, :nx].sum(), 0.0, dm.sum(), energy]
 
 
-@pytest.mark.parametrize("nx,ny,nz", [(12, 12, 6), (64, 13, 16), (65, 12, 17)])
+@pytest.mark.parametrize("nx,ny,nz", [(12, 12, 6), (64, 13, 16), (65, 12, 17), (65, 130, 17), (129, 330, 18), (12, 640, 97)])
 def test_sums_match_numpy(gpu, nx, ny, nz):
     from wrfdc.cases import make_case
     from wrfdc.device import Domain

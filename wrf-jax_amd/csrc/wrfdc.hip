@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(64) k_copy_ring(const DevCtx *xv, CopyList L) 
 //     winds averaged to the mass point, T = theta * ((pb+p)/p0)^(R/cp),
 //     cv = R/(cp/cv - 1) and the geopotential averaged from the two w levels.
 // Pass 1 writes one partial per block (vector stores, no atomics).  A wave
-// owns 64 columns of one row and marches a run of CK_LEVELS levels, so w, ph
+// owns 64 columns of one row and marches a run of up to CK_LEVELS levels, so w, ph
 // and phb of the level above are read once and carried, and no index is
 // divided per point.  At 400x400x60 with 6 moist species (538 MB) a call takes
 // 375 us with one point per thread of a strided 64-bit loop and the library's
@@ -113,6 +113,11 @@ __device__ __forceinline__ double ck_pow(double r, double c) {
   }
   return v;
 }
+// Levels of a wave's run for n (wave, level) pairs: as few as give every wave of
+// the launch a run, up to CK_LEVELS.  On a small domain the launch takes as long
+// as one run does (a call on 64x64x40: 39 us with runs of 16, 32 with runs of
+// 1; 24x20x10 with 6 species 35 and 30).
+__device__ __forceinline__ int ck_run(int n, int waves) { return imin_(imax_((n + waves - 1) / waves, 1), CK_LEVELS); }
 // sums of the block's values to out[0 .. CK_N-1]: within a wave, then over the waves
 __device__ __forceinline__ void ck_block_sum(const double s[CK_N], double *out) {
   __shared__ double red[CK_BLOCK / 64][CK_N];
@@ -135,7 +140,8 @@ __global__ void __launch_bounds__(CK_BLOCK) k_checksum_partial(const DevCtx xv, 
   const DevCtx *__restrict__ x = &xv;
   constexpr int NW = CK_BLOCK / 64;
   const int ni = x->ide - 1, nk = x->kde - 1, nj = x->jde - 1;
-  const int nt = (ni + 63) / 64, ns = (nk + CK_LEVELS - 1) / CK_LEVELS, nu = nj * nt * ns;
+  const int nt = (ni + 63) / 64, waves = (int)gridDim.x * NW;
+  const int lev = ck_run(nj * nt * nk, waves), ns = (nk + lev - 1) / lev, nu = nj * nt * ns;
   const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const double cv = (double)x->r_d / ((double)x->cpovcv - 1.0);
   const double rcp = 1.0 - 1.0 / (double)x->cpovcv;  // R/cp
@@ -144,8 +150,9 @@ __global__ void __launch_bounds__(CK_BLOCK) k_checksum_partial(const DevCtx xv, 
   const unsigned sj = (unsigned)(x->kde * x->ip), sk = (unsigned)x->ip;
   double s[CK_N] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   int nf = 0;
-  for (int u = (int)blockIdx.x * NW + wave; u < nu; u += (int)gridDim.x * NW) {
-    const int k0 = 1 + (u % ns) * CK_LEVELS, k1 = imin_(k0 + CK_LEVELS - 1, nk);
+  int u = (int)blockIdx.x * NW + wave;
+  for (; u < nu; u += waves) {
+    const int k0 = 1 + (u % ns) * lev, k1 = imin_(k0 + lev - 1, nk);
     const int i = 1 + (u / ns % nt) * 64 + lane, j = 1 + u / ns / nt;
     if (i > ni) continue;
     const float mu2 = A2(FL(mu_2), i, j);
@@ -176,12 +183,14 @@ __global__ void __launch_bounds__(CK_BLOCK) k_checksum_partial(const DevCtx xv, 
     }
   }
   // the species, a run of levels of one species at a time (their loads wait
-  // for nothing, so a whole run of them is in flight)
-  for (int u = (int)blockIdx.x * NW + wave; u < nu * x->nmoist; u += (int)gridDim.x * NW) {
-    const int v = u % nu, k0 = 1 + (v % ns) * CK_LEVELS, k1 = imin_(k0 + CK_LEVELS - 1, nk);
-    const int i = 1 + (v / ns % nt) * 64 + lane, j = 1 + v / ns / nt;
+  // for nothing, so a whole run of them is in flight), by the waves that come
+  // after the state's
+  const int slev = ck_run(nj * nt * nk * x->nmoist, waves), sns = (nk + slev - 1) / slev, snu = nj * nt * sns;
+  for (u -= nu; u < snu * x->nmoist; u += waves) {
+    const int v = u % snu, k0 = 1 + (v % sns) * slev, k1 = imin_(k0 + slev - 1, nk);
+    const int i = 1 + (v / sns % nt) * 64 + lane, j = 1 + v / sns / nt;
     if (i > ni) continue;
-    const float *q = SP(moist, u / nu);
+    const float *q = SP(moist, u / snu);
     float r[CK_LEVELS];
 #pragma unroll
     for (int n = 0; n < CK_LEVELS; n++) r[n] = A3(q, i, imin_(k0 + n, k1), j);
@@ -236,6 +245,12 @@ static const char kKinds[] = {
 };
 
 static const int kCkBlocks = 512;
+// blocks of k_checksum_partial: up to kCkBlocks, as many as have a level of 64
+// columns of the state or of a species for each wave
+static int ck_blocks(const DevCtx &h) {
+  const long long n = (long long)(h.jde - 1) * ((h.ide + 62) / 64) * (h.kde - 1) * (1 + h.nmoist);
+  return (int)std::min<long long>((n + CK_BLOCK / 64 - 1) / (CK_BLOCK / 64), kCkBlocks);
+}
 
 // Partial sums of wrfdc_checksums_noalloc: one fixed array per GPU (each
 // device that loads the library holds its own copy until the process ends).
@@ -2038,8 +2053,9 @@ int wrfdc_checksums(wrfdc_ctx *x, double out[WRFDC_NCHECKSUMS]) {
   static_assert(CK_N == WRFDC_NCHECKSUMS, "checksum count");
   if (!out) return set_err(x, WRFDC_EINVAL, "out is null");
   int rc = guarded(x, [&]() {
-    k_checksum_partial<<<kCkBlocks, CK_BLOCK, 0, x->s>>>(x->h, x->ck);
-    k_checksum_final<<<1, CK_BLOCK, 0, x->s>>>(x->ck, kCkBlocks, x->ck + kCkBlocks * CK_N);
+    const int nb = ck_blocks(x->h);
+    k_checksum_partial<<<nb, CK_BLOCK, 0, x->s>>>(x->h, x->ck);
+    k_checksum_final<<<1, CK_BLOCK, 0, x->s>>>(x->ck, nb, x->ck + kCkBlocks * CK_N);
     hchk(hipMemcpyAsync(out, x->ck + kCkBlocks * CK_N, sizeof(double) * CK_N, hipMemcpyDeviceToHost, x->s), "copy checksums");
     hchk(hipStreamSynchronize(x->s), "synchronize checksums");
     return WRFDC_OK;
@@ -2065,8 +2081,9 @@ int wrfdc_checksums_noalloc(const wrfdc_config *cfg, void *const *fields, double
   rc = noalloc_scratch(&part);
   if (rc != WRFDC_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
-  k_checksum_partial<<<kCkBlocks, CK_BLOCK, 0, s>>>(h, part);
-  k_checksum_final<<<1, CK_BLOCK, 0, s>>>(part, kCkBlocks, out_dev);
+  const int nb = ck_blocks(h);
+  k_checksum_partial<<<nb, CK_BLOCK, 0, s>>>(h, part);
+  k_checksum_final<<<1, CK_BLOCK, 0, s>>>(part, nb, out_dev);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_err(nullptr, WRFDC_EHIP, std::string("checksum kernels: ") + hipGetErrorString(e));
   return WRFDC_OK;
