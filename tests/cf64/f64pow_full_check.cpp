@@ -1,5 +1,6 @@
 // Host build of csrc/k_f64math.h: f64_pow_full against 113-bit arithmetic.
-// Prints the largest error in ulp of the result over samples of each range.
+// Prints the largest error in ulp of the result over samples of each range, then
+// the quotients of f64_div_by that differ from the IEEE division's.
 #include <quadmath.h>
 
 #include <cmath>
@@ -34,5 +35,27 @@ int main() {
     printf("%g..%g ^%.6f max_ulp=%.4f\n", r.lo, r.hi, r.c, worst);
   }
   for (double t : {1.0, 0.5, 2.0}) printf("%g ^0 max_ulp=%.4f\n", t, ulp_error(f64_pow_full(t, 0.0), 1.0Q));
+  long differ = 0, n = 0;
+  auto check = [&](double a, double c) {
+    const double q = f64_div_by(a, c, 1.0 / c), r = a / c;
+    differ += !(q == r || (q != q && r != r));
+    n++;
+  };
+  auto uniform = [&]() {
+    x ^= x << 13;
+    x ^= x >> 7;
+    x ^= x << 17;
+    return (double)(x >> 11) * 0x1p-53;
+  };
+  const double inf = __builtin_inf(), nan = __builtin_nan("");
+  for (int q = 0; q < 3000000; q++) {
+    const double c = q % 3 == 0 ? 1e5 : q % 3 == 1 ? (double)(float)(0.5 + uniform()) * (double)(float)(0.5 + uniform()) : 0.5 + uniform();
+    // a quotient near the middle between two doubles as often as not
+    check(ldexp(1.0 + uniform(), (int)(uniform() * 200.0) - 100), c);
+    check((1.0 + uniform()) * c * (1.0 + 0x1p-53 * (uniform() - 0.5)), c);
+  }
+  for (double a : {inf, -inf, nan, 0.0, -0.0, 1.5, -1e-30})
+    for (double c : {1e5, -2.0, inf, -inf, 0.0, -0.0, nan}) check(a, c);
+  printf("div checked=%ld differ=%ld\n", n, differ);
   return 0;
 }

@@ -34,6 +34,11 @@
 //    ulp of t^c: the final rounding, 0.001 for the logarithm's plain terms (2^-64
 //    of its value, for |c log t| < 2), 0.001 for the first term left out
 //    (0.347^15 / 15!) and 0.005 for the plain terms from r^4 / 24 on.
+//  f64_div_by(x, c, rc), rc = RN(1 / c): x / c rounded once, as the IEEE
+//    division rounds it (Markstein: the quotient x rc is within an ulp, its
+//    remainder by FMA is exact and the corrected quotient rounds correctly, for
+//    results in the normal range); zeros, infinities and NaN give what x / c gives
+//    (the remainder is NaN there, and the quotient stands).
 //
 // Only FMA-explicit arithmetic (__builtin_fma) and IEEE operations, so the
 // host and the device evaluate it to the same bits; tests/test_f64math.py
@@ -158,4 +163,9 @@ F64M_FN double f64_pow_full(double t, double c) {
   const double a = 1.0 + r, b = a + 0.5 * r2, g = b + u;
   const double rest = ((u - (g - b)) + ((0.5 * r2 - (b - a)) + (r - (a - 1.0)))) + (r2 * r2 * v + ((0.5 * r2l + ul) + rl * g));
   return __builtin_ldexp(g + rest, (int)n);
+}
+
+F64M_FN double f64_div_by(double x, double c, double rc) {
+  const double q = x * rc, v = __builtin_fma(__builtin_fma(-q, c, x), rc, q);
+  return v == v ? v : q;
 }

@@ -94,9 +94,9 @@ __global__ void __launch_bounds__(64) k_copy_ring(const DevCtx *xv, CopyList L) 
 // and phb of the level above are read once and carried, and no index is
 // divided per point.  At 400x400x60 with 6 moist species (538 MB) a call takes
 // 375 us with one point per thread of a strided 64-bit loop and the library's
-// pow, 165 us this way (22 us of it the power's terms in two parts and the
-// FP64 divisions by p0 and the map factors, which a reciprocal would round
-// once more).
+// pow, 160 us this way (17 us of it the power's terms in two parts and the
+// correctly rounded quotients by p0 and the map factors; with IEEE divisions
+// 165).
 #define CK_BLOCK 512
 #define CK_LEVELS 16
 #define CK_N 6
@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(CK_BLOCK) k_checksum_partial(const DevCtx xv, 
   const double cv = (double)x->r_d / ((double)x->cpovcv - 1.0);
   const double rcp = 1.0 - 1.0 / (double)x->cpovcv;  // R/cp
   const double area_g = (double)x->dx * (double)x->dy / (double)x->g;
-  const double t0 = (double)x->t0, p0 = (double)x->p0;
+  const double t0 = (double)x->t0, p0 = (double)x->p0, rp0 = 1.0 / p0;
   const unsigned sj = (unsigned)(x->kde * x->ip), sk = (unsigned)x->ip;
   double s[CK_N] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   int nf = 0;
@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(CK_BLOCK) k_checksum_partial(const DevCtx xv, 
       s[0] += mt;
       nf += isfinite(mu2) ? 0 : 1;
     }
-    const double msf2 = (double)A2(FL(msftx), i, j) * (double)A2(FL(msfty), i, j);
+    const double msf2 = (double)A2(FL(msftx), i, j) * (double)A2(FL(msfty), i, j), rmsf2 = 1.0 / msf2;
     unsigned o = XI3(i, k0, j);
     float w0 = elem(FL(w_2), o), ph0 = elem(FL(ph_2), o), phb0 = elem(FL(phb), o);
 #pragma unroll 2
@@ -171,9 +171,9 @@ __global__ void __launch_bounds__(CK_BLOCK) k_checksum_partial(const DevCtx xv, 
       const float pv = elem(FL(p), o), pbv = elem(FL(pb), o);
       nf += (isfinite(tv) ? 0 : 1) + (isfinite(uv) ? 0 : 1) + (isfinite(vv) ? 0 : 1) + (isfinite(w0) ? 0 : 1) + (isfinite(ph0) ? 0 : 1);
       s[1] += (double)tv;
-      const double dm = ((double)A1(FL(c1h), k) * mt + (double)A1(FL(c2h), k)) * -(double)A1(FL(dnw), k) * area_g / msf2;
+      const double dm = f64_div_by(((double)A1(FL(c1h), k) * mt + (double)A1(FL(c2h), k)) * -(double)A1(FL(dnw), k) * area_g, msf2, rmsf2);
       const double ub = 0.5 * ((double)uv + (double)ue), vb = 0.5 * ((double)vv + (double)vn), wb = 0.5 * ((double)w0 + (double)w1);
-      const double temp = (t0 + (double)tv) * ck_pow(((double)pbv + (double)pv) / p0, rcp);
+      const double temp = (t0 + (double)tv) * ck_pow(f64_div_by((double)pbv + (double)pv, p0, rp0), rcp);
       const double phi = 0.5 * ((double)ph0 + (double)phb0 + (double)ph1 + (double)phb1);
       s[4] += dm;
       s[5] += dm * (0.5 * (ub * ub + vb * vb + wb * wb) + cv * temp + phi);
